@@ -3,11 +3,11 @@
 Sweeps, on a frame of uneven scans into many maps (captured-graph launches,
 as the batched form runs them; by default each frame into emptied maps, the
 benchmark's workload):
-  ray_block           workgroup size of the two work-stealing ray walks
-  ray_blocks_per_cu   workgroups per CU of the cell-update walk
-  leaf_blocks_per_cu  workgroups per CU of the leaf-allocation walk
-  ray_chunk           most rays a wavefront takes per cursor atomic
-                      (rays per lane = ray_chunk / 64)
+  ray_block           workgroup size of the walks over the rays
+  ray_blocks_per_cu   most workgroups per CU of the cell-update walk
+  leaf_blocks_per_cu  most workgroups per CU of the leaf-allocation walk
+  ray_chunk           rays a wavefront of the create-and-mark walk takes, in
+                      batches of 64 one after the other
   ep_table_factor     endpoint-table slots per point (inverse load factor)
   root_slack          root-directory slots per root (inverse load factor)
   ray_window          cells a ray may run ahead of its wavefront's slowest
@@ -15,7 +15,7 @@ benchmark's workload):
   leaf_window         the same in leaves for the leaf pass
   fresh_pass          maps empty at a scan's start: one create-and-mark walk
                       (1) or the leaf and update walks (0)
-  fresh_blocks_per_cu workgroups per CU of the create-and-mark walk
+  fresh_blocks_per_cu most workgroups per CU of the create-and-mark walk
   fresh_window        its lockstep window, in cells
   ray_order           winner order: direction only (0), or classes of ray
                       length and direction (1..5)
@@ -39,15 +39,15 @@ TUNING_FILE = os.path.join(HERE, "tuning.json")
 
 CANDIDATES = {
     "ray_block": [64, 128, 256],
-    "ray_blocks_per_cu": [2, 4, 6, 8, 12, 16],
-    "leaf_blocks_per_cu": [4, 6, 8, 12, 16, 32],
+    "ray_blocks_per_cu": [16, 24, 32, 64, 128, 256],
+    "leaf_blocks_per_cu": [16, 24, 32, 64, 128, 256],
     "ray_chunk": [64, 128, 256, 512],
     "ep_table_factor": [2, 4],
     "root_slack": [2, 4],
     "ray_window": [4, 8, 16, 32, 64, 1 << 20],
     "leaf_window": [8, 16, 32, 64, 1 << 20],
     "fresh_pass": [1, 0],
-    "fresh_blocks_per_cu": [2, 4, 6, 8, 12, 16],
+    "fresh_blocks_per_cu": [16, 24, 32, 64, 128, 256],
     "fresh_window": [4, 8, 16, 32, 64, 1 << 20],
     "ray_order": [3, 4, 2, 5, 1, 0],
 }

@@ -93,24 +93,26 @@ struct bxg_ctx {
   hipEvent_t ev[64] = {};
   bool profiling = false;
   bool counting = false;
-  // tuning (bxg_ctx_set_tuning): workgroups per CU of the work-stealing
-  // update pass and leaf-allocation pass over the rays, the workgroup size
-  // of both, the most rays a wavefront takes per cursor atomic (rays per
-  // lane = ray_chunk / 64), the endpoint-table capacity per point and the
-  // root-directory capacity per root (inverse load factors); the update
-  // pass of a call with fewer points than its tuned grid has lanes runs on
-  // small_ray_blocks_per_cu workgroups per CU
-  uint32_t ray_blocks_per_cu = 4;
-  uint32_t small_ray_blocks_per_cu = 2;
-  uint32_t leaf_blocks_per_cu = 16;
-  uint32_t ray_block = 256;
+  // tuning (bxg_ctx_set_tuning): the most workgroups per CU the passes over
+  // the rays are launched with (update, leaf and fresh pass), the workgroups
+  // per CU that a small call's ray segments may fill, the workgroup size of
+  // the passes, the rays a fresh-pass wavefront walks batch after batch, the
+  // endpoint-table capacity per point and the root-directory capacity per
+  // root (inverse load factors).  One-wavefront workgroups: a workgroup's
+  // slots are free for the next one as soon as its own rays are done (256
+  // threads: update pass 4.0 against 3.75 ms a 64-map frame, 275 against 224
+  // us a LiDAR scan)
+  uint32_t ray_blocks_per_cu = 128;
+  uint32_t small_ray_blocks_per_cu = 32;
+  uint32_t leaf_blocks_per_cu = 128;
+  uint32_t ray_block = 64;
   uint32_t ray_chunk = 256;
   uint32_t ep_table_factor = 2;
   uint32_t root_slack = 2;
   uint32_t ray_window = 8;    // lockstep windows of the update pass (cells) and leaf pass (leaves)
   uint32_t leaf_window = 32;
   uint32_t fresh_pass = 1;    // maps empty at a scan's start: one create-and-mark walk
-  uint32_t fresh_blocks_per_cu = 6;  // workgroups per CU of that walk
+  uint32_t fresh_blocks_per_cu = 128;
   uint32_t fresh_window = 16;        // its lockstep window (cells)
   uint32_t ray_order = 3;            // winner order: direction sector, length class, direction
   std::vector<Prof> prof_pending;
@@ -715,31 +717,22 @@ int enqueue_scan_kernels(bxg_ctx* c, const BatchHdr* hdr, const ScanDesc* desc, 
                          uint64_t grid_points, uint32_t nscans, bool any_extra) {
   const uint32_t gp = nblocks(grid_points);
   const uint32_t gw = std::max<uint32_t>(1, std::min<uint32_t>(gp, 16384));
-  // work-stealing ray kernels: enough blocks to fill every CU, no more
-  // than the rays could use (64 rays per wavefront, 4 wavefronts a block)
-  const uint32_t cus = (uint32_t)std::max(c->cu_count, 1);
-  // leaf pass: at most one lane per point (the winners are fewer); update
-  // pass: up to 8, since a call with fewer rays than lanes walks each ray as
-  // up to 8 segments (on the leaf pass the extra wavefronts cost more in
-  // cursor traffic than the segments gain)
+  // the passes over the rays: a wavefront a batch of 64 winners (at most one
+  // per 64 points; capped, the wavefronts then walk several), and in small
+  // calls up to 8, for segments of the batches, while the workgroups per CU
+  // allow it; a multiple of the XCDs
+  const uint64_t cus = (uint64_t)std::max(c->cu_count, 1);
   const uint32_t rb = c->ray_block;
-  const uint32_t most = (uint32_t)((grid_points + rb - 1) / rb);
-  const uint32_t most8 = (uint32_t)std::min<uint64_t>((grid_points * 8 + rb - 1) / rb, 1u << 30);
-  // the tuned grid serves large calls (batched frames, lockstep batches); a
-  // call with fewer points than that grid has lanes walks ray segments on a
-  // grid of small_ray_blocks_per_cu workgroups per CU (2 by default: more
-  // lanes cut the rays into more, shorter segments, and each segment starts
-  // with a seek and a root lookup of its own)
-  const uint32_t gr_full = std::max<uint32_t>(1, cus * c->ray_blocks_per_cu);
-  const uint32_t gr = grid_points >= (uint64_t)gr_full * rb
-                          ? gr_full
-                          : std::max<uint32_t>(1, std::min<uint32_t>(cus * c->small_ray_blocks_per_cu, most8));
-  const uint32_t gl = std::max<uint32_t>(1, std::min<uint32_t>(cus * c->leaf_blocks_per_cu, most));
-  // the fresh pass: its own workgroups per CU for large calls
-  const uint32_t gf_full = std::max<uint32_t>(1, cus * c->fresh_blocks_per_cu);
-  const uint32_t gf = grid_points >= (uint64_t)gf_full * rb
-                          ? gf_full
-                          : std::max<uint32_t>(1, std::min<uint32_t>(cus * c->small_ray_blocks_per_cu, most8));
+  const uint64_t most = (grid_points + rb - 1) / rb;
+  const auto walk_grid = [&](uint64_t per_cu, uint64_t run) {
+    const uint64_t whole = std::min((most + run - 1) / run, cus * per_cu);
+    const uint64_t cut = std::min(most * (1u << kMaxSegLog), cus * c->small_ray_blocks_per_cu);
+    const uint64_t g = std::max<uint64_t>({whole, cut, 1});
+    return (uint32_t)((g + kXcds - 1) / kXcds * kXcds);
+  };
+  const uint32_t gr = walk_grid(c->ray_blocks_per_cu, 1);
+  const uint32_t gl = walk_grid(c->leaf_blocks_per_cu, 1);
+  const uint32_t gf = walk_grid(c->fresh_blocks_per_cu, c->ray_chunk / 64);
   sc.chunk_max = c->ray_chunk;
   sc.win_cells = (int32_t)c->ray_window;
   sc.win_leaves = (int32_t)c->leaf_window;
@@ -747,7 +740,7 @@ int enqueue_scan_kernels(bxg_ctx* c, const BatchHdr* hdr, const ScanDesc* desc, 
   sc.win_fresh = (int32_t)c->fresh_window;
   sc.ray_order = c->ray_order;
   // new-leaf pass: a wavefront per new leaf, grid-stride over them
-  const uint32_t gm = std::max<uint32_t>(1, std::min<uint32_t>(cus * 8, gp));
+  const uint32_t gm = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(cus * 8, gp));
   BXG_TRY(launch(c, "k_scan_begin", k_scan_begin, 1, kBlock, hdr, desc, sc));
   BXG_TRY(launch(c, "k_scan_classify", k_scan_classify, gp, kBlock, hdr, desc, sc));
   BXG_TRY(launch(c, "k_scan_winners", k_scan_winners, gp, kBlock, hdr, desc, sc));
@@ -772,7 +765,7 @@ int enqueue_scan_kernels(bxg_ctx* c, const BatchHdr* hdr, const ScanDesc* desc, 
     BXG_TRY(launch(c, "k_scan_new_endpoints", k_scan_new_endpoints<false>, gw, kBlock, desc, sc));
   }
   BXG_TRY(launch(c, "k_scan_new_leaves", k_scan_new_leaves, gm, kBlock, hdr, desc));
-  BXG_TRY(launch(c, "k_scan_finalize", k_scan_finalize, 1, kBlock, hdr, desc, sc));
+  BXG_TRY(launch(c, "k_scan_finalize", k_scan_finalize, 1, kBlock, hdr, desc));
   return BXG_OK;
 }
 

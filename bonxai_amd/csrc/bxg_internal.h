@@ -146,14 +146,12 @@ struct alignas(16) BatchHdr {
 constexpr uint32_t kDirBits = 12;  // direction and length-class bits of a bucket
 constexpr uint32_t kMaxTagBits = 6;
 constexpr uint32_t kMaxBuckets = 1u << (kDirBits + kMaxTagBits);
-constexpr uint32_t kRegions = 8;   // winner-list regions, one per XCD
+constexpr uint32_t kXcds = 8;      // workgroups are dispatched round the XCDs
 constexpr uint32_t kScanTile = 4096;  // buckets one block of the bucket scan covers
 constexpr uint32_t kTiles = kMaxBuckets / kScanTile;
 static_assert((1u << kDirBits) % kScanTile == 0 && kTiles <= 64, "bucket scan tiles");
-// scan counter words: [0] winner count, [1, 1 + 6 * kRegions) region cursors
-// and exhausted flags of the three walks (leaf pass, update pass, fresh
-// pass), [kFreshWords, + 4) the fresh-pass split (below), [kTileWords, +
-// kTiles) bucket-tile sums, [kClipWords, + 64) per scan (index mod 64) the
+// scan counter words: [0] winner count, [kFreshWords, + 4) the fresh-pass
+// split (below), [kTileWords, + kTiles) bucket-tile sums, [kClipWords, + 64) per scan (index mod 64) the
 // points clipped at the max range among those of one wavefront in 16
 constexpr uint32_t kTileWords = 64;
 constexpr uint32_t kClipWords = kTileWords + kTiles;
@@ -163,7 +161,7 @@ constexpr uint32_t kCounterWords = kClipWords + 64;
 // list: [kFreshWords, +1] the 64-bit mask of those scans, [+2] the first of
 // their tags (kNone: no split, every pass walks the whole list and skips the
 // other pipeline's rays), [+3] the index of their first winner.
-constexpr uint32_t kFreshWords = 1 + 6 * kRegions;
+constexpr uint32_t kFreshWords = 1;
 static_assert(kFreshWords + 4 <= kTileWords, "counter words");
 
 // scratch of one integration call, owned by the context
@@ -183,7 +181,7 @@ struct ScanScratch {
   uint32_t* tpos;       // per point: endpoint-table slot of its endpoint
   EpSlot* ep;           // endpoint table
   uint32_t ep_mask;     // capacity - 1
-  uint32_t chunk_max;   // most rays a wavefront takes per cursor atomic (64..1024)
+  uint32_t chunk_max;   // rays a wavefront of the fresh pass walks one batch after the other (64..1024)
   int32_t win_cells;    // lockstep window of the update pass, in cells (0: the default)
   int32_t win_leaves;   // lockstep window of the leaf pass, in leaves (0: the default)
   uint32_t fresh_pass;  // 1: the rays of maps empty at the scan's start take the fresh pass
@@ -193,9 +191,7 @@ struct ScanScratch {
   uint32_t* wkey;       // per point: bucket of a winner, kNone otherwise
   uint32_t* hist;       // [kMaxBuckets] winners per bucket (zero between calls)
   uint32_t* offs;       // [kMaxBuckets] bucket write cursors
-  uint32_t* counters;   // [0] winner count, [1..16] leaf-pass region cursors
-                        // and exhausted flags, [17..32] the same for the ray
-                        // pass, [33..48] for the fresh pass
+  uint32_t* counters;   // kCounterWords words (above)
 };
 
 // rec.w flag bits

@@ -202,6 +202,49 @@ __device__ __forceinline__ MapView load_view(const MapDev* p) {
   return v;
 }
 
+// A map header read through scalar loads: p is the same in every lane of the
+// wavefront (a header changes only between kernels).
+#define BXG_C __attribute__((address_space(4)))
+template <class T>
+__device__ __forceinline__ T* uniform_ptr(T* p) {
+  const uint64_t a = (uint64_t)p;
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32));
+  return (T*)(((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ int32_t uniform_i32(const int32_t* p) {
+  return *(const int32_t BXG_C*)uniform_ptr(p);
+}
+__device__ __forceinline__ MapView uniform_view(const MapDev* p) {
+  const MapDev BXG_C* q = (const MapDev BXG_C*)uniform_ptr(p);
+  MapView v;
+  v.root_keys = gp((uint64_t*)q->root_keys);
+  v.children = gp((uint32_t*)q->children);
+  v.masks = gp((uint64_t*)q->leaf_masks);
+  v.cells = gp((uint8_t*)q->cells);
+  v.touched = gp((uint8_t*)q->touched);
+  v.origin = q->leaf_origin;
+  v.ctr = q->ctr;
+  v.inv_res = q->inv_res;
+  v.ib = q->inner_bits;
+  v.lb = q->leaf_bits;
+  v.log2n = q->log2n;
+  v.isz = q->inner_size;
+  v.lsz = q->leaf_size;
+  v.lw = q->leaf_words;
+  v.vb = q->value_bytes;
+  v.flags = q->flags;
+  v.root_mask = q->root_mask;
+  v.max_probe = q->max_probe;
+  v.leaf_cap = q->leaf_cap;
+  v.miss = q->opt_miss;
+  v.hit = q->opt_hit;
+  v.cmin = q->opt_cmin;
+  v.cmax = q->opt_cmax;
+  v.thr = q->opt_thr;
+  return v;
+}
+
 // counter words read at kernel start (written by earlier kernels)
 __device__ __forceinline__ uint32_t map_status(const MapView& m) { return *gp(&m.ctr->status); }
 __device__ __forceinline__ int32_t map_cur(const MapView& m) { return *gp(&m.ctr->cur); }
@@ -413,6 +456,15 @@ struct LeafWalk {
     }
     // axis steps from the origin to the first cell of the next leaf
     const int64_t N = (int64_t)n + (s > 0 ? (int64_t)L - (c & lm) : (int64_t)(c & lm) + 1);
+    if (m <= kRay32) {  // the same in 32 bits: (2N - 1) m < 2^32
+      const uint32_t A = (uint32_t)(2 * N - 1) * (uint32_t)m, LM = L * (uint32_t)m;
+      q = A / b;
+      r = A - q * b;
+      Q = LM / (uint32_t)d;
+      R = 2u * (LM - Q * (uint32_t)d);
+      kc = (int32_t)(q + (r > 0 ? 1u : 0u));
+      return;
+    }
     const uint64_t A = (uint64_t)(2 * N - 1) * (uint64_t)m;
     const uint64_t q64 = A / b;
     const uint64_t LM = (uint64_t)L * (uint64_t)m;
@@ -430,11 +482,9 @@ struct LeafWalk {
     const uint32_t L = 1u << lb;
     k = w.k;
     kend = w.kend;
-    const int64_t m2 = 2 * (int64_t)w.mx;
     // axis steps already taken at cell k (none at k = 0)
-    const int32_t nx = k ? (int32_t)((2 * (int64_t)k * w.dx + w.mx) / m2) : 0;
-    const int32_t ny = k ? (int32_t)((2 * (int64_t)k * w.dy + w.mx) / m2) : 0;
-    const int32_t nz = k ? (int32_t)((2 * (int64_t)k * w.dz + w.mx) / m2) : 0;
+    int32_t nx = 0, ny = 0, nz = 0;
+    if (k) w.steps(k, nx, ny, nz);
     axis(w.cx, w.sx, w.dx, nx, w.mx, L, lx, stx, kx, qx, rx, Qx, Rx, bx);
     axis(w.cy, w.sy, w.dy, ny, w.mx, L, ly, sty, ky, qy, ry, Qy, Ry, by);
     axis(w.cz, w.sz, w.dz, nz, w.mx, L, lz, stz, kz, qz, rz, Qz, Rz, bz);
@@ -1059,251 +1109,192 @@ __global__ void __launch_bounds__(256) k_scan_scatter(const BatchHdr* __restrict
   if (win) sc.winners[pos] = (uint32_t)gi;
 }
 
-// The passes over the winners' rays (walk_winners, start_ray).
+// The passes over the winners' rays (walk_winners).
 enum : int { kPassLeaves = 0, kPassUpdate = 1, kPassFresh = 2 };
 
-// Start the ray of winner `idx`; false if it has no cells to walk (origin
-// voxel endpoint, endpoint-only call, or a map whose call failed), or if the
-// ray belongs to the other pipeline: with sc.fresh_pass set, the rays of a
-// map that was empty when the scan started (leaf_base 0: every leaf the scan
-// touches is new) take only the fresh pass, and the other maps' rays only the
-// leaf and update passes.
-// With lg > 0, work unit `unit` is segment unit & (2^lg - 1) of winner
-// unit >> lg: segment s of n = 2^lg walks cells [ceil(s mx / n), ceil((s + 1)
-// mx / n)), so segment 0 holds cell 0 and the segments cover the ray once.
-// `first` tells the caller the unit holds the ray's cell 0.
-__device__ __forceinline__ bool start_ray(const ScanDesc* __restrict__ sd, const ScanScratch& sc,
-                                          uint32_t unit, uint32_t lg, MapView& m, RayWalk& w,
-                                          RootCache& rc, int32_t& cur, uint32_t& lbase,
-                                          int pass, bool& first, uint32_t& win) {
-  // the leaf and fresh passes walk the endpoint's cell too (they create
-  // leaves); the update pass only the ray's cells
-  const bool leaf_pass = pass != kPassUpdate;
-  const uint32_t idx = unit >> lg, seg = unit & ((1u << lg) - 1u);
-  first = seg == 0;
-  const uint32_t gi = sc.winners[idx];
-  win = gi;
-  const int4 r = sc.rec[gi];
-  const ScanDesc& d = sd[(uint32_t)r.w >> 16];
-  const bool no_rays = (d.flags & kScanNoRays) != 0;
-  const bool at_origin = r.x == d.ox && r.y == d.oy && r.z == d.oz;
-  // the update pass walks cells [0, mx) of the ray (none for an endpoint in
-  // the origin's voxel or a scan without rays); the leaf pass also the
-  // endpoint's cell mx, so that it creates the winner's endpoint leaf with
-  // the ray's (only that cell for a scan without rays)
-  if (!leaf_pass && (no_rays || at_origin)) return false;
-  if (leaf_pass && no_rays && seg != 0) return false;
-  m = load_view(d.map);
-  if (pass != kPassLeaves && (map_status(m) & kFatal)) return false;
-  cur = map_cur(m);
-  lbase = *gp(&m.ctr->leaf_base);
-  if (sc.fresh_pass ? ((pass == kPassFresh) != (lbase == 0)) : pass == kPassFresh) return false;
-  w.init(d.ox, d.oy, d.oz, r.x, r.y, r.z);
-  const int32_t last = w.mx + (leaf_pass ? 1 : 0);
-  int32_t k0 = 0, k1 = last;
-  if (no_rays) {
-    k0 = w.mx;
-  } else if (lg) {
-    const int64_t n = 1ll << lg;
-    k0 = (int32_t)(((int64_t)last * seg + n - 1) >> lg);
-    k1 = (int32_t)(((int64_t)last * (seg + 1) + n - 1) >> lg);
-  }
-  if (k0 >= k1) return false;
-  if (k0 == 0)
-    w.kend = k1;  // from the origin (and mx may be 0: no division)
-  else
-    w.seek(k0, k1);
-  rc.reset();
-  return true;
-}
-
-constexpr uint32_t kChunk = 256;  // default of ScanScratch::chunk_max
-// cells a lane may run ahead of its wavefront's slowest ray in lockstep
-// batches: update pass and leaf pass (defaults; the tuning keys ray_window
-// and leaf_window set them per context.  Measured on 64 scans re-inserted
-// into filled maps: 8 beats 4 and 16 for the update pass, 32 beats 16 for
-// the leaf pass)
+// cells a lane may run ahead of its wavefront's slowest ray when rays are
+// walked whole: update pass and leaf pass (defaults; the tuning keys
+// ray_window and leaf_window set them per context.  Measured on 64 scans
+// re-inserted into filled maps: 8 beats 4 and 16 for the update pass, 32
+// beats 16 for the leaf pass)
 constexpr int32_t kSyncWindowCells = 8;
 constexpr int32_t kSyncWindowLeaves = 32;
-constexpr uint32_t kLockstepRays = 1;  // rays a lane from which batches run in lockstep
-constexpr uint32_t kMaxSegLog = 3;     // at most 8 segments a ray when rays are fewer than lanes
+constexpr uint32_t kMaxSegLog = 3;  // at most 8 segments a ray
+constexpr uint32_t kGroupLog = 3;   // batches side by side on one XCD in a short list
 
-// Work-stealing walk over the winner list.  The list is split into kRegions
-// ranges; a wavefront starts in the range of its XCD (workgroups are
-// dispatched round-robin over the XCDs) and takes up to chunk_max rays per
-// atomic on the range's cursor.  Every lane works on its own ray, one leaf
-// per step.  With at least kLockstepRays rays a lane, the wavefront takes its
-// next 64 rays only when all 64 are done (lockstep batches): consecutive
-// winners are rays of one map in neighbouring directions (and, with the ray
-// order of k_scan_winners, of about one length), so a batch's rays stay side
-// by side and cross the same cache lines at about the same time, where lanes
-// refilled one by one drift apart (measured on 64 scans a call: the update
-// pass 23 % and the leaf pass 18 % faster).  With fewer rays (one scan a
-// call) lanes refill one by one: there, a batch waiting for its longest ray
-// leaves the GPU idle (measured again with length-ordered rays: the LiDAR
-// sequence 26 % slower in lockstep).  A range found empty
-// is flagged so that idle wavefronts stop touching its cursor.  kMode 0: leaf
-// allocation pass; 1: update pass; 2: counted update; 3: fresh pass (maps
-// empty at the scan's start: create and mark in one walk); 4: counted fresh
-// pass.
-// cursors[0..kRegions) are the cursors, cursors[kRegions..2*kRegions) the
-// exhausted flags.
+// The walk over the winner list.  A batch is 64 consecutive winners, rays of
+// one map in neighbouring directions and (with the ray order of
+// k_scan_winners) of about one length, so that they cross the same leaves
+// and cache lines at about the same time; a wavefront walks one batch, one
+// ray a lane, one leaf a step.  Which batch follows from the wavefront's
+// number alone: no cursor, no work stealing (the grid holds a wavefront a
+// batch, and the workgroups waiting for a free slot balance the load).
+//
+// A short list (one scan a call) has fewer batches than the GPU has wavefront
+// slots, and a walk is a chain of dependent loads about 1.5 us a step: there
+// each ray is cut into up to 8 segments, and a wavefront walks one segment of
+// a batch.  The tasks of a group of up to 8 batches follow each other on one
+// XCD (workgroups go round the XCDs), segment by segment, so that its L2
+// sees neighbours at one distance from the sensor.  A long list is cut into
+// one contiguous part an XCD (a map's rays stay on one XCD or two); there the
+// rays are walked whole, in lockstep: a lane more than the window's cells
+// ahead of the wavefront's slowest ray waits a step.  The fresh pass takes
+// ray_chunk / 64 consecutive batches a wavefront: neighbouring batches that
+// run at the same time race for the same leaves (1: 3.6 ms, 4: 3.0 ms, 8:
+// 3.5 ms a 64-map frame).
+//
+// Measured against persistent wavefronts that took rays from 8 cursors and
+// refilled their lanes one by one in short lists (us a call; leaf pass /
+// update pass): 2,001-point scan 61 / 31 -> 14 / 25, 307k-point depth frame
+// 70 / 61 -> 10 / 14, 65k-point LiDAR scan at 50 m 210 / 385 -> 99 / 224;
+// 64 maps 1149 / 4538 -> 600 / 3750, fresh pass 3047 -> 3000.  Bound: the
+// dependent loads of a step (entry, cells) and the scattered lines they touch.
+//
+// kMode 0: leaf allocation pass; 1: update pass; 2: counted update; 3: fresh
+// pass (maps empty at the scan's start: create and mark in one walk); 4:
+// counted fresh pass.
 template <int kMode>
-__device__ void walk_winners(const ScanDesc* __restrict__ sd, const ScanScratch& sc,
-                             uint32_t* cursors) {
-  if (kMode >= 3 && !sc.fresh_pass) return;
+__device__ void walk_winners(const ScanDesc* __restrict__ sd, const ScanScratch& sc) {
+  constexpr bool kCounted = kMode == 2 || kMode == 4;
+  constexpr bool kFreshPass = kMode >= 3;
+  constexpr int kPass = kMode == 0 ? kPassLeaves : (kFreshPass ? kPassFresh : kPassUpdate);
+  constexpr bool leaf_pass = kPass != kPassUpdate;
+  if (kFreshPass && !sc.fresh_pass) return;
   // the pass's part of the winner list: with a split, the fresh scans'
   // winners end the list
   const uint32_t total = sc.counters[0];
   const bool split = sc.counters[kFreshWords + 2] != kNone;
   const uint32_t at = split ? sc.counters[kFreshWords + 3] : 0u;
-  const uint32_t w0 = (split && kMode >= 3) ? at : 0u;
-  const uint32_t nwin = split ? (kMode >= 3 ? total - at : at) : total;
+  const uint32_t w0 = (split && kFreshPass) ? at : 0u;
+  const uint32_t nwin = split ? (kFreshPass ? total - at : at) : total;
+  const uint32_t nb = (nwin + 63u) >> 6;
+  // the wavefront's number among those of its XCD (the grid is a multiple of
+  // kXcds workgroups)
+  const uint32_t wpb = blockDim.x >> 6;
+  const uint32_t xcd = blockIdx.x % kXcds;
+  const uint32_t wave = (blockIdx.x / kXcds) * wpb +
+                        (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t waves = (gridDim.x / kXcds) * wpb;
   const uint32_t lane = lane_id();
-  const uint32_t lanes = gridDim.x * blockDim.x;
-  const bool lockstep = nwin >= kLockstepRays * lanes;
-  // fewer rays than lanes (one scan a call): each ray is walked as 2^lg
-  // segments by different lanes, so the short list still fills the GPU
   uint32_t lg = 0;
-  while (!lockstep && lg < kMaxSegLog && ((uint64_t)nwin << (lg + 1)) <= lanes) ++lg;
-  const uint32_t nunits = nwin << lg;
-  uint32_t chunk_pos = 0, chunk_end = 0;
-  // small lists are one region: splitting them only multiplies cursor traffic
-  const uint32_t cmax = sc.chunk_max ? sc.chunk_max : kChunk;
-  constexpr bool kCounted = kMode == 2 || kMode == 4;
-  constexpr bool kFreshPass = kMode >= 3;
-  constexpr int kPass = kMode == 0 ? kPassLeaves : (kFreshPass ? kPassFresh : kPassUpdate);
+  while (lg < kMaxSegLog && ((uint64_t)nb << (lg + 1)) <= (uint64_t)waves * kXcds) ++lg;
+  const bool lockstep = lg == 0;
+  uint32_t gl = kGroupLog;  // fewer batches a group where that would leave XCDs idle
+  while (gl > 0 && (nb >> gl) < 8u * kXcds) --gl;
+  const uint32_t per_xcd = (nb + kXcds - 1) / kXcds;
+  const uint32_t run = kFreshPass ? max(sc.chunk_max / 64u, 1u) : 1u;
   const int32_t wcells = sc.win_cells > 0 ? sc.win_cells : kSyncWindowCells;
   const int32_t win = kMode == 0 ? (sc.win_leaves > 0 ? sc.win_leaves : kSyncWindowLeaves)
                                  : (kFreshPass && sc.win_fresh > 0 ? sc.win_fresh : wcells);
-  const uint32_t nreg = nunits >= kRegions * 8 * cmax ? kRegions : 1u;
-  // chunk size: kChunk units when there is work for every wavefront, down
-  // to one unit a lane on small lists
-  uint32_t chunk = (nunits / (gridDim.x * (blockDim.x / 64u))) & ~63u;
-  chunk = chunk < 64u ? 64u : (chunk > cmax ? cmax : chunk);
-  uint32_t region = blockIdx.x % nreg, tried = 0;
-  bool first = false;
-  bool exhausted = false;
-  bool have = false;
-  MapView m;
-  RayWalk w;
-  LeafWalk lw;  // the leaf pass walks leaves, not cells
-  RootCache rc;
-  int32_t cur = 0;
-  uint32_t lbase = 0;
-  uint32_t nupd = 0;
-  uint32_t next_leaf = kNone;
-  // fresh pass: root slot and inner-grid entry of the current cell's leaf
-  int32_t slot = -1;
-  uint32_t entry = kEmptyChild;
-  bool stopped = false;
-  bool ray_first = false;
-  uint32_t wgi = 0;  // the ray's winner (its point index)
-  // counted form: per-lane totals, flushed when the lane's map changes
-  MapCounters* cmap = nullptr;
-  uint64_t c_upd = 0, c_rays = 0, c_vis = 0;
+  uint32_t round = 0, in_run = 0;  // rounds of the grid over the list
   for (;;) {
-    // lockstep: a new batch once every lane's ray is done (wave-uniform
-    // control flow); rays are handed out until every lane has one or the
-    // list is exhausted
-    const bool refill = !lockstep || __ballot(have) == 0;
-    for (;;) {
-      const uint64_t need = __ballot(!have);
-      if (!refill || need == 0 || exhausted) break;
-      if (chunk_pos == chunk_end) {
-        const uint32_t lo = (uint32_t)((uint64_t)nunits * region / nreg);
-        const uint32_t hi = (uint32_t)((uint64_t)nunits * (region + 1) / nreg);
-        uint32_t base = hi - lo;
-        // plain reads first: an exhausted range costs no atomic
-        if (lane == 0 && !*gp(&cursors[kRegions + region]) && *gp(&cursors[region]) < hi - lo)
-          base = add32(&cursors[region], chunk);
-        base = (uint32_t)__shfl((int)base, 0);
-        if (base >= hi - lo) {
-          if (lane == 0) *gp(&cursors[kRegions + region]) = 1u;
-          if (++tried == nreg) {
-            exhausted = true;
-            break;
+    uint32_t batch, seg = 0;
+    if (lockstep) {
+      const uint32_t first = round * waves * run;
+      if (first >= per_xcd) break;
+      const uint32_t j = first + wave * run + in_run;
+      if (++in_run == run) {
+        in_run = 0;
+        ++round;
+      }
+      batch = j < per_xcd ? xcd * per_xcd + j : nb;
+    } else {
+      const uint32_t j = round * waves + wave;
+      ++round;
+      const uint32_t group = (j >> (gl + lg)) * kXcds + xcd;
+      if ((group << gl) >= nb) break;
+      batch = (group << gl) + (j & ((1u << gl) - 1u));
+      seg = (j >> gl) & ((1u << lg) - 1u);
+    }
+    if (batch >= nb) continue;
+    const uint32_t idx = batch * 64u + lane;
+    const bool valid = idx < nwin;
+    const uint32_t gi = valid ? sc.winners[w0 + idx] : 0u;
+    const int4 r = valid ? sc.rec[gi] : make_int4(0, 0, 0, 0);
+    const uint32_t s = (uint32_t)r.w >> 16;
+    // one scan at a time (a batch seldom holds two), so that the scan's and
+    // the map's header sit in scalar registers
+    uint64_t pending = __ballot(valid);
+    while (pending) {
+      const uint32_t s0 =
+          (uint32_t)__builtin_amdgcn_readlane((int)s, __ffsll((unsigned long long)pending) - 1);
+      const bool act = valid && s == s0;
+      pending &= ~__ballot(act);
+      const ScanDesc& d = sd[s0];
+      const MapView m = uniform_view(d.map);
+      const int32_t cur = uniform_i32(&m.ctr->cur);
+      const uint32_t lbase = (uint32_t)uniform_i32((const int32_t*)&m.ctr->leaf_base);
+      // with sc.fresh_pass set, the rays of a map that was empty when the scan
+      // started (leaf_base 0: every leaf the scan touches is new) take only
+      // the fresh pass, and the other maps' rays only the leaf and update passes
+      if (sc.fresh_pass ? ((kPass == kPassFresh) != (lbase == 0)) : kPass == kPassFresh) continue;
+      if (kPass != kPassLeaves && (map_status(m) & kFatal)) continue;
+      const int32_t ox = d.ox, oy = d.oy, oz = d.oz;
+      const bool no_rays = (d.flags & kScanNoRays) != 0;
+      RayWalk w;
+      w.init(ox, oy, oz, r.x, r.y, r.z);
+      // the update pass walks cells [0, mx) of the ray (none for an endpoint
+      // in the origin's voxel or a scan without rays); the leaf and fresh
+      // passes also the endpoint's cell mx, so that they create the winner's
+      // endpoint leaf (only that cell for a scan without rays)
+      bool have = act && (leaf_pass || !no_rays);
+      const int32_t last = w.mx + (leaf_pass ? 1 : 0);
+      // segment seg of n = 2^lg walks cells [ceil(seg last / n), ceil((seg +
+      // 1) last / n)): segment 0 holds cell 0, and they cover the ray once
+      const int64_t up = (1ll << lg) - 1;
+      int32_t k0 = (int32_t)(((int64_t)last * seg + up) >> lg);
+      int32_t k1 = (int32_t)(((int64_t)last * (seg + 1u) + up) >> lg);
+      if (no_rays) {
+        k0 = w.mx;
+        k1 = seg == 0 ? last : k0;
+      }
+      if (k0 >= k1) have = false;
+      if (have) {
+        if (k0 == 0)
+          w.kend = k1;  // from the origin (and mx may be 0: no division)
+        else
+          w.seek(k0, k1);
+      }
+      LeafWalk lw;  // the leaf pass walks leaves, not cells
+      RootCache rc;
+      rc.reset();
+      uint32_t next_leaf = kNone;
+      // fresh pass: root slot and inner-grid entry of the current cell's leaf
+      int32_t slot = -1;
+      uint32_t entry = kEmptyChild;
+      bool stopped = false;
+      uint32_t nupd = 0;
+      uint64_t c_vis = 0;
+      const bool ray_first = have && seg == 0 && w.k < w.mx;
+      if (kMode == 0 && have) lw.init(w, m.lb);
+      if (kPass == kPassUpdate && have) next_leaf = walk_leaf(m, w, rc);
+      if (kFreshPass && have) fresh_entry(m, w, rc, slot, entry);
+      if (kCounted && have) c_vis = (uint32_t)max(0, min(w.kend, w.mx) - w.k);
+      while (__ballot(have)) {
+        bool go = have;
+        if (lockstep) {
+          const int32_t kk = kMode == 0 ? lw.k : w.k;
+          int32_t kmin = wave_min(have ? kk : 0x7fffffff);
+          go = have && kk < kmin + win;
+          if (__ballot(go) == 0) go = have;
+        }
+        if (go) {
+          if (kMode == 0) {
+            leaves_step(m, lw, rc);
+          } else if (kFreshPass) {
+            nupd += fresh_step<kCounted>(m, w, rc, slot, entry, stopped, &sc.tpos[gi]);
+          } else {
+            nupd += apply_step<kCounted>(m, w, rc, cur, lbase, next_leaf);
           }
-          region = (region + 1) % nreg;
-          continue;
-        }
-        chunk_pos = lo + base;
-        chunk_end = chunk_pos + chunk < hi ? chunk_pos + chunk : hi;
-        continue;
-      }
-      const uint32_t avail = chunk_end - chunk_pos;
-      const uint32_t want = (uint32_t)__popcll(need);
-      const uint32_t take = want < avail ? want : avail;
-      const uint32_t rank = (uint32_t)__popcll(need & lanes_below());
-      if (!have && rank < take) {
-        have = start_ray(sd, sc, chunk_pos + rank + (w0 << lg), lg, m, w, rc, cur, lbase, kPass, first, wgi);
-        nupd = 0;
-        stopped = false;
-        // the unit holds cell 0 of a ray with cells (the fresh pass also
-        // walks origin-voxel endpoints and endpoint-only calls: no ray)
-        ray_first = have && first && w.k < w.mx;
-        if (kMode == 0 && have) lw.init(w, m.lb);
-        if ((kMode == 1 || kMode == 2) && have) next_leaf = walk_leaf(m, w, rc);
-        if (kFreshPass && have) fresh_entry(m, w, rc, slot, entry);
-        if (kCounted && have && m.ctr != cmap) {
-          if (cmap) {
-            add64(&cmap->stat_ray_updates, c_upd);
-            add64(&cmap->stat_rays, c_rays);
-            add64(&cmap->stat_ray_visits, c_vis);
-          }
-          cmap = m.ctr;
-          c_upd = c_rays = c_vis = 0;
-        }
-        if (kMode == 2 && have) c_vis += (uint32_t)(w.kend - w.k);
-        // the fresh pass also walks the endpoint's cell mx, not a ray cell
-        if (kMode == 4 && have) c_vis += (uint32_t)max(0, min(w.kend, w.mx) - w.k);
-      }
-      chunk_pos += take;
-    }
-    if (__ballot(have) == 0) break;
-    // lockstep: a lane more than the window's cells ahead of the wavefront's
-    // slowest ray waits a step, so the batch stays at about one distance
-    // from the sensor (runs end at leaf borders, so rays drift apart
-    // otherwise; measured: the update pass about 8 % faster)
-    const int32_t kk = kMode == 0 ? lw.k : w.k;
-    int32_t kmin = have ? kk : 0x7fffffff;
-    bool go = have;
-    if (lockstep && kMode == 0) {
-      // the leaf pass: DPP minimum (it also frees the registers that keep
-      // the pass at 5 waves a SIMD; the update pass measured no gain); a
-      // wavefront with no lane free to move lets every lane with a ray move
-      kmin = wave_min(kmin);
-      go = have && kk < kmin + win;
-      if (__ballot(go) == 0) go = have;
-    } else if (lockstep) {
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        const int32_t t = __shfl_xor(kmin, o);
-        kmin = t < kmin ? t : kmin;
-      }
-      go = have && kk < kmin + win;
-    }
-    if (go) {
-      if (kMode == 0) {
-        leaves_step(m, lw, rc);
-      } else if (kFreshPass) {
-        nupd += fresh_step<kCounted>(m, w, rc, slot, entry, stopped, &sc.tpos[wgi]);
-      } else {
-        nupd += apply_step<kCounted>(m, w, rc, cur, lbase, next_leaf);
-      }
-      if (kMode == 0 ? lw.done() : (w.done() || stopped)) {
-        have = false;
-        if (kCounted) {
-          c_upd += nupd;
-          c_rays += ray_first ? 1u : 0u;
+          if (kMode == 0 ? lw.done() : (w.done() || stopped)) have = false;
         }
       }
+      if (kCounted && act) {
+        add64(&m.ctr->stat_ray_updates, nupd);
+        add64(&m.ctr->stat_rays, ray_first ? 1u : 0u);
+        add64(&m.ctr->stat_ray_visits, c_vis);
+      }
     }
-  }
-  if (kCounted && cmap) {
-    add64(&cmap->stat_ray_updates, c_upd);
-    add64(&cmap->stat_rays, c_rays);
-    add64(&cmap->stat_ray_visits, c_vis);
   }
 }
 
@@ -1311,7 +1302,7 @@ __device__ void walk_winners(const ScanDesc* __restrict__ sd, const ScanScratch&
 // written (so a pool overflow leaves the map's cells untouched).
 __global__ void __launch_bounds__(256) k_scan_ray_leaves(const ScanDesc* __restrict__ sd,
                                                          ScanScratch sc) {
-  walk_winners<0>(sd, sc, &sc.counters[1]);
+  walk_winners<0>(sd, sc);
 }
 
 // Phase 2c (one block per scan): leaves of the rays still due from
@@ -1449,7 +1440,7 @@ __global__ void __launch_bounds__(256) k_scan_new_endpoints(const ScanDesc* __re
 template <bool kCount>
 __global__ void __launch_bounds__(256) k_scan_rays(const ScanDesc* __restrict__ sd,
                                                    ScanScratch sc) {
-  walk_winners<kCount ? 2 : 1>(sd, sc, &sc.counters[1 + 2 * kRegions]);
+  walk_winners<kCount ? 2 : 1>(sd, sc);
 }
 
 // Phase 4' (per winner of a map empty at the scan's start, with
@@ -1458,7 +1449,7 @@ __global__ void __launch_bounds__(256) k_scan_rays(const ScanDesc* __restrict__ 
 template <bool kCount>
 __global__ void __launch_bounds__(256) k_scan_fresh_rays(const ScanDesc* __restrict__ sd,
                                                          ScanScratch sc) {
-  walk_winners<kCount ? 4 : 3>(sd, sc, &sc.counters[1 + 4 * kRegions]);
+  walk_winners<kCount ? 4 : 3>(sd, sc);
 }
 
 // Phase 4b (one block per scan): rays due from addHitPoint / addMissPoint.
@@ -1645,11 +1636,9 @@ __global__ void k_scan_begin(const BatchHdr* __restrict__ hdr, const ScanDesc* _
 }
 
 // Phase 5 (per scan): advance update_count 1 -> 2 -> 3 -> 1
-// (probabilistic_map.cpp:103-105) unless the scan failed; reset the batch;
-// copy every scanned map's counters to its pinned host mirror, so the host
+// (probabilistic_map.cpp:103-105) unless the scan failed; copy every scanned map's counters to its pinned host mirror, so the host
 // learns pool use and errors from one event after the call (no copy a map).
-__global__ void k_scan_finalize(const BatchHdr* __restrict__ hdr, const ScanDesc* __restrict__ sd,
-                                ScanScratch sc) {
+__global__ void k_scan_finalize(const BatchHdr* __restrict__ hdr, const ScanDesc* __restrict__ sd) {
   for (uint32_t s = threadIdx.x; s < hdr->nscans; s += blockDim.x) {
     const MapDev BXG_G* md = (const MapDev BXG_G*)sd[s].map;
     MapCounters BXG_G* ctr = gp(md->ctr);
@@ -1666,7 +1655,6 @@ __global__ void k_scan_finalize(const BatchHdr* __restrict__ hdr, const ScanDesc
 #pragma unroll
     for (uint32_t k = 0; k < sizeof(MapCounters) / 8; ++k) dst[k] = v[k];
   }
-  if (threadIdx.x <= 6 * kRegions) sc.counters[threadIdx.x] = 0;
 }
 
 // ------------------------------------------------------ bulk cell ops

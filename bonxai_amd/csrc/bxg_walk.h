@@ -16,6 +16,9 @@
 namespace bxg {
 
 constexpr int kRun = 8;  // cells of one leaf handled per step of a ray
+// longest ray (cells) whose closed forms fit 32 bits: a 32-bit division costs
+// about a fifth of a 64-bit one
+constexpr int32_t kRay32 = 32767;
 
 // Cell 0 is the origin voxel, then max|d|-1 further cells; the end voxel is
 // not part of the ray and a zero-length ray is empty.  (cx, cy, cz) is cell
@@ -50,19 +53,31 @@ struct RayWalk {
   // closed form (n steps along an axis after k cells: n = floor((2k|d| +
   // mx) / (2mx)), error k|d| - n mx), the same state stepping from 0 reaches
   BXG_HD void seek(int32_t k0, int32_t k1) {
-    const int64_t m2 = 2 * (int64_t)mx;
-    const int64_t nx = (2 * (int64_t)k0 * dx + mx) / m2;
-    const int64_t ny = (2 * (int64_t)k0 * dy + mx) / m2;
-    const int64_t nz = (2 * (int64_t)k0 * dz + mx) / m2;
-    cx += sx * (int32_t)nx;
-    cy += sy * (int32_t)ny;
-    cz += sz * (int32_t)nz;
+    int32_t nx, ny, nz;
+    steps(k0, nx, ny, nz);
+    cx += sx * nx;
+    cy += sy * ny;
+    cz += sz * nz;
     const int32_t h = (mx + 1) >> 1;
-    ex = (int32_t)((int64_t)k0 * dx - nx * mx) - h;
-    ey = (int32_t)((int64_t)k0 * dy - ny * mx) - h;
-    ez = (int32_t)((int64_t)k0 * dz - nz * mx) - h;
+    ex = (int32_t)((int64_t)k0 * dx - (int64_t)nx * mx) - h;
+    ey = (int32_t)((int64_t)k0 * dy - (int64_t)ny * mx) - h;
+    ez = (int32_t)((int64_t)k0 * dz - (int64_t)nz * mx) - h;
     k = k0;
     kend = k1;
+  }
+  // steps the walk has taken along each axis when it reaches cell k0 (mx > 0)
+  BXG_HD void steps(int32_t k0, int32_t& nx, int32_t& ny, int32_t& nz) const {
+    if (mx <= kRay32) {  // 2 k |d| + mx < 2^31 + 2^15
+      const uint32_t m2 = 2u * (uint32_t)mx, k2 = 2u * (uint32_t)k0;
+      nx = (int32_t)((k2 * (uint32_t)dx + (uint32_t)mx) / m2);
+      ny = (int32_t)((k2 * (uint32_t)dy + (uint32_t)mx) / m2);
+      nz = (int32_t)((k2 * (uint32_t)dz + (uint32_t)mx) / m2);
+      return;
+    }
+    const int64_t m2 = 2 * (int64_t)mx;
+    nx = (int32_t)((2 * (int64_t)k0 * dx + mx) / m2);
+    ny = (int32_t)((2 * (int64_t)k0 * dy + mx) / m2);
+    nz = (int32_t)((2 * (int64_t)k0 * dz + mx) / m2);
   }
   BXG_HD bool done() const { return k >= kend; }
 };
