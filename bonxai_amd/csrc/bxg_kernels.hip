@@ -584,7 +584,7 @@ __device__ __forceinline__ uint32_t walk_leaf(const MapView& m, const RayWalk& w
 // 1, every writer agreeing; no read, no atomic), and k_scan_new_leaves writes
 // the leaf's cells and mask words from those bytes after the scan's endpoints
 // are marked.  In older leaves each cell is read, updated unless its
-// update_id is cur, and a cell turned on sets its mask bit with an atomicOr.
+// update_id is cur, and the cells turned on set their mask bits with atomicOrs.
 template <bool kCount>
 __device__ __forceinline__ uint32_t apply_step(const MapView& m, RayWalk& w, RootCache& rc,
                                                int32_t cur, uint32_t lbase, uint32_t& next_leaf) {
@@ -616,6 +616,14 @@ __device__ __forceinline__ uint32_t apply_step(const MapView& m, RayWalk& w, Roo
   for (int j = 0; j < kRun; ++j)
     v[j] = base[li[j]];  // slots j >= n re-read the run's first cell
   uint32_t nupd = 0;
+  // Mask bits of the cells turned on, gathered per mask word (a plane of the
+  // leaf: a ray's cells in it seldom change words more than once), so that a
+  // run takes one or two device-wide atomics instead of up to 8: they bound
+  // the update pass of scans that turn many cells on (LiDAR scans 1 m apart
+  // at 50 m: 357 -> 275 us a scan with 256-thread workgroups)
+  uint64_t BXG_G* mw = m.masks + (uint64_t)leaf * m.lw;
+  uint32_t word = 0;
+  uint64_t bits = 0;
 #pragma unroll
   for (int j = 0; j < kRun; ++j) {
     const bool upd = ((uint32_t)j < n) & (cell_id(v[j]) != cur);  // one branch, not two
@@ -634,10 +642,17 @@ __device__ __forceinline__ uint32_t apply_step(const MapView& m, RayWalk& w, Roo
       } else {
         base[li[j]] = cell_miss(old, m.miss, m.cmin, cur);
       }
-      if (old == 0)
-        or64((uint64_t*)&m.masks[(uint64_t)leaf * m.lw + (li[j] >> 6)], 1ull << (li[j] & 63));
+      if (old == 0) {
+        if (bits != 0 && (li[j] >> 6) != word) {
+          or64((uint64_t*)&mw[word], bits);
+          bits = 0;
+        }
+        word = li[j] >> 6;
+        bits |= 1ull << (li[j] & 63u);
+      }
     }
   }
+  if (bits) or64((uint64_t*)&mw[word], bits);
   return nupd;
 }
 
