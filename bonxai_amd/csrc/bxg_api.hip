@@ -219,6 +219,18 @@ uint32_t lookup_blocks(uint64_t n) {
   return (uint32_t)((n + (uint64_t)kBlock * kLookups - 1) / ((uint64_t)kBlock * kLookups));
 }
 
+// k_export over n leaves: mask words a wavefront (a power of two, 4096
+// wavefronts or more where the map has the words) and workgroups
+uint32_t export_words(const MapDev& h, uint64_t n) {
+  uint32_t w = 4;
+  while (w < kExportMostWords && n * h.leaf_words >= 2ull * w * 4096) w *= 2;
+  return w;
+}
+uint32_t export_blocks(const MapDev& h, uint64_t n) {
+  const uint64_t per = (uint64_t)kExportBlock / 64 * export_words(h, n);
+  return (uint32_t)((n * h.leaf_words + per - 1) / per);
+}
+
 // launch on a stream of the context, bracketed by events when profiling
 template <typename... KArgs, typename... Args>
 int launch_on(bxg_ctx* c, hipStream_t stream, const char* name, void (*k)(KArgs...), uint32_t grid,
@@ -1735,8 +1747,8 @@ int bxg_export(bxg_map* m, int filter, int32_t* coords, void* vals, uint64_t cap
   uint32_t nl = 0;
   BXG_TRY(known_leaf_count(m, &nl));
   BXG_HIP(c, hipMemsetAsync(c->d_small, 0, 8, c->stream));
-  BXG_TRY(launch(c, "k_export", k_export, nblocks((uint64_t)nl * m->h.leaf_size), kBlock,
-                 (const MapDev*)m->d, nl, (uint32_t)filter, coords, (uint8_t*)vals, cap,
+  BXG_TRY(launch(c, "k_export", k_export, export_blocks(m->h, nl), kExportBlock,
+                 (const MapDev*)m->d, nl, export_words(m->h, nl), (uint32_t)filter, coords, (uint8_t*)vals, cap,
                  c->d_small));
   BXG_TRY(d2h_sync(c, c->h_small, c->d_small, 8));
   *count = c->h_small[0];

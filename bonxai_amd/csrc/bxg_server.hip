@@ -138,8 +138,8 @@ void srv_launch_read(bxg_server* s, SrvReq* r) {
       uint64_t* dc = s->d_counts + r->slot;
       rc = hipMemsetAsync(dc, 0, 8, st) == hipSuccess ? BXG_OK : fail(c, BXG_ERR_HIP, "hipMemsetAsync");
       if (rc == BXG_OK)
-        rc = launch_on(c, st, "k_export", k_export, nblocks((uint64_t)nl * m->h.leaf_size), kBlock,
-                       (const MapDev*)m->d, nl, (uint32_t)r->filter, r->out_coords, (uint8_t*)r->vals,
+        rc = launch_on(c, st, "k_export", k_export, export_blocks(m->h, nl), kExportBlock,
+                       (const MapDev*)m->d, nl, export_words(m->h, nl), (uint32_t)r->filter, r->out_coords, (uint8_t*)r->vals,
                        r->cap, dc);
       if (rc == BXG_OK && hipMemcpyAsync(s->h_counts + r->slot, dc, 8, hipMemcpyDeviceToHost, st) != hipSuccess)
         rc = fail(c, BXG_ERR_HIP, "hipMemcpyAsync");
