@@ -544,6 +544,7 @@ int ensure_scan_scratch(bxg_ctx* c, uint64_t points, uint32_t nscans) {
     dfree(c->sc.tpos);
     dfree(c->sc.winners);
     dfree(c->sc.wkey);
+    dfree(c->sc.wrank);
     dfree(c->sc.ep);
     uint32_t* hist = c->sc.hist;
     uint32_t* offs = c->sc.offs;
@@ -562,6 +563,8 @@ int ensure_scan_scratch(bxg_ctx* c, uint64_t points, uint32_t nscans) {
     c->sc.winners = (uint32_t*)p;
     BXG_TRY(dmalloc(c, &p, cap * 4));
     c->sc.wkey = (uint32_t*)p;
+    BXG_TRY(dmalloc(c, &p, cap * 4));
+    c->sc.wrank = (uint32_t*)p;
     if (!c->sc.hist) {
       BXG_TRY(dmalloc(c, &p, (uint64_t)kMaxBuckets * 4));
       c->sc.hist = (uint32_t*)p;
@@ -724,6 +727,13 @@ int upload_extra(bxg_map* m) {
   return upload(c, m->d_extra, m->extra.data(), m->extra.size() * sizeof(int4));
 }
 
+// bits of the scan index kept in a winner's bucket
+uint32_t tag_bits_for(uint32_t nscans) {
+  uint32_t b = 0;
+  while (b < kMaxTagBits && (1u << b) < nscans) ++b;
+  return b;
+}
+
 // the kernel sequence of one wave of scans on given scratch/descriptors
 int enqueue_scan_kernels(bxg_ctx* c, const BatchHdr* hdr, const ScanDesc* desc, ScanScratch sc,
                          uint64_t grid_points, uint32_t nscans, bool any_extra) {
@@ -756,9 +766,16 @@ int enqueue_scan_kernels(bxg_ctx* c, const BatchHdr* hdr, const ScanDesc* desc, 
   BXG_TRY(launch(c, "k_scan_begin", k_scan_begin, 1, kBlock, hdr, desc, sc));
   BXG_TRY(launch(c, "k_scan_classify", k_scan_classify, gp, kBlock, hdr, desc, sc));
   BXG_TRY(launch(c, "k_scan_winners", k_scan_winners, gp, kBlock, hdr, desc, sc));
-  BXG_TRY(launch(c, "k_scan_bucket_reduce", k_scan_bucket_reduce, kTiles, 1024, hdr, sc));
-  BXG_TRY(launch(c, "k_scan_bucket_scan", k_scan_bucket_scan, kTiles, 1024, hdr, sc));
-  BXG_TRY(launch(c, "k_scan_scatter", k_scan_scatter, gp, kBlock, hdr, sc));
+  // a tile of buckets a scan (the scan index mod 64)
+  const uint32_t tiles = (1u << (kDirBits + tag_bits_for(nscans))) / kScanTile;
+  if (tiles == 1) {
+    BXG_TRY(launch(c, "k_scan_scatter", k_scan_scatter<true>, std::max(gp, 1u), kBlock, hdr, sc));
+  } else {
+    if (tiles > kUnreducedTiles)
+      BXG_TRY(launch(c, "k_scan_bucket_reduce", k_scan_bucket_reduce, tiles, 1024, hdr, sc));
+    BXG_TRY(launch(c, "k_scan_bucket_scan", k_scan_bucket_scan, tiles, 1024, hdr, sc));
+    BXG_TRY(launch(c, "k_scan_scatter", k_scan_scatter<false>, gp, kBlock, hdr, sc));
+  }
   BXG_TRY(launch(c, "k_scan_ray_leaves", k_scan_ray_leaves, gl, rb, desc, sc));
   if (any_extra)
     BXG_TRY(launch(c, "k_scan_extra_leaves", k_scan_extra_leaves, nscans, kBlock, hdr, desc));
@@ -768,13 +785,13 @@ int enqueue_scan_kernels(bxg_ctx* c, const BatchHdr* hdr, const ScanDesc* desc, 
     BXG_TRY(launch(c, "k_scan_rays", k_scan_rays<true>, gr, rb, desc, sc));
     if (any_extra)
       BXG_TRY(launch(c, "k_scan_extra_rays", k_scan_extra_rays<true>, nscans, kBlock, hdr, desc));
-    BXG_TRY(launch(c, "k_scan_new_endpoints", k_scan_new_endpoints<true>, gw, kBlock, desc, sc));
+    BXG_TRY(launch(c, "k_scan_new_endpoints", k_scan_new_endpoints<true>, gw, kBlock, hdr, desc, sc));
   } else {
     BXG_TRY(launch(c, "k_scan_fresh_rays", k_scan_fresh_rays<false>, gf, rb, desc, sc));
     BXG_TRY(launch(c, "k_scan_rays", k_scan_rays<false>, gr, rb, desc, sc));
     if (any_extra)
       BXG_TRY(launch(c, "k_scan_extra_rays", k_scan_extra_rays<false>, nscans, kBlock, hdr, desc));
-    BXG_TRY(launch(c, "k_scan_new_endpoints", k_scan_new_endpoints<false>, gw, kBlock, desc, sc));
+    BXG_TRY(launch(c, "k_scan_new_endpoints", k_scan_new_endpoints<false>, gw, kBlock, hdr, desc, sc));
   }
   BXG_TRY(launch(c, "k_scan_new_leaves", k_scan_new_leaves, gm, kBlock, hdr, desc));
   BXG_TRY(launch(c, "k_scan_finalize", k_scan_finalize, 1, kBlock, hdr, desc));
@@ -786,13 +803,6 @@ int reset_scan_stats(bxg_map* m) {
   bxg_ctx* c = m->ctx;
   const uint64_t z[3] = {0, 0, 0};  // stat_rays, stat_ray_updates, stat_ray_visits
   return upload(c, &m->ctr->stat_rays, z, sizeof(z));
-}
-
-// bits of the scan index kept in a winner's bucket
-uint32_t tag_bits_for(uint32_t nscans) {
-  uint32_t b = 0;
-  while (b < kMaxTagBits && (1u << b) < nscans) ++b;
-  return b;
 }
 
 // one wave of scans, each into a different map
@@ -1022,7 +1032,8 @@ constexpr uint64_t kNaOffRec = kNaOffOffs + (uint64_t)kMaxBuckets * 4;
 constexpr uint64_t kNaOffTpos = kNaOffRec + kNaPoints * sizeof(int4);
 constexpr uint64_t kNaOffWinners = kNaOffTpos + kNaPoints * 4;
 constexpr uint64_t kNaOffWkey = kNaOffWinners + kNaPoints * 4;
-constexpr uint64_t kNaOffEp = kNaOffWkey + kNaPoints * 4;
+constexpr uint64_t kNaOffWrank = kNaOffWkey + kNaPoints * 4;
+constexpr uint64_t kNaOffEp = kNaOffWrank + kNaPoints * 4;
 constexpr uint64_t kNaBytes = kNaOffEp + kNaEpSlots * sizeof(EpSlot);
 static_assert(sizeof(BatchHdr) <= kNaOffDesc - kNaOffHdr, "batch header slot");
 static_assert(sizeof(ScanDesc) <= kNaOffCounters - kNaOffDesc, "descriptor slot");
@@ -1064,6 +1075,7 @@ ScanScratch na_layout(uint8_t* base, uint64_t n, uint64_t* ep_slots) {
   sc.tpos = (uint32_t*)(base + kNaOffTpos);
   sc.winners = (uint32_t*)(base + kNaOffWinners);
   sc.wkey = (uint32_t*)(base + kNaOffWkey);
+  sc.wrank = (uint32_t*)(base + kNaOffWrank);
   sc.hist = (uint32_t*)(base + kNaOffHist);
   sc.offs = (uint32_t*)(base + kNaOffOffs);
   sc.counters = (uint32_t*)(base + kNaOffCounters);
@@ -1200,6 +1212,7 @@ int bxg_ctx_destroy(bxg_ctx* c) {
   dfree(c->sc.tpos);
   dfree(c->sc.winners);
   dfree(c->sc.wkey);
+  dfree(c->sc.wrank);
   dfree(c->sc.hist);
   dfree(c->sc.offs);
   dfree(c->sc.ep);
@@ -2187,6 +2200,7 @@ int bxg_graph_create(bxg_ctx* c, uint32_t max_scans, uint64_t max_points, bxg_gr
   if (rc == BXG_OK) rc = dmalloc(c, &p, cap * 4), g->sc.tpos = (uint32_t*)p;
   if (rc == BXG_OK) rc = dmalloc(c, &p, cap * 4), g->sc.winners = (uint32_t*)p;
   if (rc == BXG_OK) rc = dmalloc(c, &p, cap * 4), g->sc.wkey = (uint32_t*)p;
+  if (rc == BXG_OK) rc = dmalloc(c, &p, cap * 4), g->sc.wrank = (uint32_t*)p;
   if (rc == BXG_OK) rc = dmalloc(c, &p, (uint64_t)kMaxBuckets * 4), g->sc.hist = (uint32_t*)p;
   if (rc == BXG_OK) rc = dmalloc(c, &p, (uint64_t)kMaxBuckets * 4), g->sc.offs = (uint32_t*)p;
   if (rc == BXG_OK) rc = fill32(c, g->sc.hist, kMaxBuckets, 0);
@@ -2305,6 +2319,7 @@ int bxg_graph_destroy(bxg_graph* g) {
   dfree(g->sc.tpos);
   dfree(g->sc.winners);
   dfree(g->sc.wkey);
+  dfree(g->sc.wrank);
   dfree(g->sc.hist);
   dfree(g->sc.offs);
   dfree(g->sc.ep);

@@ -178,7 +178,8 @@ static_assert(kEmptyKey == ~0ull && kNone == 0xFFFFFFFFu, "an empty EpSlot is al
 
 struct ScanScratch {
   int4* rec;            // per flattened point: endpoint xyz, flags | scan << 16
-  uint32_t* tpos;       // per point: endpoint-table slot of its endpoint
+  uint32_t* tpos;       // per point: endpoint-table slot of its endpoint; from the scatter on,
+                        // per winner: leaf index of its endpoint if new, kLeafLater or kNone
   EpSlot* ep;           // endpoint table
   uint32_t ep_mask;     // capacity - 1
   uint32_t chunk_max;   // rays a wavefront of the fresh pass walks one batch after the other (64..1024)
@@ -189,8 +190,9 @@ struct ScanScratch {
   uint32_t ray_order;   // winner order (0..5, k_scan_winners): 0 direction only
   uint32_t* winners;    // flattened point indices of per-voxel winners, bucketed
   uint32_t* wkey;       // per point: bucket of a winner, kNone otherwise
+  uint32_t* wrank;      // per winner: its place in its bucket
   uint32_t* hist;       // [kMaxBuckets] winners per bucket (zero between calls)
-  uint32_t* offs;       // [kMaxBuckets] bucket write cursors
+  uint32_t* offs;       // [kMaxBuckets] first place of each bucket (calls of several scans)
   uint32_t* counters;   // kCounterWords words (above)
 };
 

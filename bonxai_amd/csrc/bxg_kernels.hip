@@ -899,24 +899,6 @@ __global__ void __launch_bounds__(256) k_scan_classify(const BatchHdr* __restric
   }
 }
 
-// Lanes of a wavefront that share a key form one group: one atomic add of
-// the group size per group; returns this lane's rank-offset (base + rank).
-__device__ __forceinline__ uint32_t wave_add_by_key(uint32_t* table, uint32_t key, bool pred) {
-  uint64_t pending = __ballot(pred);
-  uint32_t pos = 0;
-  while (pending) {
-    const int leader = __ffsll((unsigned long long)pending) - 1;
-    const uint32_t lk = (uint32_t)__shfl((int)key, leader);
-    const uint64_t same = __ballot(pred && key == lk);
-    uint32_t base = 0;
-    if ((int)lane_id() == leader) base = add32(&table[lk], (uint32_t)__popcll(same));
-    base = (uint32_t)__shfl((int)base, leader);
-    if ((same >> lane_id()) & 1ull) pos = base + (uint32_t)__popcll(same & lanes_below());
-    pending &= ~same;
-  }
-  return pos;
-}
-
 // octahedral direction bin of (dx, dy, dz), 2^b x 2^b bins in Morton order
 // (b = 3..6)
 __device__ __forceinline__ uint32_t dir_bin(int32_t dx, int32_t dy, int32_t dz, uint32_t b) {
@@ -960,7 +942,11 @@ __device__ __forceinline__ RayOrder ray_order(uint32_t k) {
 
 // Phase 2 (per point): the lowest-index point of each claimed voxel is its
 // winner (probabilistic_map.cpp:30-54 lets only the first point of a voxel
-// through the update_id test); winners are counted per bucket.
+// through the update_id test); winners are counted per bucket, and each
+// keeps its place in its bucket, so that k_scan_scatter needs no atomics.
+// The returning atomics of a wavefront are in flight together (one after the
+// other, here and again in the scatter, took 10 + 23 us for 2,001 points, up
+// to 64 round trips; now 8 + 6).
 __global__ void __launch_bounds__(256) k_scan_winners(const BatchHdr* __restrict__ hdr,
                                                       const ScanDesc* __restrict__ sd,
                                                       ScanScratch sc) {
@@ -1009,7 +995,26 @@ __global__ void __launch_bounds__(256) k_scan_winners(const BatchHdr* __restrict
     }
     sc.wkey[gi] = win ? key : kNone;
   }
-  wave_add_by_key(sc.hist, key, win);
+  // the wavefront's lanes of one bucket form a group, so that its rays stay
+  // together in the bucket (groups of neighbouring lanes only: update pass of
+  // 64 maps 4.28 against 3.9 ms, and 350 against 120 us here)
+  uint64_t pending = __ballot(win);
+  uint32_t lead = 0, rank = 0, size = 0;
+  while (pending) {
+    const uint32_t l = (uint32_t)__ffsll((unsigned long long)pending) - 1u;
+    const bool mine = win && key == (uint32_t)__builtin_amdgcn_readlane((int)key, (int)l);
+    const uint64_t same = __ballot(mine);
+    if (mine) {
+      lead = l;
+      rank = (uint32_t)__popcll(same & lanes_below());
+      size = (uint32_t)__popcll(same);
+    }
+    pending &= ~same;
+  }
+  uint32_t base = 0;
+  if (win && lead == lane_id()) base = add32(&sc.hist[key], size);
+  base = (uint32_t)__shfl((int)base, (int)lead);
+  if (win) sc.wrank[gi] = base + rank;
 }
 
 // inclusive prefix sum over the 64 lanes of a wavefront
@@ -1043,9 +1048,14 @@ __global__ void __launch_bounds__(1024) k_scan_bucket_reduce(const BatchHdr* __r
   }
 }
 
+// Calls of up to this many bucket tiles (a scan a tile) have no pass for the
+// tile sums: each tile adds up the earlier ones itself (a launch saved, about
+// 5 us; with more tiles the sums would take longer than the launch).
+constexpr uint32_t kUnreducedTiles = 8;
+
 // Phase 2s' (per bucket tile): exclusive scan of the bucket counts into the
-// bucket write cursors, carried over the earlier tiles; the counts are zeroed
-// for the next call and the last tile writes the winner count to counters[0].
+// buckets' first places, carried over the earlier tiles; the last tile writes
+// the winner count to counters[0].
 __global__ void __launch_bounds__(1024) k_scan_bucket_scan(const BatchHdr* __restrict__ hdr,
                                                            ScanScratch sc) {
   __shared__ uint32_t wsum[16];
@@ -1054,18 +1064,25 @@ __global__ void __launch_bounds__(1024) k_scan_bucket_scan(const BatchHdr* __res
   const uint32_t base = blockIdx.x * kScanTile;
   if (base >= nb) return;
   const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
-  if (wid == 0) {
+  const bool reduced = gridDim.x > kUnreducedTiles;
+  uint32_t sum = 0;  // this thread's part of the earlier tiles
+  if (reduced) {
     // blockIdx.x < kTiles <= 64: one lane per earlier tile
-    const uint32_t t = lane < blockIdx.x ? sc.counters[kTileWords + lane] : 0u;
-    const uint32_t tot = (uint32_t)__shfl((int)wave_scan(t), 63);
-    if (lane == 0) carry = tot;
+    if (threadIdx.x < blockIdx.x) sum = sc.counters[kTileWords + threadIdx.x];
+  } else {
+    for (uint32_t t = 0; t < blockIdx.x; ++t) {
+      const uint4 e = reinterpret_cast<const uint4*>(sc.hist + t * kScanTile)[threadIdx.x];
+      sum += e.x + e.y + e.z + e.w;
+    }
   }
-  uint4* h4 = reinterpret_cast<uint4*>(sc.hist + base);
-  const uint4 v = h4[threadIdx.x];
+  if (threadIdx.x == 0) carry = 0;
+  const uint4 v = reinterpret_cast<const uint4*>(sc.hist + base)[threadIdx.x];
   const uint32_t s = v.x + v.y + v.z + v.w;
   const uint32_t incl = wave_scan(s);
   if (lane == 63) wsum[wid] = incl;
+  sum = wave_scan(sum);
   __syncthreads();
+  if (lane == 63 && sum) atomicAdd(&carry, sum);
   if (wid == 0) {
     const uint32_t w = lane < 16u ? wsum[lane] : 0u;
     const uint32_t wi = wave_scan(w);
@@ -1079,7 +1096,6 @@ __global__ void __launch_bounds__(1024) k_scan_bucket_scan(const BatchHdr* __res
   o.z = run; run += v.z;
   o.w = run;
   reinterpret_cast<uint4*>(sc.offs + base)[threadIdx.x] = o;
-  h4[threadIdx.x] = make_uint4(0u, 0u, 0u, 0u);
   // the fresh scans' winners start at bucket split << kDirBits (a tile's
   // first bucket: kScanTile divides 2^kDirBits); with no fresh scan, at the end
   const uint32_t split = sc.counters[kFreshWords + 2];
@@ -1090,15 +1106,61 @@ __global__ void __launch_bounds__(1024) k_scan_bucket_scan(const BatchHdr* __res
   }
 }
 
-// Phase 2t (per point): winners written into their buckets.
+constexpr uint32_t kLeafLater = 0xFFFFFFFEu;  // tpos: look the endpoint's leaf up after the fresh pass
+
+// Phase 2t (per point): winners written into their buckets, and their
+// endpoint-table slots released (every point has read its slot by now).
+// kOne: a call of one scan (one tile of buckets), whose workgroups each scan
+// the 4096 bucket counts themselves, in LDS: no passes for the bucket sums.
+template <bool kOne>
 __global__ void __launch_bounds__(256) k_scan_scatter(const BatchHdr* __restrict__ hdr,
                                                       ScanScratch sc) {
+  __shared__ uint32_t first[kOne ? kScanTile : 1];
+  __shared__ uint32_t wsum[4];
   const uint64_t gi = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  uint32_t key = kNone;
-  if (gi < hdr->total) key = sc.wkey[gi];
-  const bool win = key != kNone;
-  const uint32_t pos = wave_add_by_key(sc.offs, win ? key : 0u, win);
-  if (win) sc.winners[pos] = (uint32_t)gi;
+  const uint32_t key = gi < hdr->total ? sc.wkey[gi] : kNone;
+  const uint32_t rank = key != kNone ? sc.wrank[gi] : 0u;
+  const uint32_t t = key != kNone ? sc.tpos[gi] : 0u;
+  if (kOne) {
+    const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
+    constexpr uint32_t kPer = kScanTile / 256 / 4;  // uint4s a thread
+    const uint4* h = reinterpret_cast<const uint4*>(sc.hist) + threadIdx.x * kPer;
+    uint4 v[kPer];
+    uint32_t s = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+      v[k] = h[k];
+      s += v[k].x + v[k].y + v[k].z + v[k].w;
+    }
+    const uint32_t incl = wave_scan(s);
+    if (lane == 63) wsum[wid] = incl;
+    __syncthreads();
+    uint32_t run = incl - s;
+    for (uint32_t w = 0; w < wid; ++w) run += wsum[w];
+    uint4* f = reinterpret_cast<uint4*>(first) + threadIdx.x * kPer;
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+      uint4 o;
+      o.x = run; run += v[k].x;
+      o.y = run; run += v[k].y;
+      o.z = run; run += v[k].z;
+      o.w = run; run += v[k].w;
+      f[k] = o;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 255) {
+      sc.counters[0] = run;
+      // the one scan's winners are all the fresh pass's (split 0) or none
+      if (sc.counters[kFreshWords + 2] != kNone)
+        sc.counters[kFreshWords + 3] = sc.counters[kFreshWords + 2] == 0u ? 0u : run;
+    }
+    __syncthreads();
+  }
+  if (key == kNone) return;
+  sc.winners[(kOne ? first[key] : sc.offs[key]) + rank] = (uint32_t)gi;
+  EpSlot BXG_G* e = gp(&sc.ep[t]);
+  e->key = kEmptyKey;
+  e->first = kNone;
+  sc.tpos[gi] = kLeafLater;
 }
 
 // The passes over the winners' rays (walk_winners).
@@ -1318,16 +1380,18 @@ __global__ void __launch_bounds__(256) k_scan_extra_leaves(const BatchHdr* __res
   }
 }
 
-constexpr uint32_t kLeafLater = 0xFFFFFFFEu;  // tpos: look the endpoint's leaf up after the fresh pass
-
-// Phase 3 (per winner): endpoint hit/miss update (probabilistic_map.cpp:30-54)
-// of the endpoints in leaves that existed before the scan, and release of
-// the endpoint-table slot.  One writer per endpoint cell.  An endpoint in a
-// leaf the scan created is left for k_scan_new_endpoints (after the ray
-// pass): its leaf index goes to tpos.
+// Phase 3 (per winner of a map not empty at the scan's start): endpoint
+// hit/miss update (probabilistic_map.cpp:30-54) of the endpoints in leaves
+// that existed before the scan.  One writer per endpoint cell.  An endpoint
+// in a leaf the scan created is left for k_scan_new_endpoints (after the ray
+// pass): its leaf index goes to tpos.  In a map empty at the scan's start
+// every endpoint leaf is new: the fresh pass, which runs after this kernel,
+// creates it and stores its index in tpos (kLeafLater until then:
+// k_scan_new_endpoints looks up any it did not), so there is nothing to do.
 __global__ void __launch_bounds__(256) k_scan_endpoints(const ScanDesc* __restrict__ sd,
                                                         ScanScratch sc) {
-  const uint32_t nwin = sc.counters[0];
+  // with a split the fresh scans' winners end the list
+  const uint32_t nwin = sc.counters[kFreshWords + 2] != kNone ? sc.counters[kFreshWords + 3] : sc.counters[0];
   const uint32_t stride = gridDim.x * blockDim.x;
   const uint32_t start = blockIdx.x * blockDim.x + threadIdx.x;
   // every lane runs the same number of iterations so the count reduction
@@ -1339,18 +1403,10 @@ __global__ void __launch_bounds__(256) k_scan_endpoints(const ScanDesc* __restri
     if (idx < nwin) {
       const uint32_t gi = sc.winners[idx];
       const int4 r = sc.rec[gi];
-      const uint32_t t = sc.tpos[gi];
-      EpSlot BXG_G* e = gp(&sc.ep[t]);
-      e->key = kEmptyKey;
-      e->first = kNone;
       const ScanDesc& d = sd[(uint32_t)r.w >> 16];
       const MapView m = load_view(d.map);
       const bool failed = (map_status(m) & kFatal) != 0;
       const uint32_t lbase = *gp(&m.ctr->leaf_base);
-      // in a map empty at the scan's start every endpoint leaf is new: the
-      // fresh pass, which runs after this kernel, creates it and stores its
-      // index here (k_scan_new_endpoints looks up any it did not), so there
-      // is nothing to look up now
       const uint32_t leaf = (failed || lbase == 0) ? kNone : find_leaf(m, r.x, r.y, r.z);
       const bool fresh = leaf != kNone && leaf >= lbase;
       sc.tpos[gi] = fresh ? leaf : (lbase == 0 && !failed ? kLeafLater : kNone);
@@ -1387,12 +1443,17 @@ __global__ void __launch_bounds__(256) k_scan_endpoints(const ScanDesc* __restri
 // voxel, and k_scan_new_leaves writes the word.  The counted form takes back
 // the ray update the ray pass counted for a cell that turns out to be an
 // endpoint.
+// It also zeroes the bucket counts for the next call.
 template <bool kCount>
-__global__ void __launch_bounds__(256) k_scan_new_endpoints(const ScanDesc* __restrict__ sd,
+__global__ void __launch_bounds__(256) k_scan_new_endpoints(const BatchHdr* __restrict__ hdr,
+                                                            const ScanDesc* __restrict__ sd,
                                                             ScanScratch sc) {
   const uint32_t nwin = sc.counters[0];
   const uint32_t stride = gridDim.x * blockDim.x;
   const uint32_t start = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t nb4 = (1u << (kDirBits + hdr->tag_bits)) / 4;
+  for (uint32_t i = start; i < nb4; i += stride)
+    reinterpret_cast<uint4*>(sc.hist)[i] = make_uint4(0u, 0u, 0u, 0u);
   for (uint32_t base = start - (start & 63u); base < nwin; base += stride) {
     const uint32_t idx = base + (start & 63u);
     uint32_t updated = 0, retracted = 0;

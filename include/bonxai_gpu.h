@@ -265,7 +265,7 @@ int bxg_insert_point_cloud_tf_host(bxg_map* map, const float* points, uint64_t n
  * reference: it is for callers that cannot allocate device memory (code that
  * must not call hipMalloc, such as a tight serving loop or a harness that
  * forbids it).  Same scan and results, but the call's scratch is a static
- * device buffer of the library (32 MiB on each GPU it runs on, held
+ * device buffer of the library (34 MiB on each GPU it runs on, held
  * until the process ends) for at most BXG_NOALLOC_MAX_POINTS points, and the
  * map's pools are used as reserved (bxg_map_reserve): nothing is allocated
  * or grown.  Blocks until the scan is done.  Returns BXG_ERR_INVALID_ARG for

@@ -71,3 +71,10 @@ def test_long_rays(ctx, cells):
     """Rays of about 2^15 cells: closed forms in 32 and in 64 bits."""
     p = np.array([[cells, 7, -3], [-cells, cells - 5, 11], [100, -cells, cells]], np.float32) * np.float32(0.1)
     _check(ctx, [p + np.float32(0.05)], 0.1, 1e6, "long rays")
+
+
+@pytest.mark.parametrize("nscans", [2, 8, 9])
+def test_bucket_tiles(ctx, nscans):
+    """Calls of several scans around the number of bucket tiles up to which
+    the bucket scan sums the earlier tiles itself."""
+    _check(ctx, [_sphere(300 + 37 * k, 4.0 + k, k) for k in range(nscans)], 0.1, 8.0, f"{nscans} scans")
