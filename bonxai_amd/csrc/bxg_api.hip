@@ -537,6 +537,10 @@ int ensure_room(bxg_map* m, uint64_t leaves, uint64_t roots) {
 
 // ----------------------------------------------------------- scratch
 
+// a batch's descriptors follow its header, kDescOffset bytes on
+constexpr uint64_t kDescOffset = 256;
+ScanDesc* descs_of(BatchHdr* hdr) { return (ScanDesc*)((uint8_t*)hdr + kDescOffset); }
+
 int ensure_scan_scratch(bxg_ctx* c, uint64_t points, uint32_t nscans) {
   if (points > c->scan_cap) {
     BXG_TRY(ctx_sync(c));
@@ -581,12 +585,14 @@ int ensure_scan_scratch(bxg_ctx* c, uint64_t points, uint32_t nscans) {
   c->sc.counters = c->d_counters;
   if (nscans > c->desc_cap) {
     BXG_TRY(ctx_sync(c));
-    dfree(c->d_desc);
-    c->d_desc = nullptr;
+    dfree(c->d_hdr);
+    c->d_hdr = nullptr;
+    c->desc_cap = 0;
     const uint32_t cap = (uint32_t)pow2_at_least(std::max<uint32_t>(nscans, 64));
     void* p;
-    BXG_TRY(dmalloc(c, &p, (uint64_t)cap * sizeof(ScanDesc)));
-    c->d_desc = (ScanDesc*)p;
+    BXG_TRY(dmalloc(c, &p, kDescOffset + (uint64_t)cap * sizeof(ScanDesc)));
+    c->d_hdr = (BatchHdr*)p;
+    c->d_desc = descs_of(c->d_hdr);
     c->desc_cap = cap;
   }
   return BXG_OK;
@@ -734,9 +740,27 @@ uint32_t tag_bits_for(uint32_t nscans) {
   return b;
 }
 
-// the kernel sequence of one wave of scans on given scratch/descriptors
-int enqueue_scan_kernels(bxg_ctx* c, const BatchHdr* hdr, const ScanDesc* desc, ScanScratch sc,
-                         uint64_t grid_points, uint32_t nscans, bool any_extra) {
+// What the host knows about a call's maps: every one empty (no leaf, no work
+// on it under way), every one not empty (a map's leaf count only falls in
+// clear and release_unused, which the host runs), or neither.
+enum class Maps { kMixed, kEmpty, kFilled };
+
+// the first kernel of a call, with its scans as arguments: writes hdr and desc
+template <uint32_t kN>
+int begin_args(bxg_ctx* c, const BatchHdr& h, const ScanDesc* scans, BatchHdr* hdr, ScanDesc* desc,
+               const ScanScratch& sc, bool reset_stats) {
+  ScanArgs<kN> a{};
+  std::copy(scans, scans + h.nscans, a.d);
+  return launch(c, "k_scan_begin", k_scan_begin_args<kN>, 1, kBlock, h, a, hdr, desc, sc,
+                reset_stats ? 1u : 0u);
+}
+
+// The kernel sequence of one wave of scans on given scratch and descriptors.
+// args: the batch's header and descriptors (at most kMostArgs), which the
+// first kernel writes to hdr and desc; null where they are there already.
+int enqueue_scan_kernels(bxg_ctx* c, BatchHdr* hdr, ScanDesc* desc, ScanScratch sc, uint64_t grid_points,
+                         uint32_t nscans, bool any_extra, Maps maps = Maps::kMixed,
+                         const BatchHdr* args_hdr = nullptr, const ScanDesc* args = nullptr) {
   const uint32_t gp = nblocks(grid_points);
   const uint32_t gw = std::max<uint32_t>(1, std::min<uint32_t>(gp, 16384));
   // the passes over the rays: a wavefront a batch of 64 winners (at most one
@@ -763,7 +787,17 @@ int enqueue_scan_kernels(bxg_ctx* c, const BatchHdr* hdr, const ScanDesc* desc, 
   sc.ray_order = c->ray_order;
   // new-leaf pass: a wavefront per new leaf, grid-stride over them
   const uint32_t gm = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(cus * 8, gp));
-  BXG_TRY(launch(c, "k_scan_begin", k_scan_begin, 1, kBlock, hdr, desc, sc));
+  // the passes that have nothing to do in such maps are not launched (about 5
+  // us each): the fresh pass in filled maps; the leaf, endpoint and update
+  // passes in empty ones, which the fresh pass walks
+  const bool fresh = maps != Maps::kFilled;
+  const bool old = maps != Maps::kEmpty || !c->fresh_pass;
+  if (!args)
+    BXG_TRY(launch(c, "k_scan_begin", k_scan_begin, 1, kBlock, hdr, desc, sc));
+  else if (nscans == 1)
+    BXG_TRY(begin_args<1>(c, *args_hdr, args, hdr, desc, sc, c->counting));
+  else
+    BXG_TRY(begin_args<kMostArgs>(c, *args_hdr, args, hdr, desc, sc, c->counting));
   BXG_TRY(launch(c, "k_scan_classify", k_scan_classify, gp, kBlock, hdr, desc, sc));
   BXG_TRY(launch(c, "k_scan_winners", k_scan_winners, gp, kBlock, hdr, desc, sc));
   // a tile of buckets a scan (the scan index mod 64)
@@ -776,19 +810,19 @@ int enqueue_scan_kernels(bxg_ctx* c, const BatchHdr* hdr, const ScanDesc* desc, 
     BXG_TRY(launch(c, "k_scan_bucket_scan", k_scan_bucket_scan, tiles, 1024, hdr, sc));
     BXG_TRY(launch(c, "k_scan_scatter", k_scan_scatter<false>, gp, kBlock, hdr, sc));
   }
-  BXG_TRY(launch(c, "k_scan_ray_leaves", k_scan_ray_leaves, gl, rb, desc, sc));
+  if (old) BXG_TRY(launch(c, "k_scan_ray_leaves", k_scan_ray_leaves, gl, rb, desc, sc));
   if (any_extra)
     BXG_TRY(launch(c, "k_scan_extra_leaves", k_scan_extra_leaves, nscans, kBlock, hdr, desc));
-  BXG_TRY(launch(c, "k_scan_endpoints", k_scan_endpoints, gw, kBlock, desc, sc));
+  if (old) BXG_TRY(launch(c, "k_scan_endpoints", k_scan_endpoints, gw, kBlock, desc, sc));
   if (c->counting) {
-    BXG_TRY(launch(c, "k_scan_fresh_rays", k_scan_fresh_rays<true>, gf, rb, desc, sc));
-    BXG_TRY(launch(c, "k_scan_rays", k_scan_rays<true>, gr, rb, desc, sc));
+    if (fresh) BXG_TRY(launch(c, "k_scan_fresh_rays", k_scan_fresh_rays<true>, gf, rb, desc, sc));
+    if (old) BXG_TRY(launch(c, "k_scan_rays", k_scan_rays<true>, gr, rb, desc, sc));
     if (any_extra)
       BXG_TRY(launch(c, "k_scan_extra_rays", k_scan_extra_rays<true>, nscans, kBlock, hdr, desc));
     BXG_TRY(launch(c, "k_scan_new_endpoints", k_scan_new_endpoints<true>, gw, kBlock, hdr, desc, sc));
   } else {
-    BXG_TRY(launch(c, "k_scan_fresh_rays", k_scan_fresh_rays<false>, gf, rb, desc, sc));
-    BXG_TRY(launch(c, "k_scan_rays", k_scan_rays<false>, gr, rb, desc, sc));
+    if (fresh) BXG_TRY(launch(c, "k_scan_fresh_rays", k_scan_fresh_rays<false>, gf, rb, desc, sc));
+    if (old) BXG_TRY(launch(c, "k_scan_rays", k_scan_rays<false>, gr, rb, desc, sc));
     if (any_extra)
       BXG_TRY(launch(c, "k_scan_extra_rays", k_scan_extra_rays<false>, nscans, kBlock, hdr, desc));
     BXG_TRY(launch(c, "k_scan_new_endpoints", k_scan_new_endpoints<false>, gw, kBlock, hdr, desc, sc));
@@ -805,12 +839,22 @@ int reset_scan_stats(bxg_map* m) {
   return upload(c, &m->ctr->stat_rays, z, sizeof(z));
 }
 
+// a batch's header and descriptors in one copy
+int upload_scans(bxg_ctx* c, BatchHdr* dst, const BatchHdr& hdr, const std::vector<ScanDesc>& descs) {
+  std::vector<uint8_t> both(kDescOffset + descs.size() * sizeof(ScanDesc));
+  std::memcpy(both.data(), &hdr, sizeof(hdr));
+  if (!descs.empty()) std::memcpy(both.data() + kDescOffset, descs.data(), descs.size() * sizeof(ScanDesc));
+  return upload(c, dst, both.data(), both.size());
+}
+
 // one wave of scans, each into a different map
 int run_wave(bxg_ctx* c, const bxg_scan_desc* scans, uint32_t nscans, uint32_t extra_flags) {
   std::vector<ScanDesc> descs;
   uint64_t total = 0;
   BXG_TRY(build_descs(c, scans, nscans, extra_flags, descs, &total));
   bool any_extra = false;
+  uint32_t empty = 0, filled = 0;
+  const bool as_args = nscans <= kMostArgs;
   for (uint32_t s = 0; s < nscans; ++s) {
     bxg_map* m = scans[s].map;
     // head-room for a scan: about one new leaf per point covers a first
@@ -822,15 +866,20 @@ int run_wave(bxg_ctx* c, const bxg_scan_desc* scans, uint32_t nscans, uint32_t e
       BXG_TRY(upload_extra(m));
       descs[s].extra = m->d_extra;
     }
-    if (c->counting) BXG_TRY(reset_scan_stats(m));
+    if (m->known_leaves)
+      ++filled;
+    else if (!m->ctr_pending && m->pending.empty())
+      ++empty;
+    if (c->counting && !as_args) BXG_TRY(reset_scan_stats(m));
   }
+  const Maps state = filled == nscans ? Maps::kFilled : (empty == nscans ? Maps::kEmpty : Maps::kMixed);
   // the maps may have grown: descriptors point at device headers, which
   // stay put, so nothing to rebuild
   BXG_TRY(ensure_scan_scratch(c, std::max<uint64_t>(total, 1), nscans));
   BatchHdr hdr{nscans, tag_bits_for(nscans), total};
-  BXG_TRY(upload(c, c->d_desc, descs.data(), descs.size() * sizeof(ScanDesc)));
-  BXG_TRY(upload(c, c->d_hdr, &hdr, sizeof(hdr)));
-  BXG_TRY(enqueue_scan_kernels(c, c->d_hdr, c->d_desc, c->sc, total, nscans, any_extra));
+  if (!as_args) BXG_TRY(upload_scans(c, c->d_hdr, hdr, descs));
+  BXG_TRY(enqueue_scan_kernels(c, c->d_hdr, c->d_desc, c->sc, total, nscans, any_extra, state,
+                               as_args ? &hdr : nullptr, as_args ? descs.data() : nullptr));
   // k_scan_finalize wrote every map's counters to its host mirror
   std::vector<bxg_map*> maps(nscans);
   for (uint32_t s = 0; s < nscans; ++s) maps[s] = scans[s].map;
@@ -1124,9 +1173,7 @@ int insert_noalloc(bxg_map* m, const bxg_scan_desc& in) {
   BXG_TRY(fill64(c, (uint64_t*)sc.ep, slots * 2, ~0ull));
   BXG_TRY(fill32(c, sc.hist, kMaxBuckets, 0));
   BXG_TRY(fill32(c, sc.counters, kCounterWords, 0));
-  BXG_TRY(launch(c, "k_na_setup", k_na_setup, 1, 64, hdr, d, d_hdr, d_desc, m->ctr,
-                 c->counting ? 1u : 0u));
-  BXG_TRY(enqueue_scan_kernels(c, d_hdr, d_desc, sc, in.n, 1, false));
+  BXG_TRY(enqueue_scan_kernels(c, d_hdr, d_desc, sc, in.n, 1, false, Maps::kMixed, &hdr, &d));
   BXG_TRY(read_counters(m));  // waits for the scan
   const uint32_t st = m->h_ctr->status;
   if (st & ~overflow) return map_status(m);
@@ -1184,8 +1231,6 @@ int bxg_ctx_create(int device, uint64_t budget_bytes, bxg_ctx** out) {
   if (rc == BXG_OK) rc = dmalloc(c, &p, kCounterWords * 4);
   c->d_counters = (uint32_t*)p;
   if (rc == BXG_OK) rc = dmalloc(c, &p, 64);
-  c->d_hdr = (BatchHdr*)p;
-  if (rc == BXG_OK) rc = dmalloc(c, &p, 64);
   c->d_small = (uint64_t*)p;
   if (rc == BXG_OK && hipHostMalloc((void**)&c->h_small, 64, hipHostMallocDefault) != hipSuccess)
     rc = BXG_ERR_HIP;
@@ -1217,7 +1262,6 @@ int bxg_ctx_destroy(bxg_ctx* c) {
   dfree(c->sc.offs);
   dfree(c->sc.ep);
   dfree(c->d_counters);
-  dfree(c->d_desc);
   dfree(c->d_hdr);
   dfree(c->op_slots);
   dfree(c->op_tpos);
@@ -2206,8 +2250,8 @@ int bxg_graph_create(bxg_ctx* c, uint32_t max_scans, uint64_t max_points, bxg_gr
   if (rc == BXG_OK) rc = fill32(c, g->sc.hist, kMaxBuckets, 0);
   if (rc == BXG_OK) rc = dmalloc(c, &p, tcap * sizeof(EpSlot)), g->sc.ep = (EpSlot*)p;
   if (rc == BXG_OK) rc = dmalloc(c, &p, kCounterWords * 4), g->d_counters = (uint32_t*)p;
-  if (rc == BXG_OK) rc = dmalloc(c, &p, (uint64_t)max_scans * sizeof(ScanDesc)), g->d_desc = (ScanDesc*)p;
-  if (rc == BXG_OK) rc = dmalloc(c, &p, sizeof(BatchHdr)), g->d_hdr = (BatchHdr*)p;
+  if (rc == BXG_OK) rc = dmalloc(c, &p, kDescOffset + (uint64_t)max_scans * sizeof(ScanDesc)), g->d_hdr = (BatchHdr*)p;
+  if (rc == BXG_OK) g->d_desc = descs_of(g->d_hdr);
   g->sc.ep_mask = (uint32_t)(tcap - 1);
   g->sc.counters = g->d_counters;
   if (rc == BXG_OK) rc = fill64(c, (uint64_t*)g->sc.ep, tcap * 2, ~0ull);  // empty: all ones
@@ -2268,8 +2312,7 @@ int bxg_graph_set_scans(bxg_graph* g, const bxg_scan_desc* scans, uint32_t nscan
     maps.push_back(m);
   }
   BatchHdr hdr{nscans, tag_bits_for(nscans), total};
-  BXG_TRY(upload(c, g->d_desc, descs.data(), descs.size() * sizeof(ScanDesc)));
-  BXG_TRY(upload(c, g->d_hdr, &hdr, sizeof(hdr)));
+  BXG_TRY(upload_scans(c, g->d_hdr, hdr, descs));
   g->maps = maps;
   g->npoints.clear();
   g->ranges.clear();
@@ -2324,7 +2367,6 @@ int bxg_graph_destroy(bxg_graph* g) {
   dfree(g->sc.offs);
   dfree(g->sc.ep);
   dfree(g->d_counters);
-  dfree(g->d_desc);
   dfree(g->d_hdr);
   delete g;
   return BXG_OK;

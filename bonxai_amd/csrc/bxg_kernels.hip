@@ -1637,22 +1637,6 @@ __global__ void __launch_bounds__(256) k_scan_new_leaves(const BatchHdr* __restr
   }
 }
 
-// Allocation-free scans (bxg_insert_point_cloud_noalloc): the batch header
-// and the one scan descriptor, passed by value, are written into the
-// caller-side scratch; a counted call also clears the map's scan statistics.
-__global__ void k_na_setup(BatchHdr hdr, ScanDesc desc, BatchHdr* __restrict__ hdr_out,
-                           ScanDesc* __restrict__ desc_out, MapCounters* __restrict__ ctr,
-                           uint32_t reset_stats) {
-  if (threadIdx.x != 0) return;
-  *hdr_out = hdr;
-  *desc_out = desc;
-  if (reset_stats) {
-    ctr->stat_rays = 0;
-    ctr->stat_ray_updates = 0;
-    ctr->stat_ray_visits = 0;
-  }
-}
-
 // After a scan that ran out of nodes (it wrote no cell): the overflow bits
 // are cleared and the bump counter, which ran past the pool, comes back to
 // the pool's size.  The leaves allocated below it stay, every cell off.
@@ -1667,13 +1651,12 @@ __global__ void k_na_recover(MapCounters* __restrict__ ctr, uint32_t leaf_cap) {
 // With the fresh pass, also the scans whose map is empty (their winners get
 // the highest bucket tags: the fresh pass walks the end of the list, the
 // other passes the rest).
-__global__ void k_scan_begin(const BatchHdr* __restrict__ hdr, const ScanDesc* __restrict__ sd,
-                             ScanScratch sc) {
-  const uint32_t nscans = hdr->nscans;
+template <class Desc>
+__device__ __forceinline__ void scan_begin(uint32_t nscans, const Desc* sd, const ScanScratch& sc) {
   for (uint32_t s = threadIdx.x; s < nscans; s += blockDim.x) {
-    const MapView m = load_view(sd[s].map);
-    MapCounters BXG_G* ctr = gp(m.ctr);
-    const uint32_t base = min(ctr->leaf_count, m.leaf_cap);
+    const MapDev BXG_G* m = gp((const MapDev*)sd[s].map);
+    MapCounters BXG_G* ctr = gp(m->ctr);
+    const uint32_t base = min(ctr->leaf_count, m->leaf_cap);
     ctr->leaf_base = base;
     if (nscans <= 64u) {  // the first wavefront holds every scan
       const uint64_t fresh = __ballot(sc.fresh_pass && base == 0);
@@ -1686,6 +1669,39 @@ __global__ void k_scan_begin(const BatchHdr* __restrict__ hdr, const ScanDesc* _
   }
   if ((nscans > 64u || nscans == 0u) && threadIdx.x == 0) sc.counters[kFreshWords + 2] = kNone;
   if (threadIdx.x < 64u) sc.counters[kClipWords + threadIdx.x] = 0;
+}
+__global__ void k_scan_begin(const BatchHdr* __restrict__ hdr, const ScanDesc* __restrict__ sd,
+                             ScanScratch sc) {
+  scan_begin(hdr->nscans, sd, sc);
+}
+
+// The same for a call whose batch header and up to kN scan descriptors come
+// as kernel arguments, written here into the device buffers that the later
+// kernels read: no copy to the device before the call (two small copies and
+// the waits around them cost about 35 us at the head of a call).  kN 16 fits
+// the 4 KB of a launch's arguments.  With reset_stats (counted calls) the
+// maps' scan statistics are cleared.
+template <uint32_t kN>
+struct ScanArgs {
+  ScanDesc d[kN];
+};
+constexpr uint32_t kMostArgs = 16;
+static_assert(sizeof(ScanArgs<kMostArgs>) + sizeof(ScanScratch) + 64 <= 4096, "kernel arguments");
+template <uint32_t kN>
+__global__ void k_scan_begin_args(BatchHdr hdr, ScanArgs<kN> a, BatchHdr* __restrict__ hdr_out,
+                                  ScanDesc* __restrict__ desc_out, ScanScratch sc, uint32_t reset_stats) {
+  if (threadIdx.x == 0) *hdr_out = hdr;
+  const uint32_t* src = reinterpret_cast<const uint32_t*>(&a);
+  uint32_t* dst = reinterpret_cast<uint32_t*>(desc_out);
+  const uint32_t words = hdr.nscans * (uint32_t)(sizeof(ScanDesc) / 4);
+  for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) dst[i] = src[i];
+  if (reset_stats && threadIdx.x < hdr.nscans) {
+    MapCounters* ctr = gp((const MapDev*)a.d[threadIdx.x].map)->ctr;
+    ctr->stat_rays = 0;
+    ctr->stat_ray_updates = 0;
+    ctr->stat_ray_visits = 0;
+  }
+  scan_begin(hdr.nscans, a.d, sc);
 }
 
 // Phase 5 (per scan): advance update_count 1 -> 2 -> 3 -> 1

@@ -78,3 +78,58 @@ def test_bucket_tiles(ctx, nscans):
     """Calls of several scans around the number of bucket tiles up to which
     the bucket scan sums the earlier tiles itself."""
     _check(ctx, [_sphere(300 + 37 * k, 4.0 + k, k) for k in range(nscans)], 0.1, 8.0, f"{nscans} scans")
+
+
+@pytest.mark.parametrize("nscans", [16, 17])
+def test_scans_as_arguments(ctx, nscans):
+    """Descriptors passed as kernel arguments (up to 16 scans) and copied."""
+    _check(ctx, [_sphere(100 + 11 * k, 3.0 + 0.2 * k, k) for k in range(nscans)], 0.1, 8.0, f"{nscans} scans")
+
+
+@pytest.mark.parametrize("fresh_pass", [1, 0])
+def test_passes_left_out(fresh_pass):
+    """Maps the host knows to be empty, filled, or neither (an asynchronous
+    insert under way), alone and together in one call, before and after a
+    clear, and with rays due from addHitPoint."""
+    import bonxai_amd as bx
+    import oracle
+    c = bx.Context(0)
+    c.set_tuning("fresh_pass", fresh_pass)
+    pts = [_sphere(2_000, 6.0 + k, k) for k in range(3)]
+    dev = [c.to_device(p) for p in pts]
+    o = np.array([0.1, 0.2, 0.3])
+    m, om = bx.ProbabilisticMap(c, 0.1), oracle.ProbMap(0.1)
+    for rep in range(2):
+        for d, p in zip(dev, pts):  # empty, then under way, then filled
+            m.insert_point_cloud(d, o, 9.0, sync=False)
+            om.insert_point_cloud(p, o, 9.0)
+        assert m.sync() == 0
+        assert_same_cells(m.cells(), om.cells(), f"asynchronous, round {rep}")
+        m.insert_point_cloud(dev[0], o, 9.0)
+        om.insert_point_cloud(pts[0], o, 9.0)
+        assert_same_cells(m.cells(), om.cells(), f"filled, round {rep}")
+        m.clear()
+        om.close()
+        om = oracle.ProbMap(0.1)
+        m.update_count = 1
+    # one call over an empty, a filled and a cleared map
+    others = [bx.ProbabilisticMap(c, 0.1) for _ in range(2)]
+    models = [om, oracle.ProbMap(0.1), oracle.ProbMap(0.1)]
+    others[0].insert_point_cloud(dev[1], o, 9.0)
+    models[1].insert_point_cloud(pts[1], o, 9.0)
+    maps = [m] + others
+    bx.insert_batch(c, [(x, dev[2], o, 9.0) for x in maps])
+    for x, model in zip(maps, models):
+        model.insert_point_cloud(pts[2], o, 9.0)
+        assert_same_cells(x.cells(), model.cells(), "one call")
+    # rays due into an empty map
+    e, oe = bx.ProbabilisticMap(c, 0.1), oracle.ProbMap(0.1)
+    for x in ([1.0, 2.0, 0.5], [-3.0, 0.2, 1.1]):
+        e.add_hit_point(x)
+        oe.add_hit_point(x)
+    e.insert_point_cloud(pts[0], o, 9.0)
+    oe.insert_point_cloud(pts[0], o, 9.0)
+    assert_same_cells(e.cells(), oe.cells(), "rays due")
+    for x in maps + models + [e, oe]:
+        x.close()
+    c.close()
