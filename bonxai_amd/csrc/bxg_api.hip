@@ -138,6 +138,7 @@ struct bxg_map {
   uint64_t known_roots = 0;
   uint64_t known_scans = 0;
   uint64_t max_leaf_growth = 0;  // largest leaf-count increase seen between snapshots
+  bool cleared = false;  // a clear may still run on the context's stream (other streams wait for it)
   int4* d_extra = nullptr;  // rays due from addHit/MissPoint
   uint32_t extra_cap = 0;
   std::vector<int4> extra;
@@ -376,7 +377,22 @@ void take_counters(bxg_map* m) {
   m->known_scans = m->h_ctr->scans_applied;
 }
 
-// read the device counters of a map (blocking)
+// The counters of a map as its enqueued work leaves them, from the host
+// mirror: every call that changes them ends with a copy into the mirror (a
+// scan's last kernel writes it, the others enqueue one) and an event, waited
+// for here; the host's own changes go to the mirror too.  No copy of its own:
+// a blocking copy cost about 20 us a map, 64 of them a frame's read-back.
+int landed_counters(bxg_map* m) {
+  if (m->ctr_pending) {
+    BXG_HIP(m->ctx, hipEventSynchronize(m->snap->e));
+    m->ctr_pending = false;
+    m->snap.reset();
+  }
+  take_counters(m);
+  return BXG_OK;
+}
+
+// copy the device counters of a map to the mirror (waits for the stream)
 int read_counters(bxg_map* m) {
   bxg_ctx* c = m->ctx;
   BXG_HIP(c, hipMemcpyAsync(m->h_ctr, m->ctr, sizeof(MapCounters), hipMemcpyDeviceToHost, c->stream));
@@ -468,6 +484,7 @@ int grow_leaves(bxg_map* m, uint64_t need) {
   BXG_HIP(c, hipMemcpyAsync(&m->ctr->leaf_count, &lc, 4, hipMemcpyHostToDevice, c->stream));
   BXG_TRY(ctx_sync(c));
   m->known_leaves = used;
+  m->h_ctr->leaf_count = lc;
   return push_header(m);
 }
 
@@ -910,7 +927,7 @@ int status_code(uint32_t st) {
 }
 
 int map_status(bxg_map* m) {
-  BXG_TRY(read_counters(m));
+  BXG_TRY(landed_counters(m));
   const uint32_t st = m->h_ctr->status;
   if (st) {
     const int code = status_code(st);
@@ -954,13 +971,11 @@ void pending_push(bxg_map* m, const bxg_scan_desc& s) {
 }
 
 // Start a pending window on m if none is open: the device's scans_applied
-// before the scans about to be enqueued, from the counter mirror when no
-// snapshot is in flight (else read, blocking).  A map holding a device error
-// reports it instead.
+// before the scans about to be enqueued, once the mirror has landed.  A map
+// holding a device error reports it instead.
 int pending_begin(bxg_map* m) {
   if (!m->pending.empty()) return BXG_OK;
-  poll_counters(m);
-  if (m->ctr_pending) BXG_TRY(read_counters(m));
+  BXG_TRY(landed_counters(m));
   if (m->h_ctr->status) return map_status(m);
   m->pending_base = m->h_ctr->scans_applied;
   return BXG_OK;
@@ -980,7 +995,7 @@ int settle(bxg_map* m) {
   todo.swap(m->pending);
   std::deque<std::array<float, 16>> tfs;  // what todo's transforms point at
   tfs.swap(m->pending_tfs);
-  BXG_TRY(read_counters(m));
+  BXG_TRY(landed_counters(m));
   const uint32_t overflow = kStOutOfPool | kStRootFull;
   if ((m->h_ctr->status & ~overflow) || !(m->h_ctr->status & overflow)) return BXG_OK;
   const uint64_t applied = m->h_ctr->scans_applied - m->pending_base;
@@ -992,7 +1007,7 @@ int settle(bxg_map* m) {
       }
       ++m->replays;
       BXG_TRY(run_batch(c, &todo[i], 1, 0));
-      BXG_TRY(read_counters(m));
+      BXG_TRY(landed_counters(m));
       if (m->h_ctr->status & ~overflow) return BXG_OK;
       if (!(m->h_ctr->status & overflow)) break;
     }
@@ -1051,7 +1066,7 @@ int cell_op(bxg_map* m, const int32_t* coords, const void* vals, uint64_t n, uin
 }
 
 int known_leaf_count(bxg_map* m, uint32_t* out) {
-  BXG_TRY(read_counters(m));
+  BXG_TRY(landed_counters(m));
   *out = (uint32_t)m->known_leaves;
   return BXG_OK;
 }
@@ -1579,14 +1594,15 @@ int bxg_map_clear(bxg_map* m, int option) {
   }
   if (option != BXG_CLEAR_MEMORY) return fail(c, BXG_ERR_INVALID_ARG, "unknown clear option");
   // CLEAR_MEMORY: empty directory and pool (the pools keep their capacity;
-  // the old leaves' bytes stay: a leaf is written whole when it is created)
-  BXG_TRY(fill64(c, m->h.root_keys, m->root_cap, kEmptyKey));
-  BXG_TRY(fill32(c, m->h.children, (uint64_t)m->root_cap * m->h.inner_size, kEmptyChild));
-  static const uint32_t z[2] = {0, 0};  // leaf_count, root_count; then status
-  BXG_HIP(c, hipMemcpyAsync(&m->ctr->leaf_count, z, 8, hipMemcpyHostToDevice, c->stream));
-  BXG_HIP(c, hipMemcpyAsync(&m->ctr->status, z, 4, hipMemcpyHostToDevice, c->stream));
+  // the old leaves' bytes stay: a leaf is written whole when it is created).
+  // Enqueued like the other calls on the map (two fills, two copies and a
+  // wait cost 60 us a map)
+  const uint64_t n16 = (uint64_t)m->root_cap * root_bytes(m) / 16;
+  BXG_TRY(launch(c, "k_map_clear", k_map_clear, (uint32_t)std::min<uint64_t>(nblocks(n16), 4096), kBlock,
+                 m->h.root_keys, m->h.children, (uint64_t)m->root_cap, m->h.inner_size, m->ctr));
+  m->cleared = true;
   m->extra.clear();
-  BXG_TRY(ctx_sync(c));
+  m->h_ctr->leaf_count = m->h_ctr->root_count = m->h_ctr->status = 0;
   m->known_leaves = m->known_roots = 0;
   return BXG_OK;
 }
@@ -1595,6 +1611,7 @@ int bxg_map_sync(bxg_map* m) {
   if (!m) return BXG_ERR_INVALID_ARG;
   std::lock_guard<std::recursive_mutex> lk(m->ctx->mu);
   BXG_TRY(settle(m));
+  BXG_TRY(ctx_sync(m->ctx));
   return map_status(m);
 }
 
@@ -1833,7 +1850,7 @@ static int host_cell_op(bxg_map* m, const int32_t* coords, const void* vals, uin
   if (was_on) BXG_TRY(stage_in(c, 2, nullptr, n, &dw));
   for (int attempt = 0;; ++attempt) {
     BXG_TRY(cell_op(m, (const int32_t*)dc, dv, n, (uint8_t*)dw, op));
-    BXG_TRY(read_counters(m));
+    BXG_TRY(landed_counters(m));
     if (!m->h_ctr->status) break;
     if (m->h_ctr->status & kStCoordRange) {
       BXG_TRY(clear_status(m));
@@ -2011,7 +2028,7 @@ int bxg_get_update_count(bxg_map* m, uint32_t* out) {
   if (!m || !out) return BXG_ERR_INVALID_ARG;
   std::lock_guard<std::recursive_mutex> lk(m->ctx->mu);
   BXG_TRY(settle(m));
-  BXG_TRY(read_counters(m));
+  BXG_TRY(landed_counters(m));
   *out = (uint32_t)m->h_ctr->cur;
   return BXG_OK;
 }
@@ -2019,9 +2036,12 @@ int bxg_set_update_count(bxg_map* m, uint32_t v) {
   if (!m || v < 1 || v > 3) return BXG_ERR_INVALID_ARG;
   std::lock_guard<std::recursive_mutex> lk(m->ctx->mu);
   BXG_TRY(settle(m));
+  BXG_TRY(landed_counters(m));
   const int32_t cur = (int32_t)v;
   BXG_HIP(m->ctx, hipMemcpyAsync(&m->ctr->cur, &cur, 4, hipMemcpyHostToDevice, m->ctx->stream));
-  return ctx_sync(m->ctx);
+  BXG_TRY(ctx_sync(m->ctx));
+  m->h_ctr->cur = cur;
+  return BXG_OK;
 }
 
 }  // extern "C"
@@ -2040,7 +2060,7 @@ int insert_async(bxg_map* m, const bxg_scan_desc& s) {
     BXG_TRY(settle(m));
     for (int attempt = 0;; ++attempt) {
       BXG_TRY(run_batch(c, &s, 1, 0));
-      BXG_TRY(read_counters(m));
+      BXG_TRY(landed_counters(m));
       const uint32_t st = m->h_ctr->status;
       if (!(st & (kStOutOfPool | kStRootFull))) break;
       if (attempt > 8) return fail(c, BXG_ERR_OUT_OF_POOL, "could not grow the node pool");
@@ -2069,7 +2089,7 @@ int insert_host(bxg_map* m, bxg_scan_desc s, const void* points) {
   s.points_dev = dp;
   for (int attempt = 0;; ++attempt) {
     BXG_TRY(run_batch(c, &s, 1, 0));
-    BXG_TRY(read_counters(m));
+    BXG_TRY(landed_counters(m));
     const uint32_t st = m->h_ctr->status;
     if (!st) break;
     if (st & (kStCoordRange | kStScratchFull)) {
@@ -2131,11 +2151,10 @@ int bxg_insert_point_cloud_noalloc(bxg_map* m, const void* points, uint64_t n, u
 // whose map ran out of nodes; a failed scan left its map's cells untouched.
 static int run_wave_checked(bxg_ctx* c, const bxg_scan_desc* scans, uint32_t nscans) {
   BXG_TRY(run_wave(c, scans, nscans, 0));
-  BXG_TRY(ctx_sync(c));
   for (uint32_t s = 0; s < nscans; ++s) {
     bxg_map* m = scans[s].map;
     for (int attempt = 0;; ++attempt) {
-      BXG_TRY(read_counters(m));
+      BXG_TRY(landed_counters(m));
       const uint32_t st = m->h_ctr->status;
       if (!st) break;
       if (st & (kStCoordRange | kStScratchFull)) {
@@ -2205,10 +2224,10 @@ int bxg_add_point_host(bxg_map* m, const double xyz[3], int is_hit) {
   std::memcpy(s.origin, xyz, sizeof(s.origin));
   s.max_range = 0.0;
   for (int attempt = 0;; ++attempt) {
-    BXG_TRY(read_counters(m));
+    BXG_TRY(landed_counters(m));
     const uint64_t before = m->h_ctr->stat_endpoint_updates;
     BXG_TRY(run_batch(c, &s, 1, kScanNoRays | (is_hit ? kScanForceHit : kScanForceMiss)));
-    BXG_TRY(read_counters(m));
+    BXG_TRY(landed_counters(m));
     const uint32_t st = m->h_ctr->status;
     if (!st) {
       if (m->h_ctr->stat_endpoint_updates != before) m->extra.push_back(make_int4(e[0], e[1], e[2], 0));

@@ -2372,6 +2372,20 @@ __global__ void __launch_bounds__(256) k_compact_leaves(
   }
 }
 
+// clear(CLEAR_MEMORY): directory keys and entries to all ones (kEmptyKey,
+// kEmptyChild), bump counters and status to zero.  cap is a power of two >=
+// 1024, so both arrays are whole 16-byte words.
+__global__ void __launch_bounds__(256) k_map_clear(uint64_t* __restrict__ keys, uint32_t* __restrict__ children,
+                                                   uint64_t cap, uint32_t isz, MapCounters* __restrict__ ctr) {
+  static_assert(kEmptyKey == ~0ull && kEmptyChild == ~0u, "all ones");
+  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  const uint4 ones = make_uint4(~0u, ~0u, ~0u, ~0u);
+  for (uint64_t i = t; i < cap / 2; i += stride) reinterpret_cast<uint4*>(keys)[i] = ones;
+  for (uint64_t i = t; i < cap * isz / 4; i += stride) reinterpret_cast<uint4*>(children)[i] = ones;
+  if (t == 0) ctr->leaf_count = ctr->root_count = ctr->status = 0;
+}
+
 __global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * blockDim.x)

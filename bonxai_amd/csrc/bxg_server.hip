@@ -125,6 +125,10 @@ void srv_launch_read(bxg_server* s, SrvReq* r) {
     r->t_admit = now_ns();
     // inserts the map took outside the engine are confirmed first
     rc = settle(m);
+    if (rc == BXG_OK && m->cleared) {
+      rc = ctx_sync(c);
+      m->cleared = false;
+    }
     if (rc != BXG_OK) {
       // reported below
     } else if (r->kind == kReqLookup) {
