@@ -15,8 +15,8 @@ hold it is reported beside it as "steady".
 
 Prints one JSON line.  Extra fields: the plain per-scan rate, the
 batched/plain ratio, voxel updates/s, per-frame p50/p99 latency, the
-roofline of the dominant scan kernel (the fresh pass, k_scan_fresh_rays, on
-empty maps; k_scan_rays on steady frames), of the leaf assembly, and of the
+roofline of the dominant scan kernel (the leaf assembly or
+the update pass on empty maps; k_scan_rays on steady frames), of the leaf assembly, and of the
 bulk lookup and insert
 kernels (VoxelGrid<float>, 2M inserts / 8M lookups), the serving form (16
 resident maps, a Poisson stream of depth-frame inserts, lookups and exports;
@@ -394,8 +394,8 @@ def run_box_scan(ctx, bx, scenes, reps=10):
 
 
 SCAN_KERNELS = ("k_scan_begin", "k_scan_classify", "k_scan_winners", "k_scan_bucket_reduce",
-                "k_scan_bucket_scan", "k_scan_scatter", "k_scan_ray_leaves", "k_scan_endpoints",
-                "k_scan_fresh_rays", "k_scan_rays", "k_scan_new_endpoints", "k_scan_new_leaves",
+                "k_scan_bucket_scan", "k_scan_scatter", "k_scan_ray_leaves", "k_scan_new_entries",
+                "k_scan_endpoints", "k_scan_rays", "k_scan_new_endpoints", "k_scan_new_leaves",
                 "k_scan_finalize")
 
 
@@ -909,21 +909,15 @@ def main():
     # voxel updates per frame: endpoint updates (one per traced ray) + ray
     # updates (every distinct cell a ray crossed whose update_id was not cur)
     upd = fc["rays"] + fc["ray_updates"]
-    # the dominant kernel of a fresh frame: the fresh pass (maps empty at the
-    # scan's start), or the update pass where the fresh pass is switched off.
-    # Algorithmic bytes of one fresh-pass launch: per ray its 16-byte record
-    # and 4-byte list entry, per updated cell its 1-byte mark, per new leaf
-    # its 16-byte origin and 4-byte inner-grid entry.  Of one update-pass
-    # launch: per ray 20 bytes, per updated cell one 4-byte read and one
-    # 4-byte write (every distinct cell once).
+    # the dominant kernel of a fresh frame: the update pass, which in a map
+    # empty at the scan's start marks cells (algorithmic bytes of a launch: per
+    # ray its 16-byte record and 4-byte list entry, per updated cell its 1-byte
+    # mark), or the leaf assembly (per new leaf 512 mark bytes read, 2048 cell
+    # bytes and 64 mask bytes written).
     kf = b["kern_fresh"]
-    fresh_pass = kf.get("k_scan_fresh_rays", 0.0) > kf["k_scan_rays"]
-    if fresh_pass:
-        dom = "k_scan_fresh_rays"
-        alg_bytes = 20 * fc["rays"] + 1 * fc["ray_updates"] + 20 * fc["leaves"]
-    else:
-        dom = "k_scan_rays"
-        alg_bytes = 20 * fc["rays"] + 8 * fc["ray_updates"]
+    kernel_bytes = {"k_scan_rays": 20 * fc["rays"] + fc["ray_updates"], "k_scan_new_leaves": 2624 * fc["leaves"]}
+    dom = max(kernel_bytes, key=lambda k: kf.get(k, 0.0))
+    alg_bytes = kernel_bytes[dom]
     k_ms = kf[dom]
     achieved = alg_bytes / (k_ms / 1e3) / 1e9
     # the leaf assembly: per new leaf 512 mark bytes read, 2048 cell bytes

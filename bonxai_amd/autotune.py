@@ -6,20 +6,16 @@ benchmark's workload):
   ray_block           workgroup size of the walks over the rays
   ray_blocks_per_cu   most workgroups per CU of the cell-update walk
   leaf_blocks_per_cu  most workgroups per CU of the leaf-allocation walk
-  ray_chunk           rays a wavefront of the create-and-mark walk takes, in
-                      batches of 64 one after the other
   ep_table_factor     endpoint-table slots per point (inverse load factor)
   root_slack          root-directory slots per root (inverse load factor)
   ray_window          cells a ray may run ahead of its wavefront's slowest
                       ray in the update pass (1 << 20: no window)
-  leaf_window         the same in leaves for the leaf pass
-  fresh_pass          maps empty at a scan's start: one create-and-mark walk
-                      (1) or the leaf and update walks (0)
-  fresh_blocks_per_cu most workgroups per CU of the create-and-mark walk
-  fresh_window        its lockstep window, in cells
+  leaf_window         the same for the leaf pass
+  fresh_window        the same for the update pass in maps empty at a scan's
+                      start
   ray_order           winner order: direction only (0), or classes of ray
                       length and direction (1..5)
-by coordinate descent (the fresh-pass and shared keys on frames into
+by coordinate descent (the shared keys and fresh_window on frames into
 emptied maps, the workload; the update- and leaf-pass keys on frames
 re-inserted into filled maps) from the defaults, and records the fastest setting per
 device (architecture name + CU count) in bonxai_amd/tuning.json.
@@ -41,21 +37,16 @@ CANDIDATES = {
     "ray_block": [64, 128, 256],
     "ray_blocks_per_cu": [16, 24, 32, 64, 128, 256],
     "leaf_blocks_per_cu": [16, 24, 32, 64, 128, 256],
-    "ray_chunk": [64, 128, 256, 512],
     "ep_table_factor": [2, 4],
     "root_slack": [2, 4],
     "ray_window": [4, 8, 16, 32, 64, 1 << 20],
     "leaf_window": [8, 16, 32, 64, 1 << 20],
-    "fresh_pass": [1, 0],
-    "fresh_blocks_per_cu": [16, 24, 32, 64, 128, 256],
     "fresh_window": [4, 8, 16, 32, 64, 1 << 20],
     "ray_order": [3, 4, 2, 5, 1, 0],
 }
-# keys searched on each kind of frame: frames into empty maps (the workload)
-# run the fresh pass; frames re-inserted into filled maps the leaf and
-# update passes.  Keys of both are searched on fresh frames.
-FRESH_KEYS = ["ray_block", "ray_chunk", "ep_table_factor", "root_slack", "fresh_pass",
-              "fresh_blocks_per_cu", "fresh_window", "ray_order"]
+# keys searched on each kind of frame: into empty maps (the workload), and
+# re-inserted into filled maps.  Keys of both are searched on fresh frames.
+FRESH_KEYS = ["ray_block", "ep_table_factor", "root_slack", "fresh_window", "ray_order"]
 STEADY_KEYS = ["ray_blocks_per_cu", "leaf_blocks_per_cu", "ray_window", "leaf_window"]
 
 
@@ -167,7 +158,7 @@ def main(argv=None):
     ap.add_argument("--maps", type=int, default=64)
     ap.add_argument("--state", choices=["both", "fresh", "steady"], default="both",
                     help="time frames into emptied maps (fresh, the workload), re-inserted ones, "
-                         "or both: the fresh-pass keys on fresh frames, then the update-pass keys on "
+                         "or both: the shared keys on fresh frames, then the update-pass keys on "
                          "re-inserted ones")
     ap.add_argument("--passes", type=int, default=2)
     ap.add_argument("--out", default=TUNING_FILE)

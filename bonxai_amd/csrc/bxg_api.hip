@@ -94,26 +94,28 @@ struct bxg_ctx {
   bool profiling = false;
   bool counting = false;
   // tuning (bxg_ctx_set_tuning): the most workgroups per CU the passes over
-  // the rays are launched with (update, leaf and fresh pass), the workgroups
-  // per CU that a small call's ray segments may fill, the workgroup size of
-  // the passes, the rays a fresh-pass wavefront walks batch after batch, the
-  // endpoint-table capacity per point and the root-directory capacity per
-  // root (inverse load factors).  One-wavefront workgroups: a workgroup's
-  // slots are free for the next one as soon as its own rays are done (256
-  // threads: update pass 4.0 against 3.75 ms a 64-map frame, 275 against 224
-  // us a LiDAR scan)
+  // the rays are launched with (update and leaf pass), the workgroups per CU
+  // that a small call's ray segments may fill, the workgroup size of the
+  // passes, the endpoint-table capacity per point and the root-directory
+  // capacity per root (inverse load factors).  One-wavefront workgroups: a
+  // workgroup's slots are free for the next one as soon as its own rays are
+  // done (256 threads: update pass 4.0 against 3.75 ms a 64-map frame, 275
+  // against 224 us a LiDAR scan)
   uint32_t ray_blocks_per_cu = 128;
   uint32_t small_ray_blocks_per_cu = 32;
   uint32_t leaf_blocks_per_cu = 128;
   uint32_t ray_block = 64;
-  uint32_t ray_chunk = 256;
   uint32_t ep_table_factor = 2;
   uint32_t root_slack = 2;
-  uint32_t ray_window = 8;    // lockstep windows of the update pass (cells) and leaf pass (leaves)
-  uint32_t leaf_window = 32;
-  uint32_t fresh_pass = 1;    // maps empty at a scan's start: one create-and-mark walk
-  uint32_t fresh_blocks_per_cu = 128;
-  uint32_t fresh_window = 16;        // its lockstep window (cells)
+  // lockstep windows (cells) of the update pass, of the leaf pass, and of the
+  // update pass in maps empty at the scan's start
+  uint32_t ray_window = kUpdateWindow;
+  uint32_t leaf_window = kLeafWindow;
+  uint32_t fresh_window = kFreshWindow;
+  // accepted for settings recorded by earlier versions; without effect
+  uint32_t ray_chunk = 256;
+  uint32_t fresh_pass = 1;
+  uint32_t fresh_blocks_per_cu = 6;
   uint32_t ray_order = 3;            // winner order: direction sector, length class, direction
   std::vector<Prof> prof_pending;
   std::vector<hipEvent_t> ev_free;
@@ -357,6 +359,11 @@ uint64_t leaf_bytes(const bxg_map* m) {
          touched_bytes(m);
 }
 uint64_t root_bytes(const bxg_map* m) { return 8 + (uint64_t)m->h.inner_size * 4; }
+// words of the have or want bits of a directory of cap roots (probabilistic
+// maps; working memory of the scans, not counted in the map's size)
+uint64_t entry_bits(const bxg_map* m, uint64_t cap) {
+  return (m->h.flags & kMapProbabilistic) ? cap * entry_words(m->h.inner_size) : 0;
+}
 
 int push_header(bxg_map* m) { return upload(m->ctx, m->d, &m->h, sizeof(MapDev)); }
 
@@ -438,6 +445,18 @@ void poll_counters(bxg_map* m) {
   }
 }
 
+// have and want bits for a directory of cap roots, all zero, in h's arrays
+// (the caller frees the old ones)
+int alloc_entry_bits(bxg_map* m, uint64_t cap, uint64_t** have, uint64_t** want) {
+  *have = *want = nullptr;
+  const uint64_t n = entry_bits(m, cap);
+  if (!n) return BXG_OK;
+  BXG_TRY(dmalloc(m->ctx, (void**)have, n * 8));
+  BXG_TRY(dmalloc(m->ctx, (void**)want, n * 8));
+  BXG_TRY(fill64(m->ctx, *have, n, 0));
+  return fill64(m->ctx, *want, n, 0);
+}
+
 int grow_leaves(bxg_map* m, uint64_t need) {
   bxg_ctx* c = m->ctx;
   if (need <= m->leaf_cap) return BXG_OK;
@@ -501,9 +520,13 @@ int grow_roots(bxg_map* m, uint64_t need_roots) {
   BXG_TRY(dmalloc(c, &children, cap * m->h.inner_size * 4));
   BXG_TRY(fill64(c, (uint64_t*)keys, cap, kEmptyKey));
   BXG_TRY(fill32(c, (uint32_t*)children, cap * m->h.inner_size, kEmptyChild));
+  uint64_t *have = nullptr, *want = nullptr;
+  BXG_TRY(alloc_entry_bits(m, cap, &have, &want));
   uint64_t* old_keys = m->h.root_keys;
   uint32_t* old_children = m->h.children;
   const uint32_t old_cap = m->root_cap;
+  std::swap(m->h.leaf_have, have);  // now the old ones
+  std::swap(m->h.leaf_want, want);
   m->h.root_keys = (uint64_t*)keys;
   m->h.children = (uint32_t*)children;
   m->h.root_mask = (uint32_t)(cap - 1);
@@ -517,6 +540,8 @@ int grow_roots(bxg_map* m, uint64_t need_roots) {
   BXG_TRY(ctx_sync(c));
   dfree(old_keys);
   dfree(old_children);
+  dfree(have);
+  dfree(want);
   c->used += more;
   m->bytes += more;
   return BXG_OK;
@@ -757,11 +782,6 @@ uint32_t tag_bits_for(uint32_t nscans) {
   return b;
 }
 
-// What the host knows about a call's maps: every one empty (no leaf, no work
-// on it under way), every one not empty (a map's leaf count only falls in
-// clear and release_unused, which the host runs), or neither.
-enum class Maps { kMixed, kEmpty, kFilled };
-
 // the first kernel of a call, with its scans as arguments: writes hdr and desc
 template <uint32_t kN>
 int begin_args(bxg_ctx* c, const BatchHdr& h, const ScanDesc* scans, BatchHdr* hdr, ScanDesc* desc,
@@ -775,8 +795,10 @@ int begin_args(bxg_ctx* c, const BatchHdr& h, const ScanDesc* scans, BatchHdr* h
 // The kernel sequence of one wave of scans on given scratch and descriptors.
 // args: the batch's header and descriptors (at most kMostArgs), which the
 // first kernel writes to hdr and desc; null where they are there already.
+// all_empty: the host knows every map of the call to be empty (no leaf, no
+// work on it under way).
 int enqueue_scan_kernels(bxg_ctx* c, BatchHdr* hdr, ScanDesc* desc, ScanScratch sc, uint64_t grid_points,
-                         uint32_t nscans, bool any_extra, Maps maps = Maps::kMixed,
+                         uint32_t nscans, bool any_extra, bool all_empty = false,
                          const BatchHdr* args_hdr = nullptr, const ScanDesc* args = nullptr) {
   const uint32_t gp = nblocks(grid_points);
   const uint32_t gw = std::max<uint32_t>(1, std::min<uint32_t>(gp, 16384));
@@ -787,28 +809,20 @@ int enqueue_scan_kernels(bxg_ctx* c, BatchHdr* hdr, ScanDesc* desc, ScanScratch 
   const uint64_t cus = (uint64_t)std::max(c->cu_count, 1);
   const uint32_t rb = c->ray_block;
   const uint64_t most = (grid_points + rb - 1) / rb;
-  const auto walk_grid = [&](uint64_t per_cu, uint64_t run) {
-    const uint64_t whole = std::min((most + run - 1) / run, cus * per_cu);
+  const auto walk_grid = [&](uint64_t per_cu) {
+    const uint64_t whole = std::min(most, cus * per_cu);
     const uint64_t cut = std::min(most * (1u << kMaxSegLog), cus * c->small_ray_blocks_per_cu);
     const uint64_t g = std::max<uint64_t>({whole, cut, 1});
     return (uint32_t)((g + kXcds - 1) / kXcds * kXcds);
   };
-  const uint32_t gr = walk_grid(c->ray_blocks_per_cu, 1);
-  const uint32_t gl = walk_grid(c->leaf_blocks_per_cu, 1);
-  const uint32_t gf = walk_grid(c->fresh_blocks_per_cu, c->ray_chunk / 64);
-  sc.chunk_max = c->ray_chunk;
+  const uint32_t gr = walk_grid(c->ray_blocks_per_cu);
+  const uint32_t gl = walk_grid(c->leaf_blocks_per_cu);
   sc.win_cells = (int32_t)c->ray_window;
   sc.win_leaves = (int32_t)c->leaf_window;
-  sc.fresh_pass = c->fresh_pass;
   sc.win_fresh = (int32_t)c->fresh_window;
   sc.ray_order = c->ray_order;
   // new-leaf pass: a wavefront per new leaf, grid-stride over them
   const uint32_t gm = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(cus * 8, gp));
-  // the passes that have nothing to do in such maps are not launched (about 5
-  // us each): the fresh pass in filled maps; the leaf, endpoint and update
-  // passes in empty ones, which the fresh pass walks
-  const bool fresh = maps != Maps::kFilled;
-  const bool old = maps != Maps::kEmpty || !c->fresh_pass;
   if (!args)
     BXG_TRY(launch(c, "k_scan_begin", k_scan_begin, 1, kBlock, hdr, desc, sc));
   else if (nscans == 1)
@@ -827,19 +841,19 @@ int enqueue_scan_kernels(bxg_ctx* c, BatchHdr* hdr, ScanDesc* desc, ScanScratch 
     BXG_TRY(launch(c, "k_scan_bucket_scan", k_scan_bucket_scan, tiles, 1024, hdr, sc));
     BXG_TRY(launch(c, "k_scan_scatter", k_scan_scatter<false>, gp, kBlock, hdr, sc));
   }
-  if (old) BXG_TRY(launch(c, "k_scan_ray_leaves", k_scan_ray_leaves, gl, rb, desc, sc));
+  BXG_TRY(launch(c, "k_scan_ray_leaves", k_scan_ray_leaves, gl, rb, desc, sc));
   if (any_extra)
     BXG_TRY(launch(c, "k_scan_extra_leaves", k_scan_extra_leaves, nscans, kBlock, hdr, desc));
-  if (old) BXG_TRY(launch(c, "k_scan_endpoints", k_scan_endpoints, gw, kBlock, desc, sc));
+  BXG_TRY(launch(c, "k_scan_new_entries", k_scan_new_entries, (uint32_t)cus * 4, kBlock, hdr, desc));
+  // an empty map has no endpoint in an older leaf (a launch saved, about 5 us)
+  if (!all_empty) BXG_TRY(launch(c, "k_scan_endpoints", k_scan_endpoints, gw, kBlock, desc, sc));
   if (c->counting) {
-    if (fresh) BXG_TRY(launch(c, "k_scan_fresh_rays", k_scan_fresh_rays<true>, gf, rb, desc, sc));
-    if (old) BXG_TRY(launch(c, "k_scan_rays", k_scan_rays<true>, gr, rb, desc, sc));
+    BXG_TRY(launch(c, "k_scan_rays", k_scan_rays<true>, gr, rb, desc, sc));
     if (any_extra)
       BXG_TRY(launch(c, "k_scan_extra_rays", k_scan_extra_rays<true>, nscans, kBlock, hdr, desc));
     BXG_TRY(launch(c, "k_scan_new_endpoints", k_scan_new_endpoints<true>, gw, kBlock, hdr, desc, sc));
   } else {
-    if (fresh) BXG_TRY(launch(c, "k_scan_fresh_rays", k_scan_fresh_rays<false>, gf, rb, desc, sc));
-    if (old) BXG_TRY(launch(c, "k_scan_rays", k_scan_rays<false>, gr, rb, desc, sc));
+    BXG_TRY(launch(c, "k_scan_rays", k_scan_rays<false>, gr, rb, desc, sc));
     if (any_extra)
       BXG_TRY(launch(c, "k_scan_extra_rays", k_scan_extra_rays<false>, nscans, kBlock, hdr, desc));
     BXG_TRY(launch(c, "k_scan_new_endpoints", k_scan_new_endpoints<false>, gw, kBlock, hdr, desc, sc));
@@ -870,7 +884,7 @@ int run_wave(bxg_ctx* c, const bxg_scan_desc* scans, uint32_t nscans, uint32_t e
   uint64_t total = 0;
   BXG_TRY(build_descs(c, scans, nscans, extra_flags, descs, &total));
   bool any_extra = false;
-  uint32_t empty = 0, filled = 0;
+  bool all_empty = true;
   const bool as_args = nscans <= kMostArgs;
   for (uint32_t s = 0; s < nscans; ++s) {
     bxg_map* m = scans[s].map;
@@ -883,19 +897,16 @@ int run_wave(bxg_ctx* c, const bxg_scan_desc* scans, uint32_t nscans, uint32_t e
       BXG_TRY(upload_extra(m));
       descs[s].extra = m->d_extra;
     }
-    if (m->known_leaves)
-      ++filled;
-    else if (!m->ctr_pending && m->pending.empty())
-      ++empty;
+    // (a map's leaf count only falls in clear and release_unused, on the host)
+    if (m->known_leaves || m->ctr_pending || !m->pending.empty()) all_empty = false;
     if (c->counting && !as_args) BXG_TRY(reset_scan_stats(m));
   }
-  const Maps state = filled == nscans ? Maps::kFilled : (empty == nscans ? Maps::kEmpty : Maps::kMixed);
   // the maps may have grown: descriptors point at device headers, which
   // stay put, so nothing to rebuild
   BXG_TRY(ensure_scan_scratch(c, std::max<uint64_t>(total, 1), nscans));
   BatchHdr hdr{nscans, tag_bits_for(nscans), total};
   if (!as_args) BXG_TRY(upload_scans(c, c->d_hdr, hdr, descs));
-  BXG_TRY(enqueue_scan_kernels(c, c->d_hdr, c->d_desc, c->sc, total, nscans, any_extra, state,
+  BXG_TRY(enqueue_scan_kernels(c, c->d_hdr, c->d_desc, c->sc, total, nscans, any_extra, all_empty,
                                as_args ? &hdr : nullptr, as_args ? descs.data() : nullptr));
   // k_scan_finalize wrote every map's counters to its host mirror
   std::vector<bxg_map*> maps(nscans);
@@ -1188,7 +1199,7 @@ int insert_noalloc(bxg_map* m, const bxg_scan_desc& in) {
   BXG_TRY(fill64(c, (uint64_t*)sc.ep, slots * 2, ~0ull));
   BXG_TRY(fill32(c, sc.hist, kMaxBuckets, 0));
   BXG_TRY(fill32(c, sc.counters, kCounterWords, 0));
-  BXG_TRY(enqueue_scan_kernels(c, d_hdr, d_desc, sc, in.n, 1, false, Maps::kMixed, &hdr, &d));
+  BXG_TRY(enqueue_scan_kernels(c, d_hdr, d_desc, sc, in.n, 1, false, false, &hdr, &d));
   BXG_TRY(read_counters(m));  // waits for the scan
   const uint32_t st = m->h_ctr->status;
   if (st & ~overflow) return map_status(m);
@@ -1554,6 +1565,8 @@ int bxg_map_destroy(bxg_map* m) {
   hipStreamSynchronize(c->stream);
   dfree(m->h.root_keys);
   dfree(m->h.children);
+  dfree(m->h.leaf_have);
+  dfree(m->h.leaf_want);
   dfree(m->h.leaf_masks);
   dfree(m->h.cells);
   dfree(m->h.leaf_origin);
@@ -1599,7 +1612,7 @@ int bxg_map_clear(bxg_map* m, int option) {
   // wait cost 60 us a map)
   const uint64_t n16 = (uint64_t)m->root_cap * root_bytes(m) / 16;
   BXG_TRY(launch(c, "k_map_clear", k_map_clear, (uint32_t)std::min<uint64_t>(nblocks(n16), 4096), kBlock,
-                 m->h.root_keys, m->h.children, (uint64_t)m->root_cap, m->h.inner_size, m->ctr));
+                 m->h.root_keys, m->h.children, m->h.leaf_have, (uint64_t)m->root_cap, m->h.inner_size, m->ctr));
   m->cleared = true;
   m->extra.clear();
   m->h_ctr->leaf_count = m->h_ctr->root_count = m->h_ctr->status = 0;
@@ -1736,6 +1749,10 @@ int bxg_map_release_unused(bxg_map* m) {
   BXG_TRY(dmalloc(c, &children, rcap * m->h.inner_size * 4));
   BXG_TRY(fill64(c, (uint64_t*)keys, rcap, kEmptyKey));
   BXG_TRY(fill32(c, (uint32_t*)children, rcap * m->h.inner_size, kEmptyChild));
+  uint64_t *have = nullptr, *want = nullptr;
+  BXG_TRY(alloc_entry_bits(m, rcap, &have, &want));
+  std::swap(m->h.leaf_have, have);  // now the old ones
+  std::swap(m->h.leaf_want, want);
   uint64_t* old_keys = m->h.root_keys;
   uint32_t* old_children = m->h.children;
   const uint32_t old_rcap = m->root_cap;
@@ -1763,6 +1780,8 @@ int bxg_map_release_unused(bxg_map* m) {
   BXG_TRY(ctx_sync(c));
   dfree(old_keys);
   dfree(old_children);
+  dfree(have);
+  dfree(want);
   dfree(old_masks);
   dfree(old_cells);
   dfree(old_orig);

@@ -9,6 +9,12 @@
 //                    is claimed with a single 64-bit atomicCAS.  The slot
 //                    index IS the inner node: children[slot * inner_size + i]
 //                    holds the leaf index of inner cell i, or EMPTY.
+//                    Probabilistic maps: one bit an inner cell in two arrays of
+//                    entry_words(inner_size) words a slot.  leaf_have: the
+//                    entry's leaf is known to exist (never set for an EMPTY
+//                    entry, but a leaf may exist without it); leaf_want: a ray
+//                    of the running scan enters the leaf and its have bit is
+//                    not set (all zero between scans).
 //   leaf pool        leaf_cap leaves handed out by an atomic bump counter:
 //                    leaf_masks[leaf * leaf_words + w]  (bit n of a leaf is
 //                    word n >> 6, bit n & 63, as mask.hpp:329-365)
@@ -92,6 +98,8 @@ struct alignas(64) MapDev {
   uint32_t* children;
   uint32_t root_mask;  // root_cap - 1
   uint32_t max_probe;
+  uint64_t* leaf_have;  // probabilistic maps, root_cap * entry_words (below)
+  uint64_t* leaf_want;
   uint64_t* leaf_masks;
   uint8_t* cells;
   int4* leaf_origin;
@@ -101,6 +109,11 @@ struct alignas(64) MapDev {
   MapCounters* ctr;
   MapCounters* ctr_host;  // pinned host mirror, written at the end of every scan
 };
+
+// 64-bit words of the inner-cell bits of one root
+__host__ __device__ inline uint32_t entry_words(uint32_t inner_size) {
+  return inner_size >= 64 ? inner_size / 64 : 1;
+}
 
 // one scan of a (possibly batched) insertPointCloud call
 struct alignas(16) ScanDesc {
@@ -150,19 +163,12 @@ constexpr uint32_t kXcds = 8;      // workgroups are dispatched round the XCDs
 constexpr uint32_t kScanTile = 4096;  // buckets one block of the bucket scan covers
 constexpr uint32_t kTiles = kMaxBuckets / kScanTile;
 static_assert((1u << kDirBits) % kScanTile == 0 && kTiles <= 64, "bucket scan tiles");
-// scan counter words: [0] winner count, [kFreshWords, + 4) the fresh-pass
-// split (below), [kTileWords, + kTiles) bucket-tile sums, [kClipWords, + 64) per scan (index mod 64) the
-// points clipped at the max range among those of one wavefront in 16
+// scan counter words: [0] winner count, [kTileWords, + kTiles) bucket-tile
+// sums, [kClipWords, + 64) per scan (index mod 64) the points clipped at the
+// max range among those of one wavefront in 16
 constexpr uint32_t kTileWords = 64;
 constexpr uint32_t kClipWords = kTileWords + kTiles;
 constexpr uint32_t kCounterWords = kClipWords + 64;
-// With at most 2^kMaxTagBits scans (one bucket tag each), the scans whose map
-// is empty at the start take the highest tags, so their winners end the
-// list: [kFreshWords, +1] the 64-bit mask of those scans, [+2] the first of
-// their tags (kNone: no split, every pass walks the whole list and skips the
-// other pipeline's rays), [+3] the index of their first winner.
-constexpr uint32_t kFreshWords = 1;
-static_assert(kFreshWords + 4 <= kTileWords, "counter words");
 
 // scratch of one integration call, owned by the context
 // One slot of the per-call endpoint table: key (scan tag, root slot, inner
@@ -182,11 +188,9 @@ struct ScanScratch {
                         // per winner: leaf index of its endpoint if new, kLeafLater or kNone
   EpSlot* ep;           // endpoint table
   uint32_t ep_mask;     // capacity - 1
-  uint32_t chunk_max;   // rays a wavefront of the fresh pass walks one batch after the other (64..1024)
-  int32_t win_cells;    // lockstep window of the update pass, in cells (0: the default)
-  int32_t win_leaves;   // lockstep window of the leaf pass, in leaves (0: the default)
-  uint32_t fresh_pass;  // 1: the rays of maps empty at the scan's start take the fresh pass
-  int32_t win_fresh;    // lockstep window of the fresh pass, in cells (0: the update pass's)
+  int32_t win_cells;    // lockstep window of the update pass, in cells
+  int32_t win_leaves;   // lockstep window of the leaf pass, in cells
+  int32_t win_fresh;    // window of the update pass in maps empty at the scan's start
   uint32_t ray_order;   // winner order (0..5, k_scan_winners): 0 direction only
   uint32_t* winners;    // flattened point indices of per-voxel winners, bucketed
   uint32_t* wkey;       // per point: bucket of a winner, kNone otherwise

@@ -68,6 +68,9 @@ __device__ __forceinline__ uint64_t xor64(uint64_t* p, uint64_t v) {
 __device__ __forceinline__ uint32_t min32(uint32_t* p, uint32_t v) {
   return __hip_atomic_fetch_min(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ uint64_t ld64(const uint64_t* p) {
+  return __hip_atomic_load(gp(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ uint32_t max32(uint32_t* p, uint32_t v) {
   return __hip_atomic_fetch_max(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -87,6 +90,27 @@ __device__ __forceinline__ int32_t wave_min(int32_t v) {
   v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xA, 0xF, false));
   v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xC, 0xF, false));
   return __builtin_amdgcn_readlane(v, 63);
+}
+
+// bitwise or over the 64 lanes of a wavefront, every lane active (the steps
+// of wave_min)
+__device__ __forceinline__ uint32_t wave_or32(uint32_t v) {
+  v |= (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0xB1, 0xF, 0xF, false);
+  v |= (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x4E, 0xF, 0xF, false);
+  v |= (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x124, 0xF, 0xF, false);
+  v |= (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x128, 0xF, 0xF, false);
+  v |= (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x142, 0xA, 0xF, false);
+  v |= (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x143, 0xC, 0xF, false);
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+__device__ __forceinline__ uint64_t wave_or(uint64_t v) {
+  return (uint64_t)wave_or32((uint32_t)v) | ((uint64_t)wave_or32((uint32_t)(v >> 32)) << 32);
+}
+
+// value of lane l (the same l in every lane), 64 bits
+__device__ __forceinline__ uint64_t lane_value(uint64_t v, uint32_t l) {
+  return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, (int)l) |
+         ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), (int)l) << 32);
 }
 
 // Bump allocation from per-map counters, aggregated over a wavefront: the
@@ -145,6 +169,8 @@ struct MapView {
   MapCounters* ctr;
   double inv_res;
   uint32_t ib, lb, log2n, isz, lsz, lw, vb, flags;
+  uint64_t BXG_G* have;
+  uint64_t BXG_G* want;
   uint32_t root_mask, max_probe, leaf_cap;
   int32_t miss, hit, cmin, cmax, thr;
 };
@@ -168,6 +194,8 @@ __device__ __forceinline__ MapView load_view(const MapDev* p) {
   v.lw = q->leaf_words;
   v.vb = q->value_bytes;
   v.flags = q->flags;
+  v.have = gp((uint64_t*)q->leaf_have);
+  v.want = gp((uint64_t*)q->leaf_want);
   v.root_mask = q->root_mask;
   v.max_probe = q->max_probe;
   v.leaf_cap = q->leaf_cap;
@@ -211,6 +239,8 @@ __device__ __forceinline__ MapView uniform_view(const MapDev* p) {
   v.lw = q->leaf_words;
   v.vb = q->value_bytes;
   v.flags = q->flags;
+  v.have = gp((uint64_t*)q->leaf_have);
+  v.want = gp((uint64_t*)q->leaf_want);
   v.root_mask = q->root_mask;
   v.max_probe = q->max_probe;
   v.leaf_cap = q->leaf_cap;
@@ -285,13 +315,6 @@ __device__ __forceinline__ bool leaf_claim(uint32_t* cp, uint32_t& seen) {
   if (v == kEmptyChild) v = cas32(cp, kEmptyChild, kPendingChild);
   seen = v;
   return v == kEmptyChild;
-}
-
-// leaf_claim for a caller that has just loaded the entry and found it EMPTY:
-// straight to the CAS (no second load round trip)
-__device__ __forceinline__ bool leaf_claim_empty(uint32_t* cp, uint32_t& seen) {
-  seen = cas32(cp, kEmptyChild, kPendingChild);
-  return seen == kEmptyChild;
 }
 
 // Leaf indices for the lanes that claimed an entry (allocateLeafGrid and
@@ -494,48 +517,61 @@ struct LeafWalk {
 };
 
 // Allocation pass, one step of a ray: the root of its current leaf (created
-// if missing) and up to kLeafRun of its next leaves in that root; their
-// inner-grid entries are loaded together (one memory round trip, not one a
-// leaf), and only those still empty take the creating path.
-constexpr int kLeafRun = 2;
-__device__ __forceinline__ void leaves_step(const MapView& m, LeafWalk& lw, RootCache& rc) {
-  const int32_t slot = root_slot<true>(m, rc, lw.lx, lw.ly, lw.lz);
-  const int32_t rmask = ~((1 << m.log2n) - 1);
-  int32_t lx[kLeafRun] = {}, ly[kLeafRun] = {}, lz[kLeafRun] = {};
-  int n = 0;
+// if missing) and the ray's next leaves of that root, up to kLeafRun, as bits
+// of the root's inner cells.  One load of `known` tells which of them exist
+// (the have bits; in a map empty at the scan's start the want bits: those put
+// down already); the others are put down in the root's want bits, and
+// k_scan_new_entries creates them.  (Leaves created by the rays themselves, a
+// claim each and one bump of the map's leaf counter a wavefront and step,
+// were bound by the counter, about 6 ns an atomic: 97 us for a LiDAR scan
+// that adds 38k leaves to a map, now 40; and a first scan's rays, creating
+// leaves and marking cells in one walk, took 465 us, now 60 + 230.)
+constexpr int kLeafRun = 8;
+__device__ __forceinline__ void leaves_step(const MapView& m, LeafWalk& lw, RootCache& rc,
+                                            const uint64_t BXG_G* known, bool go) {
+  uint64_t miss = 0;
+  uint32_t e = 0;  // word of the directory (at most 2^24 roots of 64 words)
+  if (go) {
+    const int32_t slot = root_slot<true>(m, rc, lw.lx, lw.ly, lw.lz);
+    const int32_t rmask = ~((1 << m.log2n) - 1);
+    const uint32_t ci = inner_index(lw.lx, lw.ly, lw.lz, m.lb, m.ib);
+    const uint32_t word = ci >> 6;
+    uint64_t bits = 1ull << (ci & 63u);
+    lw.next();
 #pragma unroll
-  for (int j = 0; j < kLeafRun; ++j) {
-    if (j == 0 || (n == j && !lw.done() && (lw.lx & rmask) == rc.rx && (lw.ly & rmask) == rc.ry &&
-                   (lw.lz & rmask) == rc.rz)) {
-      lx[j] = lw.lx;
-      ly[j] = lw.ly;
-      lz[j] = lw.lz;
-      n = j + 1;
+    for (int j = 1; j < kLeafRun; ++j) {
+      const uint32_t c = inner_index(lw.lx, lw.ly, lw.lz, m.lb, m.ib);
+      const bool in = !lw.done() & ((((lw.lx & rmask) ^ rc.rx) | ((lw.ly & rmask) ^ rc.ry) |
+                                     ((lw.lz & rmask) ^ rc.rz)) == 0) & ((c >> 6) == word);
+      if (!in) break;
+      bits |= 1ull << (c & 63u);
       lw.next();
     }
+    if (slot >= 0) {  // else the root directory is full: the call fails
+      e = (uint32_t)slot * entry_words(m.isz) + word;
+      miss = bits & ~known[e];
+    }
   }
-  if (slot < 0) return;  // root directory full: the call fails
-  uint32_t v[kLeafRun];
-  uint32_t* cp[kLeafRun];
-#pragma unroll
-  for (int j = 0; j < kLeafRun; ++j) {
-    cp[j] = (uint32_t*)&m.children[(uint64_t)slot * m.isz + inner_index(lx[j], ly[j], lz[j], m.lb, m.ib)];
-    v[j] = j < n ? *gp(cp[j]) : 0u;
+  if (__ballot(miss != 0) == 0) return;
+  // Fewer atomics: a lane leaves the bits that the lane before it puts down,
+  // and the lanes of the first few words of the wavefront go together on one
+  // of them (near the sensor all 64 rays cross one root: a 100k-point room 37
+  // us, 120 us without; grouping every word costs more than its atomics where
+  // the rays have spread).
+  const uint32_t plo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)miss, 0x138, 0xF, 0xF, false);
+  const uint32_t phi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(miss >> 32), 0x138, 0xF, 0xF, false);
+  const uint32_t pe = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)e, 0x138, 0xF, 0xF, false);
+  uint64_t put = miss;
+  if (lane_id() > 0 && pe == e) put &= ~(((uint64_t)phi << 32) | plo);
+  uint64_t pending = __ballot(put != 0);
+  for (int g = 0; g < 4 && pending; ++g) {
+    const uint32_t l = (uint32_t)__ffsll((unsigned long long)pending) - 1u;
+    const bool mine = put != 0 && e == (uint32_t)__builtin_amdgcn_readlane((int)e, (int)l);
+    pending &= ~__ballot(mine);
+    const uint64_t all = wave_or(mine ? put : 0ull);
+    if (mine) put = lane_id() == l ? all : 0ull;
   }
-  // claims first, then one aggregated allocation per run slot for the
-  // whole wavefront (every active lane takes part, claimed or not)
-  bool won[kLeafRun];
-#pragma unroll
-  for (int j = 0; j < kLeafRun; ++j) {
-    // neighbouring rays in neighbouring lanes often reach the same missing
-    // leaf at the same step: the lowest lane of each such run claims it
-    const bool missing = j < n && v[j] == kEmptyChild;
-    const int lead = run_leader(missing, (uint64_t)cp[j], 0u);
-    uint32_t seen;
-    won[j] = (missing && lead == (int)lane_id()) ? leaf_claim_empty(cp[j], seen) : false;
-  }
-#pragma unroll
-  for (int j = 0; j < kLeafRun; ++j) leaf_publish(m, won[j], cp[j], (uint32_t)slot, lx[j], ly[j], lz[j]);
+  if (put) or64((uint64_t*)&m.want[e], put);
 }
 
 // One leaf of a ray, update pass: the cells of the ray in the current leaf
@@ -630,87 +666,6 @@ __device__ __forceinline__ uint32_t apply_step(const MapView& m, RayWalk& w, Roo
     }
   }
   if (bits) or64((uint64_t*)&mw[word], bits);
-  return nupd;
-}
-
-// The fresh pass: rays of a map that was empty when the scan started, so
-// every leaf they cross is new.  One walk creates the leaves (as the leaf
-// pass) and marks the ray's cells (as the update pass does in new leaves),
-// where the two-pass pipeline walks each ray twice.  Nothing it writes is
-// visible in the map's cells until k_scan_new_leaves, and a failed call's
-// marks are dropped there, so the pass may stop at an overflow like the leaf
-// pass.  Per lane: the root slot and inner-grid entry of the current cell's
-// leaf, loaded one step ahead.
-
-// root slot (created if missing) and inner-grid entry of the walk's current
-// cell (a plain load: a stale EMPTY only sends the lane to the claim's CAS, a
-// stale PENDING to an atomic re-read)
-__device__ __forceinline__ void fresh_entry(const MapView& m, const RayWalk& w, RootCache& rc,
-                                            int32_t& slot, uint32_t& entry) {
-  slot = root_slot<true>(m, rc, w.cx, w.cy, w.cz);
-  entry = slot >= 0
-              ? *gp(&m.children[(uint64_t)slot * m.isz + inner_index(w.cx, w.cy, w.cz, m.lb, m.ib)])
-              : kEmptyChild;
-}
-
-// One leaf of a fresh-pass ray: the leaf is created if missing (the lowest
-// lane of each run of lanes at one entry claims it, one aggregated bump per
-// wavefront), then the run's cells before the endpoint are marked in the
-// leaf's touched bytes.  A leaf another wavefront is still creating
-// (PENDING) is re-read and the step taken again on the lane's next turn; its
-// creator publishes it within its own step.  A full root directory or pool
-// (the call fails) stops the ray.  The run that holds the endpoint's cell
-// stores its leaf index in *ep_leaf.  Returns the cells marked first (counted
-// form, exact, by atomics).
-template <bool kCount>
-__device__ __forceinline__ uint32_t fresh_step(const MapView& m, RayWalk& w, RootCache& rc,
-                                               int32_t& slot, uint32_t& entry, bool& stopped,
-                                               uint32_t* ep_leaf) {
-  uint32_t* cp = slot >= 0 ? (uint32_t*)&m.children[(uint64_t)slot * m.isz +
-                                                    inner_index(w.cx, w.cy, w.cz, m.lb, m.ib)]
-                           : nullptr;
-  const bool missing = slot >= 0 && entry == kEmptyChild;
-  const int lead = run_leader(missing, (uint64_t)cp, 0u);
-  bool won = false;
-  uint32_t seen = entry;
-  if (missing && lead == (int)lane_id()) won = leaf_claim_empty(cp, seen);
-  const int32_t lmask = ~((1 << m.lb) - 1);
-  const uint32_t idx = leaf_publish(m, won, cp, (uint32_t)slot, w.cx & lmask, w.cy & lmask, w.cz & lmask);
-  if (won) seen = idx;
-  // the other lanes of a leader's run take its outcome
-  const uint32_t led = (uint32_t)__shfl((int)seen, lead);
-  if (missing) seen = led;
-  if (slot < 0 || seen == kEmptyChild) {
-    stopped = true;
-    return 0;
-  }
-  if (seen == kPendingChild) {
-    entry = ld32(cp);
-    return 0;
-  }
-  const int32_t k0 = w.k;
-  uint32_t li[kRun];
-  const uint32_t n = collect_run(m, w, li);
-  // cells k0 .. k0 + n - 1 of the walk; the ray's are those before mx
-  const int32_t rest = w.mx - k0;
-  const uint32_t nray = rest <= 0 ? 0u : (n < (uint32_t)rest ? n : (uint32_t)rest);
-  uint8_t BXG_G* tb = m.touched + (uint64_t)seen * m.lsz;
-  uint32_t nupd = 0;
-#pragma unroll
-  for (int j = 0; j < kRun; ++j) {
-    if ((uint32_t)j < nray) {
-      if (kCount) {
-        const uint32_t sh = (li[j] & 3u) * 8u;
-        nupd += ((or32((uint32_t*)(tb + (li[j] & ~3u)), 1u << sh) >> sh) & 0xFFu) == 0u ? 1u : 0u;
-      } else {
-        tb[li[j]] = 1;
-      }
-    }
-  }
-  // the run holding the endpoint's cell (mx) leaves its leaf for
-  // k_scan_new_endpoints, which then needs no lookup
-  if (k0 <= w.mx && w.mx < k0 + (int32_t)n) *ep_leaf = seen;
-  if (!w.done()) fresh_entry(m, w, rc, slot, entry);
   return nupd;
 }
 
@@ -959,17 +914,7 @@ __global__ void __launch_bounds__(256) k_scan_winners(const BatchHdr* __restrict
       win = true;
       const uint32_t s = (uint32_t)r.w >> 16;
       const ScanDesc& d = sd[s];
-      uint32_t tag = s & ((1u << hdr->tag_bits) - 1u);
-      const uint32_t split = sc.counters[kFreshWords + 2];
-      if (split != kNone) {
-        // the other scans keep their order in tags [0, split), the fresh
-        // scans theirs in [split, nscans)
-        const uint64_t fresh = (uint64_t)sc.counters[kFreshWords] |
-                               ((uint64_t)sc.counters[kFreshWords + 1] << 32);
-        const uint64_t below = (1ull << s) - 1ull;
-        tag = ((fresh >> s) & 1ull) ? split + (uint32_t)__popcll(fresh & below)
-                                    : (uint32_t)__popcll(~fresh & below);
-      }
+      const uint32_t tag = s & ((1u << hdr->tag_bits) - 1u);
       const int32_t dx = r.x - d.ox, dy = r.y - d.oy, dz = r.z - d.oz;
       // The ray's length class (its cell count mx against the max range, in
       // 2^cb equal parts) sits between a coarse direction sector (hb bits)
@@ -1096,17 +1041,10 @@ __global__ void __launch_bounds__(1024) k_scan_bucket_scan(const BatchHdr* __res
   o.z = run; run += v.z;
   o.w = run;
   reinterpret_cast<uint4*>(sc.offs + base)[threadIdx.x] = o;
-  // the fresh scans' winners start at bucket split << kDirBits (a tile's
-  // first bucket: kScanTile divides 2^kDirBits); with no fresh scan, at the end
-  const uint32_t split = sc.counters[kFreshWords + 2];
-  if (split != kNone && (split << kDirBits) == base && threadIdx.x == 0) sc.counters[kFreshWords + 3] = o.x;
-  if (base + kScanTile >= nb && threadIdx.x == 1023) {
-    sc.counters[0] = carry + wsum[15];
-    if (split != kNone && (split << kDirBits) >= nb) sc.counters[kFreshWords + 3] = carry + wsum[15];
-  }
+  if (base + kScanTile >= nb && threadIdx.x == 1023) sc.counters[0] = carry + wsum[15];
 }
 
-constexpr uint32_t kLeafLater = 0xFFFFFFFEu;  // tpos: look the endpoint's leaf up after the fresh pass
+constexpr uint32_t kLeafLater = 0xFFFFFFFEu;  // tpos: the endpoint's leaf is not looked up yet
 
 // Phase 2t (per point): winners written into their buckets, and their
 // endpoint-table slots released (every point has read its slot by now).
@@ -1147,12 +1085,7 @@ __global__ void __launch_bounds__(256) k_scan_scatter(const BatchHdr* __restrict
       o.w = run; run += v[k].w;
       f[k] = o;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 255) {
-      sc.counters[0] = run;
-      // the one scan's winners are all the fresh pass's (split 0) or none
-      if (sc.counters[kFreshWords + 2] != kNone)
-        sc.counters[kFreshWords + 3] = sc.counters[kFreshWords + 2] == 0u ? 0u : run;
-    }
+    if (blockIdx.x == 0 && threadIdx.x == 255) sc.counters[0] = run;
     __syncthreads();
   }
   if (key == kNone) return;
@@ -1163,16 +1096,15 @@ __global__ void __launch_bounds__(256) k_scan_scatter(const BatchHdr* __restrict
   sc.tpos[gi] = kLeafLater;
 }
 
-// The passes over the winners' rays (walk_winners).
-enum : int { kPassLeaves = 0, kPassUpdate = 1, kPassFresh = 2 };
-
 // cells a lane may run ahead of its wavefront's slowest ray when rays are
-// walked whole: update pass and leaf pass (defaults; the tuning keys
-// ray_window and leaf_window set them per context.  Measured on 64 scans
-// re-inserted into filled maps: 8 beats 4 and 16 for the update pass, 32
-// beats 16 for the leaf pass)
-constexpr int32_t kSyncWindowCells = 8;
-constexpr int32_t kSyncWindowLeaves = 32;
+// walked whole: update pass (in a map empty at the scan's start, and in
+// others) and leaf pass; the defaults of the tuning keys fresh_window,
+// ray_window and leaf_window.  Measured on 64 scans: re-inserted 8 beats 4 and
+// 16 (3.7 against 4.2 and 4.1 ms); leaf pass 64: 0.50, 16: 0.60, none: 0.49
+// re-inserted, 0.92, 1.04, 0.98 ms into empty maps
+constexpr int32_t kFreshWindow = 16;
+constexpr int32_t kUpdateWindow = 8;
+constexpr int32_t kLeafWindow = 64;
 constexpr uint32_t kMaxSegLog = 3;  // at most 8 segments a ray
 constexpr uint32_t kGroupLog = 3;   // batches side by side on one XCD in a short list
 
@@ -1192,35 +1124,21 @@ constexpr uint32_t kGroupLog = 3;   // batches side by side on one XCD in a shor
 // sees neighbours at one distance from the sensor.  A long list is cut into
 // one contiguous part an XCD (a map's rays stay on one XCD or two); there the
 // rays are walked whole, in lockstep: a lane more than the window's cells
-// ahead of the wavefront's slowest ray waits a step.  The fresh pass takes
-// ray_chunk / 64 consecutive batches a wavefront: neighbouring batches that
-// run at the same time race for the same leaves (1: 3.6 ms, 4: 3.0 ms, 8:
-// 3.5 ms a 64-map frame).
+// ahead of the wavefront's slowest ray waits a step.
 //
 // Measured against persistent wavefronts that took rays from 8 cursors and
 // refilled their lanes one by one in short lists (us a call; leaf pass /
 // update pass): 2,001-point scan 61 / 31 -> 14 / 25, 307k-point depth frame
-// 70 / 61 -> 10 / 14, 65k-point LiDAR scan at 50 m 210 / 385 -> 99 / 224;
-// 64 maps 1149 / 4538 -> 600 / 3750, fresh pass 3047 -> 3000.  Bound: the
-// dependent loads of a step (entry, cells) and the scattered lines they touch.
+// 70 / 61 -> 10 / 14, 65k-point LiDAR scan at 50 m 210 / 385 -> 40 / 224;
+// 64 maps 1149 / 4538 -> 500 / 3750 (leaf pass with its want bits).  Bound:
+// the dependent loads of a step (entry, cells) and the scattered lines they
+// touch.
 //
-// kMode 0: leaf allocation pass; 1: update pass; 2: counted update; 3: fresh
-// pass (maps empty at the scan's start: create and mark in one walk); 4:
-// counted fresh pass.
+// kMode 0: leaf allocation pass; 1: update pass; 2: counted update.
 template <int kMode>
 __device__ void walk_winners(const ScanDesc* __restrict__ sd, const ScanScratch& sc) {
-  constexpr bool kCounted = kMode == 2 || kMode == 4;
-  constexpr bool kFreshPass = kMode >= 3;
-  constexpr int kPass = kMode == 0 ? kPassLeaves : (kFreshPass ? kPassFresh : kPassUpdate);
-  constexpr bool leaf_pass = kPass != kPassUpdate;
-  if (kFreshPass && !sc.fresh_pass) return;
-  // the pass's part of the winner list: with a split, the fresh scans'
-  // winners end the list
-  const uint32_t total = sc.counters[0];
-  const bool split = sc.counters[kFreshWords + 2] != kNone;
-  const uint32_t at = split ? sc.counters[kFreshWords + 3] : 0u;
-  const uint32_t w0 = (split && kFreshPass) ? at : 0u;
-  const uint32_t nwin = split ? (kFreshPass ? total - at : at) : total;
+  constexpr bool kLeaves = kMode == 0;
+  const uint32_t nwin = sc.counters[0];
   const uint32_t nb = (nwin + 63u) >> 6;
   // the wavefront's number among those of its XCD (the grid is a multiple of
   // kXcds workgroups)
@@ -1236,25 +1154,12 @@ __device__ void walk_winners(const ScanDesc* __restrict__ sd, const ScanScratch&
   uint32_t gl = kGroupLog;  // fewer batches a group where that would leave XCDs idle
   while (gl > 0 && (nb >> gl) < 8u * kXcds) --gl;
   const uint32_t per_xcd = (nb + kXcds - 1) / kXcds;
-  const uint32_t run = kFreshPass ? max(sc.chunk_max / 64u, 1u) : 1u;
-  const int32_t wcells = sc.win_cells > 0 ? sc.win_cells : kSyncWindowCells;
-  const int32_t win = kMode == 0 ? (sc.win_leaves > 0 ? sc.win_leaves : kSyncWindowLeaves)
-                                 : (kFreshPass && sc.win_fresh > 0 ? sc.win_fresh : wcells);
-  uint32_t round = 0, in_run = 0;  // rounds of the grid over the list
-  for (;;) {
+  for (uint32_t j = wave;; j += waves) {
     uint32_t batch, seg = 0;
     if (lockstep) {
-      const uint32_t first = round * waves * run;
-      if (first >= per_xcd) break;
-      const uint32_t j = first + wave * run + in_run;
-      if (++in_run == run) {
-        in_run = 0;
-        ++round;
-      }
-      batch = j < per_xcd ? xcd * per_xcd + j : nb;
+      if (j >= per_xcd) break;
+      batch = xcd * per_xcd + j;
     } else {
-      const uint32_t j = round * waves + wave;
-      ++round;
       const uint32_t group = (j >> (gl + lg)) * kXcds + xcd;
       if ((group << gl) >= nb) break;
       batch = (group << gl) + (j & ((1u << gl) - 1u));
@@ -1263,7 +1168,7 @@ __device__ void walk_winners(const ScanDesc* __restrict__ sd, const ScanScratch&
     if (batch >= nb) continue;
     const uint32_t idx = batch * 64u + lane;
     const bool valid = idx < nwin;
-    const uint32_t gi = valid ? sc.winners[w0 + idx] : 0u;
+    const uint32_t gi = valid ? sc.winners[idx] : 0u;
     const int4 r = valid ? sc.rec[gi] : make_int4(0, 0, 0, 0);
     const uint32_t s = (uint32_t)r.w >> 16;
     // one scan at a time (a batch seldom holds two), so that the scan's and
@@ -1278,21 +1183,18 @@ __device__ void walk_winners(const ScanDesc* __restrict__ sd, const ScanScratch&
       const MapView m = uniform_view(d.map);
       const int32_t cur = uniform_i32(&m.ctr->cur);
       const uint32_t lbase = (uint32_t)uniform_i32((const int32_t*)&m.ctr->leaf_base);
-      // with sc.fresh_pass set, the rays of a map that was empty when the scan
-      // started (leaf_base 0: every leaf the scan touches is new) take only
-      // the fresh pass, and the other maps' rays only the leaf and update passes
-      if (sc.fresh_pass ? ((kPass == kPassFresh) != (lbase == 0)) : kPass == kPassFresh) continue;
-      if (kPass != kPassLeaves && (map_status(m) & kFatal)) continue;
+      if (!kLeaves && (map_status(m) & kFatal)) continue;
+      const int32_t win = kLeaves ? sc.win_leaves : (lbase == 0 ? sc.win_fresh : sc.win_cells);
       const int32_t ox = d.ox, oy = d.oy, oz = d.oz;
       const bool no_rays = (d.flags & kScanNoRays) != 0;
       RayWalk w;
       w.init(ox, oy, oz, r.x, r.y, r.z);
       // the update pass walks cells [0, mx) of the ray (none for an endpoint
-      // in the origin's voxel or a scan without rays); the leaf and fresh
-      // passes also the endpoint's cell mx, so that they create the winner's
-      // endpoint leaf (only that cell for a scan without rays)
-      bool have = act && (leaf_pass || !no_rays);
-      const int32_t last = w.mx + (leaf_pass ? 1 : 0);
+      // in the origin's voxel or a scan without rays); the leaf pass also the
+      // endpoint's cell mx, so that it creates the winner's endpoint leaf
+      // (only that cell for a scan without rays)
+      bool have = act && (kLeaves || !no_rays);
+      const int32_t last = w.mx + (kLeaves ? 1 : 0);
       // segment seg of n = 2^lg walks cells [ceil(seg last / n), ceil((seg +
       // 1) last / n)): segment 0 holds cell 0, and they cover the ray once
       const int64_t up = (1ll << lg) - 1;
@@ -1313,47 +1215,37 @@ __device__ void walk_winners(const ScanDesc* __restrict__ sd, const ScanScratch&
       RootCache rc;
       rc.reset();
       uint32_t next_leaf = kNone;
-      // fresh pass: root slot and inner-grid entry of the current cell's leaf
-      int32_t slot = -1;
-      uint32_t entry = kEmptyChild;
-      bool stopped = false;
       uint32_t nupd = 0;
-      uint64_t c_vis = 0;
-      const bool ray_first = have && seg == 0 && w.k < w.mx;
-      if (kMode == 0 && have) lw.init(w, m.lb);
-      if (kPass == kPassUpdate && have) next_leaf = walk_leaf(m, w, rc);
-      if (kFreshPass && have) fresh_entry(m, w, rc, slot, entry);
-      if (kCounted && have) c_vis = (uint32_t)max(0, min(w.kend, w.mx) - w.k);
+      const uint32_t ncells = have ? (uint32_t)(w.kend - w.k) : 0u;
+      if (kLeaves && have) lw.init(w, m.lb);
+      if (!kLeaves && have) next_leaf = walk_leaf(m, w, rc);
       while (__ballot(have)) {
         bool go = have;
         if (lockstep) {
-          const int32_t kk = kMode == 0 ? lw.k : w.k;
-          int32_t kmin = wave_min(have ? kk : 0x7fffffff);
-          go = have && kk < kmin + win;
-          if (__ballot(go) == 0) go = have;
+          const int32_t k = kLeaves ? lw.k : w.k;
+          go = have && k < wave_min(have ? k : 0x7fffffff) + win;
+          if (__ballot(go) == 0) go = have;  // a window that wraps past 2^31
         }
-        if (go) {
-          if (kMode == 0) {
-            leaves_step(m, lw, rc);
-          } else if (kFreshPass) {
-            nupd += fresh_step<kCounted>(m, w, rc, slot, entry, stopped, &sc.tpos[gi]);
-          } else {
-            nupd += apply_step<kCounted>(m, w, rc, cur, lbase, next_leaf);
-          }
-          if (kMode == 0 ? lw.done() : (w.done() || stopped)) have = false;
+        if (kLeaves) {
+          leaves_step(m, lw, rc, lbase == 0 ? m.want : m.have, go);
+          have = have && !(go && lw.done());
+        } else if (go) {
+          nupd += apply_step<kMode == 2>(m, w, rc, cur, lbase, next_leaf);
+          have = !w.done();
         }
       }
-      if (kCounted && act) {
+      if (kMode == 2 && ncells) {
         add64(&m.ctr->stat_ray_updates, nupd);
-        add64(&m.ctr->stat_rays, ray_first ? 1u : 0u);
-        add64(&m.ctr->stat_ray_visits, c_vis);
+        add64(&m.ctr->stat_rays, seg == 0 ? 1u : 0u);
+        add64(&m.ctr->stat_ray_visits, ncells);
       }
     }
   }
 }
 
-// Phase 2b: every leaf on every winner's ray is created before any cell is
-// written (so a pool overflow leaves the map's cells untouched).
+// Phase 2b: the leaves on every winner's ray that do not exist yet are put
+// down as wants (k_scan_new_entries creates them before any cell is written,
+// so a pool overflow leaves the map's cells untouched).
 __global__ void __launch_bounds__(256) k_scan_ray_leaves(const ScanDesc* __restrict__ sd,
                                                          ScanScratch sc) {
   walk_winners<0>(sd, sc);
@@ -1367,16 +1259,99 @@ __global__ void __launch_bounds__(256) k_scan_extra_leaves(const BatchHdr* __res
   const ScanDesc& d = sd[blockIdx.x];
   if (d.flags & kScanNoRays) return;
   const MapView m = load_view(d.map);
-  for (uint32_t j = threadIdx.x; j < d.nextra; j += blockDim.x) {
-    const int4 e = d.extra[j];
-    if (e.x == d.ox && e.y == d.oy && e.z == d.oz) continue;
+  // whole wavefronts: leaves_step is a wavefront collective
+  for (uint32_t j0 = threadIdx.x & ~63u; j0 < d.nextra; j0 += blockDim.x) {
+    const uint32_t j = j0 + lane_id();
+    const int4 e = j < d.nextra ? d.extra[j] : make_int4(d.ox, d.oy, d.oz, 0);
+    bool have = !(e.x == d.ox && e.y == d.oy && e.z == d.oz);
     RayWalk w;
     RootCache rc;
     rc.reset();
     w.init(d.ox, d.oy, d.oz, e.x, e.y, e.z);
     LeafWalk lw;
     lw.init(w, m.lb);
-    while (!lw.done()) leaves_step(m, lw, rc);
+    while (__ballot(have)) {
+      leaves_step(m, lw, rc, m.have, have);
+      if (have && lw.done()) have = false;
+    }
+  }
+}
+
+// Phase 2d (per root directory word of each scan's map): the leaves wanted by
+// the leaf pass are created (allocateLeafGrid and GridBlockAllocator::
+// allocateBlock, bonxai.hpp:572-586 and grid_allocator.hpp:94-123): a
+// wavefront takes the words of 64 inner cells that have wants, reads their
+// entries, takes one bump of the map's leaf counter for up to
+// kEntryRun words, writes origins and entries and the have bits, and clears
+// the wants.  Entries that hold a leaf after all (have bits are hints) are
+// passed over.  A map whose pool is too small is flagged, the entries past
+// its end stay EMPTY, and no cell has been written (the host grows the pool
+// and runs the call again).  Bound: reading the want words of the whole
+// directory (8 KB a 1,024-root directory), then a chain of loads, one
+// atomic and stores.
+constexpr uint32_t kEntryRun = 8;
+__global__ void __launch_bounds__(256) k_scan_new_entries(const BatchHdr* __restrict__ hdr,
+                                                          const ScanDesc* __restrict__ sd) {
+  const uint32_t lane = lane_id();
+  const uint32_t wave = blockIdx.x * (blockDim.x >> 6) +
+                        (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t nwaves = gridDim.x * (blockDim.x >> 6);
+  const uint32_t nscans = hdr->nscans;
+  uint32_t turn = wave;  // the maps' words follow each other round the wavefronts
+  for (uint32_t s = 0; s < nscans; ++s) {
+    const MapView m = uniform_view(sd[s].map);
+    const uint32_t ew = entry_words(m.isz);
+    const uint64_t nwords = (uint64_t)(m.root_mask + 1) * ew;
+    const uint32_t first = turn;
+    turn = (turn + nwaves - (uint32_t)((nwords / 64) % nwaves)) % nwaves;
+    for (uint64_t e0 = (uint64_t)first * 64; e0 < nwords; e0 += (uint64_t)nwaves * 64) {
+      const uint64_t want = m.want[e0 + lane];  // nwords is a multiple of 64
+      uint64_t pending = __ballot(want != 0);
+      if (!pending) continue;
+      if (want) m.want[e0 + lane] = 0;
+      while (pending) {
+        uint32_t l[kEntryRun], child[kEntryRun];
+        uint64_t make[kEntryRun];
+#pragma unroll
+        for (uint32_t k = 0; k < kEntryRun; ++k) {
+          l[k] = pending ? (uint32_t)__ffsll((unsigned long long)pending) - 1u : 64u;
+          pending &= pending - 1;
+          // a word's 64 entries (fewer in small inner grids), one a lane
+          child[k] = l[k] < 64u && lane < m.isz ? m.children[(e0 + l[k]) / ew * m.isz + (e0 + l[k]) % ew * 64 + lane]
+                                                : 0u;
+        }
+        uint32_t n = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < kEntryRun; ++k) {
+          make[k] = l[k] < 64u ? lane_value(want, l[k]) & __ballot(child[k] == kEmptyChild) : 0ull;
+          n += (uint32_t)__popcll(make[k]);
+        }
+        uint32_t base = 0;
+        if (n && lane == 0) base = add32(&m.ctr->leaf_count, n);
+        base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+#pragma unroll
+        for (uint32_t k = 0; k < kEntryRun; ++k) {
+          if (l[k] >= 64u) continue;
+          const uint64_t e = e0 + l[k];
+          const uint32_t slot = (uint32_t)(e / ew), ci = (uint32_t)(e % ew) * 64u + lane;
+          const uint32_t idx = base + (uint32_t)__popcll(make[k] & lanes_below());
+          const bool mine = (make[k] >> lane) & 1ull;
+          if (mine && idx < m.leaf_cap) {
+            int32_t x, y, z;
+            unpack_root(m.root_keys[slot], m.log2n, &x, &y, &z);
+            const uint32_t im = (1u << m.ib) - 1;
+            m.origin[idx] = make_int4(x + (int32_t)((ci & im) << m.lb), y + (int32_t)(((ci >> m.ib) & im) << m.lb),
+                                      z + (int32_t)((ci >> (2 * m.ib)) << m.lb), (int32_t)slot);
+            m.children[(uint64_t)slot * m.isz + ci] = idx;
+            child[k] = idx;
+          }
+          const uint64_t have = __ballot(lane < m.isz && child[k] < kPendingChild);
+          if (lane == 0) m.have[e] = have;
+          if (mine && idx >= m.leaf_cap) or32(&m.ctr->status, kStOutOfPool);
+          base += (uint32_t)__popcll(make[k]);
+        }
+      }
+    }
   }
 }
 
@@ -1385,13 +1360,11 @@ __global__ void __launch_bounds__(256) k_scan_extra_leaves(const BatchHdr* __res
 // that existed before the scan.  One writer per endpoint cell.  An endpoint
 // in a leaf the scan created is left for k_scan_new_endpoints (after the ray
 // pass): its leaf index goes to tpos.  In a map empty at the scan's start
-// every endpoint leaf is new: the fresh pass, which runs after this kernel,
-// creates it and stores its index in tpos (kLeafLater until then:
-// k_scan_new_endpoints looks up any it did not), so there is nothing to do.
+// every endpoint leaf is new, and k_scan_new_endpoints looks it up (tpos
+// stays kLeafLater): there is nothing to do here.
 __global__ void __launch_bounds__(256) k_scan_endpoints(const ScanDesc* __restrict__ sd,
                                                         ScanScratch sc) {
-  // with a split the fresh scans' winners end the list
-  const uint32_t nwin = sc.counters[kFreshWords + 2] != kNone ? sc.counters[kFreshWords + 3] : sc.counters[0];
+  const uint32_t nwin = sc.counters[0];
   const uint32_t stride = gridDim.x * blockDim.x;
   const uint32_t start = blockIdx.x * blockDim.x + threadIdx.x;
   // every lane runs the same number of iterations so the count reduction
@@ -1405,11 +1378,11 @@ __global__ void __launch_bounds__(256) k_scan_endpoints(const ScanDesc* __restri
       const int4 r = sc.rec[gi];
       const ScanDesc& d = sd[(uint32_t)r.w >> 16];
       const MapView m = load_view(d.map);
-      const bool failed = (map_status(m) & kFatal) != 0;
       const uint32_t lbase = *gp(&m.ctr->leaf_base);
-      const uint32_t leaf = (failed || lbase == 0) ? kNone : find_leaf(m, r.x, r.y, r.z);
+      const bool skip = lbase == 0 || (map_status(m) & kFatal) != 0;
+      const uint32_t leaf = skip ? kNone : find_leaf(m, r.x, r.y, r.z);
       const bool fresh = leaf != kNone && leaf >= lbase;
-      sc.tpos[gi] = fresh ? leaf : (lbase == 0 && !failed ? kLeafLater : kNone);
+      if (!skip) sc.tpos[gi] = fresh ? leaf : kNone;
       if (leaf != kNone && !fresh) {
         const uint32_t li = leaf_index(r.x, r.y, r.z, m.lb);
         uint32_t BXG_G* cell = (uint32_t BXG_G*)m.cells + (uint64_t)leaf * m.lsz + li;
@@ -1435,8 +1408,7 @@ __global__ void __launch_bounds__(256) k_scan_endpoints(const ScanDesc* __restri
 
 // Phase 4d (per winner): the endpoint update of the endpoints in leaves the
 // scan created (k_scan_endpoints left their leaf index in tpos, or
-// kLeafLater where the fresh pass was still to create it).  Such a
-// cell held zero before the scan, so its endpoint word is cell_hit(0) or
+// kLeafLater in maps empty at the scan's start).  Such a cell held zero before the scan, so its endpoint word is cell_hit(0) or
 // cell_miss(0), whatever ray marked it meanwhile (the reference updates
 // endpoints first and its rays skip them, probabilistic_map.cpp:30-54,
 // 81-89): its touched byte becomes 2 (hit) or 1 (miss), one writer per
@@ -1494,15 +1466,6 @@ template <bool kCount>
 __global__ void __launch_bounds__(256) k_scan_rays(const ScanDesc* __restrict__ sd,
                                                    ScanScratch sc) {
   walk_winners<kCount ? 2 : 1>(sd, sc);
-}
-
-// Phase 4' (per winner of a map empty at the scan's start, with
-// ScanScratch::fresh_pass): leaf creation and the ray clear in one walk (the
-// leaf pass and the update pass skip these rays).
-template <bool kCount>
-__global__ void __launch_bounds__(256) k_scan_fresh_rays(const ScanDesc* __restrict__ sd,
-                                                         ScanScratch sc) {
-  walk_winners<kCount ? 4 : 3>(sd, sc);
 }
 
 // Phase 4b (one block per scan): rays due from addHitPoint / addMissPoint.
@@ -1648,26 +1611,13 @@ __global__ void k_na_recover(MapCounters* __restrict__ ctr, uint32_t leaf_cap) {
 
 // Phase 0 (per scan): the leaf count at the start of the scan, so that later
 // phases can tell the leaves the scan creates from older ones.
-// With the fresh pass, also the scans whose map is empty (their winners get
-// the highest bucket tags: the fresh pass walks the end of the list, the
-// other passes the rest).
 template <class Desc>
 __device__ __forceinline__ void scan_begin(uint32_t nscans, const Desc* sd, const ScanScratch& sc) {
   for (uint32_t s = threadIdx.x; s < nscans; s += blockDim.x) {
     const MapDev BXG_G* m = gp((const MapDev*)sd[s].map);
     MapCounters BXG_G* ctr = gp(m->ctr);
-    const uint32_t base = min(ctr->leaf_count, m->leaf_cap);
-    ctr->leaf_base = base;
-    if (nscans <= 64u) {  // the first wavefront holds every scan
-      const uint64_t fresh = __ballot(sc.fresh_pass && base == 0);
-      if (threadIdx.x == 0) {
-        sc.counters[kFreshWords] = (uint32_t)fresh;
-        sc.counters[kFreshWords + 1] = (uint32_t)(fresh >> 32);
-        sc.counters[kFreshWords + 2] = sc.fresh_pass ? nscans - (uint32_t)__popcll(fresh) : kNone;
-      }
-    }
+    ctr->leaf_base = min(ctr->leaf_count, m->leaf_cap);
   }
-  if ((nscans > 64u || nscans == 0u) && threadIdx.x == 0) sc.counters[kFreshWords + 2] = kNone;
   if (threadIdx.x < 64u) sc.counters[kClipWords + threadIdx.x] = 0;
 }
 __global__ void k_scan_begin(const BatchHdr* __restrict__ hdr, const ScanDesc* __restrict__ sd,
@@ -2052,12 +2002,6 @@ __global__ void __launch_bounds__(256) k_classify_cells(const MapDev* __restrict
 
 // ------------------------------------------------------ whole-map passes
 
-// value of lane l (the same l in every lane), 64 bits
-__device__ __forceinline__ uint64_t lane_value(uint64_t v, uint32_t l) {
-  return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, (int)l) |
-         ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), (int)l) << 32);
-}
-
 // forEachCell (bonxai.hpp:704-743) as a compaction; filter 0 all, 1 p >
 // threshold, 2 p < threshold.  A wavefront takes `words` mask words (64 cells
 // each; 4 to 32): one lane holds each word, reduced by the filter to the
@@ -2373,16 +2317,19 @@ __global__ void __launch_bounds__(256) k_compact_leaves(
 }
 
 // clear(CLEAR_MEMORY): directory keys and entries to all ones (kEmptyKey,
-// kEmptyChild), bump counters and status to zero.  cap is a power of two >=
+// kEmptyChild), have bits, bump counters and status to zero.  cap is a power of two >=
 // 1024, so both arrays are whole 16-byte words.
 __global__ void __launch_bounds__(256) k_map_clear(uint64_t* __restrict__ keys, uint32_t* __restrict__ children,
-                                                   uint64_t cap, uint32_t isz, MapCounters* __restrict__ ctr) {
+                                                   uint64_t* __restrict__ have, uint64_t cap, uint32_t isz,
+                                                   MapCounters* __restrict__ ctr) {
   static_assert(kEmptyKey == ~0ull && kEmptyChild == ~0u, "all ones");
   const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   const uint4 ones = make_uint4(~0u, ~0u, ~0u, ~0u);
   for (uint64_t i = t; i < cap / 2; i += stride) reinterpret_cast<uint4*>(keys)[i] = ones;
   for (uint64_t i = t; i < cap * isz / 4; i += stride) reinterpret_cast<uint4*>(children)[i] = ones;
+  if (have)
+    for (uint64_t i = t; i < cap * entry_words(isz); i += stride) have[i] = 0;
   if (t == 0) ctr->leaf_count = ctr->root_count = ctr->status = 0;
 }
 

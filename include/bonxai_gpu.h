@@ -138,15 +138,12 @@ int bxg_set_counting(bxg_ctx* ctx, int on);
  * "small_ray_blocks_per_cu" (1..64, default 32), the workgroups per CU that
  * the passes of a small call fill by cutting its rays into up to 8 segments;
  * "ray_block" (64..256, default 64), the workgroup size of the passes;
- * "ray_chunk" (64..1024, default 256), the rays a wavefront of the fresh
- * pass walks, 64 at a time; "ep_table_factor", "root_slack"; "ray_window"
- * (default 8) and "leaf_window" (default 32), how many cells / leaves a ray
- * may run ahead of the slowest ray of its wavefront; "fresh_pass" (default
- * 1): the rays of a map that is empty when its scan starts create their
- * leaves and mark their cells in one walk (0: the leaf pass and the update
- * pass, as for other maps); "fresh_blocks_per_cu" (default 128)
- * and "fresh_window" (default 16), that walk's most workgroups per CU and
- * lockstep window in cells; "ray_order" (0..5, default 3): the order in which the rays
+ * "ep_table_factor", "root_slack"; "ray_window" (default 8), "fresh_window"
+ * (default 16) and "leaf_window" (default 64), how many cells a ray may run
+ * ahead of the slowest ray of its wavefront in the update pass, in the
+ * update pass of maps that are empty when their scan starts, and in the leaf
+ * pass; "ray_chunk", "fresh_pass" and "fresh_blocks_per_cu" are accepted for
+ * settings recorded by earlier versions and have no effect; "ray_order" (0..5, default 3): the order in which the rays
  * of a scan are walked, by direction only (0) or by classes of length (equal
  * parts of the max range) and direction: 1 and 2 are 4 classes over 32 x 32
  * and 16 classes over 16 x 16 direction bins, 3 and 4 the latter under 8 and

@@ -133,3 +133,57 @@ def test_passes_left_out(fresh_pass):
     for x in maps + models + [e, oe]:
         x.close()
     c.close()
+
+
+@pytest.mark.parametrize("bits", [(1, 3), (2, 1), (3, 2), (4, 2), (4, 4)])
+def test_new_entries_of_other_grids(ctx, bits):
+    """Leaf creation with 1, 8 and 64 words of wanted leaves a root (and roots
+    of fewer than 64 leaves): same cells, and exactly the leaves the cells and
+    rays need (each holds a cell that is on, every scan cell being on)."""
+    import bonxai_amd as bx
+    import oracle
+
+    m = bx.ProbabilisticMap.__new__(bx.ProbabilisticMap)
+    bx.VoxelGrid.__init__(m, ctx, 0.1, *bits, np.uint32, _flags=bx.MAP_PROBABILISTIC)
+    om = oracle.ProbMap(0.1)
+    for k in range(3):
+        p = _sphere(3_000, 9.0, 60 + k)
+        o = np.array([0.5 * k, -0.3 * k, 0.05])
+        m.insert_point_cloud(p, o, 10.0)
+        om.insert_point_cloud(p, o, 10.0)
+        assert_same_cells(m.cells(), om.cells(), f"bits {bits}, scan {k}")
+        leaves = np.unique(om.cells()[0] >> bits[1], axis=0)
+        assert m.stats()["leaf_count"] == len(leaves)
+    m.close()
+    om.close()
+
+
+def test_leaves_made_and_removed_between_scans(ctx):
+    """Leaves that bulk calls create, and leaves that releaseUnusedMemory
+    removes, between the scans of one map: the scan's bits of existing leaves
+    are hints, and no leaf is made twice or missed."""
+    import bonxai_amd as bx
+    import oracle
+    m, om = bx.ProbabilisticMap(ctx, 0.1), oracle.ProbMap(0.1)
+    a, b = _sphere(2_000, 5.0, 1), _sphere(2_000, 7.0, 2)
+    far = np.stack([np.arange(400) % 100 - 50, np.arange(400) // 100 * 9, np.full(400, 3)], 1).astype(np.int32)
+    words = np.full(len(far), (1000 << 4) | 3, np.uint32)
+    m.set_values(far, words)
+    om.grid.set_values(far, words)
+    for p, o in ((a, [0.1, 0.2, 0.3]), (b, [0.4, 0.2, 0.3])):
+        m.insert_point_cloud(p, np.array(o), 8.0)
+        om.insert_point_cloud(p, np.array(o), 8.0)
+    assert_same_cells(m.cells(), om.cells(), "after bulk calls")
+    c = om.cells()[0]
+    gone = c[c[:, 0] > 10]
+    m.set_cells_off(gone)
+    om.grid.set_cells_off(gone)
+    m.release_unused_memory()
+    om.grid.release_unused()
+    for p, o in ((b, [0.2, 0.2, 0.3]), (a, [0.1, 0.3, 0.3])):
+        m.insert_point_cloud(p, np.array(o), 8.0)
+        om.insert_point_cloud(p, np.array(o), 8.0)
+    assert_same_cells(m.cells(), om.cells(), "after releaseUnusedMemory")
+    assert m.stats()["leaf_count"] == len(np.unique(om.cells()[0] >> 3, axis=0))
+    m.close()
+    om.close()
