@@ -476,7 +476,7 @@ int grow_leaves(bxg_map* m, uint64_t need) {
   if (tb) BXG_TRY(dmalloc(c, &touched, cap * tb));
   // the leaves in use move over; the rest of the pool stays uninitialised
   // (a leaf is written whole when it is created).  Touched marks start at
-  // zero, and every scan leaves them so.
+  // zero, no life's mark.
   if (tb) BXG_HIP(c, hipMemsetAsync(touched, 0, cap * tb, c->stream));
   if (used) {
     BXG_HIP(c, hipMemcpyAsync(masks, m->h.leaf_masks, used * lw * 8, hipMemcpyDeviceToDevice, c->stream));
@@ -1610,12 +1610,19 @@ int bxg_map_clear(bxg_map* m, int option) {
   // the old leaves' bytes stay: a leaf is written whole when it is created).
   // Enqueued like the other calls on the map (two fills, two copies and a
   // wait cost 60 us a map)
+  uint32_t life = m->h_ctr->life;
+  if (is_prob(m) && ++life == kLives) {  // the marks' values start over
+    life = 0;
+    BXG_TRY(fill64(c, (uint64_t*)m->h.touched, (uint64_t)m->leaf_cap * m->h.leaf_size / 8, 0));
+  }
   const uint64_t n16 = (uint64_t)m->root_cap * root_bytes(m) / 16;
   BXG_TRY(launch(c, "k_map_clear", k_map_clear, (uint32_t)std::min<uint64_t>(nblocks(n16), 4096), kBlock,
-                 m->h.root_keys, m->h.children, m->h.leaf_have, (uint64_t)m->root_cap, m->h.inner_size, m->ctr));
+                 m->h.root_keys, m->h.children, m->h.leaf_have, (uint64_t)m->root_cap, m->h.inner_size,
+                 m->ctr, life));
   m->cleared = true;
   m->extra.clear();
   m->h_ctr->leaf_count = m->h_ctr->root_count = m->h_ctr->status = 0;
+  m->h_ctr->life = life;
   m->known_leaves = m->known_roots = 0;
   return BXG_OK;
 }

@@ -21,8 +21,11 @@
 //                    cells[(leaf * leaf_size + n) * value_bytes]
 //                    leaf_origin[leaf] = min-corner coordinate of the leaf.
 //                    touched[leaf * leaf_size + n] (probabilistic maps): one
-//                    byte a cell, nonzero only while a scan runs, for the
-//                    cells that scan updates in the leaves it creates.
+//                    byte a cell, the marks of the scan that created the leaf:
+//                    mark_miss or mark_hit of the map's life for the cells it
+//                    updated.  Nobody clears them: a pool index is handed out
+//                    once in a map's life (until clear), other lives' marks
+//                    mean nothing, and the bytes are zeroed every kLives clears.
 //
 // Invariant kept by every kernel: a cell whose mask bit is off holds all-zero
 // bytes.  The reference never reads an off cell's storage (value() returns
@@ -76,7 +79,7 @@ struct alignas(128) MapCounters {
   // leaf_count when the running scan or bulk call started: leaves at or
   // above it were created by that call, and it initialises them
   uint32_t leaf_base;
-  uint32_t pad1;
+  uint32_t life;  // the map's life (clears, mod kLives): its touched marks (mark_miss)
   uint64_t scans_applied;
   uint64_t pad2[13];
   uint64_t stat_endpoint_updates;
@@ -88,6 +91,11 @@ struct alignas(128) MapCounters {
 static_assert(sizeof(MapCounters) == 384, "MapCounters is three cache lines");
 static_assert(offsetof(MapCounters, status) == 128 && offsetof(MapCounters, stat_endpoint_updates) == 256,
               "MapCounters lines");
+
+// touched marks of a life: 1 and 2, 3 and 4, ... 253 and 254
+constexpr uint32_t kLives = 127;
+__host__ __device__ inline uint32_t mark_miss(uint32_t life) { return 2 * life + 1; }
+__host__ __device__ inline uint32_t mark_hit(uint32_t life) { return 2 * life + 2; }
 
 struct alignas(64) MapDev {
   double inv_res;

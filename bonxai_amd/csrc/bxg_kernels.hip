@@ -596,13 +596,14 @@ __device__ __forceinline__ uint32_t walk_leaf(const MapView& m, const RayWalk& w
 // cells was off (zero) before it, and the ray update of such a cell gives the
 // same word whichever ray gets there first, cell_miss(0).  So a run in a new
 // leaf only marks its cells in the leaf's touched bytes (plain byte stores of
-// 1, every writer agreeing; no read, no atomic), and k_scan_new_leaves writes
+// the miss mark, every writer agreeing; no read, no atomic), and k_scan_new_leaves writes
 // the leaf's cells and mask words from those bytes after the scan's endpoints
 // are marked.  In older leaves each cell is read, updated unless its
 // update_id is cur, and the cells turned on set their mask bits with atomicOrs.
 template <bool kCount>
 __device__ __forceinline__ uint32_t apply_step(const MapView& m, RayWalk& w, RootCache& rc,
-                                               int32_t cur, uint32_t lbase, uint32_t& next_leaf) {
+                                               int32_t cur, uint32_t lbase, uint32_t mark,
+                                               uint32_t& next_leaf) {
   const uint32_t leaf = next_leaf;
   uint32_t li[kRun];
   const uint32_t n = collect_run(m, w, li);
@@ -615,11 +616,17 @@ __device__ __forceinline__ uint32_t apply_step(const MapView& m, RayWalk& w, Roo
     for (int j = 0; j < kRun; ++j) {
       if ((uint32_t)j < n) {
         if (kCount) {
-          // exact first marks: an atomic or on the byte's aligned word
+          // exact first marks: a CAS on the byte's aligned word
           const uint32_t sh = (li[j] & 3u) * 8u;
-          nupd += ((or32((uint32_t*)(tb + (li[j] & ~3u)), 1u << sh) >> sh) & 0xFFu) == 0u ? 1u : 0u;
+          uint32_t* wp = (uint32_t*)(tb + (li[j] & ~3u));
+          for (uint32_t old = ld32(wp); ((old >> sh) & 0xFFu) != mark;) {
+            const uint32_t seen = cas32(wp, old, (old & ~(0xFFu << sh)) | (mark << sh));
+            nupd += seen == old ? 1u : 0u;
+            if (seen == old) break;
+            old = seen;
+          }
         } else {
-          tb[li[j]] = 1;
+          tb[li[j]] = (uint8_t)mark;
         }
       }
     }
@@ -1203,6 +1210,7 @@ __device__ void walk_winners(const ScanDesc* __restrict__ sd, const ScanScratch&
       const MapView m = uniform_view(d.map);
       const int32_t cur = uniform_i32(&m.ctr->cur);
       const uint32_t lbase = (uint32_t)uniform_i32((const int32_t*)&m.ctr->leaf_base);
+      const uint32_t mark = mark_miss((uint32_t)uniform_i32((const int32_t*)&m.ctr->life));
       if (!kLeaves && (map_status(m) & kFatal)) continue;
       const int32_t win = kLeaves ? sc.win_leaves : (lbase == 0 ? sc.win_fresh : sc.win_cells);
       const int32_t ox = d.ox, oy = d.oy, oz = d.oz;
@@ -1250,7 +1258,7 @@ __device__ void walk_winners(const ScanDesc* __restrict__ sd, const ScanScratch&
           leaves_step(m, lw, rc, lbase == 0 ? m.want : m.have, go);
           have = have && !(go && lw.done());
         } else if (go) {
-          nupd += apply_step<kMode == 2>(m, w, rc, cur, lbase, next_leaf);
+          nupd += apply_step<kMode == 2>(m, w, rc, cur, lbase, mark, next_leaf);
           have = !w.done();
         }
       }
@@ -1431,7 +1439,7 @@ __global__ void __launch_bounds__(256) k_scan_endpoints(const ScanDesc* __restri
 // kLeafLater in maps empty at the scan's start).  Such a cell held zero before the scan, so its endpoint word is cell_hit(0) or
 // cell_miss(0), whatever ray marked it meanwhile (the reference updates
 // endpoints first and its rays skip them, probabilistic_map.cpp:30-54,
-// 81-89): its touched byte becomes 2 (hit) or 1 (miss), one writer per
+// 81-89): its touched byte becomes the hit or the miss mark, one writer per
 // voxel, and k_scan_new_leaves writes the word.  The counted form takes back
 // the ray update the ray pass counted for a cell that turns out to be an
 // endpoint.
@@ -1458,8 +1466,9 @@ __global__ void __launch_bounds__(256) k_scan_new_endpoints(const BatchHdr* __re
       if (leaf == kLeafLater) leaf = (map_status(m) & kFatal) ? kNone : find_leaf(m, r.x, r.y, r.z);
       if (leaf != kNone) {
         uint8_t BXG_G* tb = m.touched + (uint64_t)leaf * m.lsz + leaf_index(r.x, r.y, r.z, m.lb);
-        if (kCount) retracted = *tb != 0u ? 1u : 0u;
-        *tb = (r.w & kRecHit) ? 2 : 1;
+        const uint32_t life = *gp(&m.ctr->life);
+        if (kCount) retracted = *tb == mark_miss(life) ? 1u : 0u;
+        *tb = (uint8_t)((r.w & kRecHit) ? mark_hit(life) : mark_miss(life));
         updated = 1;
         ctr = m.ctr;
       }
@@ -1499,6 +1508,7 @@ __global__ void __launch_bounds__(256) k_scan_extra_rays(const BatchHdr* __restr
   if (map_status(m) & kFatal) return;
   const int32_t cur = map_cur(m);
   const uint32_t lbase = *gp(&m.ctr->leaf_base);
+  const uint32_t mark = mark_miss(*gp(&m.ctr->life));
   for (uint32_t j = threadIdx.x; j < d.nextra; j += blockDim.x) {
     const int4 e = d.extra[j];
     if (e.x == d.ox && e.y == d.oy && e.z == d.oz) continue;
@@ -1508,7 +1518,7 @@ __global__ void __launch_bounds__(256) k_scan_extra_rays(const BatchHdr* __restr
     w.init(d.ox, d.oy, d.oz, e.x, e.y, e.z);
     uint32_t n = 0;
     uint32_t next_leaf = walk_leaf(m, w, rc);
-    while (!w.done()) n += apply_step<kCount>(m, w, rc, cur, lbase, next_leaf);
+    while (!w.done()) n += apply_step<kCount>(m, w, rc, cur, lbase, mark, next_leaf);
     if (kCount) {
       add64(&m.ctr->stat_ray_updates, n);
       add64(&m.ctr->stat_rays, 1);
@@ -1520,14 +1530,16 @@ __global__ void __launch_bounds__(256) k_scan_extra_rays(const BatchHdr* __restr
 // Phase 4c: the leaves the scan created, written whole.  Their cells were
 // all off before the scan (a created leaf is initialised, as the reference's
 // Grid constructor does, bonxai.hpp:51-58), and the scan left in each
-// cell's touched byte what it did there: 0 nothing, 1 a miss (a ray, or a
-// miss endpoint: cell_miss(0)), 2 a hit endpoint (cell_hit(0)).  So every
-// cell word follows from its byte, and the mask is exactly the nonzero bytes
-// (Accessor::value(create) sets the bit, bonxai.hpp:485-490): one pass per
-// new leaf writes its cells and mask words and clears the bytes it read,
-// with no read of the cell pool and no atomic.  The new leaves of each
-// scan's map are [leaf_base, leaf_count); a map whose call failed wrote no
-// byte, and its new leaves are written off (zero).
+// cell's touched byte what it did there: the life's miss mark (a ray, or a
+// miss endpoint: cell_miss(0)), its hit mark (a hit endpoint: cell_hit(0)), or
+// neither (nothing).  So every cell word follows from its byte, and the mask
+// is exactly the marked bytes (Accessor::value(create) sets the bit,
+// bonxai.hpp:485-490): one pass per new leaf writes its cells and mask words,
+// with no read of the cell pool and no atomic.  (Clearing the marks here took
+// 2.78 ms for a frame's 4.12M new leaves; marks that belong to a life need no
+// clearing: 2.43 ms, 4.5 TB/s of the 10.8 GB.)  The new leaves of each scan's
+// map are [leaf_base, leaf_count); those of a failed call are written off
+// (zero).  Bound: HBM.
 constexpr uint32_t kNewLeafRun = 4;  // leaves a wavefront of k_scan_new_leaves has in flight
 __global__ void __launch_bounds__(256) k_scan_new_leaves(const BatchHdr* __restrict__ hdr,
                                                          const ScanDesc* __restrict__ sd) {
@@ -1542,11 +1554,12 @@ __global__ void __launch_bounds__(256) k_scan_new_leaves(const BatchHdr* __restr
     const uint32_t hi = min(ctr->leaf_count, m.leaf_cap);
     if (lo >= hi) continue;
     const int32_t cur = ctr->cur;
-    // a failed call's leaves stay off: its marks (the fresh pass may stop
-    // part-way) are cleared and give no cell
+    // a failed call's leaves stay off: no byte is its mark
     const bool failed = (ctr->status & kFatal) != 0;
-    const uint32_t wmiss = failed ? 0u : cell_miss(0u, m.miss, m.cmin, cur);
-    const uint32_t whit = failed ? 0u : cell_hit(0u, m.hit, m.cmax, cur);
+    const uint32_t bmiss = failed ? ~0u : mark_miss(ctr->life);
+    const uint32_t bhit = failed ? ~0u : mark_hit(ctr->life);
+    const uint32_t wmiss = cell_miss(0u, m.miss, m.cmin, cur);
+    const uint32_t whit = cell_hit(0u, m.hit, m.cmax, cur);
     if (m.lsz == 512) {
       // 8^3 leaves (the default leaf_bits 3): lane l has cells 4l..4l+3 and
       // 256+4l..256+4l+3, so each store instruction writes 1 KB in one piece
@@ -1560,7 +1573,7 @@ __global__ void __launch_bounds__(256) k_scan_new_leaves(const BatchHdr* __restr
         for (uint32_t k = 0; k < kNewLeafRun; ++k) {
           const uint32_t leaf = leaf0 + k * nwaves;
           const uint32_t BXG_G* tp = (const uint32_t BXG_G*)(m.touched + (uint64_t)leaf * 512u) + lane;
-          t[k][0] = leaf < hi ? tp[0] : 0u;
+          t[k][0] = leaf < hi ? tp[0] : 0u;  // (0 is no life's mark)
           t[k][1] = leaf < hi ? tp[64] : 0u;
         }
 #pragma unroll
@@ -1574,12 +1587,11 @@ __global__ void __launch_bounds__(256) k_scan_new_leaves(const BatchHdr* __restr
 #pragma unroll
             for (uint32_t b = 0; b < 4; ++b) {
               const uint32_t cls = (t[k][h] >> (8 * b)) & 0xFFu;
-              v[b] = cls == 0u ? 0u : (cls == 1u ? wmiss : whit);
-              nib |= (cls != 0u && !failed ? 1u : 0u) << b;
+              v[b] = cls == bmiss ? wmiss : (cls == bhit ? whit : 0u);
+              nib |= ((cls == bmiss) | (cls == bhit) ? 1u : 0u) << b;
             }
             u32x4 BXG_G* cp = (u32x4 BXG_G*)(m.cells + (uint64_t)leaf * 2048u + 1024u * h) + lane;
             __builtin_nontemporal_store(u32x4{v[0], v[1], v[2], v[3]}, cp);
-            if (t[k][h]) ((uint32_t BXG_G*)(m.touched + (uint64_t)leaf * 512u + 256u * h))[lane] = 0u;
             // mask word 4h + r: the nibbles of lanes 16r..16r+15, lane 16r + i
             // at bits 4i..4i+3; lanes 16r..16r+7 fill the low half, 16r+8..
             // 16r+15 the high half.  OR over each half-row of 8 lanes (DPP
@@ -1602,16 +1614,13 @@ __global__ void __launch_bounds__(256) k_scan_new_leaves(const BatchHdr* __restr
       }
     } else {
       for (uint32_t leaf = lo + wave; leaf < hi; leaf += nwaves) {
-        uint8_t BXG_G* tb = m.touched + (uint64_t)leaf * m.lsz;
+        const uint8_t BXG_G* tb = m.touched + (uint64_t)leaf * m.lsz;
         uint32_t BXG_G* cells = (uint32_t BXG_G*)m.cells + (uint64_t)leaf * m.lsz;
         for (uint32_t w = 0; w < m.lw; ++w) {
           const uint32_t i = w * 64u + lane;
           const uint32_t cls = i < m.lsz ? tb[i] : 0u;
-          if (i < m.lsz) {
-            cells[i] = cls == 0u ? 0u : (cls == 1u ? wmiss : whit);
-            if (cls) tb[i] = 0;
-          }
-          const uint64_t b = __ballot(cls != 0u && !failed);
+          if (i < m.lsz) cells[i] = cls == bmiss ? wmiss : (cls == bhit ? whit : 0u);
+          const uint64_t b = __ballot((cls == bmiss) | (cls == bhit));
           if (lane == 0) m.masks[(uint64_t)leaf * m.lw + w] = b;
         }
       }
@@ -2336,11 +2345,11 @@ __global__ void __launch_bounds__(256) k_compact_leaves(
 }
 
 // clear(CLEAR_MEMORY): directory keys and entries to all ones (kEmptyKey,
-// kEmptyChild), have bits, bump counters and status to zero.  cap is a power of two >=
+// kEmptyChild), have bits, bump counters and status to zero, the next life.  cap is a power of two >=
 // 1024, so both arrays are whole 16-byte words.
 __global__ void __launch_bounds__(256) k_map_clear(uint64_t* __restrict__ keys, uint32_t* __restrict__ children,
                                                    uint64_t* __restrict__ have, uint64_t cap, uint32_t isz,
-                                                   MapCounters* __restrict__ ctr) {
+                                                   MapCounters* __restrict__ ctr, uint32_t life) {
   static_assert(kEmptyKey == ~0ull && kEmptyChild == ~0u, "all ones");
   const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -2349,7 +2358,10 @@ __global__ void __launch_bounds__(256) k_map_clear(uint64_t* __restrict__ keys, 
   for (uint64_t i = t; i < cap * isz / 4; i += stride) reinterpret_cast<uint4*>(children)[i] = ones;
   if (have)
     for (uint64_t i = t; i < cap * entry_words(isz); i += stride) have[i] = 0;
-  if (t == 0) ctr->leaf_count = ctr->root_count = ctr->status = 0;
+  if (t == 0) {
+    ctr->leaf_count = ctr->root_count = ctr->status = 0;
+    ctr->life = life;
+  }
 }
 
 __global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v) {

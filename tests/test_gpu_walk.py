@@ -187,3 +187,32 @@ def test_leaves_made_and_removed_between_scans(ctx):
     assert m.stats()["leaf_count"] == len(np.unique(om.cells()[0] >> 3, axis=0))
     m.close()
     om.close()
+
+
+def test_marks_of_many_lives(ctx):
+    """A map cleared more often than the marks have values: every life's scans
+    read only their own marks, though the pool keeps the bytes of earlier ones
+    (scans alternate, so that leaves reuse indices with other cells marked)."""
+    import bonxai_amd as bx
+    import oracle
+    pts = [_sphere(300, 2.0, 1), _sphere(300, 3.0, 2)]
+    o = np.array([0.1, 0.0, 0.2])
+    want = []
+    for k in range(2):
+        om = oracle.ProbMap(0.1)
+        om.insert_point_cloud(pts[k], o, 2.5)
+        om.insert_point_cloud(pts[1 - k], o, 2.5)
+        want.append((om.cells(), om.digest()))
+        om.close()
+    m = bx.ProbabilisticMap(ctx, 0.1)
+    dev = [ctx.to_device(p) for p in pts]
+    for life in range(270):
+        k = life % 2
+        m.update_count = 1
+        m.insert_point_cloud(dev[k], o, 2.5, sync=False)
+        m.insert_point_cloud(dev[1 - k], o, 2.5, sync=False)
+        assert m.digest() == want[k][1], f"life {life}"
+        if life in (0, 126, 127, 128, 255):
+            assert_same_cells(m.cells(), want[k][0], f"life {life}")
+        m.clear()
+    m.close()
