@@ -1909,101 +1909,45 @@ __global__ void __launch_bounds__(256) k_op_apply(const MapDev* __restrict__ mp,
 }
 
 
-// ConstAccessor::value / isCellOn (bonxai.hpp:496-534) for a batch.  Each
-// thread carries kLookups lookups through the chain root key -> inner entry
-// -> cell (-> mask word) together, so every stage issues kLookups
-// independent loads (lookup j of a block is element base + j * blockDim.x:
-// every stage's loads and stores stay coalesced across the wavefront).
-constexpr uint32_t kLookups = 4;
-
-__device__ __forceinline__ int32_t root_find_from(const MapView& m, uint64_t key, uint32_t h) {
-  for (uint32_t p = 0; p <= m.root_mask; ++p) {
-    const uint64_t k = m.root_keys[h];
-    if (k == key) return (int32_t)h;
-    if (k == kEmptyKey) return -1;
-    h = (h + 1) & m.root_mask;
-  }
-  return -1;
-}
-
+// ConstAccessor::value / isCellOn (bonxai.hpp:496-534) for a batch, one
+// lookup a thread: root key -> inner entry -> cell (-> mask word).  4- and
+// 8-byte cells: the cell first.  Off cells hold zero bytes, so a nonzero cell
+// is on and its mask word is not read; only a zero cell (off, or on with a
+// zero value) costs the mask load.  Bound: the chain of loads in small
+// batches, the scattered cell lines in large ones (8M random reads of a 2M-
+// cell grid: 0.107 ms; the hits' 4-byte reads alone take 0.075).  Four
+// lookups a thread, their loads issued together, leave too few wavefronts to
+// cover the chain: 0.113 ms, 16k lookups 9 against 6 us, 64 batches of 256k
+// 710 against 490 us; the mask loaded beside the cell: 0.132 ms.
 __global__ void __launch_bounds__(256) k_lookup(const MapDev* __restrict__ mp,
                                                 const int32_t* __restrict__ coords, uint64_t n,
                                                 uint8_t* __restrict__ vals,
                                                 uint8_t* __restrict__ found) {
-  const MapView m = load_view(mp);
-  const uint64_t base = (uint64_t)blockIdx.x * blockDim.x * kLookups + threadIdx.x;
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const MapView m = uniform_view(mp);
   const int32_t BXG_G* cg = gp(coords);
-  int32_t x[kLookups], y[kLookups], z[kLookups];
-  uint64_t key[kLookups];
-  uint32_t h[kLookups];
-  bool live[kLookups];
-#pragma unroll
-  for (uint32_t j = 0; j < kLookups; ++j) {
-    const uint64_t i = base + (uint64_t)j * blockDim.x;
-    live[j] = i < n;
-    x[j] = live[j] ? cg[3 * i] : 0;
-    y[j] = live[j] ? cg[3 * i + 1] : 0;
-    z[j] = live[j] ? cg[3 * i + 2] : 0;
-  }
-  uint64_t k0[kLookups];
-#pragma unroll
-  for (uint32_t j = 0; j < kLookups; ++j) {
-    live[j] = live[j] && pack_root(x[j], y[j], z[j], m.log2n, &key[j]);
-    h[j] = live[j] ? root_hash(key[j], m.root_mask) : 0u;
-    k0[j] = live[j] ? m.root_keys[h[j]] : kEmptyKey;
-  }
-  uint32_t c[kLookups];
-#pragma unroll
-  for (uint32_t j = 0; j < kLookups; ++j) {
-    int32_t slot = -1;
-    if (k0[j] == key[j] && live[j]) {
-      slot = (int32_t)h[j];
-    } else if (live[j] && k0[j] != kEmptyKey) {
-      slot = root_find_from(m, key[j], (h[j] + 1) & m.root_mask);  // a collision: probe on
-    }
-    c[j] = slot >= 0 ? m.children[(uint64_t)slot * m.isz + inner_index(x[j], y[j], z[j], m.lb, m.ib)]
-                     : kEmptyChild;
-  }
-  uint32_t li[kLookups];
-  uint64_t g[kLookups];
-#pragma unroll
-  for (uint32_t j = 0; j < kLookups; ++j) {
-    li[j] = leaf_index(x[j], y[j], z[j], m.lb);
-    g[j] = (uint64_t)(c[j] < kPendingChild ? c[j] : 0u) * m.lsz + li[j];
-  }
+  const int32_t x = cg[3 * i], y = cg[3 * i + 1], z = cg[3 * i + 2];
+  const uint32_t leaf = find_leaf(m, x, y, z);
   const uint32_t vb = m.vb;
-  // 4- and 8-byte cells: the cell first.  Off cells hold zero bytes, so a
-  // nonzero cell is on and its mask word is not read; only a zero cell (off,
-  // or on with a zero value) costs the mask load.
-  uint64_t cv[kLookups];
   const bool cell_first = vb == 4 || vb == 8;
-#pragma unroll
-  for (uint32_t j = 0; j < kLookups; ++j) {
-    cv[j] = 0;
-    if (cell_first && c[j] < kPendingChild)
-      cv[j] = vb == 4 ? (uint64_t)((const uint32_t BXG_G*)m.cells)[g[j]]
-                      : ((const uint64_t BXG_G*)m.cells)[g[j]];
+  uint64_t v = 0, g = 0;
+  bool on = false;
+  if (leaf != kNone) {
+    const uint32_t li = leaf_index(x, y, z, m.lb);
+    g = (uint64_t)leaf * m.lsz + li;
+    if (cell_first)
+      v = vb == 4 ? (uint64_t)((const uint32_t BXG_G*)m.cells)[g] : ((const uint64_t BXG_G*)m.cells)[g];
+    on = v != 0 || ((m.masks[(uint64_t)leaf * m.lw + (li >> 6)] >> (li & 63)) & 1ull);
   }
-  bool on[kLookups];
-#pragma unroll
-  for (uint32_t j = 0; j < kLookups; ++j) {
-    on[j] = cv[j] != 0;
-    if (!on[j] && c[j] < kPendingChild)
-      on[j] = (m.masks[(uint64_t)c[j] * m.lw + (li[j] >> 6)] >> (li[j] & 63)) & 1ull;
-  }
-#pragma unroll
-  for (uint32_t j = 0; j < kLookups; ++j) {
-    const uint64_t i = base + (uint64_t)j * blockDim.x;
-    if (i >= n) continue;
-    if (found) found[i] = on[j];
-    if (!vals || !vb) continue;
-    if (vb == 4) {
-      ((uint32_t*)vals)[i] = (uint32_t)cv[j];
-    } else if (vb == 8) {
-      ((uint64_t*)vals)[i] = cv[j];
-    } else {
-      for (uint32_t b = 0; b < vb; ++b) vals[i * vb + b] = on[j] ? m.cells[g[j] * vb + b] : 0;
-    }
+  if (found) found[i] = on;
+  if (!vals || !vb) return;
+  if (vb == 4) {
+    ((uint32_t*)vals)[i] = (uint32_t)v;
+  } else if (vb == 8) {
+    ((uint64_t*)vals)[i] = v;
+  } else {
+    for (uint32_t b = 0; b < vb; ++b) vals[i * vb + b] = on ? m.cells[g * vb + b] : 0;
   }
 }
 

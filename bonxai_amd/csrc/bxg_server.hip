@@ -132,7 +132,7 @@ void srv_launch_read(bxg_server* s, SrvReq* r) {
     if (rc != BXG_OK) {
       // reported below
     } else if (r->kind == kReqLookup) {
-      rc = launch_on(c, st, "k_lookup", k_lookup, lookup_blocks(r->n), kBlock, (const MapDev*)m->d, r->coords,
+      rc = launch_on(c, st, "k_lookup", k_lookup, nblocks(r->n), kBlock, (const MapDev*)m->d, r->coords,
                      r->n, (uint8_t*)r->vals, r->found);
     } else {
       // the map is idle: its last counter snapshot has landed or is about to
