@@ -799,19 +799,22 @@ int enqueue_scan_kernels(bxg_ctx* c, BatchHdr* hdr, ScanDesc* desc, ScanScratch 
   const uint32_t gw = std::max<uint32_t>(1, std::min<uint32_t>(gp, 16384));
   // the passes over the rays: a wavefront a batch of 64 winners (at most one
   // per 64 points; capped, the wavefronts then walk several), and in small
-  // calls up to 8, for segments of the batches, while the workgroups per CU
-  // allow it; a multiple of the XCDs
+  // calls more, for segments of the batches, while the workgroups per CU
+  // allow it; a multiple of the XCDs.  The update pass twice as many as the
+  // leaf pass (LiDAR scans at 50 m, one of 8: 32 workgroups per CU 205 us, 64
+  // 186, 128 182; the leaf pass, whose atomics meet on the roots near the
+  // sensor, 43, 47, 62, in a 100k-point room 36, 59, 111)
   const uint64_t cus = (uint64_t)std::max(c->cu_count, 1);
   const uint32_t rb = c->ray_block;
   const uint64_t most = (grid_points + rb - 1) / rb;
-  const auto walk_grid = [&](uint64_t per_cu) {
+  const auto walk_grid = [&](uint64_t per_cu, uint64_t small_per_cu) {
     const uint64_t whole = std::min(most, cus * per_cu);
-    const uint64_t cut = std::min(most * (1u << kMaxSegLog), cus * c->small_ray_blocks_per_cu);
+    const uint64_t cut = std::min(most * (1u << kMaxSegLog), cus * small_per_cu);
     const uint64_t g = std::max<uint64_t>({whole, cut, 1});
     return (uint32_t)((g + kXcds - 1) / kXcds * kXcds);
   };
-  const uint32_t gr = walk_grid(c->ray_blocks_per_cu);
-  const uint32_t gl = walk_grid(c->leaf_blocks_per_cu);
+  const uint32_t gr = walk_grid(c->ray_blocks_per_cu, 2ull * c->small_ray_blocks_per_cu);
+  const uint32_t gl = walk_grid(c->leaf_blocks_per_cu, c->small_ray_blocks_per_cu);
   sc.win_cells = (int32_t)c->ray_window;
   sc.win_leaves = (int32_t)c->leaf_window;
   sc.win_fresh = (int32_t)c->fresh_window;

@@ -1132,7 +1132,7 @@ __global__ void __launch_bounds__(256) k_scan_scatter(const BatchHdr* __restrict
 constexpr int32_t kFreshWindow = 16;
 constexpr int32_t kUpdateWindow = 8;
 constexpr int32_t kLeafWindow = 64;
-constexpr uint32_t kMaxSegLog = 3;  // at most 8 segments a ray
+constexpr uint32_t kMaxSegLog = 5;  // at most 32 segments a ray
 constexpr uint32_t kGroupLog = 3;   // batches side by side on one XCD in a short list
 
 // The walk over the winner list.  A batch is 64 consecutive winners, rays of
@@ -1145,8 +1145,8 @@ constexpr uint32_t kGroupLog = 3;   // batches side by side on one XCD in a shor
 //
 // A short list (one scan a call) has fewer batches than the GPU has wavefront
 // slots, and a walk is a chain of dependent loads about 1.5 us a step: there
-// each ray is cut into up to 8 segments, and a wavefront walks one segment of
-// a batch.  The tasks of a group of up to 8 batches follow each other on one
+// each ray is cut into up to 32 segments (2,001 points: update pass 25 us with
+// 8, 20 with 16, 16 with 32), and a wavefront walks one segment of a batch.  The tasks of a group of up to 8 batches follow each other on one
 // XCD (workgroups go round the XCDs), segment by segment, so that its L2
 // sees neighbours at one distance from the sensor.  A long list is cut into
 // one contiguous part an XCD (a map's rays stay on one XCD or two); there the

@@ -136,7 +136,8 @@ int bxg_set_counting(bxg_ctx* ctx, int on);
  * and "leaf_blocks_per_cu" (1..256, default 128), the most workgroups per CU
  * of the update pass and the leaf-allocation pass over the rays;
  * "small_ray_blocks_per_cu" (1..64, default 32), the workgroups per CU that
- * the passes of a small call fill by cutting its rays into up to 8 segments;
+ * the leaf pass of a small call, and half of those that its update pass, fills
+ * by cutting the rays into up to 32 segments;
  * "ray_block" (64..256, default 64), the workgroup size of the passes;
  * "ep_table_factor", "root_slack"; "ray_window" (default 8), "fresh_window"
  * (default 16) and "leaf_window" (default 64), how many cells a ray may run
