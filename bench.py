@@ -395,8 +395,7 @@ def run_box_scan(ctx, bx, scenes, reps=10):
 
 SCAN_KERNELS = ("k_scan_begin", "k_scan_classify", "k_scan_winners", "k_scan_bucket_reduce",
                 "k_scan_bucket_scan", "k_scan_scatter", "k_scan_ray_leaves", "k_scan_new_entries",
-                "k_scan_endpoints", "k_scan_rays", "k_scan_new_endpoints", "k_scan_new_leaves",
-                "k_scan_finalize")
+                "k_scan_endpoints", "k_scan_rays", "k_scan_new_endpoints", "k_scan_new_leaves")
 
 
 def run_sequence(ctx, bx, scenes, nscans=200, cpu_budget_s=3.0):

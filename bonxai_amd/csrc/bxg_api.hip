@@ -777,16 +777,6 @@ uint32_t tag_bits_for(uint32_t nscans) {
   return b;
 }
 
-// the first kernel of a call, with its scans as arguments: writes hdr and desc
-template <uint32_t kN>
-int begin_args(bxg_ctx* c, const BatchHdr& h, const ScanDesc* scans, BatchHdr* hdr, ScanDesc* desc,
-               const ScanScratch& sc, bool reset_stats) {
-  ScanArgs<kN> a{};
-  std::copy(scans, scans + h.nscans, a.d);
-  return launch(c, "k_scan_begin", k_scan_begin_args<kN>, 1, kBlock, h, a, hdr, desc, sc,
-                reset_stats ? 1u : 0u);
-}
-
 // The kernel sequence of one wave of scans on given scratch and descriptors.
 // args: the batch's header and descriptors (at most kMostArgs), which the
 // first kernel writes to hdr and desc; null where they are there already.
@@ -821,13 +811,21 @@ int enqueue_scan_kernels(bxg_ctx* c, BatchHdr* hdr, ScanDesc* desc, ScanScratch 
   sc.ray_order = c->ray_order;
   // new-leaf pass: a wavefront per new leaf, grid-stride over them
   const uint32_t gm = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(cus * 8, gp));
-  if (!args)
-    BXG_TRY(launch(c, "k_scan_begin", k_scan_begin, 1, kBlock, hdr, desc, sc));
-  else if (nscans == 1)
-    BXG_TRY(begin_args<1>(c, *args_hdr, args, hdr, desc, sc, c->counting));
-  else
-    BXG_TRY(begin_args<kMostArgs>(c, *args_hdr, args, hdr, desc, sc, c->counting));
-  BXG_TRY(launch(c, "k_scan_classify", k_scan_classify, gp, kBlock, hdr, desc, sc));
+  const uint32_t reset = c->counting ? 1u : 0u;
+  if (args && nscans == 1) {
+    ScanArgs<1> a{{args[0]}};
+    BXG_TRY(launch(c, "k_scan_classify", k_scan_classify_one, std::max(gp, 1u), kBlock, *args_hdr, a, hdr, desc,
+                   sc, reset));
+  } else {
+    if (args) {
+      ScanArgs<kMostArgs> a{};
+      std::copy(args, args + nscans, a.d);
+      BXG_TRY(launch(c, "k_scan_begin", k_scan_begin_args, 1, kBlock, *args_hdr, a, hdr, desc, reset));
+    } else {
+      BXG_TRY(launch(c, "k_scan_begin", k_scan_begin, 1, kBlock, hdr, desc));
+    }
+    BXG_TRY(launch(c, "k_scan_classify", k_scan_classify, gp, kBlock, hdr, desc, sc));
+  }
   BXG_TRY(launch(c, "k_scan_winners", k_scan_winners, gp, kBlock, hdr, desc, sc));
   // a tile of buckets a scan (the scan index mod 64)
   const uint32_t tiles = (1u << (kDirBits + tag_bits_for(nscans))) / kScanTile;
@@ -856,8 +854,7 @@ int enqueue_scan_kernels(bxg_ctx* c, BatchHdr* hdr, ScanDesc* desc, ScanScratch 
       BXG_TRY(launch(c, "k_scan_extra_rays", k_scan_extra_rays<false>, nscans, kBlock, hdr, desc));
     BXG_TRY(launch(c, "k_scan_new_endpoints", k_scan_new_endpoints<false>, gw, kBlock, hdr, desc, sc));
   }
-  BXG_TRY(launch(c, "k_scan_new_leaves", k_scan_new_leaves, gm, kBlock, hdr, desc));
-  BXG_TRY(launch(c, "k_scan_finalize", k_scan_finalize, 1, kBlock, hdr, desc));
+  BXG_TRY(launch(c, "k_scan_new_leaves", k_scan_new_leaves, gm, kBlock, hdr, desc, sc));
   return BXG_OK;
 }
 
@@ -906,7 +903,7 @@ int run_wave(bxg_ctx* c, const bxg_scan_desc* scans, uint32_t nscans, uint32_t e
   if (!as_args) BXG_TRY(upload_scans(c, c->d_hdr, hdr, descs));
   BXG_TRY(enqueue_scan_kernels(c, c->d_hdr, c->d_desc, c->sc, total, nscans, any_extra, all_empty,
                                as_args ? &hdr : nullptr, as_args ? descs.data() : nullptr));
-  // k_scan_finalize wrote every map's counters to its host mirror
+  // k_scan_new_leaves wrote every map's counters to its host mirror
   std::vector<bxg_map*> maps(nscans);
   for (uint32_t s = 0; s < nscans; ++s) maps[s] = scans[s].map;
   return snapshot_event(c, maps.data(), maps.size());
@@ -2382,7 +2379,7 @@ int bxg_graph_launch(bxg_graph* g) {
   for (size_t s = 0; s < g->maps.size(); ++s)
     BXG_TRY(ensure_room(g->maps[s], scan_leaf_estimate(g->maps[s], g->npoints[s], g->ranges[s]), 1024));
   BXG_HIP(c, hipGraphLaunch(g->exec, c->stream));
-  // the frame's k_scan_finalize wrote each map's counters to its mirror
+  // the frame's k_scan_new_leaves wrote each map's counters to its mirror
   BXG_TRY(snapshot_event(c, g->maps.data(), g->maps.size()));
   // each map keeps its scan of the frame until it is confirmed (settle),
   // which re-runs it should the frame have overflowed the map's pools

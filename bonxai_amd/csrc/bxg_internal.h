@@ -81,7 +81,9 @@ struct alignas(128) MapCounters {
   uint32_t leaf_base;
   uint32_t life;  // the map's life (clears, mod kLives): its touched marks (mark_miss)
   uint64_t scans_applied;
-  uint64_t pad2[13];
+  int32_t scan_cur;  // cur of the running scan (cur itself moves on in its last kernel)
+  uint32_t pad1;
+  uint64_t pad2[12];
   uint64_t stat_endpoint_updates;
   uint64_t stat_rays;
   uint64_t stat_ray_updates;
@@ -173,7 +175,7 @@ constexpr uint32_t kTiles = kMaxBuckets / kScanTile;
 static_assert((1u << kDirBits) % kScanTile == 0 && kTiles <= 64, "bucket scan tiles");
 // scan counter words: [0] winner count, [kTileWords, + kTiles) bucket-tile
 // sums, [kClipWords, + 64) per scan (index mod 64) the points clipped at the
-// max range among those of one wavefront in 16
+// max range among those of one wavefront in 16 (zero between calls)
 constexpr uint32_t kTileWords = 64;
 constexpr uint32_t kClipWords = kTileWords + kTiles;
 constexpr uint32_t kCounterWords = kClipWords + 64;

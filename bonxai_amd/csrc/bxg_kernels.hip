@@ -697,31 +697,81 @@ __device__ __forceinline__ uint64_t ep_key(uint32_t tag, uint32_t slot, uint32_t
   return ((uint64_t)tag << 48) | ((uint64_t)slot << 24) | ((uint64_t)ci << 12) | (uint64_t)li;
 }
 
+// Phase 0 (per scan): the leaf count at the start of the scan, so that later
+// phases can tell the leaves the scan creates from older ones, and the scan's
+// update id.
+__device__ __forceinline__ void scan_begin(uint32_t nscans, const ScanDesc* sd) {
+  for (uint32_t s = threadIdx.x; s < nscans; s += blockDim.x) {
+    const MapDev BXG_G* m = gp((const MapDev*)sd[s].map);
+    MapCounters BXG_G* ctr = gp(m->ctr);
+    ctr->leaf_base = min(ctr->leaf_count, m->leaf_cap);
+    ctr->scan_cur = ctr->cur;
+  }
+}
+__global__ void k_scan_begin(const BatchHdr* __restrict__ hdr, const ScanDesc* __restrict__ sd) {
+  scan_begin(hdr->nscans, sd);
+}
+
+// The same for a call whose batch header and up to kN scan descriptors come
+// as kernel arguments, written here into the device buffers that the later
+// kernels read: no copy to the device before the call (two small copies and
+// the waits around them cost about 35 us at the head of a call).  kN 16 fits
+// the 4 KB of a launch's arguments.  With reset_stats (counted calls) the
+// maps' scan statistics are cleared.
+template <uint32_t kN>
+struct ScanArgs {
+  ScanDesc d[kN];
+};
+constexpr uint32_t kMostArgs = 16;
+static_assert(sizeof(ScanArgs<kMostArgs>) + sizeof(ScanScratch) + 64 <= 4096, "kernel arguments");
+template <uint32_t kN>
+__device__ __forceinline__ void scan_begin_args(const BatchHdr& hdr, const ScanArgs<kN>& a, BatchHdr* hdr_out,
+                                                ScanDesc* desc_out, uint32_t reset_stats) {
+  if (threadIdx.x == 0) *hdr_out = hdr;
+  const uint32_t* src = reinterpret_cast<const uint32_t*>(&a);
+  uint32_t* dst = reinterpret_cast<uint32_t*>(desc_out);
+  const uint32_t words = hdr.nscans * (uint32_t)(sizeof(ScanDesc) / 4);
+  for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) dst[i] = src[i];
+  if (reset_stats && threadIdx.x < hdr.nscans) {
+    MapCounters* ctr = gp((const MapDev*)a.d[threadIdx.x].map)->ctr;
+    ctr->stat_rays = 0;
+    ctr->stat_ray_updates = 0;
+    ctr->stat_ray_visits = 0;
+  }
+  scan_begin(hdr.nscans, a.d);
+}
+__global__ void k_scan_begin_args(BatchHdr hdr, ScanArgs<kMostArgs> a, BatchHdr* __restrict__ hdr_out,
+                                  ScanDesc* __restrict__ desc_out, uint32_t reset_stats) {
+  scan_begin_args(hdr, a, hdr_out, desc_out, reset_stats);
+}
+
 // Phase 1 (per point): max-range clip and posToCoord in FP64
 // (probabilistic_map.hpp:144-157, bonxai.hpp:404-410), root and leaf of the
 // endpoint created, pre-scan update_id test, and the first-index claim of
 // the endpoint voxel among the points whose voxel is to be updated.
-__global__ void __launch_bounds__(256) k_scan_classify(const BatchHdr* __restrict__ hdr,
-                                                       const ScanDesc* __restrict__ sd,
-                                                       ScanScratch sc) {
+// kOne: a call of one scan, whose header sits in scalar registers.
+template <bool kOne>
+__device__ __forceinline__ void classify_points(uint64_t total, uint32_t nscans, const ScanDesc* sd,
+                                                const ScanScratch& sc) {
   const uint64_t gi = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t total = hdr->total;
   if (gi - lane_id() >= total) return;  // the whole wavefront lies past the last point
   // Every lane of a live wavefront stays to the end: the root, leaf and
   // endpoint claims below are wavefront collectives.
   const bool live = gi < total;
   // the scan of the wavefront's first point, searched once with uniform
   // (scalar) loads; lanes past a scan boundary step forward from it
-  const uint32_t nscans = hdr->nscans;
-  const uint64_t g0 = (uint64_t)blockIdx.x * blockDim.x +
-                      ((uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) << 6);
-  uint32_t s = find_scan(sd, nscans, g0);
-  if (live)
-    while (s + 1 < nscans && sd[s + 1].pt_off <= gi) ++s;
-  else
-    s = 0u;
+  uint32_t s = 0;
+  if (!kOne) {
+    const uint64_t g0 = (uint64_t)blockIdx.x * blockDim.x +
+                        ((uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) << 6);
+    s = find_scan(sd, nscans, g0);
+    if (live)
+      while (s + 1 < nscans && sd[s + 1].pt_off <= gi) ++s;
+    else
+      s = 0u;
+  }
   const ScanDesc& d = sd[s];
-  const MapView m = load_view(d.map);
+  const MapView m = kOne ? uniform_view(d.map) : load_view(d.map);
   int4 rec = make_int4(0, 0, 0, (int32_t)(s << 16));
   bool valid = false;
   bool clipped = false;
@@ -879,6 +929,23 @@ __global__ void __launch_bounds__(256) k_scan_classify(const BatchHdr* __restric
     if ((int)lane_id() == leader) add32(&sc.counters[kClipWords + (ls & 63u)], (uint32_t)__popcll(same));
     pend &= ~same;
   }
+}
+
+__global__ void __launch_bounds__(256) k_scan_classify(const BatchHdr* __restrict__ hdr,
+                                                       const ScanDesc* __restrict__ sd,
+                                                       ScanScratch sc) {
+  classify_points<false>(hdr->total, hdr->nscans, sd, sc);
+}
+
+// Phases 0 and 1 of a call of one scan in one kernel, the scan as an
+// argument: the first workgroup also starts the scan (the points do not need
+// what it writes).  A launch saved, about 5 us a call.
+__global__ void __launch_bounds__(256) k_scan_classify_one(BatchHdr hdr, ScanArgs<1> a,
+                                                           BatchHdr* __restrict__ hdr_out,
+                                                           ScanDesc* __restrict__ desc_out, ScanScratch sc,
+                                                           uint32_t reset_stats) {
+  if (blockIdx.x == 0) scan_begin_args(hdr, a, hdr_out, desc_out, reset_stats);
+  classify_points<true>(hdr.total, 1u, a.d, sc);
 }
 
 // octahedral direction bin of (dx, dy, dz), 2^b x 2^b bins in Morton order
@@ -1540,9 +1607,37 @@ __global__ void __launch_bounds__(256) k_scan_extra_rays(const BatchHdr* __restr
 // clearing: 2.43 ms, 4.5 TB/s of the 10.8 GB.)  The new leaves of each scan's
 // map are [leaf_base, leaf_count); those of a failed call are written off
 // (zero).  Bound: HBM.
+//
+// Phase 5 (per scan) on the first workgroup, whose results no other
+// workgroup of this kernel reads: update_count 1 -> 2 -> 3 -> 1
+// (probabilistic_map.cpp:103-105) unless the scan failed; every scanned map's
+// counters to its pinned host mirror, so that the host learns pool use and
+// errors from one event after the call (no copy a map); the clip counts back
+// to zero.
+__device__ __forceinline__ void scan_finalize(uint32_t nscans, const ScanDesc* sd, const ScanScratch& sc) {
+  if (threadIdx.x < 64u) sc.counters[kClipWords + threadIdx.x] = 0;
+  for (uint32_t s = threadIdx.x; s < nscans; s += blockDim.x) {
+    const MapDev BXG_G* md = (const MapDev BXG_G*)sd[s].map;
+    MapCounters BXG_G* ctr = gp(md->ctr);
+    if (!(sd[s].flags & kScanNoRays) && !(ctr->status & kFatal)) {
+      const int32_t c = ctr->cur + 1;
+      ctr->cur = c == 4 ? 1 : c;
+      ctr->scans_applied += 1;
+    }
+    const uint64_t BXG_G* src = (const uint64_t BXG_G*)ctr;
+    uint64_t* dst = (uint64_t*)md->ctr_host;
+    uint64_t v[sizeof(MapCounters) / 8];
+#pragma unroll
+    for (uint32_t k = 0; k < sizeof(MapCounters) / 8; ++k) v[k] = src[k];
+#pragma unroll
+    for (uint32_t k = 0; k < sizeof(MapCounters) / 8; ++k) dst[k] = v[k];
+  }
+}
+
 constexpr uint32_t kNewLeafRun = 4;  // leaves a wavefront of k_scan_new_leaves has in flight
 __global__ void __launch_bounds__(256) k_scan_new_leaves(const BatchHdr* __restrict__ hdr,
-                                                         const ScanDesc* __restrict__ sd) {
+                                                         const ScanDesc* __restrict__ sd, ScanScratch sc) {
+  if (blockIdx.x == 0) scan_finalize(hdr->nscans, sd, sc);
   const uint32_t lane = lane_id();
   const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
@@ -1553,7 +1648,7 @@ __global__ void __launch_bounds__(256) k_scan_new_leaves(const BatchHdr* __restr
     const uint32_t lo = ctr->leaf_base;
     const uint32_t hi = min(ctr->leaf_count, m.leaf_cap);
     if (lo >= hi) continue;
-    const int32_t cur = ctr->cur;
+    const int32_t cur = ctr->scan_cur;
     // a failed call's leaves stay off: no byte is its mark
     const bool failed = (ctr->status & kFatal) != 0;
     const uint32_t bmiss = failed ? ~0u : mark_miss(ctr->life);
@@ -1635,73 +1730,6 @@ __global__ void k_na_recover(MapCounters* __restrict__ ctr, uint32_t leaf_cap) {
   if (threadIdx.x != 0) return;
   ctr->status &= ~(kStOutOfPool | kStRootFull);
   ctr->leaf_count = min(ctr->leaf_count, leaf_cap);
-}
-
-// Phase 0 (per scan): the leaf count at the start of the scan, so that later
-// phases can tell the leaves the scan creates from older ones.
-template <class Desc>
-__device__ __forceinline__ void scan_begin(uint32_t nscans, const Desc* sd, const ScanScratch& sc) {
-  for (uint32_t s = threadIdx.x; s < nscans; s += blockDim.x) {
-    const MapDev BXG_G* m = gp((const MapDev*)sd[s].map);
-    MapCounters BXG_G* ctr = gp(m->ctr);
-    ctr->leaf_base = min(ctr->leaf_count, m->leaf_cap);
-  }
-  if (threadIdx.x < 64u) sc.counters[kClipWords + threadIdx.x] = 0;
-}
-__global__ void k_scan_begin(const BatchHdr* __restrict__ hdr, const ScanDesc* __restrict__ sd,
-                             ScanScratch sc) {
-  scan_begin(hdr->nscans, sd, sc);
-}
-
-// The same for a call whose batch header and up to kN scan descriptors come
-// as kernel arguments, written here into the device buffers that the later
-// kernels read: no copy to the device before the call (two small copies and
-// the waits around them cost about 35 us at the head of a call).  kN 16 fits
-// the 4 KB of a launch's arguments.  With reset_stats (counted calls) the
-// maps' scan statistics are cleared.
-template <uint32_t kN>
-struct ScanArgs {
-  ScanDesc d[kN];
-};
-constexpr uint32_t kMostArgs = 16;
-static_assert(sizeof(ScanArgs<kMostArgs>) + sizeof(ScanScratch) + 64 <= 4096, "kernel arguments");
-template <uint32_t kN>
-__global__ void k_scan_begin_args(BatchHdr hdr, ScanArgs<kN> a, BatchHdr* __restrict__ hdr_out,
-                                  ScanDesc* __restrict__ desc_out, ScanScratch sc, uint32_t reset_stats) {
-  if (threadIdx.x == 0) *hdr_out = hdr;
-  const uint32_t* src = reinterpret_cast<const uint32_t*>(&a);
-  uint32_t* dst = reinterpret_cast<uint32_t*>(desc_out);
-  const uint32_t words = hdr.nscans * (uint32_t)(sizeof(ScanDesc) / 4);
-  for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) dst[i] = src[i];
-  if (reset_stats && threadIdx.x < hdr.nscans) {
-    MapCounters* ctr = gp((const MapDev*)a.d[threadIdx.x].map)->ctr;
-    ctr->stat_rays = 0;
-    ctr->stat_ray_updates = 0;
-    ctr->stat_ray_visits = 0;
-  }
-  scan_begin(hdr.nscans, a.d, sc);
-}
-
-// Phase 5 (per scan): advance update_count 1 -> 2 -> 3 -> 1
-// (probabilistic_map.cpp:103-105) unless the scan failed; copy every scanned map's counters to its pinned host mirror, so the host
-// learns pool use and errors from one event after the call (no copy a map).
-__global__ void k_scan_finalize(const BatchHdr* __restrict__ hdr, const ScanDesc* __restrict__ sd) {
-  for (uint32_t s = threadIdx.x; s < hdr->nscans; s += blockDim.x) {
-    const MapDev BXG_G* md = (const MapDev BXG_G*)sd[s].map;
-    MapCounters BXG_G* ctr = gp(md->ctr);
-    if (!(sd[s].flags & kScanNoRays) && !(ctr->status & kFatal)) {
-      const int32_t c = ctr->cur + 1;
-      ctr->cur = c == 4 ? 1 : c;
-      ctr->scans_applied += 1;
-    }
-    const uint64_t BXG_G* src = (const uint64_t BXG_G*)ctr;
-    uint64_t* dst = (uint64_t*)md->ctr_host;
-    uint64_t v[sizeof(MapCounters) / 8];
-#pragma unroll
-    for (uint32_t k = 0; k < sizeof(MapCounters) / 8; ++k) v[k] = src[k];
-#pragma unroll
-    for (uint32_t k = 0; k < sizeof(MapCounters) / 8; ++k) dst[k] = v[k];
-  }
 }
 
 // ------------------------------------------------------ bulk cell ops
