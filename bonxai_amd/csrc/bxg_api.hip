@@ -78,10 +78,9 @@ struct bxg_ctx {
 
   // bulk-op scratch
   uint64_t op_cap = 0;
-  OpSlot* op_slots = nullptr;  // op_cap * 2 slots
-  uint32_t* op_tpos = nullptr;
-  uint32_t* op_leaf = nullptr;
-  uint8_t* op_prebit = nullptr;
+  uint64_t* op_entry = nullptr;
+  uint64_t op_starts = 0;  // 16-bit words of op_start
+  uint16_t* op_start = nullptr;
 
   // device staging of host-memory calls
   void* dstage[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -635,43 +634,48 @@ int ensure_scan_scratch(bxg_ctx* c, uint64_t points, uint32_t nscans) {
   return BXG_OK;
 }
 
-int ensure_op_scratch(bxg_ctx* c, uint64_t n) {
-  if (n <= c->op_cap) return BXG_OK;
-  BXG_TRY(ctx_sync(c));
-  dfree(c->op_slots);
-  dfree(c->op_tpos);
-  dfree(c->op_leaf);
-  dfree(c->op_prebit);
-  c->op_slots = nullptr;
-  c->op_tpos = c->op_leaf = nullptr;
-  c->op_prebit = nullptr;
-  c->op_cap = 0;
-  const uint64_t cap = std::max<uint64_t>(pow2_at_least(n), 1 << 12);
+// The scratch of a bulk call of n cells: 8 bytes an input and, per tile, a
+// 16-bit word a bucket.  Tiles of 1024 to 8192 inputs, so that about 128 to
+// 256 workgroups order them (2M inputs in tiles of 4096: 45 + 69 us for 43 +
+// 66).  Buckets: a workgroup costs some 15 us whatever it holds, so about 1024
+// inputs each where there are enough for two workgroups a CU (500k inputs:
+// 512 buckets 26 us, 1024 41; 2M: 2048 buckets 66, 4096 91); below that as
+// many as the card runs at once, of 64 inputs or more (700 inputs: 16 buckets
+// 12 us, 8 16; 20k: 256 buckets 17.6, 512 19.6).
+int op_scratch(bxg_ctx* c, uint64_t n, OpScratch* os) {
+  const uint64_t cap = std::max<uint64_t>(pow2_at_least(n), 1 << 13);
   if (cap > (1ull << 31)) return fail(c, BXG_ERR_INVALID_ARG, "too many cells in one call");
-  void* p;
-  BXG_TRY(dmalloc(c, &p, cap * 2 * sizeof(OpSlot)));
-  c->op_slots = (OpSlot*)p;
-  BXG_TRY(dmalloc(c, &p, cap * 4));
-  c->op_tpos = (uint32_t*)p;
-  BXG_TRY(dmalloc(c, &p, cap * 4));
-  c->op_leaf = (uint32_t*)p;
-  BXG_TRY(dmalloc(c, &p, cap));
-  c->op_prebit = (uint8_t*)p;
-  c->op_cap = cap;
+  os->tile = n >= (1u << 20) ? 8192 : n >= (1u << 19) ? 4096 : n >= (1u << 18) ? 2048 : 1024;
+  os->tiles = (uint32_t)((n + os->tile - 1) / os->tile);
+  const uint64_t nb = std::max({std::min<uint64_t>(pow2_at_least((n + 63) / 64), 256),
+                                std::min<uint64_t>(pow2_at_least((n + 127) / 128), 512),
+                                std::min<uint64_t>(pow2_at_least((n + 1023) / 1024), kOpMaxBuckets)});
+  os->nb = (uint32_t)std::max<uint64_t>(nb, kXcds);
+  const uint64_t starts = (uint64_t)os->tiles * (os->nb + 2);
+  if (cap > c->op_cap || starts > c->op_starts) {
+    BXG_TRY(ctx_sync(c));
+    void* p;
+    if (cap > c->op_cap) {
+      dfree(c->op_entry);
+      c->op_entry = nullptr;
+      c->op_cap = 0;
+      BXG_TRY(dmalloc(c, &p, cap * 8));
+      c->op_entry = (uint64_t*)p;
+      c->op_cap = cap;
+    }
+    if (starts > c->op_starts) {
+      dfree(c->op_start);
+      c->op_start = nullptr;
+      c->op_starts = 0;
+      const uint64_t words = pow2_at_least(starts);
+      BXG_TRY(dmalloc(c, &p, words * 2));
+      c->op_start = (uint16_t*)p;
+      c->op_starts = words;
+    }
+  }
+  os->entry = c->op_entry;
+  os->start = c->op_start;
   return BXG_OK;
-}
-
-// The scratch of a bulk call of n inputs: a table of twice the power of two
-// at or above n slots (load factor at most 1/2), emptied by the call itself.
-OpScratch op_scratch(bxg_ctx* c, uint64_t n, uint64_t* slots) {
-  OpScratch os;
-  *slots = std::max<uint64_t>(pow2_at_least(n), 1 << 12) * 2;
-  os.slots = c->op_slots;
-  os.mask = (uint32_t)(*slots - 1);
-  os.tpos = c->op_tpos;
-  os.leaf = c->op_leaf;
-  os.prebit = c->op_prebit;
-  return os;
 }
 
 // ------------------------------------------------------------ scans
@@ -1043,31 +1047,32 @@ int cell_op(bxg_map* m, const int32_t* coords, const void* vals, uint64_t n, uin
   if (!n) return BXG_OK;
   if (op != kOpSetOff)
     BXG_TRY(ensure_room(m, std::min<uint64_t>(n, 1u << 22), std::min<uint64_t>(n, 1u << 16)));
-  BXG_TRY(ensure_op_scratch(c, n));
-  uint64_t slots = 0;
-  const OpScratch os = op_scratch(c, n, &slots);
-  BXG_TRY(launch(c, "k_op_clear", k_op_clear, (uint32_t)std::min<uint64_t>(nblocks(slots), 4096), kBlock,
-                 os.slots, slots));
-  BXG_TRY(launch(c, "k_op_begin", k_op_begin, 1, 64, (const MapDev*)m->d));
-  if (op == kOpSetValue && !was_on)
-    BXG_TRY(launch(c, "k_op_resolve", k_op_resolve<true, false>, nblocks(n), kBlock, (const MapDev*)m->d,
-                   coords, n, os));
-  else if (op != kOpSetOff)
-    BXG_TRY(launch(c, "k_op_resolve", k_op_resolve<true, true>, nblocks(n), kBlock, (const MapDev*)m->d,
-                   coords, n, os));
-  else
-    BXG_TRY(launch(c, "k_op_resolve", k_op_resolve<false, true>, nblocks(n), kBlock, (const MapDev*)m->d,
-                   coords, n, os));
-  if (op != kOpSetOff) {
-    // the leaves the call created: at most one per input
-    const uint64_t words = std::min<uint64_t>(n, m->leaf_cap) *
-                           ((uint64_t)m->h.leaf_words + (uint64_t)m->h.leaf_size * m->h.value_bytes / 8);
-    const uint32_t gz = (uint32_t)std::max<uint64_t>(
-        1, std::min<uint64_t>(nblocks(words), (uint64_t)std::max(c->cu_count, 1) * 8));
-    BXG_TRY(launch(c, "k_zero_new_leaves", k_zero_new_leaves, gz, kBlock, (const MapDev*)m->d));
+  OpScratch os;
+  BXG_TRY(op_scratch(c, n, &os));
+  const bool create = op != kOpSetOff;
+  const MapDev* md = m->d;
+  auto tiles = create ? (os.tile == 8192   ? k_op_tiles<true, 8>
+                         : os.tile == 4096 ? k_op_tiles<true, 4>
+                         : os.tile == 2048 ? k_op_tiles<true, 2>
+                                           : k_op_tiles<true, 1>)
+                      : (os.tile == 8192   ? k_op_tiles<false, 8>
+                         : os.tile == 4096 ? k_op_tiles<false, 4>
+                         : os.tile == 2048 ? k_op_tiles<false, 2>
+                                           : k_op_tiles<false, 1>);
+  BXG_TRY(launch(c, "k_op_tiles", tiles, os.tiles, kOpTileThreads, md, coords, n, op, was_on, os));
+  // Calls within the leaves ensure_room has made room for create and apply in
+  // one kernel; in a larger one the pool can run out, and then no cell may be
+  // set, so its leaves are all created first.
+  const uint8_t* v = (const uint8_t*)vals;
+  bool fused = create;
+  if (create && n > (1u << 22)) {
+    BXG_TRY(launch(c, "k_op_leaves", k_op_buckets<true, false, false, false>, os.nb, kOpThreads, md, v, n, op, was_on, os));
+    fused = false;
   }
-  BXG_TRY(launch(c, "k_op_apply", k_op_apply, nblocks(n), kBlock, (const MapDev*)m->d, coords,
-                 (const uint8_t*)vals, n, op, was_on, os));
+  auto buckets = op != kOpSetValue ? (fused ? k_op_buckets<true, true, true, false> : k_op_buckets<false, true, true, false>)
+                 : was_on          ? (fused ? k_op_buckets<true, true, true, true> : k_op_buckets<false, true, true, true>)
+                          : (fused ? k_op_buckets<true, true, false, true> : k_op_buckets<false, true, false, true>);
+  BXG_TRY(launch(c, "k_op_buckets", buckets, os.nb, kOpThreads, md, v, n, op, was_on, os));
   return snapshot_counters(m);
 }
 
@@ -1284,10 +1289,8 @@ int bxg_ctx_destroy(bxg_ctx* c) {
   dfree(c->sc.ep);
   dfree(c->d_counters);
   dfree(c->d_hdr);
-  dfree(c->op_slots);
-  dfree(c->op_tpos);
-  dfree(c->op_leaf);
-  dfree(c->op_prebit);
+  dfree(c->op_entry);
+  dfree(c->op_start);
   for (int i = 0; i < 4; ++i) dfree(c->dstage[i]);
   dfree(c->d_small);
   if (c->h_small) hipHostFree(c->h_small);

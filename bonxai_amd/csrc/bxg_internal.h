@@ -36,7 +36,7 @@
 // pool is not zeroed): whatever creates a leaf writes all its cells and mask
 // words, as the reference's Grid constructor initialises a new leaf
 // (bonxai.hpp:51-58): the scan's leaf assembly (k_scan_new_leaves), the bulk
-// calls' k_zero_new_leaves, or k_write_leaves.
+// calls' k_op_buckets, or k_write_leaves.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -1734,62 +1734,411 @@ __global__ void k_na_recover(MapCounters* __restrict__ ctr, uint32_t leaf_cap) {
 
 // ------------------------------------------------------ bulk cell ops
 
-// One slot of a bulk call's cell table: the cell's key and the first and
-// last input index naming it, on one 16-byte line so that a claim touches
-// one cache line.  An empty slot is (all ones, all ones, 0).
-struct alignas(16) OpSlot {
-  uint64_t key;
-  uint32_t first;
-  uint32_t last;
-};
+// setValue / setCellOn / setCellOff for a batch, with the results of the calls
+// made one after the other (bonxai.hpp:449-466, 537-569).  Two kernels:
+// k_op_tiles orders each tile of inputs by the bucket (hash) of their leaf,
+// and k_op_buckets gives each bucket to one workgroup, which finds the first
+// and last input of every cell in LDS.  A leaf belongs to one workgroup, so
+// its cells, its mask words and its entry need no device atomics, and the
+// workgroup initialises the leaves it creates.
+//
+// A table of the cells in device memory (claim, last index, mask bits: two to
+// three device atomics an input, about 15 G/s in all) took 0.46 ms for 2M
+// inputs into a new grid, clear and leaf initialisation included, and five
+// launches; the two kernels take 0.030 + 0.059 ms (0.4 MB of bucket starts
+// aside, 64 bytes an input are moved: 1.4 TB/s).  What bounds them: the tiles'
+// claims of missing roots (12 us) and their passes through LDS; in the
+// buckets a chain of some ten dependent reads a workgroup with two or three
+// workgroups a CU (reads of the entries 14 us, LDS tables 6, leaves looked up
+// and created 13, values and cells 17).
+
+constexpr uint32_t kOpTileThreads = 1024;
+constexpr uint32_t kOpTileLog = 13;    // most inputs of a tile
+constexpr uint32_t kOpMaxBuckets = 4096;
+constexpr uint32_t kOpThreads = 512;   // of k_op_buckets (2M inputs: 256 threads 93 us, 512 66, 1024 102)
+// cell slots of a bucket's table: 2 to 3 workgroups a CU, and four times a
+// bucket's inputs on average (3072 slots, four workgroups a CU: 78 us for 66,
+// the fuller tables cost more than the wavefronts bring)
+constexpr uint32_t kOpCells = 4096;
+constexpr uint32_t kOpLeaves = 256;    // its leaf slots (at most)
+constexpr uint32_t kOpWords = 2048;    // its mask words
+constexpr uint64_t kCreated = kEmptyKey - 1;  // in place of a leaf's key, once created
+constexpr uint32_t kOpProbes = 32;     // slots looked at for a cell or leaf before the table counts as full
+
+enum : uint32_t { kOpSetValue = 0, kOpSetOn = 1, kOpSetOff = 2 };
 
 struct OpScratch {
-  OpSlot* slots;     // the call's table (mask + 1 slots)
-  uint32_t mask;
-  uint32_t* tpos;    // per input: table slot (kNone if no cell)
-  uint32_t* leaf;    // per input: its leaf index, or kNone where not known yet
-  uint8_t* prebit;   // per input: mask bit before the call
+  uint64_t* entry;   // per tile, its inputs by bucket: cell << kOpTileLog | place in the tile
+  uint16_t* start;   // per tile, each bucket's first entry, nb + 1 words (stride nb + 2)
+  uint32_t tile;     // inputs a tile
+  uint32_t tiles;
+  uint32_t nb;       // buckets (a power of two, 8 or more)
 };
 
-// empty the first n slots of a call's table
-__global__ void __launch_bounds__(256) k_op_clear(OpSlot* __restrict__ slots, uint64_t n) {
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * blockDim.x) {
-    OpSlot e;
-    e.key = kEmptyKey;
-    e.first = kNone;
-    e.last = 0;
-    slots[i] = e;
+// a key of an LDS table: the slot's key, or kEmptyKey taken by this key
+__device__ __forceinline__ uint64_t lds_claim(uint64_t* p, uint64_t key) {
+  uint64_t k = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  if (k != kEmptyKey) return k;
+  k = atomicCAS((unsigned long long*)p, kEmptyKey, key);
+  return k == kEmptyKey ? key : k;
+}
+__device__ __forceinline__ uint32_t lds_claim(uint32_t* p, uint32_t key) {
+  uint32_t k = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  if (k != kNone) return k;
+  k = atomicCAS(p, kNone, key);
+  return k == kNone ? key : k;
+}
+
+// The inputs of a tile in the order of their leaves' buckets.  kCreate:
+// missing roots are created (setCellOff leaves out inputs without one).  The
+// tile's distinct roots are found in LDS and looked up once.
+template <bool kCreate, int kPer>
+__global__ void __launch_bounds__(kOpTileThreads) k_op_tiles(const MapDev* __restrict__ mp,
+                                                             const int32_t* __restrict__ coords, uint64_t n,
+                                                             uint32_t op, uint8_t* __restrict__ was_on,
+                                                             OpScratch os) {
+  constexpr uint32_t kTile = kOpTileThreads * kPer;
+  constexpr uint32_t kRoots = kTile * 2 < 4096 ? kTile * 2 : 4096;
+  constexpr uint32_t kStage = kTile * 8 > kRoots * 12 ? kTile * 8 : kRoots * 12;
+  __shared__ __attribute__((aligned(16))) uint8_t stage[kStage];
+  __shared__ uint32_t hist[kOpMaxBuckets / 2];  // 16 bits a bucket
+  __shared__ uint32_t wsum[kOpTileThreads / 64];
+  uint64_t* rkeys = (uint64_t*)stage;
+  int32_t* rslots = (int32_t*)(stage + kRoots * 8);
+  const MapView m = uniform_view(mp);
+  const uint32_t t = threadIdx.x, lane = t & 63u, wid = t >> 6;
+  const uint64_t base = (uint64_t)blockIdx.x * kTile;
+  for (uint32_t p = t; p < kRoots; p += kOpTileThreads) rkeys[p] = kEmptyKey;
+  for (uint32_t p = t; p < os.nb / 2; p += kOpTileThreads) hist[p] = 0;
+  int32_t x[kPer], y[kPer], z[kPer];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const uint64_t i = base + (uint32_t)j * kOpTileThreads + t;
+    x[j] = y[j] = z[j] = 0;
+    if (i < n) {
+      const int32_t BXG_G* c = gp(coords) + 3 * i;
+      x[j] = c[0];
+      y[j] = c[1];
+      z[j] = c[2];
+      if (was_on) was_on[i] = op == kOpSetOff ? 0 : 1;
+    }
+  }
+  __syncthreads();
+  constexpr uint32_t kOut = 0xFFFFFFFFu, kDirect = 0xFFFFFFFEu;
+  uint32_t rp[kPer];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    rp[j] = kOut;
+    if (base + (uint32_t)j * kOpTileThreads + t < n) {
+      uint64_t key;
+      if (!pack_root(x[j], y[j], z[j], m.log2n, &key)) {
+        if (kCreate) or32(&m.ctr->status, kStCoordRange);
+      } else {
+        uint32_t h = (uint32_t)mix64(key) & (kRoots - 1);
+        rp[j] = kDirect;  // a table with no room near: the input asks the map itself
+        for (int p = 0; p < 16; ++p) {
+          if (lds_claim(&rkeys[h], key) == key) {
+            rp[j] = h;
+            break;
+          }
+          h = (h + 1) & (kRoots - 1);
+        }
+      }
+    }
+  }
+  __syncthreads();
+  // Workgroups begin at different parts of their tables: those that start
+  // together then claim different roots of a new grid, and find the rest
+  // claimed (2M cells in 1,584 new roots: 42 -> 30 us)
+  for (uint32_t q = t; q < kRoots; q += kOpTileThreads) {
+    const uint32_t p = (q + blockIdx.x * kOpTileThreads) & (kRoots - 1u);
+    const uint64_t key = rkeys[p];
+    bool inserted = false;
+    if (key != kEmptyKey) rslots[p] = kCreate ? root_probe(m, key, inserted) : root_find(m, key);
+    const uint64_t b = __ballot(inserted);
+    if (b && lane == 0) add32(&m.ctr->root_count, (uint32_t)__popcll(b));
+  }
+  __syncthreads();
+  const uint32_t cl = 3 * m.lb, il = 3 * m.ib;
+  uint64_t ent[kPer];
+  uint32_t at[kPer];  // bucket << 16 | rank in the tile's part of it
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    int32_t slot = -1;
+    if (rp[j] < kRoots) {
+      slot = rslots[rp[j]];
+    } else if (rp[j] == kDirect) {
+      uint64_t key;
+      pack_root(x[j], y[j], z[j], m.log2n, &key);
+      bool inserted = false;
+      slot = kCreate ? root_probe(m, key, inserted) : root_find(m, key);
+      if (inserted) add32(&m.ctr->root_count, 1u);
+    }
+    at[j] = kOut;
+    if (slot >= 0) {
+      const uint64_t child = ((uint64_t)slot << il) | inner_index(x[j], y[j], z[j], m.lb, m.ib);
+      const uint64_t cell = (child << cl) | leaf_index(x[j], y[j], z[j], m.lb);
+      const uint32_t bk = (uint32_t)mix64(child) & (os.nb - 1);
+      const uint32_t sh = (bk & 1u) * 16u;
+      const uint32_t r = atomicAdd(&hist[bk >> 1], 1u << sh) >> sh;
+      ent[j] = (cell << kOpTileLog) | ((uint32_t)j * kOpTileThreads + t);
+      at[j] = (bk << 16) | (r & 0xFFFFu);
+    }
+  }
+  __syncthreads();
+  // first places of the buckets: two words (four buckets) a thread
+  constexpr uint32_t kMost = kOpMaxBuckets / 2 / kOpTileThreads;
+  const uint32_t nw = os.nb / 2;
+  uint32_t c[kMost], sum = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < kMost; ++k) {
+    const uint32_t w = t * kMost + k;
+    c[k] = w < nw ? hist[w] : 0u;
+    sum += (c[k] & 0xFFFFu) + (c[k] >> 16);
+  }
+  const uint32_t incl = wave_scan(sum);
+  if (lane == 63) wsum[wid] = incl;
+  __syncthreads();
+  uint32_t run = incl - sum;
+  for (uint32_t w = 0; w < wid; ++w) run += wsum[w];
+  uint32_t* start = (uint32_t*)(os.start + (uint64_t)blockIdx.x * (os.nb + 2));
+#pragma unroll
+  for (uint32_t k = 0; k < kMost; ++k) {
+    const uint32_t w = t * kMost + k;
+    if (w < nw) {
+      const uint32_t lo = run, hi = run + (c[k] & 0xFFFFu);
+      run = hi + (c[k] >> 16);
+      hist[w] = lo | (hi << 16);
+      start[w] = lo | (hi << 16);
+      if (w == nw - 1) start[nw] = run;  // the tile's inputs in all
+    }
+  }
+  __syncthreads();
+  uint64_t* sorted = (uint64_t*)stage;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j)
+    if (at[j] != kOut) {
+      const uint32_t bk = at[j] >> 16;
+      sorted[((hist[bk >> 1] >> ((bk & 1u) * 16u)) & 0xFFFFu) + (at[j] & 0xFFFFu)] = ent[j];
+    }
+  __syncthreads();
+  uint32_t total = 0;
+  for (uint32_t w = 0; w < kOpTileThreads / 64; ++w) total += wsum[w];
+  for (uint32_t p = t; p < total; p += kOpTileThreads) gp(os.entry)[base + p] = sorted[p];
+}
+
+__device__ __forceinline__ void copy_bytes(uint8_t BXG_G* dst, const uint8_t BXG_G* src, uint32_t vb) {
+  for (uint32_t b = 0; b < vb; ++b) dst[b] = src[b];
+}
+
+// cell g of the map becomes value i of vals (null: zero bytes)
+__device__ __forceinline__ void set_cell(const MapView& m, uint64_t g, const uint8_t* vals, uint64_t i) {
+  const uint32_t vb = m.vb;
+  if (vb == 4) {
+    ((uint32_t BXG_G*)m.cells)[g] = vals ? gp((const uint32_t*)vals)[i] : 0u;
+  } else if (vb == 8 && ((uintptr_t)vals & 7u) == 0) {
+    ((uint64_t BXG_G*)m.cells)[g] = vals ? gp((const uint64_t*)vals)[i] : 0ull;
+  } else if (vals) {
+    copy_bytes(m.cells + g * vb, gp(vals) + i * vb, vb);
+  } else {
+    for (uint32_t b = 0; b < vb; ++b) m.cells[g * vb + b] = 0;
   }
 }
 
-// The leaf count when a bulk call starts: the leaves at or above it are the
-// call's, created with undefined bytes.
-__global__ void k_op_begin(const MapDev* __restrict__ mp) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  const MapView m = load_view(mp);
-  MapCounters BXG_G* ctr = gp(m.ctr);
-  ctr->leaf_base = min(ctr->leaf_count, m.leaf_cap);
-}
-
-// The leaves a bulk call created, initialised before any cell of them is
-// written: mask words and cell bytes zero (every cell off), as the
-// reference's Grid constructor leaves a new leaf (bonxai.hpp:51-58).  Grid-
-// stride over 8-byte words (a leaf's cells are a multiple of 8 bytes).
-__global__ void __launch_bounds__(256) k_zero_new_leaves(const MapDev* __restrict__ mp) {
-  const MapView m = load_view(mp);
-  const MapCounters BXG_G* ctr = gp(m.ctr);
-  const uint64_t lo = ctr->leaf_base;
-  const uint64_t hi = min(ctr->leaf_count, m.leaf_cap);
-  if (lo >= hi) return;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  const uint64_t start = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t nm = (hi - lo) * m.lw;
-  for (uint64_t i = start; i < nm; i += stride) m.masks[lo * m.lw + i] = 0;
-  const uint64_t cw = (uint64_t)m.lsz * m.vb / 8;  // 8-byte words a leaf
-  uint64_t BXG_G* cells = (uint64_t BXG_G*)m.cells + lo * cw;
-  const uint64_t nc = (hi - lo) * cw;
-  for (uint64_t i = start; i < nc; i += stride) cells[i] = 0;
+// A bucket of a bulk call.  kCreate: its missing leaves are created, all cells
+// off and zero (bonxai.hpp:51-58).  kApply: its cells are set.  kFirst: the
+// call needs each cell's first input and prior mask bit (was_on is asked for,
+// or setCellOn / setCellOff); a setValue batch without was_on needs only the
+// last input of each cell.  was_on of an input is the prior bit for the first
+// of its cell and "on" (off for setCellOff) for later ones, which k_op_tiles
+// has written; setValue keeps the last input's value, setCellOn the first
+// one's, if the cell was off.  A bucket with more cells or leaves than the
+// tables hold is done in halves by the bits of its cells' hashes.
+template <bool kCreate, bool kApply, bool kFirst, bool kLast>
+__global__ void __launch_bounds__(kOpThreads) k_op_buckets(const MapDev* __restrict__ mp,
+                                                           const uint8_t* __restrict__ vals, uint64_t n,
+                                                           uint32_t op, uint8_t* __restrict__ was_on,
+                                                           OpScratch os) {
+  __shared__ uint32_t ckey[kOpCells];    // leaf slot << 12 | cell in the leaf
+  __shared__ uint32_t clast[kLast ? kOpCells : 1];
+  __shared__ uint32_t cfirst[kFirst ? kOpCells : 1];
+  __shared__ uint64_t lkey[kOpLeaves];   // the leaf's entry among the children
+  __shared__ uint32_t lidx[kOpLeaves];
+  __shared__ uint32_t lnew[kOpLeaves];   // slots of the leaves to create
+  __shared__ uint64_t bits[kOpWords];    // mask bits of the call's cells
+  __shared__ uint32_t over, nnew, nbase;
+  const MapView m = uniform_view(mp);
+  const uint32_t t = threadIdx.x, lane = t & 63u, wid = t >> 6;
+  const bool failed = (map_status(m) & kFatal) != 0;  // such a call sets no cell
+  if (kApply && failed && was_on)
+    for (uint64_t i = (uint64_t)blockIdx.x * kOpThreads + t; i < n; i += (uint64_t)gridDim.x * kOpThreads)
+      was_on[i] = 0;
+  if (!kCreate && failed) return;
+  // buckets that follow each other (their entries share lines) on one XCD
+  const uint32_t bk = (blockIdx.x % kXcds) * (os.nb / kXcds) + blockIdx.x / kXcds;
+  const uint32_t cl = 3 * m.lb, il = 3 * m.ib;
+  const uint32_t lwl = 31u - (uint32_t)__clz((int)m.lw);  // lw is a power of two
+  const uint32_t nslots = min(kOpLeaves, kOpWords >> lwl);
+  // lanes a tile, so that the workgroup reads all tiles' entries at once
+  uint32_t gl = 0;
+  while (gl < 6 && (os.tiles << gl) < kOpThreads) ++gl;
+  uint32_t depth = 0, path = 0;
+  for (;;) {
+    for (uint32_t p = t; p < kOpCells; p += kOpThreads) {
+      ckey[p] = kNone;
+      if (kLast) clast[p] = 0;
+      if (kFirst) cfirst[p] = kNone;
+    }
+    for (uint32_t p = t; p < kOpLeaves; p += kOpThreads) lkey[p] = kEmptyKey;
+    for (uint32_t p = t; p < kOpWords; p += kOpThreads) bits[p] = 0;
+    if (t == 0) over = nnew = 0;
+    __syncthreads();
+    const uint32_t part = (uint32_t)((1ull << depth) - 1ull);
+    for (uint32_t tile = t >> gl; tile < os.tiles; tile += kOpThreads >> gl) {
+      const uint16_t BXG_G* st = gp((const uint16_t*)os.start) + (uint64_t)tile * (os.nb + 2) + bk;
+      const uint32_t hi = st[1];
+      const uint64_t tb = (uint64_t)tile * os.tile;
+      for (uint32_t k = st[0] + (t & ((1u << gl) - 1u)); k < hi; k += 1u << gl) {
+        const uint64_t e = gp((const uint64_t*)os.entry)[tb + k];
+        const uint64_t cell = e >> kOpTileLog;
+        const uint32_t i = (uint32_t)tb + ((uint32_t)e & ((1u << kOpTileLog) - 1u));
+        const uint64_t hash = mix64(cell);
+        if (((uint32_t)(hash >> 32) & part) != path) continue;
+        const uint64_t child = cell >> cl;
+        uint32_t ls = ((uint32_t)child * 0x9E3779B1u >> 20) & (nslots - 1u);
+        uint32_t p = 0;
+        for (; p < kOpProbes; ++p) {
+          if (lds_claim(&lkey[ls], child) == child) break;
+          ls = (ls + 1u) & (nslots - 1u);
+        }
+        if (p == kOpProbes) {
+          over = 1;
+          continue;
+        }
+        if (!kApply) continue;
+        const uint32_t key = (ls << 12) | ((uint32_t)cell & ((1u << cl) - 1u));
+        uint32_t h = (uint32_t)hash & (kOpCells - 1u);
+        for (p = 0; p < kOpProbes; ++p) {
+          if (lds_claim(&ckey[h], key) == key) {
+            if (kLast) atomicMax(&clast[h], i);
+            if (kFirst) atomicMin(&cfirst[h], i);
+            break;
+          }
+          h = (h + 1u) & (kOpCells - 1u);
+        }
+        if (p == kOpProbes) over = 1;
+      }
+    }
+    __syncthreads();
+    if (over) {
+      if (depth < 32) {
+        ++depth;
+        __syncthreads();
+        continue;
+      }
+      if (t == 0) or32(&m.ctr->status, kStScratchFull);  // cells of one hash: not met
+      return;
+    }
+    // the values of the cells, in flight while the leaves are looked up
+    constexpr uint32_t kMine = kOpCells / kOpThreads;
+    const bool word = kLast && (m.vb == 4 || (m.vb == 8 && ((uintptr_t)vals & 7u) == 0));
+    uint64_t val[kMine] = {};
+    if (kApply && !failed && word) {
+#pragma unroll
+      for (uint32_t j = 0; j < kMine; ++j) {
+        const uint32_t p = j * kOpThreads + t;
+        if (ckey[p] == kNone) continue;
+        if (m.vb == 4)
+          val[j] = gp((const uint32_t*)vals)[clast[p]];
+        else
+          val[j] = gp((const uint64_t*)vals)[clast[p]];
+      }
+    }
+    // the leaves: looked up, and created where missing
+    if (t < nslots && lkey[t] != kEmptyKey) {
+      const uint32_t c = m.children[lkey[t]];
+      lidx[t] = c < kPendingChild ? c : kNone;
+      if (kCreate && c >= kPendingChild) lnew[atomicAdd(&nnew, 1u)] = t;
+    }
+    if (kCreate) {
+      __syncthreads();
+      const uint32_t k = nnew;
+      if (k) {
+        if (t == 0) nbase = add32(&m.ctr->leaf_count, k);
+        __syncthreads();
+        if (t < k) {
+          const uint32_t s = lnew[t], idx = nbase + t;
+          if (idx >= m.leaf_cap) {
+            or32(&m.ctr->status, kStOutOfPool);
+          } else {
+            const uint64_t child = lkey[s];
+            const uint32_t ci = (uint32_t)child & (m.isz - 1u), im = (1u << m.ib) - 1u;
+            int32_t ox, oy, oz;
+            unpack_root(m.root_keys[child >> il], m.log2n, &ox, &oy, &oz);
+            m.origin[idx] = make_int4(ox + (int32_t)((ci & im) << m.lb), oy + (int32_t)(((ci >> m.ib) & im) << m.lb),
+                                      oz + (int32_t)((ci >> (2 * m.ib)) << m.lb), (int32_t)(child >> il));
+            m.children[child] = idx;
+            lidx[s] = idx;
+            lkey[s] = kCreated;
+          }
+        }
+        __syncthreads();
+        const uint32_t cw = (uint32_t)((uint64_t)m.lsz * m.vb / 8);  // 8-byte words a leaf
+        for (uint32_t r = wid; r < k; r += kOpThreads / 64) {
+          const uint32_t leaf = lidx[lnew[r]];
+          if (leaf == kNone) continue;
+          if (!kApply || failed)
+            for (uint32_t w = lane; w < m.lw; w += 64) m.masks[(uint64_t)leaf * m.lw + w] = 0;
+          for (uint32_t w = lane; w < cw; w += 64) ((uint64_t BXG_G*)m.cells)[(uint64_t)leaf * cw + w] = 0;
+        }
+      }
+    }
+    __syncthreads();
+    if (kApply && !failed) {
+#pragma unroll
+      for (uint32_t j = 0; j < kMine; ++j) {
+        const uint32_t p = j * kOpThreads + t, key = ckey[p];
+        if (key == kNone) continue;
+        const uint32_t ls = key >> 12, li = key & 4095u, leaf = lidx[ls];
+        if (leaf == kNone) continue;
+        const uint64_t g = (uint64_t)leaf * m.lsz + li;
+        const uint64_t bit = 1ull << (li & 63u);
+        bool pre = false;
+        if (kFirst) {
+          pre = lkey[ls] != kCreated && (m.masks[(uint64_t)leaf * m.lw + (li >> 6)] & bit) != 0;
+          if (was_on) was_on[cfirst[p]] = pre;
+        }
+        if (word) {
+          if (m.vb == 4)
+            ((uint32_t BXG_G*)m.cells)[g] = (uint32_t)val[j];
+          else
+            ((uint64_t BXG_G*)m.cells)[g] = val[j];
+        } else if (kLast) {
+          if (m.vb) set_cell(m, g, vals, clast[p]);
+        } else if (op == kOpSetOn) {
+          if (!pre && m.vb && vals) set_cell(m, g, vals, cfirst[p]);
+        } else {
+          set_cell(m, g, nullptr, 0);
+        }
+        atomicOr((unsigned long long*)&bits[(ls << lwl) + (li >> 6)], bit);
+      }
+      __syncthreads();
+      for (uint32_t w = t; w < nslots * m.lw; w += kOpThreads) {
+        const uint64_t v = bits[w];
+        const uint32_t ls = w >> lwl;
+        if (kCreate && lkey[ls] == kCreated) {  // every word of a new leaf
+          m.masks[(uint64_t)lidx[ls] * m.lw + (w & (m.lw - 1u))] = v;
+        } else if (v) {
+          uint64_t BXG_G* mw = m.masks + (uint64_t)lidx[ls] * m.lw + (w & (m.lw - 1u));
+          *mw = op == kOpSetOff ? *mw & ~v : *mw | v;
+        }
+      }
+      __syncthreads();
+    }
+    while (depth && ((path >> (depth - 1u)) & 1u)) path &= ~(1u << --depth);
+    if (!depth) return;
+    path |= 1u << (depth - 1u);
+  }
 }
 
 // create the root and leaf of every coordinate (setValue / setCellOn path)
@@ -1808,132 +2157,6 @@ __global__ void __launch_bounds__(256) k_touch(const MapDev* __restrict__ mp,
   if (slot < 0) return;
   const int32_t lmask = ~((1 << m.lb) - 1);
   leaf_request(m, (uint32_t)slot, inner_index(x, y, z, m.lb, m.ib), x & lmask, y & lmask, z & lmask);
-}
-
-// First and last input index of every distinct cell, and its prior mask
-// bit, in one pass with the creation of missing roots and leaves (kCreate:
-// setValue / setCellOn; setCellOff creates nothing and skips absent cells).
-// A cell's table key is its root slot, inner index and leaf index, known
-// before its leaf is, so a lane never waits for another lane's leaf: a leaf
-// still being created (or created in this call: index at or above the
-// call's leaf_base, its bytes not yet initialised) has all mask bits off.
-// kFirst: the call needs each cell's first input and prior mask bit (was_on
-// is asked for, or setCellOn / setCellOff); a setValue batch without was_on
-// needs only the last input of each cell (last write wins).
-template <bool kCreate, bool kFirst>
-__global__ void __launch_bounds__(256) k_op_resolve(const MapDev* __restrict__ mp,
-                                                    const int32_t* __restrict__ coords,
-                                                    uint64_t n, OpScratch os) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const MapView m = load_view(mp);
-  const int32_t x = coords[3 * i], y = coords[3 * i + 1], z = coords[3 * i + 2];
-  os.tpos[i] = kNone;
-  if (kFirst) os.prebit[i] = 0;
-  uint64_t rkey;
-  if (!pack_root(x, y, z, m.log2n, &rkey)) {
-    if (kCreate) or32(&m.ctr->status, kStCoordRange);
-    return;
-  }
-  const int32_t slot = kCreate ? root_insert(m, rkey) : root_find(m, rkey);
-  if (slot < 0) return;
-  const uint32_t ci = inner_index(x, y, z, m.lb, m.ib);
-  const uint32_t li = leaf_index(x, y, z, m.lb);
-  uint32_t leaf;
-  if (kCreate) {
-    const int32_t lmask = ~((1 << m.lb) - 1);
-    leaf = leaf_request(m, (uint32_t)slot, ci, x & lmask, y & lmask, z & lmask);
-    if (leaf == kEmptyChild) return;  // pool exhausted: the call fails
-  } else {
-    leaf = m.children[(uint64_t)slot * m.isz + ci];
-    if (leaf >= kPendingChild) return;
-  }
-  // a leaf still being created by another lane: its index is looked up by
-  // k_op_apply, after this kernel
-  os.leaf[i] = leaf < kPendingChild ? leaf : kNone;
-  if (kFirst && leaf < *gp(&m.ctr->leaf_base))
-    os.prebit[i] = (uint8_t)((m.masks[(uint64_t)leaf * m.lw + (li >> 6)] >> (li & 63)) & 1);
-  const uint64_t key = ((uint64_t)(uint32_t)slot << 24) | ((uint64_t)ci << 12) | (uint64_t)li;
-  uint32_t h = (uint32_t)mix64(key) & os.mask;
-  for (uint32_t p = 0; p <= os.mask; ++p) {
-    uint64_t k = gp(&os.slots[h])->key;
-    if (k == kEmptyKey) {
-      k = cas64(&os.slots[h].key, kEmptyKey, key);
-      if (k == kEmptyKey) k = key;
-    }
-    if (k == key) {
-      if (kFirst) min32(&os.slots[h].first, (uint32_t)i);
-      max32(&os.slots[h].last, (uint32_t)i);
-      os.tpos[i] = h;
-      return;
-    }
-    h = (h + 1) & os.mask;
-  }
-}
-
-enum : uint32_t { kOpSetValue = 0, kOpSetOn = 1, kOpSetOff = 2 };
-
-__device__ __forceinline__ void copy_bytes(uint8_t BXG_G* dst, const uint8_t BXG_G* src, uint32_t vb) {
-  for (uint32_t b = 0; b < vb; ++b) dst[b] = src[b];
-}
-
-// Sequential-order semantics of a batch of setValue / setCellOn / setCellOff
-// (bonxai.hpp:449-466, 537-569): was_on of an input is the prior bit for the
-// first occurrence of its cell and "on" (off for setCellOff) for later ones;
-// setValue keeps the last occurrence's value, setCellOn the first one's.
-__global__ void __launch_bounds__(256) k_op_apply(const MapDev* __restrict__ mp,
-                                                  const int32_t* __restrict__ coords,
-                                                  const uint8_t* __restrict__ vals, uint64_t n,
-                                                  uint32_t op, uint8_t* __restrict__ was_on,
-                                                  OpScratch os) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const MapView m = load_view(mp);
-  const uint32_t t = os.tpos[i];
-  if (t == kNone || (map_status(m) & kFatal)) {  // no cell, or the call failed
-    if (was_on) was_on[i] = 0;
-    return;
-  }
-  const uint32_t last = os.slots[t].last;
-  // first and the prior bit exist only where k_op_resolve was asked for them
-  const bool need_first = was_on != nullptr || op != kOpSetValue;
-  const uint32_t first = need_first ? os.slots[t].first : 0u;
-  const uint8_t pre = need_first ? os.prebit[i] : (uint8_t)0;
-  const int32_t x = coords[3 * i], y = coords[3 * i + 1], z = coords[3 * i + 2];
-  const uint32_t known = os.leaf[i];
-  const uint32_t leaf = known != kNone ? known : find_leaf(m, x, y, z);
-  if (leaf == kNone) {
-    if (was_on) was_on[i] = 0;
-    return;
-  }
-  const uint32_t li = leaf_index(x, y, z, m.lb);
-  const uint64_t g = (uint64_t)leaf * m.lsz + li;
-  uint64_t* mw = (uint64_t*)&m.masks[(uint64_t)leaf * m.lw + (li >> 6)];
-  const uint64_t bit = 1ull << (li & 63);
-  const uint32_t vb = m.vb;
-  if (op == kOpSetOff) {
-    if (was_on) was_on[i] = (uint8_t)((uint32_t)i == first ? pre : 0);
-    if ((uint32_t)i == last) {
-      and64(mw, ~bit);
-      for (uint32_t b = 0; b < vb; ++b) m.cells[g * vb + b] = 0;
-    }
-    return;
-  }
-  if (was_on) was_on[i] = (uint8_t)((uint32_t)i == first ? pre : 1);
-  if (op == kOpSetValue) {
-    if ((uint32_t)i == last) {
-      if (vb == 4)
-        ((uint32_t BXG_G*)m.cells)[g] = gp((const uint32_t*)vals)[i];
-      else if (vb)
-        copy_bytes(m.cells + g * vb, gp(vals) + i * vb, vb);
-      or64(mw, bit);
-    }
-  } else {  // setCellOn: the first occurrence decides, and writes only if off
-    if ((uint32_t)i == first) {
-      if (!pre && vb && vals) copy_bytes(m.cells + g * vb, gp(vals) + i * vb, vb);
-      or64(mw, bit);
-    }
-  }
 }
 
 
