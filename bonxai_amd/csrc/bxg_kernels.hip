@@ -425,99 +425,6 @@ __device__ __forceinline__ uint32_t collect_run(const MapView& m, RayWalk& w, ui
   return collect_cells(w, m.lb, li);
 }
 
-// The leaves a ray's cells [k, kend) lie in, one leaf per step, without
-// visiting the cells.  Along an axis with |d| > 0 the ray takes its n-th step
-// at cell ceil((2n - 1) m / (2|d|)) (the inverse of the closed form), so the
-// cell at which it enters the leaf N axis steps away is that value for N;
-// the next boundary is L steps further, which adds floor(L m / |d|) and a
-// remainder to the quotient, so after the set-up (a few divisions a ray)
-// each leaf costs additions and compares only.  Axes crossing at the same
-// cell move the ray diagonally, into one leaf.  Same leaves, in the same
-// order, as the cell walk.
-struct LeafWalk {
-  int32_t lx, ly, lz;  // origin of the current leaf
-  int32_t stx, sty, stz;  // +-L per leaf along each axis
-  int32_t kx, ky, kz;  // cell at which the ray enters the next leaf along each axis
-  uint32_t qx, qy, qz, rx, ry, rz;  // kx = qx + (rx > 0): (2N - 1) m = qx * 2|dx| + rx
-  uint32_t Qx, Qy, Qz, Rx, Ry, Rz;  // per further leaf: floor(L m / |d|), 2 (L m mod |d|)
-  uint32_t bx, by, bz;  // 2|d|
-  int32_t k, kend;
-  static constexpr int32_t kNever = 0x7fffffff;
-  __device__ __forceinline__ static void axis(int32_t c, int32_t s, int32_t d, int32_t n, int32_t m,
-                                              uint32_t L, int32_t& lc, int32_t& st, int32_t& kc,
-                                              uint32_t& q, uint32_t& r, uint32_t& Q, uint32_t& R,
-                                              uint32_t& b) {
-    const int32_t lm = (int32_t)L - 1;
-    lc = c & ~lm;
-    st = s * (int32_t)L;
-    b = 2u * (uint32_t)(d > 0 ? d : 1);
-    if (d == 0) {
-      kc = kNever;
-      q = r = Q = R = 0;
-      return;
-    }
-    // axis steps from the origin to the first cell of the next leaf
-    const int64_t N = (int64_t)n + (s > 0 ? (int64_t)L - (c & lm) : (int64_t)(c & lm) + 1);
-    if (m <= kRay32) {  // the same in 32 bits: (2N - 1) m < 2^32
-      const uint32_t A = (uint32_t)(2 * N - 1) * (uint32_t)m, LM = L * (uint32_t)m;
-      q = A / b;
-      r = A - q * b;
-      Q = LM / (uint32_t)d;
-      R = 2u * (LM - Q * (uint32_t)d);
-      kc = (int32_t)(q + (r > 0 ? 1u : 0u));
-      return;
-    }
-    const uint64_t A = (uint64_t)(2 * N - 1) * (uint64_t)m;
-    const uint64_t q64 = A / b;
-    const uint64_t LM = (uint64_t)L * (uint64_t)m;
-    const uint64_t Q64 = LM / (uint64_t)d;
-    // quotients past 2^30 are beyond any ray (kend < 2^30): such an axis
-    // never crosses again, and the sums below cannot overflow
-    q = (uint32_t)(q64 < (1ull << 30) ? q64 : (1ull << 30));
-    r = (uint32_t)(A - q64 * b);
-    Q = (uint32_t)(Q64 < (1ull << 30) ? Q64 : (1ull << 30));
-    R = 2u * (uint32_t)(LM - Q64 * (uint64_t)d);
-    kc = (int32_t)(q + (r > 0 ? 1u : 0u));
-  }
-  // the leaf of cell w.k, walking cells [w.k, w.kend) of w's ray
-  __device__ __forceinline__ void init(const RayWalk& w, uint32_t lb) {
-    const uint32_t L = 1u << lb;
-    k = w.k;
-    kend = w.kend;
-    // axis steps already taken at cell k (none at k = 0)
-    int32_t nx = 0, ny = 0, nz = 0;
-    if (k) w.steps(k, nx, ny, nz);
-    axis(w.cx, w.sx, w.dx, nx, w.mx, L, lx, stx, kx, qx, rx, Qx, Rx, bx);
-    axis(w.cy, w.sy, w.dy, ny, w.mx, L, ly, sty, ky, qy, ry, Qy, Ry, by);
-    axis(w.cz, w.sz, w.dz, nz, w.mx, L, lz, stz, kz, qz, rz, Qz, Rz, bz);
-  }
-  __device__ __forceinline__ bool done() const { return k >= kend; }
-  __device__ __forceinline__ static void cross(int32_t& lc, int32_t st, int32_t& kc, uint32_t& q,
-                                               uint32_t& r, uint32_t Q, uint32_t R, uint32_t b) {
-    lc += st;
-    q += Q;
-    r += R;
-    if (r >= b) {
-      ++q;
-      r -= b;
-    }
-    kc = q < (1u << 30) ? (int32_t)(q + (r > 0 ? 1u : 0u)) : kNever;
-  }
-  // move to the next leaf (or past kend)
-  __device__ __forceinline__ void next() {
-    int32_t kn = kx < ky ? kx : ky;
-    kn = kn < kz ? kn : kz;
-    if (kn >= kend) {
-      k = kend;
-      return;
-    }
-    if (kx == kn) cross(lx, stx, kx, qx, rx, Qx, Rx, bx);
-    if (ky == kn) cross(ly, sty, ky, qy, ry, Qy, Ry, by);
-    if (kz == kn) cross(lz, stz, kz, qz, rz, Qz, Rz, bz);
-    k = kn;
-  }
-};
-
 // Allocation pass, one step of a ray: the root of its current leaf (created
 // if missing) and the ray's next leaves of that root, up to kLeafRun, as bits
 // of the root's inner cells.  One load of `known` tells which of them exist
@@ -529,24 +436,30 @@ struct LeafWalk {
 // that adds 38k leaves to a map, now 40; and a first scan's rays, creating
 // leaves and marking cells in one walk, took 465 us, now 60 + 230.)
 constexpr int kLeafRun = 8;
-__device__ __forceinline__ void leaves_step(const MapView& m, LeafWalk& lw, RootCache& rc,
+constexpr int32_t kNoRoot = -2;  // the root is not looked up yet
+__device__ __forceinline__ void leaves_step(const MapView& m, LeafWalk& lw, int32_t& slot,
                                             const uint64_t BXG_G* known, bool go) {
   uint64_t miss = 0;
   uint32_t e = 0;  // word of the directory (at most 2^24 roots of 64 words)
   if (go) {
-    const int32_t slot = root_slot<true>(m, rc, lw.lx, lw.ly, lw.lz);
-    const int32_t rmask = ~((1 << m.log2n) - 1);
-    const uint32_t ci = inner_index(lw.lx, lw.ly, lw.lz, m.lb, m.ib);
+    if (!lw.inside(m.ib)) {
+      lw.enter(m.lb, m.ib);
+      slot = kNoRoot;
+    }
+    if (slot == kNoRoot) {
+      uint64_t key;
+      slot = pack_root(lw.rx, lw.ry, lw.rz, m.log2n, &key) ? root_insert(m, key) : -1;
+    }
+    const uint32_t ci = lw.cell(m.ib);
     const uint32_t word = ci >> 6;
+    const uint32_t mask = LeafWalk::inside_mask(m.ib) | LeafWalk::word_mask(m.ib);
+    const uint32_t here = lw.p & mask;  // this root, this word
     uint64_t bits = 1ull << (ci & 63u);
     lw.next();
 #pragma unroll
     for (int j = 1; j < kLeafRun; ++j) {
-      const uint32_t c = inner_index(lw.lx, lw.ly, lw.lz, m.lb, m.ib);
-      const bool in = !lw.done() & ((((lw.lx & rmask) ^ rc.rx) | ((lw.ly & rmask) ^ rc.ry) |
-                                     ((lw.lz & rmask) ^ rc.rz)) == 0) & ((c >> 6) == word);
-      if (!in) break;
-      bits |= 1ull << (c & 63u);
+      if (lw.done() | ((lw.p & mask) != here)) break;
+      bits |= 1ull << (lw.p & LeafWalk::kBit);
       lw.next();
     }
     if (slot >= 0) {  // else the root directory is full: the call fails
@@ -1194,7 +1107,7 @@ __global__ void __launch_bounds__(256) k_scan_scatter(const BatchHdr* __restrict
 // walked whole: update pass (in a map empty at the scan's start, and in
 // others) and leaf pass; the defaults of the tuning keys fresh_window,
 // ray_window and leaf_window.  Measured on 64 scans: re-inserted 8 beats 4 and
-// 16 (3.7 against 4.2 and 4.1 ms); leaf pass 64: 0.50, 16: 0.60, none: 0.49
+// 16 (3.7 against 4.2 and 4.1 ms); leaf pass (since then 0.39) 64: 0.50, 16: 0.60, none: 0.49
 // re-inserted, 0.92, 1.04, 0.98 ms into empty maps
 constexpr int32_t kFreshWindow = 16;
 constexpr int32_t kUpdateWindow = 8;
@@ -1307,12 +1220,13 @@ __device__ void walk_winners(const ScanDesc* __restrict__ sd, const ScanScratch&
           w.seek(k0, k1);
       }
       LeafWalk lw;  // the leaf pass walks leaves, not cells
+      int32_t slot = kNoRoot;
       RootCache rc;
       rc.reset();
       uint32_t next_leaf = kNone;
       uint32_t nupd = 0;
       const uint32_t ncells = have ? (uint32_t)(w.kend - w.k) : 0u;
-      if (kLeaves && have) lw.init(w, m.lb);
+      if (kLeaves && have) lw.init(w, m.lb, m.ib);
       if (!kLeaves && have) next_leaf = walk_leaf(m, w, rc);
       while (__ballot(have)) {
         bool go = have;
@@ -1322,7 +1236,7 @@ __device__ void walk_winners(const ScanDesc* __restrict__ sd, const ScanScratch&
           if (__ballot(go) == 0) go = have;  // a window that wraps past 2^31
         }
         if (kLeaves) {
-          leaves_step(m, lw, rc, lbase == 0 ? m.want : m.have, go);
+          leaves_step(m, lw, slot, lbase == 0 ? m.want : m.have, go);
           have = have && !(go && lw.done());
         } else if (go) {
           nupd += apply_step<kMode == 2>(m, w, rc, cur, lbase, mark, next_leaf);
@@ -1360,13 +1274,12 @@ __global__ void __launch_bounds__(256) k_scan_extra_leaves(const BatchHdr* __res
     const int4 e = j < d.nextra ? d.extra[j] : make_int4(d.ox, d.oy, d.oz, 0);
     bool have = !(e.x == d.ox && e.y == d.oy && e.z == d.oz);
     RayWalk w;
-    RootCache rc;
-    rc.reset();
     w.init(d.ox, d.oy, d.oz, e.x, e.y, e.z);
     LeafWalk lw;
-    lw.init(w, m.lb);
+    lw.init(w, m.lb, m.ib);
+    int32_t slot = kNoRoot;
     while (__ballot(have)) {
-      leaves_step(m, lw, rc, m.have, have);
+      leaves_step(m, lw, slot, m.have, have);
       if (have && lw.done()) have = false;
     }
   }
