@@ -83,26 +83,28 @@ __device__ __forceinline__ uint64_t lanes_below() { return (1ull << lane_id()) -
 // Minimum over the 64 lanes of a wavefront, every lane active: DPP moves
 // within quads (quad_perm [1,0,3,2], [2,3,0,1]) and rows (row_ror 4, 8), then
 // row_bcast 15 into rows 1 and 3 and row_bcast 31 into rows 2 and 3, so that
-// lane 63 holds the minimum; no LDS round trips.
+// lane 63 holds the minimum; no LDS round trips.  The value kept where a move
+// writes nothing is the operation's identity, so that the compiler makes the
+// move a modifier of the operation.
 __device__ __forceinline__ int32_t wave_min(int32_t v) {
-  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));
-  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));
-  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x124, 0xF, 0xF, false));
-  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x128, 0xF, 0xF, false));
-  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xA, 0xF, false));
-  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xC, 0xF, false));
+  v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0xB1, 0xF, 0xF, false));
+  v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x4E, 0xF, 0xF, false));
+  v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x124, 0xF, 0xF, false));
+  v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x128, 0xF, 0xF, false));
+  v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x142, 0xA, 0xF, false));
+  v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x143, 0xC, 0xF, false));
   return __builtin_amdgcn_readlane(v, 63);
 }
 
 // bitwise or over the 64 lanes of a wavefront, every lane active (the steps
 // of wave_min)
 __device__ __forceinline__ uint32_t wave_or32(uint32_t v) {
-  v |= (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0xB1, 0xF, 0xF, false);
-  v |= (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x4E, 0xF, 0xF, false);
-  v |= (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x124, 0xF, 0xF, false);
-  v |= (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x128, 0xF, 0xF, false);
-  v |= (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x142, 0xA, 0xF, false);
-  v |= (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x143, 0xC, 0xF, false);
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false);
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, false);
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xF, 0xF, false);
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xF, 0xF, false);
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);
+  v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);
   return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 __device__ __forceinline__ uint64_t wave_or(uint64_t v) {
@@ -421,7 +423,8 @@ __device__ __forceinline__ uint32_t cell_miss(uint32_t w, int32_t miss, int32_t 
 
 // The cell walk of a ray (RayWalk, collect_cells) is in bxg_walk.h, shared
 // with the host check of the walk.
-__device__ __forceinline__ uint32_t collect_run(const MapView& m, RayWalk& w, uint32_t li[kRun]) {
+template <class Walk>
+__device__ __forceinline__ uint32_t collect_run(const MapView& m, Walk& w, uint32_t li[kRun]) {
   return collect_cells(w, m.lb, li);
 }
 
@@ -494,10 +497,13 @@ __device__ __forceinline__ void leaves_step(const MapView& m, LeafWalk& lw, int3
 // its update_id already equals cur.  Returns the cells written (counted
 // form: exact, by CAS).
 // leaf index of the walk's current cell (read-only phases)
-__device__ __forceinline__ uint32_t walk_leaf(const MapView& m, const RayWalk& w, RootCache& rc) {
-  const int32_t slot = root_slot<false>(m, rc, w.cx, w.cy, w.cz);
+template <class Walk>
+__device__ __forceinline__ uint32_t walk_leaf(const MapView& m, const Walk& w, RootCache& rc) {
+  int32_t x, y, z;
+  w.cell(x, y, z);
+  const int32_t slot = root_slot<false>(m, rc, x, y, z);
   if (slot < 0) return kNone;
-  const uint32_t c = m.children[(uint64_t)slot * m.isz + inner_index(w.cx, w.cy, w.cz, m.lb, m.ib)];
+  const uint32_t c = m.children[(uint64_t)slot * m.isz + inner_index(x, y, z, m.lb, m.ib)];
   return c >= kPendingChild ? kNone : c;
 }
 
@@ -513,8 +519,8 @@ __device__ __forceinline__ uint32_t walk_leaf(const MapView& m, const RayWalk& w
 // the leaf's cells and mask words from those bytes after the scan's endpoints
 // are marked.  In older leaves each cell is read, updated unless its
 // update_id is cur, and the cells turned on set their mask bits with atomicOrs.
-template <bool kCount>
-__device__ __forceinline__ uint32_t apply_step(const MapView& m, RayWalk& w, RootCache& rc,
+template <bool kCount, class Walk>
+__device__ __forceinline__ uint32_t apply_step(const MapView& m, Walk& w, RootCache& rc,
                                                int32_t cur, uint32_t lbase, uint32_t mark,
                                                uint32_t& next_leaf) {
   const uint32_t leaf = next_leaf;
@@ -1141,6 +1147,32 @@ constexpr uint32_t kGroupLog = 3;   // batches side by side on one XCD in a shor
 // the dependent loads of a step (entry, cells) and the scattered lines they
 // touch.
 //
+// whether a lane at cell k steps with its wavefront: every lane that has a ray
+// and is less than win cells ahead of the slowest
+__device__ __forceinline__ bool in_window(bool have, int32_t k, int32_t win) {
+  const bool go = have && k < wave_min(have ? k : 0x7fffffff) + win;
+  return __ballot(go) == 0 ? have : go;  // else a window that wraps past 2^31
+}
+
+// the update walk of a wavefront's rays (lanes with have set); cells written
+// (counted form)
+template <bool kCount, class Walk>
+__device__ __forceinline__ uint32_t walk_cells(const MapView& m, Walk& w, bool have, bool lockstep, int32_t win,
+                                               int32_t cur, uint32_t lbase, uint32_t mark) {
+  RootCache rc;
+  rc.reset();
+  uint32_t next_leaf = kNone, nupd = 0;
+  if (have) next_leaf = walk_leaf(m, w, rc);
+  while (__ballot(have)) {
+    const bool go = lockstep ? in_window(have, w.k, win) : have;
+    if (go) {
+      nupd += apply_step<kCount>(m, w, rc, cur, lbase, mark, next_leaf);
+      have = !w.done();
+    }
+  }
+  return nupd;
+}
+
 // kMode 0: leaf allocation pass; 1: update pass; 2: counted update.
 template <int kMode>
 __device__ void walk_winners(const ScanDesc* __restrict__ sd, const ScanScratch& sc) {
@@ -1219,29 +1251,23 @@ __device__ void walk_winners(const ScanDesc* __restrict__ sd, const ScanScratch&
         else
           w.seek(k0, k1);
       }
-      LeafWalk lw;  // the leaf pass walks leaves, not cells
-      int32_t slot = kNoRoot;
-      RootCache rc;
-      rc.reset();
-      uint32_t next_leaf = kNone;
-      uint32_t nupd = 0;
       const uint32_t ncells = have ? (uint32_t)(w.kend - w.k) : 0u;
-      if (kLeaves && have) lw.init(w, m.lb, m.ib);
-      if (!kLeaves && have) next_leaf = walk_leaf(m, w, rc);
-      while (__ballot(have)) {
-        bool go = have;
-        if (lockstep) {
-          const int32_t k = kLeaves ? lw.k : w.k;
-          go = have && k < wave_min(have ? k : 0x7fffffff) + win;
-          if (__ballot(go) == 0) go = have;  // a window that wraps past 2^31
-        }
-        if (kLeaves) {
+      uint32_t nupd = 0;
+      if (kLeaves) {  // walks leaves, not cells
+        LeafWalk lw;
+        if (have) lw.init(w, m.lb, m.ib);
+        int32_t slot = kNoRoot;
+        while (__ballot(have)) {
+          const bool go = lockstep ? in_window(have, lw.k, win) : have;
           leaves_step(m, lw, slot, lbase == 0 ? m.want : m.have, go);
           have = have && !(go && lw.done());
-        } else if (go) {
-          nupd += apply_step<kMode == 2>(m, w, rc, cur, lbase, mark, next_leaf);
-          have = !w.done();
         }
+      } else if (__ballot(have && w.mx > kRay32)) {
+        nupd = walk_cells<kMode == 2>(m, w, have, lockstep, win, cur, lbase, mark);
+      } else {
+        RayWalk16 w16;
+        if (have) w16.init(w, m.lb);
+        nupd = walk_cells<kMode == 2>(m, w16, have, lockstep, win, cur, lbase, mark);
       }
       if (kMode == 2 && ncells) {
         add64(&m.ctr->stat_ray_updates, nupd);
