@@ -781,6 +781,15 @@ uint32_t tag_bits_for(uint32_t nscans) {
   return b;
 }
 
+// One-scan calls of up to this many points list their winners in point order,
+// not by direction and length: two atomics and a launch fewer (about 10 us a
+// call in a map in use: 2,001 points 111 -> 99 us, 16k 168 -> 164, 32k 213 ->
+// 208, where a room's random points already lose 7 us in the update pass; from
+// 65k on nothing is left).  Not in a map known to be empty, where the wants of
+// rays in random directions meet on more words (2,000 points of a room: leaf
+// pass 15 -> 47 us), and not in a graph, whose maps may be empty.
+constexpr uint64_t kListedPoints = 16384;
+
 // The kernel sequence of one wave of scans on given scratch and descriptors.
 // args: the batch's header and descriptors (at most kMostArgs), which the
 // first kernel writes to hdr and desc; null where they are there already.
@@ -830,12 +839,17 @@ int enqueue_scan_kernels(bxg_ctx* c, BatchHdr* hdr, ScanDesc* desc, ScanScratch 
     }
     BXG_TRY(launch(c, "k_scan_classify", k_scan_classify, gp, kBlock, hdr, desc, sc));
   }
-  BXG_TRY(launch(c, "k_scan_winners", k_scan_winners, gp, kBlock, hdr, desc, sc));
   // a tile of buckets a scan (the scan index mod 64)
   const uint32_t tiles = (1u << (kDirBits + tag_bits_for(nscans))) / kScanTile;
-  if (tiles == 1) {
-    BXG_TRY(launch(c, "k_scan_scatter", k_scan_scatter<true>, std::max(gp, 1u), kBlock, hdr, sc));
+  const bool listed = args && nscans == 1 && !all_empty && grid_points <= kListedPoints;
+  if (listed) {
+    BXG_TRY(launch(c, "k_scan_winners", k_scan_list_winners, std::max(gp, 1u), kBlock, hdr, sc));
   } else {
+    BXG_TRY(launch(c, "k_scan_winners", k_scan_winners, gp, kBlock, hdr, desc, sc));
+  }
+  if (!listed && tiles == 1) {
+    BXG_TRY(launch(c, "k_scan_scatter", k_scan_scatter<true>, std::max(gp, 1u), kBlock, hdr, sc));
+  } else if (!listed) {
     if (tiles > kUnreducedTiles)
       BXG_TRY(launch(c, "k_scan_bucket_reduce", k_scan_bucket_reduce, tiles, 1024, hdr, sc));
     BXG_TRY(launch(c, "k_scan_bucket_scan", k_scan_bucket_scan, tiles, 1024, hdr, sc));
@@ -1199,7 +1213,8 @@ int insert_noalloc(bxg_map* m, const bxg_scan_desc& in) {
   BXG_TRY(fill64(c, (uint64_t*)sc.ep, slots * 2, ~0ull));
   BXG_TRY(fill32(c, sc.hist, kMaxBuckets, 0));
   BXG_TRY(fill32(c, sc.counters, kCounterWords, 0));
-  BXG_TRY(enqueue_scan_kernels(c, d_hdr, d_desc, sc, in.n, 1, false, false, &hdr, &d));
+  const bool empty = m->known_leaves == 0 && !m->ctr_pending;
+  BXG_TRY(enqueue_scan_kernels(c, d_hdr, d_desc, sc, in.n, 1, false, empty, &hdr, &d));
   BXG_TRY(read_counters(m));  // waits for the scan
   const uint32_t st = m->h_ctr->status;
   if (st & ~overflow) return map_status(m);

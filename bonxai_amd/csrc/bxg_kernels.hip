@@ -908,6 +908,8 @@ __device__ __forceinline__ RayOrder ray_order(uint32_t k) {
   }
 }
 
+constexpr uint32_t kLeafLater = 0xFFFFFFFEu;  // tpos: the endpoint's leaf is not looked up yet
+
 // Phase 2 (per point): the lowest-index point of each claimed voxel is its
 // winner (probabilistic_map.cpp:30-54 lets only the first point of a voxel
 // through the update_id test); winners are counted per bucket, and each
@@ -973,6 +975,29 @@ __global__ void __launch_bounds__(256) k_scan_winners(const BatchHdr* __restrict
   if (win && lead == lane_id()) base = add32(&sc.hist[key], size);
   base = (uint32_t)__shfl((int)base, (int)lead);
   if (win) sc.wrank[gi] = base + rank;
+}
+
+// Phase 2 of a call of one scan of few points: the winners listed in point
+// order, a wavefront's together, their endpoint-table slots released, in place
+// of the buckets.  A loser that reads its voxel's slot after the release sees
+// no index, which is not its own either.
+__global__ void __launch_bounds__(256) k_scan_list_winners(const BatchHdr* __restrict__ hdr, ScanScratch sc) {
+  const uint64_t gi = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  bool win = false;
+  EpSlot BXG_G* e = nullptr;
+  if (gi < hdr->total && (sc.rec[gi].w & kRecMarked)) {
+    e = gp(&sc.ep[sc.tpos[gi]]);
+    win = e->first == (uint32_t)gi;
+  }
+  const uint64_t wins = __ballot(win);
+  uint32_t base = 0;
+  if (lane_id() == 0 && wins) base = add32(&sc.counters[0], (uint32_t)__popcll(wins));
+  base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+  if (!win) return;
+  sc.winners[base + (uint32_t)__popcll(wins & lanes_below())] = (uint32_t)gi;
+  e->key = kEmptyKey;
+  e->first = kNone;
+  sc.tpos[gi] = kLeafLater;
 }
 
 // inclusive prefix sum over the 64 lanes of a wavefront
@@ -1056,8 +1081,6 @@ __global__ void __launch_bounds__(1024) k_scan_bucket_scan(const BatchHdr* __res
   reinterpret_cast<uint4*>(sc.offs + base)[threadIdx.x] = o;
   if (base + kScanTile >= nb && threadIdx.x == 1023) sc.counters[0] = carry + wsum[15];
 }
-
-constexpr uint32_t kLeafLater = 0xFFFFFFFEu;  // tpos: the endpoint's leaf is not looked up yet
 
 // Phase 2t (per point): winners written into their buckets, and their
 // endpoint-table slots released (every point has read its slot by now).
@@ -1583,10 +1606,11 @@ __global__ void __launch_bounds__(256) k_scan_extra_rays(const BatchHdr* __restr
 // workgroup of this kernel reads: update_count 1 -> 2 -> 3 -> 1
 // (probabilistic_map.cpp:103-105) unless the scan failed; every scanned map's
 // counters to its pinned host mirror, so that the host learns pool use and
-// errors from one event after the call (no copy a map); the clip counts back
-// to zero.
+// errors from one event after the call (no copy a map); the winner count and
+// the clip counts back to zero.
 __device__ __forceinline__ void scan_finalize(uint32_t nscans, const ScanDesc* sd, const ScanScratch& sc) {
   if (threadIdx.x < 64u) sc.counters[kClipWords + threadIdx.x] = 0;
+  if (threadIdx.x == 0) sc.counters[0] = 0;
   for (uint32_t s = threadIdx.x; s < nscans; s += blockDim.x) {
     const MapDev BXG_G* md = (const MapDev BXG_G*)sd[s].map;
     MapCounters BXG_G* ctr = gp(md->ctr);
