@@ -823,8 +823,9 @@ int enqueue_scan_kernels(bxg_ctx* c, BatchHdr* hdr, ScanDesc* desc, ScanScratch 
   sc.win_fresh = (int32_t)c->fresh_window;
   sc.ray_order = c->ray_order;
   // New-leaf pass: a wavefront per new leaf, grid-stride over them, 2
-  // workgroups a CU (64 first scans 2.37 ms with 8, 2.26 with 3, 2.14 with 2,
-  // 2.83 with 1; LiDAR scans of a map in use 35, 32, 28, 34 us).  Small calls
+  // workgroups a CU (LiDAR scans of a map in use 35 us with 8, 32 with 3, 28
+  // with 2, 34 with 1; 64 first scans run at the memory's rate, 2.1 to 2.4 ms
+  // from process to process, with 2 as with 8, and 2.8 with 1).  Small calls
   // too: a sparse scan's rays create a hundred leaves a point (2,001 LiDAR
   // points into an empty map: 141 us on a workgroup per 256 points, 9 on 64).
   const uint32_t gm = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(cus * 2, 64ull * gp));
