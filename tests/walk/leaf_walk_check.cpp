@@ -13,7 +13,7 @@ int main() {
   long leaves = 0;
   for (uint32_t lb = 1; lb <= 4; ++lb) {
     for (uint32_t ib = 1; ib <= 4; ++ib) {
-      for (const int32_t m : {0, 1, 2, 7, 40, 300, 3001, 32766, 32767, 32768, 70001}) {
+      for (const int32_t m : {0, 1, 2, 7, 40, 300, 3001, 32766, 32767, 32768, 70001, 1 << 24}) {
         for (int t = 0; t < (m > 5000 ? 12 : 200); ++t) {
           int32_t o[3], d[3];
           for (int a = 0; a < 3; ++a) {
@@ -24,10 +24,12 @@ int main() {
           if (t % 5 == 0) d[(t + 1) % 3] = 0;
           if (t % 7 == 0) d[(t + 2) % 3] = d[t % 3];
           if (t % 11 == 0) d[(t + 1) % 3] = m > 0 ? 1 : 0;
-          // the whole ray with its end cell, or a part of it
+          // the whole ray with its end cell, or a part of it (of the longest, 20000 cells)
           const int32_t last = m + 1;
-          const int32_t k0 = t < 20 ? 0 : (int32_t)(rng() % (uint64_t)last);
-          const int32_t k1 = t < 20 ? last : k0 + 1 + (int32_t)(rng() % (uint64_t)(last - k0));
+          const bool whole = t < 20 && m < (1 << 20);
+          const int32_t k0 = whole ? 0 : (int32_t)(rng() % (uint64_t)last);
+          int32_t k1 = whole ? last : k0 + 1 + (int32_t)(rng() % (uint64_t)(last - k0));
+          if (m >= 1 << 20 && k1 - k0 > 20000) k1 = k0 + 20000;
           bxg::RayWalk w;
           w.init(o[0], o[1], o[2], o[0] + d[0], o[1] + d[1], o[2] + d[2]);
           if (k0 == 0)
