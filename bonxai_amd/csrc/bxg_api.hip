@@ -132,6 +132,7 @@ struct bxg_map {
   MapCounters* h_ctr = nullptr;  // pinned mirror of the counters
   std::shared_ptr<SnapEvent> snap;  // completion of the last snapshot into h_ctr
   bool ctr_pending = false;
+  uint64_t under_way = 0;  // leaves that the work since the counters last landed may create, at most
   uint32_t root_cap = 0;
   uint32_t leaf_cap = 0;
   uint64_t bytes = 0;
@@ -378,18 +379,22 @@ void take_counters(bxg_map* m) {
   m->known_scans = m->h_ctr->scans_applied;
 }
 
+// the same once the snapshot has landed: no work on the map is under way
+void take_landed(bxg_map* m) {
+  m->ctr_pending = false;
+  m->snap.reset();
+  m->under_way = 0;
+  take_counters(m);
+}
+
 // The counters of a map as its enqueued work leaves them, from the host
 // mirror: every call that changes them ends with a copy into the mirror (a
 // scan's last kernel writes it, the others enqueue one) and an event, waited
 // for here; the host's own changes go to the mirror too.  No copy of its own:
 // a blocking copy cost about 20 us a map, 64 of them a frame's read-back.
 int landed_counters(bxg_map* m) {
-  if (m->ctr_pending) {
-    BXG_HIP(m->ctx, hipEventSynchronize(m->snap->e));
-    m->ctr_pending = false;
-    m->snap.reset();
-  }
-  take_counters(m);
+  if (m->ctr_pending) BXG_HIP(m->ctx, hipEventSynchronize(m->snap->e));
+  take_landed(m);
   return BXG_OK;
 }
 
@@ -398,15 +403,15 @@ int read_counters(bxg_map* m) {
   bxg_ctx* c = m->ctx;
   BXG_HIP(c, hipMemcpyAsync(m->h_ctr, m->ctr, sizeof(MapCounters), hipMemcpyDeviceToHost, c->stream));
   BXG_TRY(ctx_sync(c));
-  m->ctr_pending = false;
-  m->snap.reset();
-  take_counters(m);
+  take_landed(m);
   return BXG_OK;
 }
 
 // Mark the snapshots enqueued so far for maps[0..n) with one event on the
-// context stream (polled lazily by poll_counters).
-int snapshot_event(bxg_ctx* c, bxg_map* const* maps, size_t n) {
+// context stream (polled lazily by poll_counters); the work they follow
+// creates at most `leaves` leaves in each map.
+constexpr uint64_t kAnyLeaves = 1ull << 40;  // more than any pool
+int snapshot_event(bxg_ctx* c, bxg_map* const* maps, size_t n, uint64_t leaves = kAnyLeaves) {
   auto ev = std::make_shared<SnapEvent>();
   ev->pool = &c->snap_pool;
   if (!c->snap_pool.empty()) {
@@ -419,24 +424,21 @@ int snapshot_event(bxg_ctx* c, bxg_map* const* maps, size_t n) {
   for (size_t i = 0; i < n; ++i) {
     maps[i]->snap = ev;
     maps[i]->ctr_pending = true;
+    maps[i]->under_way += leaves;
   }
   return BXG_OK;
 }
 
 // enqueue a counter snapshot after a mutating call (polled lazily)
-int snapshot_counters(bxg_map* m) {
+int snapshot_counters(bxg_map* m, uint64_t leaves) {
   bxg_ctx* c = m->ctx;
   BXG_HIP(c, hipMemcpyAsync(m->h_ctr, m->ctr, sizeof(MapCounters), hipMemcpyDeviceToHost, c->stream));
-  return snapshot_event(c, &m, 1);
+  return snapshot_event(c, &m, 1, leaves);
 }
 
 // take a finished snapshot into account without blocking
 void poll_counters(bxg_map* m) {
-  if (m->ctr_pending && hipEventQuery(m->snap->e) == hipSuccess) {
-    m->ctr_pending = false;
-    m->snap.reset();
-    take_counters(m);
-  }
+  if (m->ctr_pending && hipEventQuery(m->snap->e) == hipSuccess) take_landed(m);
 }
 
 // have and want bits for a directory of cap roots, all zero, in h's arrays
@@ -970,8 +972,7 @@ int clear_status(bxg_map* m) {
   BXG_HIP(m->ctx, hipMemcpyAsync(&m->ctr->status, &z, 4, hipMemcpyHostToDevice, m->ctx->stream));
   BXG_TRY(ctx_sync(m->ctx));
   // any snapshot enqueued before has landed; the mirror follows the device
-  m->ctr_pending = false;
-  m->snap.reset();
+  take_landed(m);
   m->h_ctr->status = 0;
   return BXG_OK;
 }
@@ -1079,20 +1080,21 @@ int cell_op(bxg_map* m, const int32_t* coords, const void* vals, uint64_t n, uin
                          : os.tile == 2048 ? k_op_tiles<false, 2>
                                            : k_op_tiles<false, 1>);
   BXG_TRY(launch(c, "k_op_tiles", tiles, os.tiles, kOpTileThreads, md, coords, n, op, was_on, os));
-  // Calls within the leaves ensure_room has made room for create and apply in
-  // one kernel; in a larger one the pool can run out, and then no cell may be
-  // set, so its leaves are all created first.
+  // A call sets no cell when the pool runs out, so its leaves must all exist
+  // before the first cell is set.  Where the pool has room for a leaf an input
+  // the buckets create their leaves as they go.  The host knows of that room
+  // unless much is under way on the map (the leaf count it knows is that of the
+  // last call that has landed); else k_op_leaves goes first, which looks again
+  // on the device and only creates leaves where the room is short there too.
   const uint8_t* v = (const uint8_t*)vals;
-  bool fused = create;
-  if (create && n > (1u << 22)) {
+  if (create && m->known_leaves + m->under_way + n > m->leaf_cap)
     BXG_TRY(launch(c, "k_op_leaves", k_op_buckets<true, false, false, false>, os.nb, kOpThreads, md, v, n, op, was_on, os));
-    fused = false;
-  }
-  auto buckets = op != kOpSetValue ? (fused ? k_op_buckets<true, true, true, false> : k_op_buckets<false, true, true, false>)
-                 : was_on          ? (fused ? k_op_buckets<true, true, true, true> : k_op_buckets<false, true, true, true>)
-                          : (fused ? k_op_buckets<true, true, false, true> : k_op_buckets<false, true, false, true>);
+  auto buckets = !create              ? k_op_buckets<false, true, true, false>
+                 : op != kOpSetValue ? k_op_buckets<true, true, true, false>
+                 : was_on            ? k_op_buckets<true, true, true, true>
+                                     : k_op_buckets<true, true, false, true>;
   BXG_TRY(launch(c, "k_op_buckets", buckets, os.nb, kOpThreads, md, v, n, op, was_on, os));
-  return snapshot_counters(m);
+  return snapshot_counters(m, create ? n : 0);
 }
 
 int known_leaf_count(bxg_map* m, uint32_t* out) {
@@ -2025,7 +2027,7 @@ int bxg_write_leaves_host(bxg_map* m, const int32_t* origins, uint64_t n, const 
   }
   BXG_TRY(launch(c, "k_write_leaves", k_write_leaves, (uint32_t)n, kBlock, (const MapDev*)m->d,
                  (const int32_t*)dorig, (uint32_t)n, (const uint64_t*)dm, (const uint8_t*)dc));
-  BXG_TRY(snapshot_counters(m));
+  BXG_TRY(snapshot_counters(m, 0));
   return ctx_sync(c);
 }
 

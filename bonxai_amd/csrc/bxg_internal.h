@@ -76,8 +76,9 @@ struct alignas(128) MapCounters {
   uint32_t pad0[30];
   uint32_t status;
   int32_t cur;  // ProbabilisticMap update_count, 1..3
-  // leaf_count when the running scan or bulk call started: leaves at or
-  // above it were created by that call, and it initialises them
+  // leaf_count when the running scan or creating bulk call started (at most
+  // leaf_cap): leaves at or above it were created by that call, and it
+  // initialises them
   uint32_t leaf_base;
   uint32_t life;  // the map's life (clears, mod kLives): its touched marks (mark_miss)
   uint64_t scans_applied;

@@ -1785,8 +1785,9 @@ __device__ __forceinline__ uint32_t lds_claim(uint32_t* p, uint32_t key) {
 }
 
 // The inputs of a tile in the order of their leaves' buckets.  kCreate:
-// missing roots are created (setCellOff leaves out inputs without one).  The
-// tile's distinct roots are found in LDS and looked up once.
+// missing roots are created (setCellOff leaves out inputs without one), and the
+// map's leaf count before the call is kept (k_op_buckets).  The tile's distinct
+// roots are found in LDS and looked up once.
 template <bool kCreate, int kPer>
 __global__ void __launch_bounds__(kOpTileThreads) k_op_tiles(const MapDev* __restrict__ mp,
                                                              const int32_t* __restrict__ coords, uint64_t n,
@@ -1803,6 +1804,7 @@ __global__ void __launch_bounds__(kOpTileThreads) k_op_tiles(const MapDev* __res
   const MapView m = uniform_view(mp);
   const uint32_t t = threadIdx.x, lane = t & 63u, wid = t >> 6;
   const uint64_t base = (uint64_t)blockIdx.x * kTile;
+  if (kCreate && blockIdx.x == 0 && t == 0) m.ctr->leaf_base = min(m.ctr->leaf_count, m.leaf_cap);
   for (uint32_t p = t; p < kRoots; p += kOpTileThreads) rkeys[p] = kEmptyKey;
   for (uint32_t p = t; p < os.nb / 2; p += kOpTileThreads) hist[p] = 0;
   int32_t x[kPer], y[kPer], z[kPer];
@@ -1941,7 +1943,9 @@ __device__ __forceinline__ void set_cell(const MapView& m, uint64_t g, const uin
 }
 
 // A bucket of a bulk call.  kCreate: its missing leaves are created, all cells
-// off and zero (bonxai.hpp:51-58).  kApply: its cells are set.  kFirst: the
+// off and zero (bonxai.hpp:51-58).  kApply: its cells are set.  Without kApply
+// (the pass before, for calls that the pool may be too small for) nothing is
+// done where the pool has room for a leaf an input after all.  kFirst: the
 // call needs each cell's first input and prior mask bit (was_on is asked for,
 // or setCellOn / setCellOff); a setValue batch without was_on needs only the
 // last input of each cell.  was_on of an input is the prior bit for the first
@@ -1964,6 +1968,7 @@ __global__ void __launch_bounds__(kOpThreads) k_op_buckets(const MapDev* __restr
   __shared__ uint32_t over, nnew, nbase;
   const MapView m = uniform_view(mp);
   const uint32_t t = threadIdx.x, lane = t & 63u, wid = t >> 6;
+  if (kCreate && !kApply && (uint64_t)*gp(&m.ctr->leaf_base) + n <= m.leaf_cap) return;
   const bool failed = (map_status(m) & kFatal) != 0;  // such a call sets no cell
   if (kApply && failed && was_on)
     for (uint64_t i = (uint64_t)blockIdx.x * kOpThreads + t; i < n; i += (uint64_t)gridDim.x * kOpThreads)
