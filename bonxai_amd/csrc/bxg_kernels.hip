@@ -1965,11 +1965,15 @@ __global__ void __launch_bounds__(kOpThreads) k_op_buckets(const MapDev* __restr
   __shared__ uint32_t lidx[kOpLeaves];
   __shared__ uint32_t lnew[kOpLeaves];   // slots of the leaves to create
   __shared__ uint64_t bits[kOpWords];    // mask bits of the call's cells
-  __shared__ uint32_t over, nnew, nbase;
+  __shared__ uint32_t over, nnew, nbase, fatal;
   const MapView m = uniform_view(mp);
   const uint32_t t = threadIdx.x, lane = t & 63u, wid = t >> 6;
   if (kCreate && !kApply && (uint64_t)*gp(&m.ctr->leaf_base) + n <= m.leaf_cap) return;
-  const bool failed = (map_status(m) & kFatal) != 0;  // such a call sets no cell
+  // A failed call sets no cell.  The status is read once for the workgroup: its
+  // wavefronts go through the same barriers whatever other workgroups flag.
+  if (t == 0) fatal = map_status(m) & kFatal;
+  __syncthreads();
+  const bool failed = fatal != 0;
   if (kApply && failed && was_on)
     for (uint64_t i = (uint64_t)blockIdx.x * kOpThreads + t; i < n; i += (uint64_t)gridDim.x * kOpThreads)
       was_on[i] = 0;

@@ -88,3 +88,29 @@ def test_calls_enqueued_one_after_the_other(ctx, second):
     assert_same_cells(g.export(), og.export(), second)
     for m in (g, og, busy):
         m.close()
+
+
+@pytest.mark.parametrize("n", [1000, 300_000])
+def test_calls_on_a_map_with_an_error(ctx, n):
+    """Device calls enqueued behind one that failed (a coordinate out of range)
+    set no cell, and every prior state reads 0."""
+    import bonxai_amd as bx
+    L = bx.lib()
+    c = _apart(n, 3, 6)
+    v = np.arange(1, n + 1, dtype=np.float32)
+    g = bx.VoxelGrid(ctx, 0.1)
+    g.set_values(c[: n // 2], v[: n // 2])
+    before = g.digest()
+    bad = c.copy()
+    bad[n // 3] = 1 << 30
+    dc, dv, dbad = ctx.to_device(c), ctx.to_device(v), ctx.to_device(bad)
+    was = [ctx.to_device(np.ones(n, np.uint8)) for _ in range(4)]
+    rc = [L.bxg_set_values(g._h, dbad.ptr, dv.ptr, n, was[0].ptr), L.bxg_set_values(g._h, dc.ptr, dv.ptr, n, was[1].ptr),
+          L.bxg_set_cells_on(g._h, dc.ptr, dv.ptr, n, was[2].ptr), L.bxg_set_cells_off(g._h, dc.ptr, n, was[3].ptr)]
+    assert rc == [bx.OK] * 4
+    assert g.sync() == bx.ERR_COORD_RANGE
+    for w in was:
+        assert not w.numpy().any()
+    g.clear_error()
+    assert g.digest() == before
+    g.close()
