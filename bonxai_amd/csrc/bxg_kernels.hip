@@ -18,6 +18,7 @@
 // Pointers read out of a map header are cast to the global address space
 // (BXG_G) so loads compile to global_load rather than flat_load.
 #include "bxg_internal.h"
+#include "bxg_op_parts.h"
 #include "bxg_walk.h"
 
 #define BXG_G __attribute__((address_space(1)))
@@ -1734,13 +1735,13 @@ __global__ void k_na_recover(MapCounters* __restrict__ ctr, uint32_t leaf_cap) {
 // k_op_tiles orders each tile of inputs by the bucket (hash) of their leaf,
 // and k_op_buckets gives each bucket to one workgroup, which finds the first
 // and last input of every cell in LDS.  A leaf belongs to one workgroup, so
-// its cells, its mask words and its entry need no device atomics, and the
-// workgroup initialises the leaves it creates.
+// its cells, its entry and (of up to kOpGathered leaves a bucket) its mask words
+// need no device atomics, and the workgroup initialises the leaves it creates.
 //
 // A table of the cells in device memory (claim, last index, mask bits: two to
 // three device atomics an input, about 15 G/s in all) took 0.46 ms for 2M
 // inputs into a new grid, clear and leaf initialisation included, and five
-// launches; the two kernels take 0.030 + 0.059 ms (0.4 MB of bucket starts
+// launches; the two kernels take 0.030 + 0.058 ms (0.4 MB of bucket starts
 // aside, 64 bytes an input are moved: 1.4 TB/s).  What bounds them: the tiles'
 // claims of missing roots (12 us) and their passes through LDS; in the
 // buckets a chain of some ten dependent reads a workgroup with two or three
@@ -1751,14 +1752,13 @@ constexpr uint32_t kOpTileThreads = 1024;
 constexpr uint32_t kOpTileLog = 13;    // most inputs of a tile
 constexpr uint32_t kOpMaxBuckets = 4096;
 constexpr uint32_t kOpThreads = 512;   // of k_op_buckets (2M inputs: 256 threads 93 us, 512 66, 1024 102)
-// cell slots of a bucket's table: 2 to 3 workgroups a CU, and four times a
-// bucket's inputs on average (3072 slots, four workgroups a CU: 78 us for 66,
-// the fuller tables cost more than the wavefronts bring)
-constexpr uint32_t kOpCells = 4096;
-constexpr uint32_t kOpLeaves = 256;    // its leaf slots (at most)
-constexpr uint32_t kOpWords = 2048;    // its mask words
-constexpr uint64_t kCreated = kEmptyKey - 1;  // in place of a leaf's key, once created
-constexpr uint32_t kOpProbes = 32;     // slots looked at for a cell or leaf before the table counts as full
+// Most leaves of a bucket whose mask bits are gathered in LDS (fewer where a
+// leaf has more than 8 mask words): clusters of cells have some 54 a bucket.
+// With more, few cells share a word: 1M inputs, each in a leaf of its own, 977 a
+// bucket, are set in 122 us, call and wait included, with an atomic a cell, and
+// in 448 when buckets were done in parts of at most 256 leaves (200k inputs in
+// leaves of 16^3 cells, parts of 32: 368 -> 42).
+constexpr uint32_t kOpGathered = 256;
 
 enum : uint32_t { kOpSetValue = 0, kOpSetOn = 1, kOpSetOff = 2 };
 
@@ -1804,7 +1804,8 @@ __global__ void __launch_bounds__(kOpTileThreads) k_op_tiles(const MapDev* __res
   const MapView m = uniform_view(mp);
   const uint32_t t = threadIdx.x, lane = t & 63u, wid = t >> 6;
   const uint64_t base = (uint64_t)blockIdx.x * kTile;
-  if (kCreate && blockIdx.x == 0 && t == 0) m.ctr->leaf_base = min(m.ctr->leaf_count, m.leaf_cap);
+  const bool count = kCreate && blockIdx.x == 0 && t == 0;
+  const uint32_t leaves = count ? min(*gp(&m.ctr->leaf_count), m.leaf_cap) : 0u;
   for (uint32_t p = t; p < kRoots; p += kOpTileThreads) rkeys[p] = kEmptyKey;
   for (uint32_t p = t; p < os.nb / 2; p += kOpTileThreads) hist[p] = 0;
   int32_t x[kPer], y[kPer], z[kPer];
@@ -1821,6 +1822,7 @@ __global__ void __launch_bounds__(kOpTileThreads) k_op_tiles(const MapDev* __res
     }
   }
   __syncthreads();
+  if (count) m.ctr->leaf_base = leaves;
   constexpr uint32_t kOut = 0xFFFFFFFFu, kDirect = 0xFFFFFFFEu;
   uint32_t rp[kPer];
 #pragma unroll
@@ -1951,53 +1953,66 @@ __device__ __forceinline__ void set_cell(const MapView& m, uint64_t g, const uin
 // last input of each cell.  was_on of an input is the prior bit for the first
 // of its cell and "on" (off for setCellOff) for later ones, which k_op_tiles
 // has written; setValue keeps the last input's value, setCellOn the first
-// one's, if the cell was off.  A bucket with more cells or leaves than the
-// tables hold is done in halves by the bits of its cells' hashes.
+// one's, if the cell was off.
+//
+// A bucket with more cells or leaves than the tables hold is done in parts
+// (OpPart).  The table of the leaves has room for the inputs of a bucket that
+// lie each in a leaf of its own.  Up to kOpGathered leaves are numbered, have a
+// thread each, and their cells' mask bits are gathered in LDS and written by
+// one thread a word; the bits of more leaves by an atomic a cell (they share
+// few words then).
 template <bool kCreate, bool kApply, bool kFirst, bool kLast>
-__global__ void __launch_bounds__(kOpThreads) k_op_buckets(const MapDev* __restrict__ mp,
+__global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buckets(const MapDev* __restrict__ mp,
                                                            const uint8_t* __restrict__ vals, uint64_t n,
                                                            uint32_t op, uint8_t* __restrict__ was_on,
                                                            OpScratch os) {
-  __shared__ uint32_t ckey[kOpCells];    // leaf slot << 12 | cell in the leaf
-  __shared__ uint32_t clast[kLast ? kOpCells : 1];
-  __shared__ uint32_t cfirst[kFirst ? kOpCells : 1];
-  __shared__ uint64_t lkey[kOpLeaves];   // the leaf's entry among the children
-  __shared__ uint32_t lidx[kOpLeaves];
-  __shared__ uint32_t lnew[kOpLeaves];   // slots of the leaves to create
-  __shared__ uint64_t bits[kOpWords];    // mask bits of the call's cells
-  __shared__ uint32_t over, nnew, nbase, fatal;
+  constexpr uint32_t kCells = kApply ? kOpCells : 4;
+  // cells: leaf slot << 12 | cell in the leaf
+  __shared__ __attribute__((aligned(16))) uint32_t ckey[kCells];
+  __shared__ __attribute__((aligned(16))) uint32_t clast[kLast ? kOpCells : 4];
+  __shared__ __attribute__((aligned(16))) uint32_t cfirst[kFirst ? kOpCells : 4];
+  // the leaves' entries among the children, then what became of them (below)
+  __shared__ __attribute__((aligned(16))) uint64_t leaf[kOpLeaves];
+  // of the numbered leaves: entry and slot, then what became of them
+  __shared__ uint64_t gathered[kApply ? kOpGathered : 1];
+  // the mask words of the numbered leaves, in place of inputs that are read by then
+  uint64_t* bits = (uint64_t*)(kLast ? clast : cfirst);
+  static_assert(kOpCells * 4 == kOpLeaves * 8, "a mask word a slot of the leaves' table");
+  __shared__ uint32_t leaves_full, cells_full, nleaf, nnew, nbase, fatal;
   const MapView m = uniform_view(mp);
   const uint32_t t = threadIdx.x, lane = t & 63u, wid = t >> 6;
   if (kCreate && !kApply && (uint64_t)*gp(&m.ctr->leaf_base) + n <= m.leaf_cap) return;
-  // A failed call sets no cell.  The status is read once for the workgroup: its
-  // wavefronts go through the same barriers whatever other workgroups flag.
+  // A failed call sets no cell.  The status is read once for the workgroup (and
+  // looked at behind the first barriers): its wavefronts go through the same
+  // ones whatever other workgroups flag.
   if (t == 0) fatal = map_status(m) & kFatal;
-  __syncthreads();
-  const bool failed = fatal != 0;
-  if (kApply && failed && was_on)
-    for (uint64_t i = (uint64_t)blockIdx.x * kOpThreads + t; i < n; i += (uint64_t)gridDim.x * kOpThreads)
-      was_on[i] = 0;
-  if (!kCreate && failed) return;
   // buckets that follow each other (their entries share lines) on one XCD
   const uint32_t bk = (blockIdx.x % kXcds) * (os.nb / kXcds) + blockIdx.x / kXcds;
   const uint32_t cl = 3 * m.lb, il = 3 * m.ib;
   const uint32_t lwl = 31u - (uint32_t)__clz((int)m.lw);  // lw is a power of two
-  const uint32_t nslots = min(kOpLeaves, kOpWords >> lwl);
+  const uint32_t most_gathered = min(kOpGathered, kOpLeaves >> lwl);
   // lanes a tile, so that the workgroup reads all tiles' entries at once
   uint32_t gl = 0;
   while (gl < 6 && (os.tiles << gl) < kOpThreads) ++gl;
-  uint32_t depth = 0, path = 0;
+  constexpr uint32_t kMine = kOpCells / kOpThreads, kMyLeaves = kOpLeaves / kOpThreads;
+  // what became of a leaf: its index (kNone: there is none), its number << 32,
+  // kMade if the call has created it
+  constexpr uint64_t kMade = 1ull << 63;
+  constexpr uint32_t kSlotBit = 48;  // an entry is below 2^36
+  OpPart part;
   for (;;) {
-    for (uint32_t p = t; p < kOpCells; p += kOpThreads) {
-      ckey[p] = kNone;
-      if (kLast) clast[p] = 0;
-      if (kFirst) cfirst[p] = kNone;
+    const uint4 ones = make_uint4(~0u, ~0u, ~0u, ~0u);
+    if (kApply) {
+      for (uint32_t p = t; p < kOpCells / 4; p += kOpThreads) {
+        reinterpret_cast<uint4*>(ckey)[p] = ones;  // kNone
+        if (kLast) reinterpret_cast<uint4*>(clast)[p] = make_uint4(0u, 0u, 0u, 0u);
+        if (kFirst) reinterpret_cast<uint4*>(cfirst)[p] = ones;
+      }
     }
-    for (uint32_t p = t; p < kOpLeaves; p += kOpThreads) lkey[p] = kEmptyKey;
-    for (uint32_t p = t; p < kOpWords; p += kOpThreads) bits[p] = 0;
-    if (t == 0) over = nnew = 0;
+    for (uint32_t p = t; p < kOpLeaves / 2; p += kOpThreads) reinterpret_cast<uint4*>(leaf)[p] = ones;  // kEmptyKey
+    if (t == 0) leaves_full = cells_full = nleaf = nnew = 0;
     __syncthreads();
-    const uint32_t part = (uint32_t)((1ull << depth) - 1ull);
+    const bool whole = part.whole();
     for (uint32_t tile = t >> gl; tile < os.tiles; tile += kOpThreads >> gl) {
       const uint16_t BXG_G* st = gp((const uint16_t*)os.start) + (uint64_t)tile * (os.nb + 2) + bk;
       const uint32_t hi = st[1];
@@ -2006,22 +2021,30 @@ __global__ void __launch_bounds__(kOpThreads) k_op_buckets(const MapDev* __restr
         const uint64_t e = gp((const uint64_t*)os.entry)[tb + k];
         const uint64_t cell = e >> kOpTileLog;
         const uint32_t i = (uint32_t)tb + ((uint32_t)e & ((1u << kOpTileLog) - 1u));
-        const uint64_t hash = mix64(cell);
-        if (((uint32_t)(hash >> 32) & part) != path) continue;
-        const uint64_t child = cell >> cl;
-        uint32_t ls = ((uint32_t)child * 0x9E3779B1u >> 20) & (nslots - 1u);
+        const uint64_t hash = mix64(cell), child = cell >> cl;
+        if (!whole && !part.holds(mix64(child), hash)) continue;
+        uint32_t ls = op_leaf_slot(child);
         uint32_t p = 0;
         for (; p < kOpProbes; ++p) {
-          if (lds_claim(&lkey[ls], child) == child) break;
-          ls = (ls + 1u) & (nslots - 1u);
+          uint64_t k = __hip_atomic_load(&leaf[ls], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          if (k == kEmptyKey) {
+            k = atomicCAS((unsigned long long*)&leaf[ls], kEmptyKey, child);
+            if (k == kEmptyKey) {
+              k = child;
+              const uint32_t number = atomicAdd(&nleaf, 1u);
+              if (kApply && number < kOpGathered) gathered[number] = child | ((uint64_t)ls << kSlotBit);
+            }
+          }
+          if (k == child) break;
+          ls = (ls + 1u) & (kOpLeaves - 1u);
         }
         if (p == kOpProbes) {
-          over = 1;
+          leaves_full = 1;
           continue;
         }
         if (!kApply) continue;
         const uint32_t key = (ls << 12) | ((uint32_t)cell & ((1u << cl) - 1u));
-        uint32_t h = (uint32_t)hash & (kOpCells - 1u);
+        uint32_t h = op_cell_slot(hash);
         for (p = 0; p < kOpProbes; ++p) {
           if (lds_claim(&ckey[h], key) == key) {
             if (kLast) atomicMax(&clast[h], i);
@@ -2030,87 +2053,125 @@ __global__ void __launch_bounds__(kOpThreads) k_op_buckets(const MapDev* __restr
           }
           h = (h + 1u) & (kOpCells - 1u);
         }
-        if (p == kOpProbes) over = 1;
+        if (p == kOpProbes) cells_full = 1;
       }
     }
     __syncthreads();
-    if (over) {
-      if (depth < 32) {
-        ++depth;
-        __syncthreads();
-        continue;
-      }
+    if (leaves_full | cells_full) {
+      const bool more = part.halve(leaves_full != 0);
+      __syncthreads();
+      if (more) continue;
       if (t == 0) or32(&m.ctr->status, kStScratchFull);  // cells of one hash: not met
       return;
     }
-    // the values of the cells, in flight while the leaves are looked up
-    constexpr uint32_t kMine = kOpCells / kOpThreads;
+    const bool failed = fatal != 0;
+    if (kApply && failed && was_on)
+      for (uint64_t i = (uint64_t)blockIdx.x * kOpThreads + t; i < n; i += (uint64_t)gridDim.x * kOpThreads)
+        was_on[i] = 0;
+    if (!kCreate && failed) return;
+    // the values of the cells, in flight while the leaves are looked up (or the
+    // inputs that hold them), and the words of `bits` cleared
     const bool word = kLast && (m.vb == 4 || (m.vb == 8 && ((uintptr_t)vals & 7u) == 0));
     uint64_t val[kMine] = {};
-    if (kApply && !failed && word) {
+    if (kApply && !failed) {
+      uint32_t src[kMine];  // (empty slots: input 0)
 #pragma unroll
-      for (uint32_t j = 0; j < kMine; ++j) {
-        const uint32_t p = j * kOpThreads + t;
-        if (ckey[p] == kNone) continue;
-        if (m.vb == 4)
-          val[j] = gp((const uint32_t*)vals)[clast[p]];
-        else
-          val[j] = gp((const uint64_t*)vals)[clast[p]];
+      for (uint32_t j = 0; j < kMine; ++j) src[j] = (kLast ? clast : cfirst)[j * kOpThreads + t];
+#pragma unroll
+      for (uint32_t j = 0; j < kMine; ++j) (kLast ? clast : cfirst)[j * kOpThreads + t] = 0;
+      if (word && m.vb == 4) {
+#pragma unroll
+        for (uint32_t j = 0; j < kMine; ++j) val[j] = gp((const uint32_t*)vals)[src[j]];
+      } else if (word) {
+#pragma unroll
+        for (uint32_t j = 0; j < kMine; ++j) val[j] = gp((const uint64_t*)vals)[src[j]];
+      } else {
+#pragma unroll
+        for (uint32_t j = 0; j < kMine; ++j) val[j] = src[j];
       }
     }
     // the leaves: looked up, and created where missing
-    if (t < nslots && lkey[t] != kEmptyKey) {
-      const uint32_t c = m.children[lkey[t]];
-      lidx[t] = c < kPendingChild ? c : kNone;
-      if (kCreate && c >= kPendingChild) lnew[atomicAdd(&nnew, 1u)] = t;
+    const uint32_t nl = nleaf;
+    const bool gather = kApply && nl <= most_gathered;
+    // entry of the thread's j-th leaf
+    const auto entry = [&](uint32_t j) -> uint64_t {
+      if (!gather) return leaf[j * kOpThreads + t];
+      return j == 0 && t < nl ? gathered[t] & ((1ull << kSlotBit) - 1ull) : kEmptyKey;
+    };
+    uint32_t idx[kMyLeaves];
+    uint32_t have = 0, make = 0, at = 0;  // its leaves and those missing (bits), the first new one's place
+#pragma unroll
+    for (uint32_t j = 0; j < kMyLeaves; ++j) {
+      const uint64_t child = entry(j);
+      have |= child != kEmptyKey ? 1u << j : 0u;
+      idx[j] = child != kEmptyKey ? m.children[child] : 0u;
     }
+#pragma unroll
+    for (uint32_t j = 0; j < kMyLeaves; ++j) make |= idx[j] >= kPendingChild ? 1u << j : 0u;
     if (kCreate) {
+      if (make) at = atomicAdd(&nnew, (uint32_t)__popc(make));
       __syncthreads();
       const uint32_t k = nnew;
       if (k) {
         if (t == 0) nbase = add32(&m.ctr->leaf_count, k);
         __syncthreads();
-        if (t < k) {
-          const uint32_t s = lnew[t], idx = nbase + t;
-          if (idx >= m.leaf_cap) {
+        const uint32_t first = nbase;
+        uint32_t next = first + at;
+#pragma unroll
+        for (uint32_t j = 0; j < kMyLeaves; ++j) {
+          if (!((make >> j) & 1u)) continue;
+          idx[j] = next++;
+          if (idx[j] >= m.leaf_cap) {
             or32(&m.ctr->status, kStOutOfPool);
-          } else {
-            const uint64_t child = lkey[s];
-            const uint32_t ci = (uint32_t)child & (m.isz - 1u), im = (1u << m.ib) - 1u;
-            int32_t ox, oy, oz;
-            unpack_root(m.root_keys[child >> il], m.log2n, &ox, &oy, &oz);
-            m.origin[idx] = make_int4(ox + (int32_t)((ci & im) << m.lb), oy + (int32_t)(((ci >> m.ib) & im) << m.lb),
-                                      oz + (int32_t)((ci >> (2 * m.ib)) << m.lb), (int32_t)(child >> il));
-            m.children[child] = idx;
-            lidx[s] = idx;
-            lkey[s] = kCreated;
+            idx[j] = kNone;
+            continue;
           }
+          const uint64_t child = entry(j);
+          const uint32_t ci = (uint32_t)child & (m.isz - 1u), im = (1u << m.ib) - 1u;
+          int32_t ox, oy, oz;
+          unpack_root(m.root_keys[child >> il], m.log2n, &ox, &oy, &oz);
+          m.origin[idx[j]] =
+              make_int4(ox + (int32_t)((ci & im) << m.lb), oy + (int32_t)(((ci >> m.ib) & im) << m.lb),
+                        oz + (int32_t)((ci >> (2 * m.ib)) << m.lb), (int32_t)(child >> il));
+          m.children[child] = idx[j];
         }
-        __syncthreads();
+        const bool masks = !gather || failed;  // else written below
         const uint32_t cw = (uint32_t)((uint64_t)m.lsz * m.vb / 8);  // 8-byte words a leaf
-        for (uint32_t r = wid; r < k; r += kOpThreads / 64) {
-          const uint32_t leaf = lidx[lnew[r]];
-          if (leaf == kNone) continue;
-          if (!kApply || failed)
-            for (uint32_t w = lane; w < m.lw; w += 64) m.masks[(uint64_t)leaf * m.lw + w] = 0;
-          for (uint32_t w = lane; w < cw; w += 64) ((uint64_t BXG_G*)m.cells)[(uint64_t)leaf * cw + w] = 0;
+        for (uint32_t r = first + wid; r < first + k && r < m.leaf_cap; r += kOpThreads / 64) {
+          if (masks)
+            for (uint32_t w = lane; w < m.lw; w += 64) m.masks[(uint64_t)r * m.lw + w] = 0;
+          for (uint32_t w = lane; w < cw; w += 64) ((uint64_t BXG_G*)m.cells)[(uint64_t)r * cw + w] = 0;
         }
       }
     }
-    __syncthreads();
     if (kApply && !failed) {
 #pragma unroll
+      for (uint32_t j = 0; j < kMyLeaves; ++j) {
+        if (!((have >> j) & 1u)) continue;
+        uint64_t w = idx[j] < kPendingChild ? idx[j] : kNone;
+        if (kCreate && ((make >> j) & 1u)) w |= kMade;
+        if (gather) {
+          leaf[gathered[t] >> kSlotBit] = w | ((uint64_t)t << 32);
+          gathered[t] = w;
+        } else {
+          leaf[j * kOpThreads + t] = w;
+        }
+      }
+      __syncthreads();
+#pragma unroll
       for (uint32_t j = 0; j < kMine; ++j) {
-        const uint32_t p = j * kOpThreads + t, key = ckey[p];
+        const uint32_t p = j * kOpThreads + t, key = ckey[p], li = key & 4095u;
         if (key == kNone) continue;
-        const uint32_t ls = key >> 12, li = key & 4095u, leaf = lidx[ls];
-        if (leaf == kNone) continue;
-        const uint64_t g = (uint64_t)leaf * m.lsz + li;
+        const uint64_t l = leaf[key >> 12];
+        const uint32_t at_leaf = (uint32_t)l;
+        if (at_leaf == kNone) continue;
+        const uint64_t g = (uint64_t)at_leaf * m.lsz + li;
         const uint64_t bit = 1ull << (li & 63u);
+        uint64_t* mw = (uint64_t*)&m.masks[(uint64_t)at_leaf * m.lw + (li >> 6)];
         bool pre = false;
         if (kFirst) {
-          pre = lkey[ls] != kCreated && (m.masks[(uint64_t)leaf * m.lw + (li >> 6)] & bit) != 0;
-          if (was_on) was_on[cfirst[p]] = pre;
+          pre = !(l & kMade) && (*gp(mw) & bit) != 0;
+          if (was_on) was_on[kLast ? cfirst[p] : (uint32_t)val[j]] = pre;
         }
         if (word) {
           if (m.vb == 4)
@@ -2118,30 +2179,35 @@ __global__ void __launch_bounds__(kOpThreads) k_op_buckets(const MapDev* __restr
           else
             ((uint64_t BXG_G*)m.cells)[g] = val[j];
         } else if (kLast) {
-          if (m.vb) set_cell(m, g, vals, clast[p]);
+          if (m.vb) set_cell(m, g, vals, val[j]);
         } else if (op == kOpSetOn) {
-          if (!pre && m.vb && vals) set_cell(m, g, vals, cfirst[p]);
+          if (!pre && m.vb && vals) set_cell(m, g, vals, val[j]);
         } else {
           set_cell(m, g, nullptr, 0);
         }
-        atomicOr((unsigned long long*)&bits[(ls << lwl) + (li >> 6)], bit);
-      }
-      __syncthreads();
-      for (uint32_t w = t; w < nslots * m.lw; w += kOpThreads) {
-        const uint64_t v = bits[w];
-        const uint32_t ls = w >> lwl;
-        if (kCreate && lkey[ls] == kCreated) {  // every word of a new leaf
-          m.masks[(uint64_t)lidx[ls] * m.lw + (w & (m.lw - 1u))] = v;
-        } else if (v) {
-          uint64_t BXG_G* mw = m.masks + (uint64_t)lidx[ls] * m.lw + (w & (m.lw - 1u));
-          *mw = op == kOpSetOff ? *mw & ~v : *mw | v;
+        if (gather) {
+          atomicOr((unsigned long long*)&bits[((uint32_t)(l >> 32 & 0xFFFFu) << lwl) + (li >> 6)], bit);
+        } else if (op == kOpSetOff) {
+          if (pre) and64(mw, ~bit);
+        } else if (!pre) {
+          or64(mw, bit);
         }
       }
       __syncthreads();
+      if (gather) {
+        for (uint32_t w = t; w < (nl << lwl); w += kOpThreads) {
+          const uint64_t v = bits[w], l = gathered[w >> lwl];
+          if ((uint32_t)l == kNone) continue;
+          uint64_t BXG_G* mw = m.masks + (uint64_t)(uint32_t)l * m.lw + (w & (m.lw - 1u));
+          if (kCreate && (l & kMade))
+            *mw = v;  // every word of a new leaf
+          else if (v)
+            *mw = op == kOpSetOff ? *mw & ~v : *mw | v;
+        }
+      }
     }
-    while (depth && ((path >> (depth - 1u)) & 1u)) path &= ~(1u << --depth);
-    if (!depth) return;
-    path |= 1u << (depth - 1u);
+    if (!part.next()) return;
+    __syncthreads();
   }
 }
 

@@ -1,0 +1,73 @@
+"""GPU parity of the bulk cell calls where the leaves of a bucket are more than
+those whose mask bits are gathered in LDS (256; 32 of 16^3 cells), and more than
+its table holds (2048).  Cells, values and prior states are compared bit for bit."""
+import numpy as np
+import pytest
+
+from conftest import assert_same_cells, sorted_cells
+
+pytestmark = pytest.mark.gpu
+
+
+def _scattered(n, leaves, lb, seed):
+    """n cells (some of them twice) in that many leaves, every fourth one of a cube."""
+    rng = np.random.default_rng(seed)
+    side = int(np.ceil((4 * leaves) ** (1 / 3)))
+    at = np.stack(np.unravel_index(rng.permutation(side ** 3)[:leaves], (side,) * 3), 1) - side // 2
+    which = np.concatenate([np.arange(leaves), rng.integers(0, leaves, n - leaves)])[rng.permutation(n)]
+    return ((at[which] << lb) + rng.integers(0, 1 << lb, (n, 3))).astype(np.int32)
+
+
+@pytest.mark.parametrize("n,leaves,bits,dtype", [
+    (16_000, 16_000, (2, 3), np.float32),   # about 64 leaves a bucket
+    (260_000, 65_000, (2, 3), np.float32),  # 127
+    (260_000, 131_000, (2, 3), np.int64),   # 256, some buckets more
+    (520_000, 300_000, (2, 2), np.float32),  # 586
+    (60_000, 16_000, (2, 4), np.float32),   # 31, some more
+    (60_000, 30_000, (2, 4), np.int32),     # 59
+    (130_000, 100_000, (3, 3), None),
+    (130_000, 100_000, (2, 3), np.uint8),
+])
+def test_scattered_calls(ctx, n, leaves, bits, dtype):
+    import bonxai_amd as bx
+    import oracle
+    rng = np.random.default_rng(n)
+    c = _scattered(n, leaves, bits[1], leaves)
+    v = None if dtype is None else rng.integers(1, 200, n).astype(dtype)
+    g, og = bx.VoxelGrid(ctx, 0.1, *bits, dtype=dtype), oracle.Grid(0.1, *bits, dtype=dtype)
+    some = c[rng.permutation(n)[: n // 2]]
+    w = None if v is None else v[::-1][: n // 2]
+    g.set_values(c[: n // 3], None if v is None else v[: n // 3])
+    og.set_values(c[: n // 3], None if v is None else v[: n // 3])
+    for what, got, want in (
+            ("set", g.set_values(c, v, True), og.set_values(c, v)),
+            ("off", g.set_cells_off(some, True), og.set_cells_off(some)),
+            ("on", g.set_cells_on(c, v, True), og.set_cells_on(c, v)),
+            ("off again", g.set_cells_off(c[: n // 4], True), og.set_cells_off(c[: n // 4]))):
+        assert np.array_equal(got, want), what
+    g.set_values(some, w)
+    og.set_values(some, w)
+    if dtype is None:
+        assert np.array_equal(sorted_cells(g.export()[0])[0], og.export()[0])
+    else:
+        assert_same_cells(g.export(), og.export(), f"{n} {leaves}")
+    assert g.active_cells_count() == og.active_cells_count()
+    g.close()
+    og.close()
+
+
+def test_more_leaves_a_bucket_than_its_table(ctx):
+    """9M cells, each in a leaf of its own: 2,200 leaves a bucket."""
+    import bonxai_amd as bx
+    n, half = 9_000_000, 4_500_000
+    side = 209
+    at = np.random.default_rng(9).permutation(side ** 3)[:n]
+    c = (2 * np.stack(np.unravel_index(at, (side,) * 3), 1)).astype(np.int32)
+    g = bx.VoxelGrid(ctx, 0.1, 4, 1, dtype=None)
+    assert not g.set_cells_on(c[:half], None, True).any()
+    assert np.array_equal(g.set_values(c, None, True), np.arange(n) < half)
+    assert g.active_cells_count() == n
+    assert g.set_cells_off(c[half // 2:], True).all()
+    assert g.active_cells_count() == half // 2
+    assert np.array_equal(g.lookup(c)[1], np.arange(n) < half // 2)
+    g.close()
