@@ -1930,12 +1930,19 @@ __device__ __forceinline__ void copy_bytes(uint8_t BXG_G* dst, const uint8_t BXG
   for (uint32_t b = 0; b < vb; ++b) dst[b] = src[b];
 }
 
-// cell g of the map becomes value i of vals (null: zero bytes)
+// whether values of vb bytes at vals can be read as words
+__device__ __forceinline__ bool whole_words(const uint8_t* vals, uint32_t vb) {
+  return (vb == 4 || vb == 8) && ((uintptr_t)vals & (vb - 1u)) == 0;
+}
+
+// cell g of the map becomes value i of vals (null: zero bytes; else at any
+// address)
 __device__ __forceinline__ void set_cell(const MapView& m, uint64_t g, const uint8_t* vals, uint64_t i) {
   const uint32_t vb = m.vb;
-  if (vb == 4) {
+  const bool words = whole_words(vals, vb);
+  if (words && vb == 4) {
     ((uint32_t BXG_G*)m.cells)[g] = vals ? gp((const uint32_t*)vals)[i] : 0u;
-  } else if (vb == 8 && ((uintptr_t)vals & 7u) == 0) {
+  } else if (words) {
     ((uint64_t BXG_G*)m.cells)[g] = vals ? gp((const uint64_t*)vals)[i] : 0ull;
   } else if (vals) {
     copy_bytes(m.cells + g * vb, gp(vals) + i * vb, vb);
@@ -2071,7 +2078,7 @@ __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buck
     if (!kCreate && failed) return;
     // the values of the cells, in flight while the leaves are looked up (or the
     // inputs that hold them), and the words of `bits` cleared
-    const bool word = kLast && (m.vb == 4 || (m.vb == 8 && ((uintptr_t)vals & 7u) == 0));
+    const bool word = kLast && whole_words(vals, m.vb);
     uint64_t val[kMine] = {};
     if (kApply && !failed) {
       uint32_t src[kMine];  // (empty slots: input 0)

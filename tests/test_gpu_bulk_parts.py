@@ -71,3 +71,23 @@ def test_more_leaves_a_bucket_than_its_table(ctx):
     assert g.active_cells_count() == half // 2
     assert np.array_equal(g.lookup(c)[1], np.arange(n) < half // 2)
     g.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.int64])
+@pytest.mark.parametrize("shift", [1, 2])
+def test_values_at_odd_addresses(ctx, dtype, shift):
+    """Values in a device buffer that no word of theirs is aligned in."""
+    import bonxai_amd as bx
+    L = bx.lib()
+    n = 5000
+    c = _scattered(n, 800, 3, 8)
+    v = (np.arange(1, n + 1) * 3).astype(dtype)
+    raw = ctx.to_device(np.concatenate([np.zeros(shift, np.uint8), v.view(np.uint8)]))
+    d = ctx.to_device(c)
+    for call, host in ((L.bxg_set_values, "set_values"), (L.bxg_set_cells_on, "set_cells_on")):
+        g, h = bx.VoxelGrid(ctx, 0.1, dtype=dtype), bx.VoxelGrid(ctx, 0.1, dtype=dtype)
+        assert call(g._h, d.ptr, raw.ptr + shift, n, None) == bx.OK
+        getattr(h, host)(c, v)
+        assert_same_cells(g.export(), sorted_cells(*h.export()), host)
+        g.close()
+        h.close()
