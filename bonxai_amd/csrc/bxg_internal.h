@@ -170,7 +170,6 @@ struct alignas(16) BatchHdr {
 constexpr uint32_t kDirBits = 12;  // direction and length-class bits of a bucket
 constexpr uint32_t kMaxTagBits = 6;
 constexpr uint32_t kMaxBuckets = 1u << (kDirBits + kMaxTagBits);
-constexpr uint32_t kXcds = 8;      // workgroups are dispatched round the XCDs
 constexpr uint32_t kScanTile = 4096;  // buckets one block of the bucket scan covers
 constexpr uint32_t kTiles = kMaxBuckets / kScanTile;
 static_assert((1u << kDirBits) % kScanTile == 0 && kTiles <= 64, "bucket scan tiles");

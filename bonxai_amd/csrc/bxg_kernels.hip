@@ -1142,8 +1142,6 @@ __global__ void __launch_bounds__(256) k_scan_scatter(const BatchHdr* __restrict
 constexpr int32_t kFreshWindow = 16;
 constexpr int32_t kUpdateWindow = 8;
 constexpr int32_t kLeafWindow = 64;
-constexpr uint32_t kMaxSegLog = 5;  // at most 32 segments a ray
-constexpr uint32_t kGroupLog = 3;   // batches side by side on one XCD in a short list
 
 // The walk over the winner list.  A batch is 64 consecutive winners, rays of
 // one map in neighbouring directions and (with the ray order of
@@ -1154,14 +1152,10 @@ constexpr uint32_t kGroupLog = 3;   // batches side by side on one XCD in a shor
 // batch, and the workgroups waiting for a free slot balance the load).
 //
 // A short list (one scan a call) has fewer batches than the GPU has wavefront
-// slots, and a walk is a chain of dependent loads about 1.5 us a step: there
-// each ray is cut into up to 32 segments (2,001 points: update pass 25 us with
-// 8, 20 with 16, 16 with 32), and a wavefront walks one segment of a batch.  The tasks of a group of up to 8 batches follow each other on one
-// XCD (workgroups go round the XCDs), segment by segment, so that its L2
-// sees neighbours at one distance from the sensor.  A long list is cut into
-// one contiguous part an XCD (a map's rays stay on one XCD or two); there the
-// rays are walked whole, in lockstep: a lane more than the window's cells
-// ahead of the wavefront's slowest ray waits a step.
+// slots, and a walk is a chain of dependent loads about 1.5 us a step: there a
+// wavefront walks one segment of a batch (WalkPlan).  In a long list the rays
+// are walked whole, in lockstep: a lane more than the window's cells ahead of
+// the wavefront's slowest ray waits a step.
 //
 // Measured against persistent wavefronts that took rays from 8 cursors and
 // refilled their lanes one by one in short lists (us a call; leaf pass /
@@ -1211,23 +1205,11 @@ __device__ void walk_winners(const ScanDesc* __restrict__ sd, const ScanScratch&
                         (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t waves = (gridDim.x / kXcds) * wpb;
   const uint32_t lane = lane_id();
-  uint32_t lg = 0;
-  while (lg < kMaxSegLog && ((uint64_t)nb << (lg + 1)) <= (uint64_t)waves * kXcds) ++lg;
-  const bool lockstep = lg == 0;
-  uint32_t gl = kGroupLog;  // fewer batches a group where that would leave XCDs idle
-  while (gl > 0 && (nb >> gl) < 8u * kXcds) --gl;
-  const uint32_t per_xcd = (nb + kXcds - 1) / kXcds;
-  for (uint32_t j = wave;; j += waves) {
-    uint32_t batch, seg = 0;
-    if (lockstep) {
-      if (j >= per_xcd) break;
-      batch = xcd * per_xcd + j;
-    } else {
-      const uint32_t group = (j >> (gl + lg)) * kXcds + xcd;
-      if ((group << gl) >= nb) break;
-      batch = (group << gl) + (j & ((1u << gl) - 1u));
-      seg = (j >> gl) & ((1u << lg) - 1u);
-    }
+  const WalkPlan plan(nb, waves * kXcds);
+  const uint32_t lg = plan.lg;
+  const bool lockstep = plan.whole();
+  uint32_t batch, seg;
+  for (uint32_t j = wave; plan.task(j, xcd, batch, seg); j += waves) {
     if (batch >= nb) continue;
     const uint32_t idx = batch * 64u + lane;
     const bool valid = idx < nwin;

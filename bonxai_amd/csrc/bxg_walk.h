@@ -388,4 +388,51 @@ struct LeafWalk {
   }
 };
 
+// The tasks of a walk over a list of nb batches of 64 rays by a number of
+// wavefronts spread over the XCDs (workgroups go round them): the wave-th
+// wavefront of an XCD takes the tasks j = wave, wave + (the XCD's wavefronts), ...
+// while task() gives one.
+//
+// A short list, with more wavefronts than batches: each ray is cut into up to
+// 32 segments (2,001 points: update pass 25 us with 8, 20 with 16, 16 with 32),
+// and a task is one segment of a batch.  With batches enough for 8 groups an XCD
+// or more, the tasks of a group of up to 8 batches follow each other on one XCD,
+// segment by segment, so that its L2 sees neighbours at one distance from the
+// sensor.  With fewer, the segments of each batch go round the XCDs: kept on one
+// each, those of one batch, a scan of up to 64 points, had an eighth of the
+// wavefronts to themselves while the others had none (10 points, 50 m: 129 us a
+// call, 60 so; 100: 103, 61; 1,000 to 8,000 points the same).  A long list: one
+// contiguous part of it an XCD (a map's rays stay on one XCD or two), the rays
+// walked whole.
+constexpr uint32_t kXcds = 8;
+constexpr uint32_t kMaxSegLog = 5;  // at most 32 segments a ray
+constexpr uint32_t kGroupLog = 3;   // batches side by side on one XCD in a short list
+struct WalkPlan {
+  uint32_t nb, lg, gl, per_xcd;
+  BXG_HD WalkPlan(uint32_t batches, uint32_t wavefronts) : nb(batches), lg(0), gl(kGroupLog) {
+    while (lg < kMaxSegLog && ((uint64_t)nb << (lg + 1)) <= wavefronts) ++lg;
+    while (gl > 0 && (nb >> gl) < 8u * kXcds) --gl;
+    per_xcd = (nb + kXcds - 1) / kXcds;
+  }
+  BXG_HD bool whole() const { return lg == 0; }
+  // task j of an XCD; false past its last one.  A batch at or past nb: nothing to do.
+  BXG_HD bool task(uint32_t j, uint32_t xcd, uint32_t& batch, uint32_t& seg) const {
+    seg = 0;
+    if (whole()) {
+      batch = xcd * per_xcd + j;
+      return j < per_xcd;
+    }
+    if (gl == 0) {
+      const uint32_t t = j * kXcds + xcd;
+      batch = t >> lg;
+      seg = t & ((1u << lg) - 1u);
+      return batch < nb;
+    }
+    const uint32_t group = (j >> (gl + lg)) * kXcds + xcd;
+    batch = (group << gl) + (j & ((1u << gl) - 1u));
+    seg = (j >> gl) & ((1u << lg) - 1u);
+    return (group << gl) < nb;
+  }
+};
+
 }  // namespace bxg
