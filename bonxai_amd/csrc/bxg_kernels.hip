@@ -1770,6 +1770,12 @@ __device__ __forceinline__ uint32_t lds_claim(uint32_t* p, uint32_t key) {
 // missing roots are created (setCellOff leaves out inputs without one), and the
 // map's leaf count before the call is kept (k_op_buckets).  The tile's distinct
 // roots are found in LDS and looked up once.
+//
+// A tile in which one bucket has an eighth of the inputs or more leaves out
+// those of it that no result needs.  Else the one workgroup of that bucket reads
+// them all, one after the other: 2M inputs in one leaf 2.76 ms, now 0.096 (in one
+// cell 2.75, now 0.061); 2M, half of them in one leaf, 1.45, now 0.15; 50k in one
+// leaf 105 us, now 42.
 template <bool kCreate, int kPer>
 __global__ void __launch_bounds__(kOpTileThreads) k_op_tiles(const MapDev* __restrict__ mp,
                                                              const int32_t* __restrict__ coords, uint64_t n,
@@ -1778,9 +1784,13 @@ __global__ void __launch_bounds__(kOpTileThreads) k_op_tiles(const MapDev* __res
   constexpr uint32_t kTile = kOpTileThreads * kPer;
   constexpr uint32_t kRoots = kTile * 2 < 4096 ? kTile * 2 : 4096;
   constexpr uint32_t kStage = kTile * 8 > kRoots * 12 ? kTile * 8 : kRoots * 12;
+  constexpr uint32_t kCrowd = kTile / 8;  // inputs of a bucket that is looked at for inputs to leave out
+  constexpr uint32_t kDups = kStage >= 65536 ? 4096 : kStage >= 32768 ? 2048 : 1024;  // their table
+  static_assert(kDups * 16 <= kStage, "the table of cells");
   __shared__ __attribute__((aligned(16))) uint8_t stage[kStage];
   __shared__ uint32_t hist[kOpMaxBuckets / 2];  // 16 bits a bucket
   __shared__ uint32_t wsum[kOpTileThreads / 64];
+  __shared__ uint32_t crowded;
   uint64_t* rkeys = (uint64_t*)stage;
   int32_t* rslots = (int32_t*)(stage + kRoots * 8);
   const MapView m = uniform_view(mp);
@@ -1790,6 +1800,7 @@ __global__ void __launch_bounds__(kOpTileThreads) k_op_tiles(const MapDev* __res
   const uint32_t leaves = count ? min(*gp(&m.ctr->leaf_count), m.leaf_cap) : 0u;
   for (uint32_t p = t; p < kRoots; p += kOpTileThreads) rkeys[p] = kEmptyKey;
   for (uint32_t p = t; p < os.nb / 2; p += kOpTileThreads) hist[p] = 0;
+  if (t == 0) crowded = 0;
   int32_t x[kPer], y[kPer], z[kPer];
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
@@ -1861,12 +1872,59 @@ __global__ void __launch_bounds__(kOpTileThreads) k_op_tiles(const MapDev* __res
       const uint64_t cell = (child << cl) | leaf_index(x[j], y[j], z[j], m.lb);
       const uint32_t bk = (uint32_t)mix64(child) & (os.nb - 1);
       const uint32_t sh = (bk & 1u) * 16u;
-      const uint32_t r = atomicAdd(&hist[bk >> 1], 1u << sh) >> sh;
+      const uint32_t r = atomicAdd(&hist[bk >> 1], 1u << sh) >> sh & 0xFFFFu;
+      if (r + 1u == kCrowd) crowded = 1;
       ent[j] = (cell << kOpTileLog) | ((uint32_t)j * kOpTileThreads + t);
-      at[j] = (bk << 16) | (r & 0xFFFFu);
+      at[j] = (bk << 16) | r;
     }
   }
   __syncthreads();
+  if (crowded) {
+    // Only the first (was_on is asked for, or setCellOn / setCellOff) and the
+    // last input (setValue) of a cell have a part in the results.  Cells that
+    // find no room in the table keep all their inputs.
+    uint64_t* cells = (uint64_t*)stage;
+    uint32_t* first = (uint32_t*)(stage + kDups * 8);
+    uint32_t* last = first + kDups;
+    for (uint32_t p = t; p < kDups; p += kOpTileThreads) {
+      cells[p] = kEmptyKey;
+      first[p] = kNone;
+      last[p] = 0;
+    }
+    __syncthreads();
+    const bool need_last = op == kOpSetValue, need_first = !need_last || was_on != nullptr;
+    uint32_t dup[kPer];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      dup[j] = kOut;
+      if (at[j] == kOut) continue;
+      const uint32_t bk = at[j] >> 16;
+      if (((hist[bk >> 1] >> ((bk & 1u) * 16u)) & 0xFFFFu) < kCrowd) continue;
+      const uint64_t cell = ent[j] >> kOpTileLog;
+      uint32_t h = op_cell_slot(cell) & (kDups - 1u);
+      for (int p = 0; p < 16; ++p) {
+        if (lds_claim(&cells[h], cell) == cell) {
+          dup[j] = h;
+          atomicMin(&first[h], (uint32_t)j * kOpTileThreads + t);
+          atomicMax(&last[h], (uint32_t)j * kOpTileThreads + t);
+          break;
+        }
+        h = (h + 1u) & (kDups - 1u);
+      }
+    }
+    __syncthreads();
+    for (uint32_t p = t; p < os.nb / 2; p += kOpTileThreads) hist[p] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      if (at[j] == kOut) continue;
+      const uint32_t bk = at[j] >> 16, sh = (bk & 1u) * 16u, here = (uint32_t)j * kOpTileThreads + t;
+      at[j] = kOut;
+      if (dup[j] != kOut && !(need_last && last[dup[j]] == here) && !(need_first && first[dup[j]] == here)) continue;
+      at[j] = (bk << 16) | (atomicAdd(&hist[bk >> 1], 1u << sh) >> sh & 0xFFFFu);
+    }
+    __syncthreads();
+  }
   // first places of the buckets: two words (four buckets) a thread
   constexpr uint32_t kMost = kOpMaxBuckets / 2 / kOpTileThreads;
   const uint32_t nw = os.nb / 2;
@@ -2005,14 +2063,45 @@ __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buck
   const uint32_t cl = 3 * m.lb, il = 3 * m.ib;
   const uint32_t lwl = 31u - (uint32_t)__clz((int)m.lw);  // lw is a power of two
   const uint32_t most_gathered = min(kOpGathered, kOpLeaves >> lwl);
-  // lanes a tile, so that the workgroup reads all tiles' entries at once
+  // lanes a tile, so that the workgroup reads all tiles' entries at once (more
+  // than 64 in calls of few tiles: 2,000 inputs in one leaf 40 us with 64, now 28)
   uint32_t gl = 0;
-  while (gl < 6 && (os.tiles << gl) < kOpThreads) ++gl;
+  while (((uint64_t)os.tiles << gl) < kOpThreads) ++gl;
   constexpr uint32_t kMine = kOpCells / kOpThreads, kMyLeaves = kOpLeaves / kOpThreads;
   // what became of a leaf: its index (kNone: there is none), its number << 32,
   // kMade if the call has created it
   constexpr uint64_t kMade = 1ull << 63;
   constexpr uint32_t kSlotBit = 48;  // an entry is below 2^36
+  constexpr uint32_t kTogether = 4;
+  const auto table = [](const auto* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+  const auto cell_key = [&](uint64_t cell, uint32_t ls) -> uint32_t {
+    return (ls << 12) | ((uint32_t)cell & ((1u << cl) - 1u));
+  };
+  // a leaf's or cell's slot, from the first on that may hold it; false if none
+  // of kOpProbes does
+  const auto claim_leaf = [&](uint64_t child, uint32_t& ls) -> bool {
+    for (uint32_t p = 0; p < kOpProbes; ++p) {
+      uint64_t k = __hip_atomic_load(&leaf[ls], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (k == kEmptyKey) {
+        k = atomicCAS((unsigned long long*)&leaf[ls], kEmptyKey, child);
+        if (k == kEmptyKey) {
+          k = child;
+          const uint32_t number = atomicAdd(&nleaf, 1u);
+          if (kApply && number < kOpGathered) gathered[number] = child | ((uint64_t)ls << kSlotBit);
+        }
+      }
+      if (k == child) return true;
+      ls = (ls + 1u) & (kOpLeaves - 1u);
+    }
+    return false;
+  };
+  const auto claim_cell = [&](uint32_t key, uint32_t& h) -> bool {
+    for (uint32_t p = 0; p < kOpProbes; ++p) {
+      if (lds_claim(&ckey[h], key) == key) return true;
+      h = (h + 1u) & (kOpCells - 1u);
+    }
+    return false;
+  };
   OpPart part;
   for (;;) {
     const uint4 ones = make_uint4(~0u, ~0u, ~0u, ~0u);
@@ -2031,43 +2120,62 @@ __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buck
       const uint16_t BXG_G* st = gp((const uint16_t*)os.start) + (uint64_t)tile * (os.nb + 2) + bk;
       const uint32_t hi = st[1];
       const uint64_t tb = (uint64_t)tile * os.tile;
-      for (uint32_t k = st[0] + (t & ((1u << gl) - 1u)); k < hi; k += 1u << gl) {
-        const uint64_t e = gp((const uint64_t*)os.entry)[tb + k];
-        const uint64_t cell = e >> kOpTileLog;
-        const uint32_t i = (uint32_t)tb + ((uint32_t)e & ((1u << kOpTileLog) - 1u));
-        const uint64_t hash = mix64(cell), child = cell >> cl;
-        if (!whole && !part.holds(mix64(child), hash)) continue;
-        uint32_t ls = op_leaf_slot(child);
-        uint32_t p = 0;
-        for (; p < kOpProbes; ++p) {
-          uint64_t k = __hip_atomic_load(&leaf[ls], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-          if (k == kEmptyKey) {
-            k = atomicCAS((unsigned long long*)&leaf[ls], kEmptyKey, child);
-            if (k == kEmptyKey) {
-              k = child;
-              const uint32_t number = atomicAdd(&nleaf, 1u);
-              if (kApply && number < kOpGathered) gathered[number] = child | ((uint64_t)ls << kSlotBit);
+      const uint64_t BXG_G* entry = gp((const uint64_t*)os.entry) + tb;
+      const auto input = [&](uint64_t e) -> uint32_t { return (uint32_t)tb + ((uint32_t)e & ((1u << kOpTileLog) - 1u)); };
+      const bool crowd = whole && hi - st[0] >= (8u << gl);
+      for (uint32_t k = st[0] + (t & ((1u << gl) - 1u)); k < hi;) {
+        uint32_t n_here = 1, todo = 1;  // inputs k, k + (1 << gl), ...; bits of those not in the tables yet
+        if (crowd && k + ((kTogether - 1u) << gl) < hi) {
+          // of a leaf that takes a large part of the call's inputs, all of them
+          // this workgroup's, most are: kTogether at a time, so that as many
+          // chains of reads are under way
+          uint64_t e[kTogether];
+          bool known[kTogether];
+#pragma unroll
+          for (uint32_t j = 0; j < kTogether; ++j) e[j] = entry[k + (j << gl)];
+#pragma unroll
+          for (uint32_t j = 0; j < kTogether; ++j) {
+            const uint64_t child = e[j] >> (kOpTileLog + cl);
+            known[j] = table(&leaf[op_leaf_slot(child)]) == child;
+          }
+          if (kApply) {
+#pragma unroll
+            for (uint32_t j = 0; j < kTogether; ++j) {
+              const uint64_t cell = e[j] >> kOpTileLog;
+              known[j] &= table(&ckey[op_cell_slot(cell)]) == cell_key(cell, op_leaf_slot(cell >> cl));
             }
           }
-          if (k == child) break;
-          ls = (ls + 1u) & (kOpLeaves - 1u);
-        }
-        if (p == kOpProbes) {
-          leaves_full = 1;
-          continue;
-        }
-        if (!kApply) continue;
-        const uint32_t key = (ls << 12) | ((uint32_t)cell & ((1u << cl) - 1u));
-        uint32_t h = op_cell_slot(hash);
-        for (p = 0; p < kOpProbes; ++p) {
-          if (lds_claim(&ckey[h], key) == key) {
-            if (kLast) atomicMax(&clast[h], i);
-            if (kFirst) atomicMin(&cfirst[h], i);
-            break;
+          n_here = kTogether;
+          todo = 0;
+#pragma unroll
+          for (uint32_t j = 0; j < kTogether; ++j) {
+            if (!known[j]) {
+              todo |= 1u << j;
+            } else if (kApply) {
+              const uint32_t h = op_cell_slot(e[j] >> kOpTileLog);
+              if (kLast) atomicMax(&clast[h], input(e[j]));
+              if (kFirst) atomicMin(&cfirst[h], input(e[j]));
+            }
           }
-          h = (h + 1u) & (kOpCells - 1u);
         }
-        if (p == kOpProbes) cells_full = 1;
+        for (; todo; todo &= todo - 1u) {
+          const uint64_t e = entry[k + (((uint32_t)__ffs((int)todo) - 1u) << gl)], cell = e >> kOpTileLog, child = cell >> cl;
+          if (!whole && !part.holds(mix64(child), mix64(cell))) continue;
+          uint32_t ls = op_leaf_slot(child);
+          if (!claim_leaf(child, ls)) {
+            leaves_full = 1;
+            continue;
+          }
+          if (!kApply) continue;
+          uint32_t h = op_cell_slot(cell);
+          if (!claim_cell(cell_key(cell, ls), h)) {
+            cells_full = 1;
+            continue;
+          }
+          if (kLast) atomicMax(&clast[h], input(e));
+          if (kFirst) atomicMin(&cfirst[h], input(e));
+        }
+        k += n_here << gl;
       }
     }
     __syncthreads();

@@ -26,10 +26,13 @@ constexpr uint32_t kOpCells = 4096;
 constexpr uint32_t kOpLeaves = 2048;
 constexpr uint32_t kOpProbes = 64;
 
-// first slot of a cell (by its hash) and of a leaf (by its entry among the children)
-BXG_PARTS_HD uint32_t op_cell_slot(uint64_t hash) { return (uint32_t)hash & (kOpCells - 1u); }
+// first slot of a cell and of a leaf (its entry among the children); a bucket's
+// leaves are spread by the hash that put them there, so a multiplication does
+BXG_PARTS_HD uint32_t op_cell_slot(uint64_t cell) {
+  return (((uint32_t)cell + (uint32_t)(cell >> 32) * 0x85EBCA6Bu) * 0x9E3779B1u) >> 20;
+}
 BXG_PARTS_HD uint32_t op_leaf_slot(uint64_t child) { return ((uint32_t)child * 0x9E3779B1u) >> 21; }
-static_assert(kOpLeaves == 1u << (32 - 21), "leaf slots");
+static_assert(kOpCells == 1u << (32 - 20) && kOpLeaves == 1u << (32 - 21), "slots");
 
 // The part of a bucket that its workgroup holds in its tables: the whole, or
 // after a table was full one half after the other, each halved further where it

@@ -91,3 +91,38 @@ def test_values_at_odd_addresses(ctx, dtype, shift):
         assert_same_cells(g.export(), sorted_cells(*h.export()), host)
         g.close()
         h.close()
+
+
+@pytest.mark.parametrize("n,bits,dtype", [
+    (1000, (2, 3), np.float32), (1024, (2, 3), np.int64), (5000, (2, 3), np.float32), (60_000, (2, 3), np.int32),
+    (300_000, (2, 2), None), (300_000, (2, 4), np.float32), (600_000, (2, 3), np.uint8), (1_100_000, (2, 3), np.float32)])
+@pytest.mark.parametrize("kind", ["cell", "leaf", "half"])
+def test_crowded_leaves(ctx, n, bits, dtype, kind):
+    """A leaf or a cell with a large part of the inputs, whose tiles leave out
+    those that no result needs."""
+    import bonxai_amd as bx
+    import oracle
+    rng = np.random.default_rng(n)
+    side = 1 << bits[1]
+    c = np.zeros((n, 3), np.int64) if kind == "cell" else rng.integers(0, side, (n, 3))
+    if kind != "leaf":
+        c = np.where(rng.random((n, 1)) < 0.5, c, rng.integers(-100, 100, (n, 3)))
+    c = np.ascontiguousarray(c.astype(np.int32))
+    v = None if dtype is None else rng.integers(1, 200, n).astype(dtype)
+    g, og = bx.VoxelGrid(ctx, 0.1, *bits, dtype=dtype), oracle.Grid(0.1, *bits, dtype=dtype)
+    part, w = c[n // 5:], None if v is None else v[n // 5:]
+    for what, got, want in (
+            ("on", g.set_cells_on(part, w, True), og.set_cells_on(part, w)),
+            ("set", g.set_values(c, v, True), og.set_values(c, v)),
+            ("off", g.set_cells_off(part, True), og.set_cells_off(part))):
+        assert np.array_equal(got, want), what
+    back = None if v is None else np.ascontiguousarray(v[::-1])
+    g.set_values(c, back)
+    og.set_values(c, back)
+    if dtype is None:
+        assert np.array_equal(sorted_cells(g.export()[0])[0], og.export()[0])
+    else:
+        assert_same_cells(g.export(), og.export(), f"{kind} {n}")
+    assert g.active_cells_count() == og.active_cells_count()
+    g.close()
+    og.close()

@@ -80,7 +80,7 @@ int main() {
           if (!part.whole() && !part.holds(mix64(child), hash)) continue;
           if (!claim(tl, op_leaf_slot(child), child, kOpProbes))
             leaves_full = true;
-          else if (!claim(tc, op_cell_slot(hash), cell, kOpProbes))
+          else if (!claim(tc, op_cell_slot(cell), cell, kOpProbes))
             cells_full = true;
           mine.push_back(i);
         }
