@@ -1086,13 +1086,16 @@ int cell_op(bxg_map* m, const int32_t* coords, const void* vals, uint64_t n, uin
   // unless much is under way on the map (the leaf count it knows is that of the
   // last call that has landed); else k_op_leaves goes first, which looks again
   // on the device and only creates leaves where the room is short there too.
+  // Leaves of several units (op_unit_log) are shared by buckets, so k_op_leaves
+  // creates them in every call.
   const uint8_t* v = (const uint8_t*)vals;
-  if (create && m->known_leaves + m->under_way + n > m->leaf_cap)
+  const bool units = op_unit_log(m->h.leaf_bits) < 3 * m->h.leaf_bits;
+  if (create && (units || m->known_leaves + m->under_way + n > m->leaf_cap))
     BXG_TRY(launch(c, "k_op_leaves", k_op_buckets<true, false, false, false>, os.nb, kOpThreads, md, v, n, op, was_on, os));
-  auto buckets = !create              ? k_op_buckets<false, true, true, false>
-                 : op != kOpSetValue ? k_op_buckets<true, true, true, false>
-                 : was_on            ? k_op_buckets<true, true, true, true>
-                                     : k_op_buckets<true, true, false, true>;
+  const bool fused = create && !units;
+  auto buckets = op != kOpSetValue ? (fused ? k_op_buckets<true, true, true, false> : k_op_buckets<false, true, true, false>)
+                 : was_on          ? (fused ? k_op_buckets<true, true, true, true> : k_op_buckets<false, true, true, true>)
+                          : (fused ? k_op_buckets<true, true, false, true> : k_op_buckets<false, true, false, true>);
   BXG_TRY(launch(c, "k_op_buckets", buckets, os.nb, kOpThreads, md, v, n, op, was_on, os));
   return snapshot_counters(m, create ? n : 0);
 }

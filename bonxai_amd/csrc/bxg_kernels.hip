@@ -1714,11 +1714,12 @@ __global__ void k_na_recover(MapCounters* __restrict__ ctr, uint32_t leaf_cap) {
 
 // setValue / setCellOn / setCellOff for a batch, with the results of the calls
 // made one after the other (bonxai.hpp:449-466, 537-569).  Two kernels:
-// k_op_tiles orders each tile of inputs by the bucket (hash) of their leaf,
-// and k_op_buckets gives each bucket to one workgroup, which finds the first
-// and last input of every cell in LDS.  A leaf belongs to one workgroup, so
-// its cells, its entry and (of up to kOpGathered leaves a bucket) its mask words
-// need no device atomics, and the workgroup initialises the leaves it creates.
+// k_op_tiles orders each tile of inputs by the bucket (hash) of their leaf (of
+// 512 cells of it in leaves of 16^3, op_unit_log), and k_op_buckets gives each
+// bucket to one workgroup, which finds the first and last input of every cell in
+// LDS.  Such a unit belongs to one workgroup, so its cells and (of up to
+// kOpGathered units a bucket) its mask words need no device atomics, and the
+// workgroup initialises the leaves it creates.
 //
 // A table of the cells in device memory (claim, last index, mask bits: two to
 // three device atomics an input, about 15 G/s in all) took 0.46 ms for 2M
@@ -1734,12 +1735,11 @@ constexpr uint32_t kOpTileThreads = 1024;
 constexpr uint32_t kOpTileLog = 13;    // most inputs of a tile
 constexpr uint32_t kOpMaxBuckets = 4096;
 constexpr uint32_t kOpThreads = 512;   // of k_op_buckets (2M inputs: 256 threads 93 us, 512 66, 1024 102)
-// Most leaves of a bucket whose mask bits are gathered in LDS (fewer where a
-// leaf has more than 8 mask words): clusters of cells have some 54 a bucket.
-// With more, few cells share a word: 1M inputs, each in a leaf of its own, 977 a
-// bucket, are set in 122 us, call and wait included, with an atomic a cell, and
-// in 448 when buckets were done in parts of at most 256 leaves (200k inputs in
-// leaves of 16^3 cells, parts of 32: 368 -> 42).
+// Most units of a bucket whose mask bits are gathered in LDS: clusters of cells
+// have some 54 a bucket.  With more, few cells share a word: 1M inputs, each in a
+// leaf of its own, 977 a bucket, are set in 122 us, call and wait included, with
+// an atomic a cell, and in 448 when buckets were done in parts of at most 256
+// leaves.
 constexpr uint32_t kOpGathered = 256;
 
 enum : uint32_t { kOpSetValue = 0, kOpSetOn = 1, kOpSetOff = 2 };
@@ -1851,7 +1851,7 @@ __global__ void __launch_bounds__(kOpTileThreads) k_op_tiles(const MapDev* __res
     if (b && lane == 0) add32(&m.ctr->root_count, (uint32_t)__popcll(b));
   }
   __syncthreads();
-  const uint32_t cl = 3 * m.lb, il = 3 * m.ib;
+  const uint32_t cl = 3 * m.lb, il = 3 * m.ib, ul = op_unit_log(m.lb);
   uint64_t ent[kPer];
   uint32_t at[kPer];  // bucket << 16 | rank in the tile's part of it
 #pragma unroll
@@ -1870,7 +1870,7 @@ __global__ void __launch_bounds__(kOpTileThreads) k_op_tiles(const MapDev* __res
     if (slot >= 0) {
       const uint64_t child = ((uint64_t)slot << il) | inner_index(x[j], y[j], z[j], m.lb, m.ib);
       const uint64_t cell = (child << cl) | leaf_index(x[j], y[j], z[j], m.lb);
-      const uint32_t bk = (uint32_t)mix64(child) & (os.nb - 1);
+      const uint32_t bk = (uint32_t)mix64(cell >> ul) & (os.nb - 1);
       const uint32_t sh = (bk & 1u) * 16u;
       const uint32_t r = atomicAdd(&hist[bk >> 1], 1u << sh) >> sh & 0xFFFFu;
       if (r + 1u == kCrowd) crowded = 1;
@@ -2027,70 +2027,74 @@ __device__ __forceinline__ void set_cell(const MapView& m, uint64_t g, const uin
 // has written; setValue keeps the last input's value, setCellOn the first
 // one's, if the cell was off.
 //
-// A bucket with more cells or leaves than the tables hold is done in parts
-// (OpPart).  The table of the leaves has room for the inputs of a bucket that
-// lie each in a leaf of its own.  Up to kOpGathered leaves are numbered, have a
+// A bucket with more cells or units than the tables hold is done in parts
+// (OpPart).  The table of the units has room for the inputs of a bucket that
+// lie each in a leaf of its own.  Up to kOpGathered units are numbered, have a
 // thread each, and their cells' mask bits are gathered in LDS and written by
-// one thread a word; the bits of more leaves by an atomic a cell (they share
-// few words then).
+// one thread a word; the bits of more units by an atomic a cell (they share
+// few words then).  Leaves of several units are created without kApply only,
+// each by the workgroup that claims it.
 template <bool kCreate, bool kApply, bool kFirst, bool kLast>
 __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buckets(const MapDev* __restrict__ mp,
                                                            const uint8_t* __restrict__ vals, uint64_t n,
                                                            uint32_t op, uint8_t* __restrict__ was_on,
                                                            OpScratch os) {
   constexpr uint32_t kCells = kApply ? kOpCells : 4;
-  // cells: leaf slot << 12 | cell in the leaf
+  // cells: the unit's slot << kOpUnitLog | cell in the unit
   __shared__ __attribute__((aligned(16))) uint32_t ckey[kCells];
   __shared__ __attribute__((aligned(16))) uint32_t clast[kLast ? kOpCells : 4];
   __shared__ __attribute__((aligned(16))) uint32_t cfirst[kFirst ? kOpCells : 4];
-  // the leaves' entries among the children, then what became of them (below)
+  // the units (entry among the children, place in the leaf), then what became of them (below)
   __shared__ __attribute__((aligned(16))) uint64_t leaf[kOpLeaves];
-  // of the numbered leaves: entry and slot, then what became of them
+  // of the numbered units: unit and slot, then what became of them
   __shared__ uint64_t gathered[kApply ? kOpGathered : 1];
-  // the mask words of the numbered leaves, in place of inputs that are read by then
+  // the mask words of the numbered units, in place of inputs that are read by then
   uint64_t* bits = (uint64_t*)(kLast ? clast : cfirst);
-  static_assert(kOpCells * 4 == kOpLeaves * 8, "a mask word a slot of the leaves' table");
+  static_assert(kOpCells * 4 >= kOpGathered * 8 << (kOpUnitLog - 6u), "their mask words");
   __shared__ uint32_t leaves_full, cells_full, nleaf, nnew, nbase, fatal;
   const MapView m = uniform_view(mp);
   const uint32_t t = threadIdx.x, lane = t & 63u, wid = t >> 6;
-  if (kCreate && !kApply && (uint64_t)*gp(&m.ctr->leaf_base) + n <= m.leaf_cap) return;
+  const uint32_t il = 3 * m.ib, ul = op_unit_log(m.lb), sl = 3 * m.lb - ul;  // 2^sl units a leaf
+  if (kCreate && !kApply && sl == 0 && (uint64_t)*gp(&m.ctr->leaf_base) + n <= m.leaf_cap) return;
   // A failed call sets no cell.  The status is read once for the workgroup (and
   // looked at behind the first barriers): its wavefronts go through the same
   // ones whatever other workgroups flag.
   if (t == 0) fatal = map_status(m) & kFatal;
   // buckets that follow each other (their entries share lines) on one XCD
   const uint32_t bk = (blockIdx.x % kXcds) * (os.nb / kXcds) + blockIdx.x / kXcds;
-  const uint32_t cl = 3 * m.lb, il = 3 * m.ib;
-  const uint32_t lwl = 31u - (uint32_t)__clz((int)m.lw);  // lw is a power of two
-  const uint32_t most_gathered = min(kOpGathered, kOpLeaves >> lwl);
+  const uint32_t lwl = ul > 6u ? ul - 6u : 0u;  // log2 of a unit's mask words
   // lanes a tile, so that the workgroup reads all tiles' entries at once (more
   // than 64 in calls of few tiles: 2,000 inputs in one leaf 40 us with 64, now 28)
   uint32_t gl = 0;
   while (((uint64_t)os.tiles << gl) < kOpThreads) ++gl;
   constexpr uint32_t kMine = kOpCells / kOpThreads, kMyLeaves = kOpLeaves / kOpThreads;
-  // what became of a leaf: its index (kNone: there is none), its number << 32,
-  // kMade if the call has created it
+  // what became of a unit: its leaf's index (kNone: there is none), its number <<
+  // 32 (below kOpGathered), its place in the leaf << kPartBit, kMade if this
+  // kernel has created the leaf
   constexpr uint64_t kMade = 1ull << 63;
-  constexpr uint32_t kSlotBit = 48;  // an entry is below 2^36
+  constexpr uint32_t kPartBit = 40;
+  static_assert(kOpGathered <= 256, "a unit's number");
+  const auto part_of = [](uint64_t w) -> uint32_t { return (uint32_t)(w >> kPartBit) & 7u; };
+  constexpr uint32_t kSlotBit = 48;  // a unit is below 2^39
   constexpr uint32_t kTogether = 4;
   const auto table = [](const auto* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
   const auto cell_key = [&](uint64_t cell, uint32_t ls) -> uint32_t {
-    return (ls << 12) | ((uint32_t)cell & ((1u << cl) - 1u));
+    return (ls << kOpUnitLog) | ((uint32_t)cell & ((1u << ul) - 1u));
   };
   // a leaf's or cell's slot, from the first on that may hold it; false if none
   // of kOpProbes does
-  const auto claim_leaf = [&](uint64_t child, uint32_t& ls) -> bool {
+  const auto claim_leaf = [&](uint64_t unit, uint32_t& ls) -> bool {
     for (uint32_t p = 0; p < kOpProbes; ++p) {
       uint64_t k = __hip_atomic_load(&leaf[ls], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       if (k == kEmptyKey) {
-        k = atomicCAS((unsigned long long*)&leaf[ls], kEmptyKey, child);
+        k = atomicCAS((unsigned long long*)&leaf[ls], kEmptyKey, unit);
         if (k == kEmptyKey) {
-          k = child;
+          k = unit;
           const uint32_t number = atomicAdd(&nleaf, 1u);
-          if (kApply && number < kOpGathered) gathered[number] = child | ((uint64_t)ls << kSlotBit);
+          if (kApply && number < kOpGathered) gathered[number] = unit | ((uint64_t)ls << kSlotBit);
         }
       }
-      if (k == child) return true;
+      if (k == unit) return true;
       ls = (ls + 1u) & (kOpLeaves - 1u);
     }
     return false;
@@ -2135,14 +2139,14 @@ __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buck
           for (uint32_t j = 0; j < kTogether; ++j) e[j] = entry[k + (j << gl)];
 #pragma unroll
           for (uint32_t j = 0; j < kTogether; ++j) {
-            const uint64_t child = e[j] >> (kOpTileLog + cl);
-            known[j] = table(&leaf[op_leaf_slot(child)]) == child;
+            const uint64_t unit = e[j] >> (kOpTileLog + ul);
+            known[j] = table(&leaf[op_leaf_slot(unit)]) == unit;
           }
           if (kApply) {
 #pragma unroll
             for (uint32_t j = 0; j < kTogether; ++j) {
               const uint64_t cell = e[j] >> kOpTileLog;
-              known[j] &= table(&ckey[op_cell_slot(cell)]) == cell_key(cell, op_leaf_slot(cell >> cl));
+              known[j] &= table(&ckey[op_cell_slot(cell)]) == cell_key(cell, op_leaf_slot(cell >> ul));
             }
           }
           n_here = kTogether;
@@ -2159,10 +2163,10 @@ __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buck
           }
         }
         for (; todo; todo &= todo - 1u) {
-          const uint64_t e = entry[k + (((uint32_t)__ffs((int)todo) - 1u) << gl)], cell = e >> kOpTileLog, child = cell >> cl;
-          if (!whole && !part.holds(mix64(child), mix64(cell))) continue;
-          uint32_t ls = op_leaf_slot(child);
-          if (!claim_leaf(child, ls)) {
+          const uint64_t e = entry[k + (((uint32_t)__ffs((int)todo) - 1u) << gl)], cell = e >> kOpTileLog, unit = cell >> ul;
+          if (!whole && !part.holds(mix64(unit), mix64(cell))) continue;
+          uint32_t ls = op_leaf_slot(unit);
+          if (!claim_leaf(unit, ls)) {
             leaves_full = 1;
             continue;
           }
@@ -2214,9 +2218,9 @@ __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buck
     }
     // the leaves: looked up, and created where missing
     const uint32_t nl = nleaf;
-    const bool gather = kApply && nl <= most_gathered;
-    // entry of the thread's j-th leaf
-    const auto entry = [&](uint32_t j) -> uint64_t {
+    const bool gather = kApply && nl <= kOpGathered;
+    // the thread's j-th unit
+    const auto unit_of = [&](uint32_t j) -> uint64_t {
       if (!gather) return leaf[j * kOpThreads + t];
       return j == 0 && t < nl ? gathered[t] & ((1ull << kSlotBit) - 1ull) : kEmptyKey;
     };
@@ -2224,12 +2228,17 @@ __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buck
     uint32_t have = 0, make = 0, at = 0;  // its leaves and those missing (bits), the first new one's place
 #pragma unroll
     for (uint32_t j = 0; j < kMyLeaves; ++j) {
-      const uint64_t child = entry(j);
-      have |= child != kEmptyKey ? 1u << j : 0u;
-      idx[j] = child != kEmptyKey ? m.children[child] : 0u;
+      const uint64_t unit = unit_of(j);
+      have |= unit != kEmptyKey ? 1u << j : 0u;
+      idx[j] = unit != kEmptyKey ? m.children[unit >> sl] : 0u;
     }
 #pragma unroll
-    for (uint32_t j = 0; j < kMyLeaves; ++j) make |= idx[j] >= kPendingChild ? 1u << j : 0u;
+    for (uint32_t j = 0; j < kMyLeaves; ++j) {
+      if (idx[j] < kPendingChild) continue;
+      // a leaf of several units belongs to the workgroup that claims it
+      if (!kApply && sl && !leaf_claim((uint32_t*)&m.children[unit_of(j) >> sl], idx[j])) continue;
+      make |= 1u << j;
+    }
     if (kCreate) {
       if (make) at = atomicAdd(&nnew, (uint32_t)__popc(make));
       __syncthreads();
@@ -2242,20 +2251,21 @@ __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buck
 #pragma unroll
         for (uint32_t j = 0; j < kMyLeaves; ++j) {
           if (!((make >> j) & 1u)) continue;
+          const uint64_t child = unit_of(j) >> sl;
           idx[j] = next++;
           if (idx[j] >= m.leaf_cap) {
             or32(&m.ctr->status, kStOutOfPool);
             idx[j] = kNone;
+            st32((uint32_t*)&m.children[child], kEmptyChild);
             continue;
           }
-          const uint64_t child = entry(j);
           const uint32_t ci = (uint32_t)child & (m.isz - 1u), im = (1u << m.ib) - 1u;
           int32_t ox, oy, oz;
           unpack_root(m.root_keys[child >> il], m.log2n, &ox, &oy, &oz);
           m.origin[idx[j]] =
               make_int4(ox + (int32_t)((ci & im) << m.lb), oy + (int32_t)(((ci >> m.ib) & im) << m.lb),
                         oz + (int32_t)((ci >> (2 * m.ib)) << m.lb), (int32_t)(child >> il));
-          m.children[child] = idx[j];
+          st32((uint32_t*)&m.children[child], idx[j]);
         }
         const bool masks = !gather || failed;  // else written below
         const uint32_t cw = (uint32_t)((uint64_t)m.lsz * m.vb / 8);  // 8-byte words a leaf
@@ -2272,6 +2282,7 @@ __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buck
         if (!((have >> j) & 1u)) continue;
         uint64_t w = idx[j] < kPendingChild ? idx[j] : kNone;
         if (kCreate && ((make >> j) & 1u)) w |= kMade;
+        w |= (unit_of(j) & ((1ull << sl) - 1ull)) << kPartBit;
         if (gather) {
           leaf[gathered[t] >> kSlotBit] = w | ((uint64_t)t << 32);
           gathered[t] = w;
@@ -2282,11 +2293,12 @@ __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buck
       __syncthreads();
 #pragma unroll
       for (uint32_t j = 0; j < kMine; ++j) {
-        const uint32_t p = j * kOpThreads + t, key = ckey[p], li = key & 4095u;
+        const uint32_t p = j * kOpThreads + t, key = ckey[p], lu = key & ((1u << kOpUnitLog) - 1u);
         if (key == kNone) continue;
-        const uint64_t l = leaf[key >> 12];
+        const uint64_t l = leaf[key >> kOpUnitLog];
         const uint32_t at_leaf = (uint32_t)l;
         if (at_leaf == kNone) continue;
+        const uint32_t li = part_of(l) << ul | lu;
         const uint64_t g = (uint64_t)at_leaf * m.lsz + li;
         const uint64_t bit = 1ull << (li & 63u);
         uint64_t* mw = (uint64_t*)&m.masks[(uint64_t)at_leaf * m.lw + (li >> 6)];
@@ -2308,7 +2320,7 @@ __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buck
           set_cell(m, g, nullptr, 0);
         }
         if (gather) {
-          atomicOr((unsigned long long*)&bits[((uint32_t)(l >> 32 & 0xFFFFu) << lwl) + (li >> 6)], bit);
+          atomicOr((unsigned long long*)&bits[((uint32_t)(l >> 32 & 0xFFu) << lwl) + (lu >> 6)], bit);
         } else if (op == kOpSetOff) {
           if (pre) and64(mw, ~bit);
         } else if (!pre) {
@@ -2320,7 +2332,7 @@ __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buck
         for (uint32_t w = t; w < (nl << lwl); w += kOpThreads) {
           const uint64_t v = bits[w], l = gathered[w >> lwl];
           if ((uint32_t)l == kNone) continue;
-          uint64_t BXG_G* mw = m.masks + (uint64_t)(uint32_t)l * m.lw + (w & (m.lw - 1u));
+          uint64_t BXG_G* mw = m.masks + (uint64_t)(uint32_t)l * m.lw + (part_of(l) << lwl) + (w & ((1u << lwl) - 1u));
           if (kCreate && (l & kMade))
             *mw = v;  // every word of a new leaf
           else if (v)

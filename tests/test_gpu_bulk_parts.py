@@ -126,3 +126,28 @@ def test_crowded_leaves(ctx, n, bits, dtype, kind):
     assert g.active_cells_count() == og.active_cells_count()
     g.close()
     og.close()
+
+
+@pytest.mark.parametrize("n,span", [(1, 16), (4000, 16), (40_000, 32), (300_000, 48), (1_100_000, 40)])
+def test_dense_leaves_of_16(ctx, n, span):
+    """Leaves of 16^3 cells, of which a bucket has an eighth: created by one of
+    the workgroups that share them."""
+    import bonxai_amd as bx
+    import oracle
+    rng = np.random.default_rng(n)
+    c = rng.integers(-span, span, (n, 3)).astype(np.int32)
+    v = rng.integers(1, 1 << 30, n).astype(np.int32)
+    dc, dv, was = ctx.to_device(c), ctx.to_device(v), ctx.array(n, np.uint8)
+    for bits in ((1, 4), (4, 4)):
+        g, og = bx.VoxelGrid(ctx, 0.1, *bits, dtype=np.int32), oracle.Grid(0.1, *bits, dtype=np.int32)
+        for _ in range(2):
+            assert bx.lib().bxg_set_values(g._h, dc.ptr, dv.ptr, n, was.ptr) == bx.OK
+            assert g.sync() == bx.OK
+            assert np.array_equal(was.numpy(), og.set_values(c, v))
+            assert_same_cells(g.export(), og.export(), f"{n} {bits}")
+            off = c[: n // 2]
+            assert np.array_equal(g.set_cells_off(off, True), og.set_cells_off(off))
+        assert np.array_equal(g.set_cells_on(c, v, True), og.set_cells_on(c, v))
+        assert_same_cells(g.export(), og.export(), f"{n} {bits}")
+        g.close()
+        og.close()

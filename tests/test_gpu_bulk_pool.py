@@ -46,21 +46,21 @@ def test_more_inputs_than_the_pool_holds(ctx):
     g.close()
 
 
+@pytest.mark.parametrize("n,lb", [(100_000, 2), (20_000, 4)])
 @pytest.mark.parametrize("second", ["device", "set", "on"])
-def test_calls_enqueued_one_after_the_other(ctx, second):
+def test_calls_enqueued_one_after_the_other(ctx, second, n, lb):
     """The second call starts before the host has learnt how many leaves the
     first one created."""
     import bonxai_amd as bx
     import oracle
     rng = np.random.default_rng(3)
-    n = 100_000
     busy = bx.VoxelGrid(ctx, 0.1, dtype=np.float32)
     q = rng.integers(-200, 200, (4_000_000, 3)).astype(np.int32)
     busy.set_values(q[:100_000], np.ones(100_000, np.float32))
     dq, out = ctx.to_device(q), ctx.array(len(q), np.float32)
-    g, og = bx.VoxelGrid(ctx, 0.1, 2, 2, dtype=np.int32), oracle.Grid(0.1, 2, 2, dtype=np.int32)
-    a = _apart(n, 2, 4)
-    b = np.concatenate([_apart(n, 2, 5, 1 << 10), a[::7], _apart(n, 2, 5, 1 << 10)[::3]])  # new, set before, twice
+    g, og = bx.VoxelGrid(ctx, 0.1, 2, lb, dtype=np.int32), oracle.Grid(0.1, 2, lb, dtype=np.int32)
+    a = _apart(n, lb, 4)
+    b = np.concatenate([_apart(n, lb, 5, 1 << 11), a[::7], _apart(n, lb, 5, 1 << 11)[::3]])  # new, set before, twice
     va, vb = np.arange(1, n + 1, dtype=np.int32), -np.arange(1, len(b) + 1, dtype=np.int32)
     da, dva, db, dvb = (ctx.to_device(x) for x in (a, va, b, vb))
     was = ctx.array(len(b), np.uint8)

@@ -43,11 +43,10 @@ int main() {
     double most;  // passes a bucket on average (a pass for each part, and for each one that had to be halved)
   } cases[] = {
       {54, 18, 9, 1.0},    // clusters
-      {300, 4, 9, 1.0},   {1000, 1, 9, 1.5}, {98, 1, 12, 1.0}, {200, 5, 12, 1.0},
+      {300, 4, 9, 1.0},   {1000, 1, 9, 1.5}, {98, 1, 12, 1.0}, {200, 5, 12, 1.0}, {2, 512, 12, 1.0},
       {300, 18, 9, 4.0},   // 5,400 cells: two halves, most of which fit
       {300, 80, 9, 31.0},  // 24,000 cells: 8 to 16 parts
       {4900, 1, 9, 15.0},  // 4 to 8 parts
-      {5, 4096, 12, 31.0},
   };
   long checks = 0;
   for (const auto& k : cases) {
@@ -63,6 +62,8 @@ int main() {
         std::vector<uint32_t> in(1u << k.cell_bits);
         for (uint32_t i = 0; i < in.size(); ++i) in[i] = i;
         std::shuffle(in.begin(), in.end(), rng);
+        if (k.cell_bits > kOpUnitLog)  // one unit of the leaf
+          for (uint32_t& c : in) c = (c & ((1u << kOpUnitLog) - 1u)) | ((l & 7u) << kOpUnitLog);
         for (uint32_t c = 0; c < k.cells; ++c) cells.push_back((child << k.cell_bits) | in[c]);
       }
       std::sort(cells.begin(), cells.end());
@@ -76,9 +77,9 @@ int main() {
         std::vector<size_t> mine;
         bool leaves_full = false, cells_full = false;
         for (size_t i = 0; i < cells.size(); ++i) {
-          const uint64_t cell = cells[i], child = cell >> k.cell_bits, hash = mix64(cell);
-          if (!part.whole() && !part.holds(mix64(child), hash)) continue;
-          if (!claim(tl, op_leaf_slot(child), child, kOpProbes))
+          const uint64_t cell = cells[i], unit = cell >> op_unit_log(k.cell_bits / 3), hash = mix64(cell);
+          if (!part.whole() && !part.holds(mix64(unit), hash)) continue;
+          if (!claim(tl, op_leaf_slot(unit), unit, kOpProbes))
             leaves_full = true;
           else if (!claim(tc, op_cell_slot(cell), cell, kOpProbes))
             cells_full = true;
