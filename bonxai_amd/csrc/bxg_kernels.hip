@@ -1990,7 +1990,7 @@ __device__ __forceinline__ void copy_value(uint8_t BXG_G* dst, const uint8_t BXG
                                            const void* at, bool on = true) {
   const uint32_t odd = (uint32_t)(uintptr_t)at | vb;
   if ((odd & 15u) == 0)
-    copy_words<u32x4, 2>(dst, src, vb / 16, on);
+    copy_words<u32x4, 4>(dst, src, vb / 16, on);
   else if ((odd & 3u) == 0)
     copy_words<uint32_t, 4>(dst, src, vb / 4, on);
   else
@@ -2000,20 +2000,6 @@ __device__ __forceinline__ void copy_value(uint8_t BXG_G* dst, const uint8_t BXG
 // whether values of vb bytes at vals can be read as words
 __device__ __forceinline__ bool whole_words(const uint8_t* vals, uint32_t vb) {
   return (vb == 4 || vb == 8) && ((uintptr_t)vals & (vb - 1u)) == 0;
-}
-
-// cell g of the map becomes value i of vals (null: zero bytes; else at any
-// address)
-__device__ __forceinline__ void set_cell(const MapView& m, uint64_t g, const uint8_t* vals, uint64_t i) {
-  const uint32_t vb = m.vb;
-  const bool words = whole_words(vals, vb);
-  if (words && vb == 4) {
-    ((uint32_t BXG_G*)m.cells)[g] = vals ? gp((const uint32_t*)vals)[i] : 0u;
-  } else if (words) {
-    ((uint64_t BXG_G*)m.cells)[g] = vals ? gp((const uint64_t*)vals)[i] : 0ull;
-  } else {
-    copy_value(m.cells + g * vb, gp(vals) + i * vb, vb, vals, vals != nullptr);
-  }
 }
 
 // A bucket of a bulk call.  kCreate: its missing leaves are created, all cells
@@ -2197,18 +2183,19 @@ __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buck
     if (!kCreate && failed) return;
     // the values of the cells, in flight while the leaves are looked up (or the
     // inputs that hold them), and the words of `bits` cleared
-    const bool word = kLast && whole_words(vals, m.vb);
-    uint64_t val[kMine] = {};
+    const bool word = whole_words(vals, m.vb);
+    uint32_t* inputs = kLast ? clast : cfirst;
+    std::conditional_t<kLast, uint64_t, uint32_t> val[kMine] = {};
     if (kApply && !failed) {
       uint32_t src[kMine];  // (empty slots: input 0)
 #pragma unroll
-      for (uint32_t j = 0; j < kMine; ++j) src[j] = (kLast ? clast : cfirst)[j * kOpThreads + t];
+      for (uint32_t j = 0; j < kMine; ++j) src[j] = inputs[j * kOpThreads + t];
 #pragma unroll
-      for (uint32_t j = 0; j < kMine; ++j) (kLast ? clast : cfirst)[j * kOpThreads + t] = 0;
-      if (word && m.vb == 4) {
+      for (uint32_t j = 0; j < kMine; ++j) inputs[j * kOpThreads + t] = 0;
+      if (kLast && word && m.vb == 4) {
 #pragma unroll
         for (uint32_t j = 0; j < kMine; ++j) val[j] = gp((const uint32_t*)vals)[src[j]];
-      } else if (word) {
+      } else if (kLast && word) {
 #pragma unroll
         for (uint32_t j = 0; j < kMine; ++j) val[j] = gp((const uint64_t*)vals)[src[j]];
       } else {
@@ -2291,6 +2278,21 @@ __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buck
         }
       }
       __syncthreads();
+      // the prior mask bits, read together
+      uint32_t pres = 0;
+      if (kFirst) {
+        uint64_t masks[kMine];
+#pragma unroll
+        for (uint32_t j = 0; j < kMine; ++j) {
+          const uint32_t key = ckey[j * kOpThreads + t];
+          const uint64_t l = key != kNone ? leaf[key >> kOpUnitLog] : (uint64_t)kNone;
+          masks[j] = 0;
+          if ((uint32_t)l != kNone && !(kCreate && (l & kMade)))
+            masks[j] = m.masks[(uint64_t)(uint32_t)l * m.lw + (part_of(l) << lwl) + ((key & ((1u << kOpUnitLog) - 1u)) >> 6)];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kMine; ++j) pres |= (uint32_t)(masks[j] >> (ckey[j * kOpThreads + t] & 63u) & 1u) << j;
+      }
 #pragma unroll
       for (uint32_t j = 0; j < kMine; ++j) {
         const uint32_t p = j * kOpThreads + t, key = ckey[p], lu = key & ((1u << kOpUnitLog) - 1u);
@@ -2302,22 +2304,15 @@ __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buck
         const uint64_t g = (uint64_t)at_leaf * m.lsz + li;
         const uint64_t bit = 1ull << (li & 63u);
         uint64_t* mw = (uint64_t*)&m.masks[(uint64_t)at_leaf * m.lw + (li >> 6)];
-        bool pre = false;
-        if (kFirst) {
-          pre = !(l & kMade) && (*gp(mw) & bit) != 0;
-          if (was_on) was_on[kLast ? cfirst[p] : (uint32_t)val[j]] = pre;
-        }
-        if (word) {
+        const bool pre = kFirst && ((pres >> j) & 1u);
+        if (kFirst && was_on) was_on[kLast ? cfirst[p] : (uint32_t)val[j]] = pre;
+        if (word && (kLast || op == kOpSetOff || (vals && !pre))) {
+          uint64_t v = kLast ? (uint64_t)val[j] : 0ull;
+          if (!kLast && vals) v = m.vb == 4 ? gp((const uint32_t*)vals)[val[j]] : gp((const uint64_t*)vals)[val[j]];
           if (m.vb == 4)
-            ((uint32_t BXG_G*)m.cells)[g] = (uint32_t)val[j];
+            ((uint32_t BXG_G*)m.cells)[g] = (uint32_t)v;
           else
-            ((uint64_t BXG_G*)m.cells)[g] = val[j];
-        } else if (kLast) {
-          if (m.vb) set_cell(m, g, vals, val[j]);
-        } else if (op == kOpSetOn) {
-          if (!pre && m.vb && vals) set_cell(m, g, vals, val[j]);
-        } else {
-          set_cell(m, g, nullptr, 0);
+            ((uint64_t BXG_G*)m.cells)[g] = v;
         }
         if (gather) {
           atomicOr((unsigned long long*)&bits[((uint32_t)(l >> 32 & 0xFFu) << lwl) + (lu >> 6)], bit);
@@ -2337,6 +2332,21 @@ __global__ void __launch_bounds__(kOpThreads, kFirst && kLast ? 4 : 6) k_op_buck
             *mw = v;  // every word of a new leaf
           else if (v)
             *mw = op == kOpSetOff ? *mw & ~v : *mw | v;
+        }
+      }
+      // cells of other sizes, and values at any address (inputs: own slots again)
+      if (m.vb && !word && (op != kOpSetOn || vals)) {
+        __syncthreads();
+#pragma unroll
+        for (uint32_t j = 0; j < kMine; ++j)
+          inputs[j * kOpThreads + t] = op == kOpSetOn && ((pres >> j) & 1u) ? kNone : (uint32_t)val[j];
+#pragma unroll 1
+        for (uint32_t p = t; p < kOpCells; p += kOpThreads) {
+          const uint32_t key = ckey[p], src = inputs[p];
+          const uint64_t l = key != kNone && src != kNone ? leaf[key >> kOpUnitLog] : (uint64_t)kNone;
+          if ((uint32_t)l == kNone) continue;
+          const uint64_t g = (uint64_t)(uint32_t)l * m.lsz + (part_of(l) << ul | (key & ((1u << kOpUnitLog) - 1u)));
+          copy_value(m.cells + g * m.vb, gp(vals) + (uint64_t)src * m.vb, m.vb, vals, op != kOpSetOff);
         }
       }
     }
