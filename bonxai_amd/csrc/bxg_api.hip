@@ -1097,7 +1097,9 @@ int cell_op(bxg_map* m, const int32_t* coords, const void* vals, uint64_t n, uin
                  : was_on          ? (fused ? k_op_buckets<true, true, true, true> : k_op_buckets<false, true, true, true>)
                           : (fused ? k_op_buckets<true, true, false, true> : k_op_buckets<false, true, false, true>);
   BXG_TRY(launch(c, "k_op_buckets", buckets, os.nb, kOpThreads, md, v, n, op, was_on, os));
-  return snapshot_counters(m, create ? n : 0);
+  // setCellOff creates nothing: the counters stay as they are, and the copy
+  // (2 us) is left out
+  return create ? snapshot_counters(m, n) : BXG_OK;
 }
 
 int known_leaf_count(bxg_map* m, uint32_t* out) {
