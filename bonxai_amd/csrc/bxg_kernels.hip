@@ -2755,17 +2755,22 @@ __global__ void __launch_bounds__(256) k_compact_leaves(
 
 // clear(CLEAR_MEMORY): directory keys and entries to all ones (kEmptyKey,
 // kEmptyChild), have bits, bump counters and status to zero, the next life.  cap
-// is a power of two >= 1024, so both arrays are whole 16-byte words.  A workgroup
-// writes one part of each array: with all of them going through it side by side
-// a directory of 2^24 roots (4.4 GB) took 1.03 ms, now 0.80.  Bound: HBM.
+// is a power of two >= 1024, so both arrays are whole 16-byte words.  Bound: HBM.
+// In large directories a workgroup writes one part of each array: with all of
+// them going through it side by side 2^24 roots (4.4 GB) took 1.03 ms, now 0.80,
+// 2^20 46.4 us, now 44.7; 2^18 take 14.4 either way, 2^17 9.4 side by side, 10.0
+// in parts.
+constexpr uint64_t kClearParts = 1ull << 18;  // largest directory cleared side by side
 __global__ void __launch_bounds__(256) k_map_clear(uint64_t* __restrict__ keys, uint32_t* __restrict__ children,
                                                    uint64_t* __restrict__ have, uint64_t cap, uint32_t isz,
                                                    MapCounters* __restrict__ ctr, uint32_t life) {
   static_assert(kEmptyKey == ~0ull && kEmptyChild == ~0u, "all ones");
   const uint4 ones = make_uint4(~0u, ~0u, ~0u, ~0u);
-  const auto fill = [](auto* p, uint64_t n, auto v) {
-    const uint64_t part = (n + gridDim.x - 1) / gridDim.x, end = min(n, (blockIdx.x + 1) * part);
-    for (uint64_t i = blockIdx.x * part + threadIdx.x; i < end; i += blockDim.x) p[i] = v;
+  const bool parts = cap > kClearParts;
+  const auto fill = [parts](auto* p, uint64_t n, auto v) {
+    const uint64_t part = parts ? (n + gridDim.x - 1) / gridDim.x : blockDim.x;
+    const uint64_t end = parts ? min(n, (blockIdx.x + 1) * part) : n, step = parts ? blockDim.x : (uint64_t)gridDim.x * part;
+    for (uint64_t i = blockIdx.x * part + threadIdx.x; i < end; i += step) p[i] = v;
   };
   fill(reinterpret_cast<uint4*>(keys), cap / 2, ones);
   fill(reinterpret_cast<uint4*>(children), cap * isz / 4, ones);
