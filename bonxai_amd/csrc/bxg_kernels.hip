@@ -71,12 +71,6 @@ __device__ __forceinline__ uint64_t xor64(uint64_t* p, uint64_t v) {
 __device__ __forceinline__ uint32_t min32(uint32_t* p, uint32_t v) {
   return __hip_atomic_fetch_min(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ uint64_t ld64(const uint64_t* p) {
-  return __hip_atomic_load(gp(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ uint32_t max32(uint32_t* p, uint32_t v) {
-  return __hip_atomic_fetch_max(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 __device__ __forceinline__ uint64_t lanes_below() { return (1ull << lane_id()) - 1ull; }
@@ -493,10 +487,6 @@ __device__ __forceinline__ void leaves_step(const MapView& m, LeafWalk& lw, int3
   if (put) or64((uint64_t*)&m.want[e], put);
 }
 
-// One leaf of a ray, update pass: the cells of the ray in the current leaf
-// (up to kRun) are loaded together, then each takes the miss update unless
-// its update_id already equals cur.  Returns the cells written (counted
-// form: exact, by CAS).
 // leaf index of the walk's current cell (read-only phases)
 template <class Walk>
 __device__ __forceinline__ uint32_t walk_leaf(const MapView& m, const Walk& w, RootCache& rc) {
@@ -508,7 +498,12 @@ __device__ __forceinline__ uint32_t walk_leaf(const MapView& m, const Walk& w, R
   return c >= kPendingChild ? kNone : c;
 }
 
-// `leaf` is the leaf of the walk's current cell on entry; on return it is the
+// One leaf of a ray, update pass: the cells of the ray in the current leaf
+// (up to kRun) are loaded together, then each takes the miss update unless
+// its update_id already equals cur.  Returns the cells written (counted
+// form: exact, by CAS).
+//
+// next_leaf is the leaf of the walk's current cell on entry; on return it is the
 // leaf of the next run (looked up before this run's cells are loaded, so the
 // two memory round trips overlap).
 //
