@@ -75,7 +75,7 @@ typedef struct bxg_map_stats {
   uint64_t root_count;
   uint64_t root_capacity;
   uint64_t scans_applied;       /* insertPointCloud calls completed */
-  uint64_t device_bytes;        /* device memory held by the map */
+  uint64_t device_bytes;        /* device memory of the map's node pools */
   uint64_t last_rays;           /* counted runs only (bxg_set_counting) */
   uint64_t last_ray_updates;
   uint32_t update_count;        /* ProbabilisticMap::_update_count (1..3) */
@@ -105,7 +105,9 @@ typedef struct bxg_graph bxg_graph;
 /* ----------------------------------------------------------- context */
 
 /* One context per GPU: a stream, scratch buffers and a memory budget for
- * the node pools of its maps (0 = no limit). */
+ * the node pools of its maps (0 = no limit).  The scans' working memory is
+ * not counted: scratch, and two bits an inner cell of a probabilistic map's
+ * root directory (16 bytes a root slot with the default bits, 6 % of it). */
 int bxg_ctx_create(int device, uint64_t budget_bytes, bxg_ctx** out);
 int bxg_ctx_destroy(bxg_ctx* ctx);
 int bxg_ctx_sync(bxg_ctx* ctx);
