@@ -140,7 +140,9 @@ struct bxg_map {
   uint64_t known_roots = 0;
   uint64_t known_scans = 0;
   uint64_t max_leaf_growth = 0;  // largest leaf-count increase seen between snapshots
-  bool cleared = false;  // a clear may still run on the context's stream (other streams wait for it)
+  // a clear or setCellOff, which leave no event, may still run on the context's
+  // stream: other streams wait for the stream first
+  bool unmarked = false;
   int4* d_extra = nullptr;  // rays due from addHit/MissPoint
   uint32_t extra_cap = 0;
   std::vector<int4> extra;
@@ -1098,8 +1100,10 @@ int cell_op(bxg_map* m, const int32_t* coords, const void* vals, uint64_t n, uin
                           : (fused ? k_op_buckets<true, true, false, true> : k_op_buckets<false, true, false, true>);
   BXG_TRY(launch(c, "k_op_buckets", buckets, os.nb, kOpThreads, md, v, n, op, was_on, os));
   // setCellOff creates nothing: the counters stay as they are, and the copy
-  // (2 us) is left out
-  return create ? snapshot_counters(m, n) : BXG_OK;
+  // and its event (4 us) are left out
+  if (create) return snapshot_counters(m, n);
+  m->unmarked = true;
+  return BXG_OK;
 }
 
 int known_leaf_count(bxg_map* m, uint32_t* out) {
@@ -1644,7 +1648,7 @@ int bxg_map_clear(bxg_map* m, int option) {
   BXG_TRY(launch(c, "k_map_clear", k_map_clear, (uint32_t)std::min<uint64_t>(nblocks(n16), 4096), kBlock,
                  m->h.root_keys, m->h.children, m->h.leaf_have, (uint64_t)m->root_cap, m->h.inner_size,
                  m->ctr, life));
-  m->cleared = true;
+  m->unmarked = true;
   m->extra.clear();
   m->h_ctr->leaf_count = m->h_ctr->root_count = m->h_ctr->status = 0;
   m->h_ctr->life = life;

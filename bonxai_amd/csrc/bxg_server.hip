@@ -125,9 +125,9 @@ void srv_launch_read(bxg_server* s, SrvReq* r) {
     r->t_admit = now_ns();
     // inserts the map took outside the engine are confirmed first
     rc = settle(m);
-    if (rc == BXG_OK && m->cleared) {
+    if (rc == BXG_OK && m->unmarked) {
       rc = ctx_sync(c);
-      m->cleared = false;
+      m->unmarked = false;
     }
     if (rc != BXG_OK) {
       // reported below
